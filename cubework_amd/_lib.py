@@ -34,6 +34,7 @@ SIGNATURES = {
     "cw_gemm_ksteps": (_int, [_int, _i64, _i64, _i64, _int, _pp, _i64, _pp, _i64, _ptr, _int, _ptr, _i64, _ptr, _i64,
                               _pp, _int, _i64, _int, _ptr]),
     "cw_gemm_workspace_bytes": (_i64, [_int, _i64, _i64, _i64, _int, _int]),
+    "cw_gemm_scratch_bytes": (_i64, [_int, _i64, _i64, _i64, _int, _i64, _i64, _int, _int, _int, _int]),
     "cw_gemm_ksteps_ws": (_int, [_int, _i64, _i64, _i64, _int, _pp, _i64, _pp, _i64, _ptr, _int, _ptr, _i64, _ptr, _i64,
                                  _pp, _int, _i64, _ptr, _i64, _int, _ptr]),
     "cw_multi_norm_workspace_bytes": (_i64, [_int, _ptr]),

@@ -16,9 +16,12 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(HERE, "libcubework_hip.so")
 
-SOURCES = ["gemm_bf16_tn.hip", "gemm_f16_tn.hip", "gemm_bf16_nn.hip", "gemm_f16_nn.hip", "gemm_bf16_nt.hip", "gemm_f16_nt.hip",  # slowest first
-           "gemm_bf16_dma_nn.hip", "gemm_bf16_dma_nt.hip", "gemm_bf16_dma_tn.hip", "gemm_f16_dma_nn.hip", "gemm_f16_dma_nt.hip", "gemm_f16_dma_tn.hip",
-           "cw_runtime.hip", "cw_api.hip", "gemm_plan.hip", "gemm_bf16.hip", "gemm_half_small.hip", "gemm_f32.hip", "epilogue.hip", "layernorm.hip", "vpce.hip", "attention.hip", "attention_bwd.hip", "embedding.hip", "embed_sort.hip", "clip_grad.hip"]
+# gemm_tile.hip is compiled once per (element type, orientation, configuration)
+TILE_OBJECTS = ["gemm_tile.hip:%s:%s:%d" % (e, layout, cfg) for cfg in range(5) for layout in ("NN", "NT", "TN") for e in ("bf16_t", "f16_t")]
+SOURCES = TILE_OBJECTS + [  # slowest first
+    "gemm_bf16_tn.hip", "gemm_f16_tn.hip", "gemm_bf16_nn.hip", "gemm_f16_nn.hip", "gemm_bf16_nt.hip", "gemm_f16_nt.hip",
+    "cw_runtime.hip", "cw_api.hip", "gemm_plan.hip", "gemm_bf16.hip", "gemm_f32.hip", "epilogue.hip", "layernorm.hip", "vpce.hip",
+    "attention.hip", "attention_bwd.hip", "embedding.hip", "embed_sort.hip", "clip_grad.hip"]
 # the measurement library: its own kernels plus the runtime services (error text, device check), nothing else
 DIAG_SOURCES = ["diag_gemm.hip", "diag.hip"]
 DIAG_LIB_PATH = os.path.join(HERE, "libcubework_diag.so")
@@ -43,8 +46,10 @@ def _hipcc():
 
 
 def _compile(src, extra=(), obj_dir=None):
-    obj = os.path.join(obj_dir or OBJ_DIR, os.path.splitext(src)[0] + ".o")
-    cmd = [_hipcc(), *HIPCC_FLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
+    src, *variant = src.split(":")
+    obj = os.path.join(obj_dir or OBJ_DIR, "_".join([os.path.splitext(src)[0], *variant]) + ".o")
+    defines = ["-D%s=%s" % kv for kv in zip(("CW_TILE_E", "CW_TILE_LAYOUT", "CW_TILE_CFG"), variant)]
+    cmd = [_hipcc(), *HIPCC_FLAGS, *extra, *defines, "-c", os.path.join(CSRC, src), "-o", obj]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError("hipcc failed for %s:\n%s\n%s" % (src, proc.stdout, proc.stderr))

@@ -9,6 +9,14 @@ extern "C" int64_t cw_gemm_workspace_bytes(int layout, int64_t M, int64_t N, int
     return gemm_workspace_bytes(layout, M, N, K, n_steps, io_dtype);
 }
 
+extern "C" int64_t cw_gemm_scratch_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int64_t lda, int64_t ldb, int aligned_a,
+                                         int aligned_b, int unaligned_addends, int io_dtype) {
+    if ((layout != CW_NN && layout != CW_NT && layout != CW_TN) || (io_dtype != CW_BF16 && io_dtype != CW_F16)) return 0;
+    const TilePlan plan = tile_plan(layout, M, N, K, n_steps, lda, ldb, aligned_a != 0 && lda % 8 == 0, aligned_b != 0 && ldb % 8 == 0,
+                                    unaligned_addends < 0 || unaligned_addends > CW_MAX_ADDENDS ? 0 : unaligned_addends, -1);
+    return plan.cfg < 0 ? 0 : plan.scratch();
+}
+
 extern "C" int cw_gemm_ksteps(int layout, int64_t M, int64_t N, int64_t K, int n_steps, const void* const* A_steps,
                               int64_t lda, const void* const* B_steps, int64_t ldb, const void* bias, int epilogue,
                               void* C, int64_t ldc, void* preact, int64_t ldp, const void* const* addends,

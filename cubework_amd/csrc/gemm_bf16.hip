@@ -1,128 +1,130 @@
-// bf16 / fp16 block GEMM: choice of kernel and tile configuration (the same for both element types).
-//   - large tile-aligned problems (>= 128 tiles of 256x256, K a multiple of 64,
-//     16-byte aligned rows, at most 4 k-steps and 2 addends): the LDS-DMA
-//     kernel (gemm_bf16_dma.h);
-//   - the same kernel split along k when the output has too few 256x256 tiles
-//     to occupy the chip but the reduction is long (the weight-gradient shape
-//     X^T dY), given scratch for the fp32 partial sums: `slices` blocks per
-//     tile, then splitk_reduce_kernel adds them in slice order and applies the
-//     epilogue;
-//   - everything else: the register-staged kernel (gemm_bf16_kernel.h), with
-//     256x256 or 128x128 tiles, guarded when the shape is ragged or unaligned.
-// CW_GEMM_IMPL=staged in the environment forces the register-staged kernel.
+// bf16 / fp16 block GEMM: choice of kernel and launch (the same for both element types).
+//   - the tile kernels (gemm_tile.h) take every shape whose operand rows are 16-byte aligned, and the others after a copy to
+//     aligned rows, which the caller's scratch holds. tile_plan (gemm_plan.hip) chooses the tile size and which tiles are
+//     cut along k, by a cost model of the launch;
+//   - a call with less scratch than that (or none) is planned by gemm_half_plan;
+//   - the register-staged kernel (gemm_bf16_kernel.h) takes what is left: unaligned operands without scratch for the copy,
+//     and an activation on the weight-gradient orientation.
+// CW_GEMM_IMPL=staged in the environment forces the register-staged kernel, CW_GEMM_IMPL=onelaunch one launch per product.
 #include <cstdlib>
 #include <cstring>
 
 #include "gemm_bf16_kernel.h"
 #include "gemm_plan.h"
+#include "gemm_tile.h"
 
 namespace cw {
 
-int gemm_bf16_dma_launch_nn(const GemmArgs& args, int epilogue, hipStream_t s, const void* tail_a, const void* tail_b);
-int gemm_bf16_dma_launch_nt(const GemmArgs& args, int epilogue, hipStream_t s, const void* tail_a, const void* tail_b);
-int gemm_bf16_dma_launch_tn(const GemmArgs& args, int epilogue, hipStream_t s, const void* tail_a, const void* tail_b);
+#define CW_TILE_CFGS(e, l) {gemm_tile_##e##_##l##_0, gemm_tile_##e##_##l##_1, gemm_tile_##e##_##l##_2, gemm_tile_##e##_##l##_3, gemm_tile_##e##_##l##_4}
+#define CW_TILE_DECL(e, l)                                              \
+    int gemm_tile_##e##_##l##_0(const TileArgs&, int, hipStream_t);     \
+    int gemm_tile_##e##_##l##_1(const TileArgs&, int, hipStream_t);     \
+    int gemm_tile_##e##_##l##_2(const TileArgs&, int, hipStream_t);     \
+    int gemm_tile_##e##_##l##_3(const TileArgs&, int, hipStream_t);     \
+    int gemm_tile_##e##_##l##_4(const TileArgs&, int, hipStream_t);
+CW_TILE_DECL(bf16_t, NN)
+CW_TILE_DECL(bf16_t, NT)
+CW_TILE_DECL(bf16_t, TN)
+CW_TILE_DECL(f16_t, NN)
+CW_TILE_DECL(f16_t, NT)
+CW_TILE_DECL(f16_t, TN)
 
-int gemm_bf16_dma_split_launch_nn(const GemmArgs& args, int slices, hipStream_t s);
-int gemm_bf16_dma_split_launch_nt(const GemmArgs& args, int slices, hipStream_t s);
-int gemm_bf16_dma_split_launch_tn(const GemmArgs& args, int slices, hipStream_t s);
+using TileLaunch = int (*)(const TileArgs&, int, hipStream_t);
+static constexpr TileLaunch kTileLaunch[2][3][kTileConfigCount] = {
+    {CW_TILE_CFGS(bf16_t, NN), CW_TILE_CFGS(bf16_t, NT), CW_TILE_CFGS(bf16_t, TN)},
+    {CW_TILE_CFGS(f16_t, NN), CW_TILE_CFGS(f16_t, NT), CW_TILE_CFGS(f16_t, TN)},
+};
+static_assert(CW_NN == 0 && CW_NT == 1 && CW_TN == 2, "kTileLaunch is indexed by layout");
 
-int gemm_f16_dma_launch_nn(const GemmArgs& args, int epilogue, hipStream_t s, const void* tail_a, const void* tail_b);
-int gemm_f16_dma_launch_nt(const GemmArgs& args, int epilogue, hipStream_t s, const void* tail_a, const void* tail_b);
-int gemm_f16_dma_launch_tn(const GemmArgs& args, int epilogue, hipStream_t s, const void* tail_a, const void* tail_b);
-
-int gemm_f16_dma_split_launch_nn(const GemmArgs& args, int slices, hipStream_t s);
-int gemm_f16_dma_split_launch_nt(const GemmArgs& args, int slices, hipStream_t s);
-int gemm_f16_dma_split_launch_tn(const GemmArgs& args, int slices, hipStream_t s);
-
-int gemm_half_small_launch(const GemmArgs& args, int layout, int epilogue, bool f16, hipStream_t s);
-
-namespace {
-
-// C = epilogue(sum over slices of partial + addends + bias). One thread per 8
-// consecutive columns of a row; slices are added in index order.
-template <int EPI, typename E>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ partial, int slices, int64_t M,
-                                                            int64_t N, const E* __restrict__ bias,
-                                                            const E* __restrict__ add0, const E* __restrict__ add1,
-                                                            int64_t ldadd, E* __restrict__ C, int64_t ldc,
-                                                            E* __restrict__ preact, int64_t ldp) {
-    const int64_t vec_per_row = N / 8;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= M * vec_per_row) return;
-    const int64_t row = idx / vec_per_row, col = (idx - row * vec_per_row) * 8;
-    const float* p = partial + row * N + col;
-    float v[8];
+// rows x cols elements at `src` (any alignment, row pitch ld) to rows of `out` (pitch ldo, a multiple of 8): one thread per 16
+// bytes of output. Memory-bound: one read and one write of the operand (global accesses need no alignment).
+__global__ __launch_bounds__(256) void pack_rows_kernel(const uint16_t* __restrict__ src, int64_t ld, int64_t rows, int64_t cols,
+                                                        uint16_t* __restrict__ out, int64_t ldo) {
+    const int64_t per_row = ldo / 8, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= rows * per_row) return;
+    const int64_t r = idx / per_row, c = (idx - r * per_row) * 8;
+    const uint16_t* p = src + r * ld + c;
+    raw16_t v = {0u, 0u, 0u, 0u};
+    if (c + 8 <= cols) {
+        __builtin_memcpy(&v, p, 16);
+    } else {
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = 0.0f;
-    for (int z = 0; z < slices; ++z) {
-        float lo[4], hi[4];
-        unpack_raw(load_raw_stream(p + (int64_t)z * M * N), lo, (const float*)nullptr);
-        unpack_raw(load_raw_stream(p + (int64_t)z * M * N + 4), hi, (const float*)nullptr);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] += lo[e];
-            v[4 + e] += hi[e];
-        }
+        for (int e = 0; e < 7; ++e)
+            if (c + e < cols) w[e >> 1] |= (uint32_t)p[e] << ((e & 1) * 16);
+        v = raw16_t{w[0], w[1], w[2], w[3]};
     }
-    float t[8];
-    if (EPI != CW_EPI_NONE && bias != nullptr) {
-        unpack_raw(load_raw(bias + col), t, (const E*)nullptr);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += t[e];
-    }
-    if (add0 != nullptr) {
-        unpack_raw(load_raw_stream(add0 + row * ldadd + col), t, (const E*)nullptr);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += t[e];
-    }
-    if (add1 != nullptr) {
-        unpack_raw(load_raw_stream(add1 + row * ldadd + col), t, (const E*)nullptr);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += t[e];
-    }
-    if (preact != nullptr) store_raw_stream(preact + row * ldp + col, pack_raw(v, (const E*)nullptr));
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = gemm_bf16::epi_act<EPI>(v[e]);
-    store_raw_stream(C + row * ldc + col, pack_raw(v, (const E*)nullptr));
+    *reinterpret_cast<raw16_t*>(out + r * ldo + c) = v;
 }
 
-template <int EPI, typename E>
-int launch_splitk_reduce(const GemmArgs& a, int slices, hipStream_t s) {
-    const int64_t threads = (int64_t)a.M * (a.N / 8);
-    hipLaunchKernelGGL((splitk_reduce_kernel<EPI, E>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s,
-                       (const float*)a.workspace, slices, (int64_t)a.M, (int64_t)a.N, (const E*)a.bias,
-                       (const E*)(a.n_addends > 0 ? a.addend[0] : nullptr),
-                       (const E*)(a.n_addends > 1 ? a.addend[1] : nullptr), a.ldadd, (E*)a.C, a.ldc, (E*)a.preact, a.ldp);
-    return check_launch("splitk_reduce_kernel");
-}
-
-template <typename E>
-int splitk_reduce(const GemmArgs& a, int slices, int epilogue, hipStream_t s) {
-    switch (epilogue) {
-        case CW_EPI_NONE: return launch_splitk_reduce<CW_EPI_NONE, E>(a, slices, s);
-        case CW_EPI_BIAS: return launch_splitk_reduce<CW_EPI_BIAS, E>(a, slices, s);
-        case CW_EPI_BIAS_GELU_TANH: return launch_splitk_reduce<CW_EPI_BIAS_GELU_TANH, E>(a, slices, s);
-        case CW_EPI_BIAS_GELU_ERF: return launch_splitk_reduce<CW_EPI_BIAS_GELU_ERF, E>(a, slices, s);
-        case CW_EPI_BIAS_RELU: return launch_splitk_reduce<CW_EPI_BIAS_RELU, E>(a, slices, s);
-        default: return fail(CW_ERR_INVALID, "cw_gemm_ksteps: bad epilogue %d", epilogue);
+static int pack_rows(const void* const* src, int n, int64_t ld, int64_t rows, int64_t cols, char* out, int64_t ldo, const void** packed,
+                     hipStream_t s) {
+    const int64_t chunks = rows * (ldo / 8);
+    if (chunks > ((int64_t)1 << 38)) return fail(CW_ERR_UNSUPPORTED, "cw_gemm_ksteps: operand too large");
+    for (int i = 0; i < n; ++i) {
+        packed[i] = out + (int64_t)i * rows * ldo * 2;
+        hipLaunchKernelGGL(pack_rows_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, s, (const uint16_t*)src[i], ld, rows, cols,
+                           (uint16_t*)packed[i], ldo);
+        if (const int rc = check_launch("pack_rows_kernel"); rc != CW_OK) return rc;
     }
+    return CW_OK;
 }
 
-}  // namespace
+static TileArgs to_tile_args(const GemmArgs& g) {
+    TileArgs a;
+    memcpy(a.A, g.A, sizeof(a.A));
+    memcpy(a.B, g.B, sizeof(a.B));
+    memcpy(a.addend, g.addend, sizeof(a.addend));
+    a.bias = g.bias; a.C = g.C; a.preact = g.preact;
+    a.lda = g.lda; a.ldb = g.ldb; a.ldc = g.ldc; a.ldp = g.ldp; a.ldadd = g.ldadd;
+    a.M = g.M; a.N = g.N; a.K = g.K; a.n_steps = g.n_steps; a.n_addends = g.n_addends;
+    a.vec_out = g.vec_c && (g.preact == nullptr || g.vec_p);
+    a.full = 0;
+    a.slices = 1;
+    a.rotate = 0;
+    a.partial = nullptr;
+    return a;
+}
 
-// Rows K-32 .. K-1 of a [K, N] operand (row pitch ld) into `out` (same pitch), the first `zero_rows` of
-// them as zeros: the k-slow operand of the short extra step that finishes a reduction length K which is
-// not a multiple of 32. The step covers k in [K-32, K); the part that overlaps the regular steps
-// (zero_rows = 32 - K % 32 rows) must not count twice, and a zero row of this operand takes it out.
-__global__ __launch_bounds__(256) void ktail_rows_kernel(const uint16_t* __restrict__ src, int64_t ld, int64_t K, int N,
-                                                         int zero_rows, uint16_t* __restrict__ out) {
-    const int vec_per_row = N / 8;
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (idx >= 32 * vec_per_row) return;
-    const int r = idx / vec_per_row, c = (idx - r * vec_per_row) * 8;
-    raw16_t v = (raw16_t){0u, 0u, 0u, 0u};
-    if (r >= zero_rows) v = load_raw(src + (K - 32 + r) * ld + c);
-    *reinterpret_cast<raw16_t*>(out + (int64_t)r * ld + c) = v;
+static int tile_launch(const GemmArgs& g, const TilePlan& plan, int layout, int epilogue, bool f16, hipStream_t s) {
+    TileArgs a = to_tile_args(g);
+    char* ws = reinterpret_cast<char*>(g.workspace);
+    if (plan.pack_a) {
+        const bool tn = layout == CW_TN;
+        if (const int rc = pack_rows(g.A, g.n_steps, g.lda, tn ? g.K : g.M, tn ? g.M : g.K, ws, plan.lda, a.A, s); rc != CW_OK) return rc;
+    }
+    if (plan.pack_b) {
+        const bool nt = layout == CW_NT;
+        if (const int rc = pack_rows(g.B, g.n_steps, g.ldb, nt ? g.N : g.K, nt ? g.K : g.N, ws + plan.pack_a_bytes, plan.ldb, a.B, s); rc != CW_OK)
+            return rc;
+    }
+    if (plan.pack_add_bytes > 0) {
+        const int64_t ld = ((int64_t)g.N + 7) / 8 * 8;
+        if (const int rc = pack_rows(g.addend, g.n_addends, g.ldadd, g.M, g.N, ws + plan.pack_a_bytes + plan.pack_b_bytes, ld, a.addend, s); rc != CW_OK)
+            return rc;
+        a.ldadd = ld;
+    }
+    a.lda = plan.lda;
+    a.ldb = plan.ldb;
+    a.full = plan.full;
+    a.slices = plan.slices;
+    a.rotate = plan.rotate ? 1 : 0;
+    a.partial = reinterpret_cast<float*>(ws + plan.pack_a_bytes + plan.pack_b_bytes + plan.pack_add_bytes);
+    return kTileLaunch[f16 ? 1 : 0][layout][plan.cfg](a, epilogue, s);
+}
+
+// A plan of one configuration without scratch for operand copies (slices > 1: every tile sliced, partial sums in g.workspace).
+static TilePlan tile_plan_of(const GemmArgs& g, int cfg, int slices = 1) {
+    TilePlan p = {};
+    const int bm = 64 * kTileConfigs[cfg].tm, bn = 64 * kTileConfigs[cfg].tn;
+    p.cfg = cfg;
+    p.tiles = (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn);
+    p.full = slices > 1 ? 0 : (int)p.tiles;
+    p.slices = slices;
+    p.rotate = slices == 1 && cfg == 0 && g.M % 256 == 0 && g.N % 256 == 0;
+    p.lda = g.lda;
+    p.ldb = g.ldb;
+    return p;
 }
 
 static bool dma_kernel_enabled() {
@@ -142,61 +144,45 @@ static bool strip_split_enabled() {
     return enabled;
 }
 
-static int staged_launch(const GemmArgs& a, int layout, int epilogue, bool big, bool exact, bool f16, hipStream_t s) {
+static int staged_launch(const GemmArgs& a, int layout, int epilogue, bool big, bool f16, hipStream_t s) {
     switch (layout) {
-        case CW_NN: return f16 ? gemm_f16_launch_nn(a, epilogue, big, exact, s) : gemm_bf16_launch_nn(a, epilogue, big, exact, s);
-        case CW_NT: return f16 ? gemm_f16_launch_nt(a, epilogue, big, exact, s) : gemm_bf16_launch_nt(a, epilogue, big, exact, s);
-        case CW_TN: return f16 ? gemm_f16_launch_tn(a, epilogue, big, exact, s) : gemm_bf16_launch_tn(a, epilogue, big, exact, s);
-        default: return fail(CW_ERR_INVALID, "cw_gemm_ksteps: bad layout %d", layout);
-    }
-}
-
-static int dma_launch(const GemmArgs& a, int layout, int epilogue, bool f16, hipStream_t s, const void* tail_a = nullptr,
-                      const void* tail_b = nullptr) {
-    switch (layout) {
-        case CW_NN:
-            return f16 ? gemm_f16_dma_launch_nn(a, epilogue, s, tail_a, tail_b) : gemm_bf16_dma_launch_nn(a, epilogue, s, tail_a, tail_b);
-        case CW_NT:
-            return f16 ? gemm_f16_dma_launch_nt(a, epilogue, s, tail_a, tail_b) : gemm_bf16_dma_launch_nt(a, epilogue, s, tail_a, tail_b);
-        case CW_TN:
-            return f16 ? gemm_f16_dma_launch_tn(a, epilogue, s, tail_a, tail_b) : gemm_bf16_dma_launch_tn(a, epilogue, s, tail_a, tail_b);
+        case CW_NN: return f16 ? gemm_f16_launch_nn(a, epilogue, big, s) : gemm_bf16_launch_nn(a, epilogue, big, s);
+        case CW_NT: return f16 ? gemm_f16_launch_nt(a, epilogue, big, s) : gemm_bf16_launch_nt(a, epilogue, big, s);
+        case CW_TN: return f16 ? gemm_f16_launch_tn(a, epilogue, big, s) : gemm_bf16_launch_tn(a, epilogue, big, s);
         default: return fail(CW_ERR_INVALID, "cw_gemm_ksteps: bad layout %d", layout);
     }
 }
 
 // f16: the operands, bias, addends and outputs are IEEE half instead of bfloat16; everything else is shared.
-// The choice of kernel and the cuts are gemm_half_plan's (gemm_plan.hip); this function only launches.
 int gemm_half_launch(const GemmArgs& args, int layout, int epilogue, bool f16, hipStream_t s) {
-    const GemmPlan plan = gemm_half_plan(args, layout, dma_kernel_enabled(), strip_split_enabled());
-    switch (plan.route) {
-        case kRouteSmallRing: return gemm_half_small_launch(plan.head, layout, epilogue, f16, s);
-        case kRouteRing: return dma_launch(plan.head, layout, epilogue, f16, s);
-        case kRouteRingThenSmall: {
-            if (const int rc = dma_launch(plan.head, layout, epilogue, f16, s); rc != CW_OK) return rc;
-            return gemm_half_small_launch(plan.tail, layout, epilogue, f16, s);
-        }
-        case kRouteRingKTail: {
-            uint16_t* tail_b = reinterpret_cast<uint16_t*>(args.workspace);
-            const int vecs = 32 * (args.N / 8);
-            hipLaunchKernelGGL(ktail_rows_kernel, dim3((vecs + 255) / 256), dim3(256), 0, s,
-                               reinterpret_cast<const uint16_t*>(args.B[0]), args.ldb, (int64_t)args.K, args.N,
-                               plan.ktail_zero_rows, tail_b);
-            if (const int rc = check_launch("ktail_rows_kernel"); rc != CW_OK) return rc;
-            return dma_launch(plan.head, layout, epilogue, f16, s, plan.ktail_a, tail_b);
-        }
-        case kRouteSplitK: {
-            int rc;
-            switch (layout) {
-                case CW_NN: rc = f16 ? gemm_f16_dma_split_launch_nn(args, plan.slices, s) : gemm_bf16_dma_split_launch_nn(args, plan.slices, s); break;
-                case CW_NT: rc = f16 ? gemm_f16_dma_split_launch_nt(args, plan.slices, s) : gemm_bf16_dma_split_launch_nt(args, plan.slices, s); break;
-                case CW_TN: rc = f16 ? gemm_f16_dma_split_launch_tn(args, plan.slices, s) : gemm_bf16_dma_split_launch_tn(args, plan.slices, s); break;
-                default: return fail(CW_ERR_INVALID, "cw_gemm_ksteps: bad layout %d", layout);
-            }
-            if (rc != CW_OK) return rc;
-            return f16 ? splitk_reduce<f16_t>(args, plan.slices, epilogue, s) : splitk_reduce<bf16_t>(args, plan.slices, epilogue, s);
-        }
-        default: return staged_launch(args, layout, epilogue, plan.big, plan.exact, f16, s);
+    const bool tiles_ok = dma_kernel_enabled() && args.n_steps > 0 &&
+                          (layout != CW_TN || epilogue == CW_EPI_NONE || epilogue == CW_EPI_BIAS);
+    const bool one_launch = !strip_split_enabled();
+    const int pack_addends = args.vec_add ? 0 : args.n_addends;
+    if (tiles_ok) {
+        const int64_t scratch = aligned16(args.workspace) ? args.workspace_bytes : 0;
+        const TilePlan want = tile_plan(layout, args.M, args.N, args.K, args.n_steps, args.lda, args.ldb, args.vec_a != 0, args.vec_b != 0,
+                                        pack_addends, one_launch ? 0 : -1);
+        if (want.cfg >= 0 && want.scratch() <= scratch) return tile_launch(args, want, layout, epilogue, f16, s);
     }
+    const GemmPlan plan = gemm_half_plan(args, layout, tiles_ok, strip_split_enabled());
+    switch (plan.route) {
+        case kRouteSmallRing: return tile_launch(args, tile_plan_of(args, 2), layout, epilogue, f16, s);
+        case kRouteRing:
+        case kRouteRingKTail: return tile_launch(args, tile_plan_of(args, 0), layout, epilogue, f16, s);
+        case kRouteRingThenSmall: {
+            if (const int rc = tile_launch(plan.head, tile_plan_of(plan.head, 0), layout, epilogue, f16, s); rc != CW_OK) return rc;
+            return tile_launch(plan.tail, tile_plan_of(plan.tail, 2), layout, epilogue, f16, s);
+        }
+        case kRouteSplitK: return tile_launch(args, tile_plan_of(args, 0, plan.slices), layout, epilogue, f16, s);
+        default: break;
+    }
+    if (tiles_ok) {
+        const TilePlan fits = tile_plan(layout, args.M, args.N, args.K, args.n_steps, args.lda, args.ldb, args.vec_a != 0, args.vec_b != 0,
+                                        pack_addends, aligned16(args.workspace) ? args.workspace_bytes : 0);
+        if (fits.cfg >= 0) return tile_launch(args, fits, layout, epilogue, f16, s);
+    }
+    return staged_launch(args, layout, epilogue, plan.big, f16, s);
 }
 
 }  // namespace cw

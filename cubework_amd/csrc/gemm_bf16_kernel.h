@@ -1,5 +1,6 @@
-// SUMMA block GEMM for gfx950: C = act(sum_i op(A_i) op(B_i) + addends + bias),
-// 16-bit operands (bf16, or fp16 with E = f16_t: the same kernels, another MFMA opcode and conversion),
+// Register-staged block GEMM for gfx950, guarded: C = act(sum_i op(A_i) op(B_i) + addends + bias) for what the tile
+// kernels (gemm_tile.h) do not take - operands with unaligned rows and no scratch for a copy of them - and the pieces
+// that both share. 16-bit operands (bf16, or fp16 with E = f16_t: the same kernels, another MFMA opcode and conversion),
 // fp32 accumulation in v_mfma_f32_32x32x16_bf16 / _f16.
 //
 // Shape of the kernel
@@ -99,7 +100,7 @@ __device__ __forceinline__ u32x4_t load8_guarded(const uint16_t* __restrict__ ba
 //     tile is (row c/8, k-chunk c%8); thread handles chunks tid, tid+256, ...
 //   TRANS == true : memory is [k][rows] (rows contiguous). Thread owns the 8x8
 //     block (k-block tid%8, row-block tid/8) and loads its 8 k-rows.
-template <int ROWS, bool TRANS, bool GUARD>
+template <int ROWS, bool TRANS>
 __device__ __forceinline__ void tile_g2r(u32x4_t (&reg)[8], const uint16_t* __restrict__ base, int64_t ld, int row0,
                                          int k0, int rmax, int kmax, int tid, bool vec_ok) {
     if constexpr (!TRANS) {
@@ -109,10 +110,7 @@ __device__ __forceinline__ void tile_g2r(u32x4_t (&reg)[8], const uint16_t* __re
             const int c = it * kThreads + tid;
             const int row = row0 + (c >> 3);
             const int k = k0 + (c & 7) * 8;
-            if constexpr (GUARD)
-                reg[it] = load8_guarded(base, ld, row, k, rmax, kmax, vec_ok);
-            else
-                reg[it] = *reinterpret_cast<const u32x4_t*>(base + (int64_t)row * ld + k);
+            reg[it] = load8_guarded(base, ld, row, k, rmax, kmax, vec_ok);
         }
     } else {
         const int kb = tid & 7;
@@ -122,36 +120,8 @@ __device__ __forceinline__ void tile_g2r(u32x4_t (&reg)[8], const uint16_t* __re
             for (int j = 0; j < 8; ++j) {
                 const int k = k0 + kb * 8 + j;
                 const int row = row0 + rb * 8;
-                if constexpr (GUARD)
-                    reg[j] = load8_guarded(base, ld, k, row, kmax, rmax, vec_ok);
-                else
-                    reg[j] = *reinterpret_cast<const u32x4_t*>(base + (int64_t)k * ld + row);
+                reg[j] = load8_guarded(base, ld, k, row, kmax, rmax, vec_ok);
             }
-        }
-    }
-}
-
-// Fast-path variant of tile_g2r for in-bounds, 16-byte aligned tiles: the
-// address is (uniform base of the tile row block) + (one 32-bit per-thread byte
-// offset `voff`, invariant over the k loop), so the loads use the scalar-base
-// addressing form and need no per-load address registers.
-//   TRANS == false: voff = ((row0 + tid/8) * ld + (tid%8)*8) * 2
-//   TRANS == true : voff = (((tid%8)*8) * ld + row0 + (tid/8)*8) * 2
-template <int ROWS, bool TRANS>
-__device__ __forceinline__ void tile_g2r_fast(u32x4_t (&reg)[8], const char* __restrict__ base, uint32_t voff,
-                                              int64_t ld_bytes, int k0, int tid) {
-    if constexpr (!TRANS) {
-        constexpr int CH = ROWS * 8 / kThreads;
-        static_for<CH>([&](auto it) {
-            const char* p = base + ((int64_t)it.value * 32 * ld_bytes + (int64_t)k0 * 2);
-            reg[it.value] = *reinterpret_cast<const u32x4_t*>(p + voff);
-        });
-    } else {
-        if ((tid >> 3) < ROWS / 8) {
-            static_for<8>([&](auto j) {
-                const char* p = base + (int64_t)(k0 + j.value) * ld_bytes;
-                reg[j.value] = *reinterpret_cast<const u32x4_t*>(p + voff);
-            });
         }
     }
 }
@@ -221,23 +191,12 @@ constexpr int c_pitch() { return BN + 8; }
 
 // Write the staged tile out row by row: 16 bytes per lane, a wavefront covers
 // whole 512-byte rows (BN = 256), so global stores are full cache lines.
-template <int BM, int BN, bool FAST>
+template <int BM, int BN>
 __device__ __forceinline__ void tile_store(const uint16_t* __restrict__ lds_c, uint16_t* __restrict__ C, int64_t ldc,
                                            int m0, int n0, int M, int N, int tid) {
     constexpr int CP = c_pitch<BN>();
     constexpr int CHUNKS_PER_ROW = BN / 8;
     constexpr int TOTAL = BM * CHUNKS_PER_ROW;
-    if constexpr (FAST) {
-        // whole tile in bounds, rows 16-byte aligned: thread -> (row q/32.., chunk q%32), no checks
-        uint16_t* base = C + (int64_t)(m0 + tid / CHUNKS_PER_ROW) * ldc + n0 + (tid % CHUNKS_PER_ROW) * 8;
-        const uint16_t* src = lds_c + (tid / CHUNKS_PER_ROW) * CP + (tid % CHUNKS_PER_ROW) * 8;
-        constexpr int ROWS_PER_PASS = kThreads / CHUNKS_PER_ROW;
-#pragma unroll 8
-        for (int pass = 0; pass < BM / ROWS_PER_PASS; ++pass)
-            *reinterpret_cast<u32x4_t*>(base + (int64_t)pass * ROWS_PER_PASS * ldc) =
-                *reinterpret_cast<const u32x4_t*>(src + pass * ROWS_PER_PASS * CP);
-        return;
-    }
     const bool vec16 = ((reinterpret_cast<uintptr_t>(C) & 15u) == 0) && ((ldc & 7) == 0);
 #pragma unroll 4
     for (int q = tid; q < TOTAL; q += kThreads) {
@@ -267,9 +226,7 @@ __device__ __forceinline__ void tile_store(const uint16_t* __restrict__ lds_c, u
 // 32x32 MFMA tile at a time), never written back.
 // acc[i][j][v]: row  m = m0 + wm*(BM/2) + i*32 + (lane & 31)
 //               col  n = n0 + wn*(BN/2) + j*32 + 8*(v/4) + 4*(lane>>5) + (v%4)
-// FAST: the tile is entirely in bounds and every pointer / leading dimension
-// allows the vector accesses (checked on the host): no per-element guards.
-template <int BM, int BN, int TM, int TN, int EPI, bool FAST, typename E, typename Args>
+template <int BM, int BN, int TM, int TN, int EPI, typename E, typename Args>
 __device__ __forceinline__ void gemm_epilogue(f32x16_t (&acc)[TM][TN], const Args& args, uint16_t* lds, int m0,
                                               int n0, int wm, int wn, int lane, int tid) {
     constexpr int WTM = BM / 2, WTN = BN / 2;
@@ -289,8 +246,8 @@ __device__ __forceinline__ void gemm_epilogue(f32x16_t (&acc)[TM][TN], const Arg
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int ncol = n0 + col_l + j * 32 + 8 * g;
-                if (use_bias && (FAST || ncol < N)) {
-                    load4_half<E>(bias + ncol, FAST ? 4 : N - ncol, FAST || args.vec_bias != 0, bv[g]);
+                if (use_bias && ncol < N) {
+                    load4_half<E>(bias + ncol, N - ncol, args.vec_bias != 0, bv[g]);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) bv[g][e] = 0.0f;
@@ -305,12 +262,12 @@ __device__ __forceinline__ void gemm_epilogue(f32x16_t (&acc)[TM][TN], const Arg
                     float v[4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * g + e] + bv[g][e];
-                    if (args.n_addends > 0 && (FAST || (mrow < M && ncol < N))) {
+                    if (args.n_addends > 0 && mrow < M && ncol < N) {
 #pragma unroll 1
                         for (int a = 0; a < args.n_addends; ++a) {
                             float t[4];
                             load4_half<E>(reinterpret_cast<const uint16_t*>(pick_ptr(args.addend, a)) + (int64_t)mrow * args.ldadd + ncol,
-                                          FAST ? 4 : N - ncol, FAST || args.vec_add != 0, t);
+                                          N - ncol, args.vec_add != 0, t);
 #pragma unroll
                             for (int e = 0; e < 4; ++e) v[e] += t[e];
                         }
@@ -331,109 +288,15 @@ __device__ __forceinline__ void gemm_epilogue(f32x16_t (&acc)[TM][TN], const Arg
     if (args.preact != nullptr) {
         stage_tile(std::false_type{});
         __syncthreads();
-        tile_store<BM, BN, FAST>(lds_c, reinterpret_cast<uint16_t*>(args.preact), args.ldp, m0, n0, M, N, tid);
+        tile_store<BM, BN>(lds_c, reinterpret_cast<uint16_t*>(args.preact), args.ldp, m0, n0, M, N, tid);
         __syncthreads();
     }
     stage_tile(std::true_type{});
     __syncthreads();
-    tile_store<BM, BN, FAST>(lds_c, reinterpret_cast<uint16_t*>(args.C), args.ldc, m0, n0, M, N, tid);
+    tile_store<BM, BN>(lds_c, reinterpret_cast<uint16_t*>(args.C), args.ldc, m0, n0, M, N, tid);
 }
 
-// Epilogue of the 256x256 LDS-DMA kernel (whole tile in bounds, aligned): the
-// tile goes out in four slabs of 2 x 32 rows (accumulator row index i of both
-// wavefront rows), staged through two alternating LDS buffers. The global
-// stores of slab i drain while slab i+1 is computed, and one barrier per slab
-// is enough: a buffer is rewritten two slabs after it was read.
-// bias_raw[j][g]: the lane's 4 bias values (bf16 pairs) for accumulator
-// columns j*32 + 8g .. +3, loaded by the caller ahead of the k loop.
-template <int EPI, typename E, typename Args>
-__device__ __forceinline__ void gemm_epilogue_slabs(f32x16_t (&acc)[4][4], const Args& args,
-                                                    const u32x2_t (&bias_raw)[4][4], uint16_t* lds, int m0, int n0,
-                                                    int wm, int wn, int lane, int tid) {
-    constexpr int CP = c_pitch<256>();
-    constexpr int BUF = 64 * CP;  // elements per staging buffer
-    const int lrow = wm * 32 + (lane & 31);
-    const int col_l = wn * 128 + 4 * (lane >> 5);
-    int buf = 0;
-
-    auto stage = [&](auto slab, auto activated) {
-        constexpr int I = decltype(slab)::value;
-        constexpr bool ACT = decltype(activated)::value;
-        const int mrow = m0 + wm * 128 + I * 32 + (lane & 31);
-        uint16_t* dst = lds + buf * BUF + lrow * CP + col_l;
-        // the first addend's 16 pieces of this slab are requested together, ahead of the arithmetic (a load in
-        // front of each use would expose its latency sixteen times); further addends, rare, are read where used
-        u32x2_t add0[4][4];
-        if (args.n_addends > 0) {
-            const uint16_t* ap = reinterpret_cast<const uint16_t*>(pick_ptr(args.addend, 0)) + (int64_t)mrow * args.ldadd + n0 + col_l;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) add0[j][g] = *reinterpret_cast<const u32x2_t*>(ap + j * 32 + 8 * g);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x2_t b = bias_raw[j][g];
-                float v[4];
-                v[0] = acc[I][j][4 * g] + half_conv<E>::lo(b.x);
-                v[1] = acc[I][j][4 * g + 1] + half_conv<E>::hi(b.x);
-                v[2] = acc[I][j][4 * g + 2] + half_conv<E>::lo(b.y);
-                v[3] = acc[I][j][4 * g + 3] + half_conv<E>::hi(b.y);
-                if (args.n_addends > 0) {
-                    const int ncol = n0 + col_l + j * 32 + 8 * g;
-                    v[0] += half_conv<E>::lo(add0[j][g].x);
-                    v[1] += half_conv<E>::hi(add0[j][g].x);
-                    v[2] += half_conv<E>::lo(add0[j][g].y);
-                    v[3] += half_conv<E>::hi(add0[j][g].y);
-#pragma unroll 1
-                    for (int a = 1; a < args.n_addends; ++a) {
-                        float t[4];
-                        load4_half<E>(reinterpret_cast<const uint16_t*>(pick_ptr(args.addend, a)) + (int64_t)mrow * args.ldadd + ncol,
-                                      4, true, t);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] += t[e];
-                    }
-                }
-                if constexpr (ACT) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = epi_act<EPI>(v[e]);
-                }
-                u32x2_t p;
-                p.x = half_conv<E>::pack2(v[0], v[1]);
-                p.y = half_conv<E>::pack2(v[2], v[3]);
-                *reinterpret_cast<u32x2_t*>(dst + j * 32 + 8 * g) = p;
-            }
-        }
-    };
-    // 64 staged rows x 32 chunks of 16 bytes: 8 per thread, whole 512-byte rows per wavefront pass
-    auto store = [&](int slab, uint16_t* out, int64_t ld) {
-        const int r = tid >> 5, cq = tid & 31;
-        const uint16_t* src = lds + buf * BUF + r * CP + cq * 8;
-#pragma unroll
-        for (int pass = 0; pass < 8; ++pass) {
-            const int lr = r + 8 * pass;
-            const int grow = m0 + (lr >= 32 ? 128 : 0) + slab * 32 + (lr & 31);
-            *reinterpret_cast<u32x4_t*>(out + (int64_t)grow * ld + n0 + cq * 8) =
-                *reinterpret_cast<const u32x4_t*>(src + pass * 8 * CP);
-        }
-    };
-    static_for<4>([&](auto slab) {
-        if (args.preact != nullptr) {
-            stage(slab, std::false_type{});
-            __syncthreads();
-            store(decltype(slab)::value, reinterpret_cast<uint16_t*>(args.preact), args.ldp);
-            buf ^= 1;
-        }
-        stage(slab, std::true_type{});
-        __syncthreads();
-        store(decltype(slab)::value, reinterpret_cast<uint16_t*>(args.C), args.ldc);
-        buf ^= 1;
-    });
-}
-
-template <int BM, int BN, bool TRANS_A, bool TRANS_B, bool GUARD, int EPI, typename E>
+template <int BM, int BN, bool TRANS_A, bool TRANS_B, int EPI, typename E>
 __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const GemmArgs args) {
     constexpr int WTM = BM / 2, WTN = BN / 2;  // wavefront sub-tile
     constexpr int TM = WTM / 32, TN = WTN / 32;
@@ -485,26 +348,13 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const GemmArgs args
     const int a_frag = (wm * WTM + (lane & 31)) * kPitch + (lane >> 5) * 8;
     const int b_frag = A_ELEMS + (wn * WTN + (lane & 31)) * kPitch + (lane >> 5) * 8;
 
-    // fast path: per-thread byte offsets that do not change over the k loop
-    const uint32_t a_voff =
-        TRANS_A ? (uint32_t)((((tid & 7) * 8) * args.lda + m0 + (tid >> 3) * 8) * 2)
-                : (uint32_t)(((m0 + (tid >> 3)) * args.lda + (tid & 7) * 8) * 2);
-    const uint32_t b_voff =
-        TRANS_B ? (uint32_t)((((tid & 7) * 8) * args.ldb + n0 + (tid >> 3) * 8) * 2)
-                : (uint32_t)(((n0 + (tid >> 3)) * args.ldb + (tid & 7) * 8) * 2);
-
     auto issue_loads = [&](int kt) {
         const int step = kt / kt_per_step;
         const int k0 = (kt - step * kt_per_step) * kBK;
-        if constexpr (GUARD) {
-            const uint16_t* Ap = reinterpret_cast<const uint16_t*>(args.A[step]);
-            const uint16_t* Bp = reinterpret_cast<const uint16_t*>(args.B[step]);
-            tile_g2r<BM, TRANS_A, true>(ra, Ap, args.lda, m0, k0, M, K, tid, vec_a);
-            tile_g2r<BN, TRANS_B, true>(rb, Bp, args.ldb, n0, k0, N, K, tid, vec_b);
-        } else {
-            tile_g2r_fast<BM, TRANS_A>(ra, reinterpret_cast<const char*>(args.A[step]), a_voff, args.lda * 2, k0, tid);
-            tile_g2r_fast<BN, TRANS_B>(rb, reinterpret_cast<const char*>(args.B[step]), b_voff, args.ldb * 2, k0, tid);
-        }
+        const uint16_t* Ap = reinterpret_cast<const uint16_t*>(args.A[step]);
+        const uint16_t* Bp = reinterpret_cast<const uint16_t*>(args.B[step]);
+        tile_g2r<BM, TRANS_A>(ra, Ap, args.lda, m0, k0, M, K, tid, vec_a);
+        tile_g2r<BN, TRANS_B>(rb, Bp, args.ldb, n0, k0, N, K, tid, vec_b);
     };
     auto commit_loads = [&](int stage) {
         uint16_t* s = lds + stage * STAGE;
@@ -546,7 +396,7 @@ __global__ __launch_bounds__(kThreads) void gemm_bf16_kernel(const GemmArgs args
         __syncthreads();
     }
 
-    gemm_epilogue<BM, BN, TM, TN, EPI, !GUARD, E>(acc, args, lds, m0, n0, wm, wn, lane, tid);
+    gemm_epilogue<BM, BN, TM, TN, EPI, E>(acc, args, lds, m0, n0, wm, wn, lane, tid);
 }
 
 template <int BM, int BN>
@@ -556,9 +406,9 @@ constexpr size_t lds_bytes() {
     return stages > ctile ? stages : ctile;
 }
 
-template <int BM, int BN, bool TA, bool TB, bool GUARD, int EPI, typename E>
+template <int BM, int BN, bool TA, bool TB, int EPI, typename E>
 int launch_cfg(const GemmArgs& args, hipStream_t s) {
-    auto kern = gemm_bf16_kernel<BM, BN, TA, TB, GUARD, EPI, E>;
+    auto kern = gemm_bf16_kernel<BM, BN, TA, TB, EPI, E>;
     constexpr size_t lds = lds_bytes<BM, BN>();
     static_assert(lds <= 160 * 1024, "LDS tile does not fit the CU");
     if (lds > 48 * 1024) {
@@ -570,37 +420,32 @@ int launch_cfg(const GemmArgs& args, hipStream_t s) {
     return check_launch("gemm_bf16_kernel");
 }
 
-template <int BM, int BN, bool TA, bool TB, bool GUARD, typename E>
+template <int BM, int BN, bool TA, bool TB, typename E>
 int launch_epi(const GemmArgs& args, int epilogue, hipStream_t s) {
     switch (epilogue) {
-        case CW_EPI_NONE: return launch_cfg<BM, BN, TA, TB, GUARD, CW_EPI_NONE, E>(args, s);
-        case CW_EPI_BIAS: return launch_cfg<BM, BN, TA, TB, GUARD, CW_EPI_BIAS, E>(args, s);
-        case CW_EPI_BIAS_GELU_TANH: return launch_cfg<BM, BN, TA, TB, GUARD, CW_EPI_BIAS_GELU_TANH, E>(args, s);
-        case CW_EPI_BIAS_GELU_ERF: return launch_cfg<BM, BN, TA, TB, GUARD, CW_EPI_BIAS_GELU_ERF, E>(args, s);
-        case CW_EPI_BIAS_RELU: return launch_cfg<BM, BN, TA, TB, GUARD, CW_EPI_BIAS_RELU, E>(args, s);
+        case CW_EPI_NONE: return launch_cfg<BM, BN, TA, TB, CW_EPI_NONE, E>(args, s);
+        case CW_EPI_BIAS: return launch_cfg<BM, BN, TA, TB, CW_EPI_BIAS, E>(args, s);
+        case CW_EPI_BIAS_GELU_TANH: return launch_cfg<BM, BN, TA, TB, CW_EPI_BIAS_GELU_TANH, E>(args, s);
+        case CW_EPI_BIAS_GELU_ERF: return launch_cfg<BM, BN, TA, TB, CW_EPI_BIAS_GELU_ERF, E>(args, s);
+        case CW_EPI_BIAS_RELU: return launch_cfg<BM, BN, TA, TB, CW_EPI_BIAS_RELU, E>(args, s);
         default: return fail(CW_ERR_INVALID, "cw_gemm_ksteps: bad epilogue %d", epilogue);
     }
 }
 
-// All tile configurations of one operand orientation. `big` selects 256x256
-// tiles, `exact` the unguarded kernels (tile-multiple, 16-byte aligned shapes).
+// Both tile sizes of one operand orientation, guarded (ragged and unaligned shapes).
 template <bool TA, bool TB, typename E>
-int launch_orientation(const GemmArgs& args, int epilogue, bool big, bool exact, hipStream_t s) {
-    if (big)
-        return exact ? launch_epi<256, 256, TA, TB, false, E>(args, epilogue, s)
-                     : launch_epi<256, 256, TA, TB, true, E>(args, epilogue, s);
-    return exact ? launch_epi<128, 128, TA, TB, false, E>(args, epilogue, s)
-                 : launch_epi<128, 128, TA, TB, true, E>(args, epilogue, s);
+int launch_orientation(const GemmArgs& args, int epilogue, bool big, hipStream_t s) {
+    return big ? launch_epi<256, 256, TA, TB, E>(args, epilogue, s) : launch_epi<128, 128, TA, TB, E>(args, epilogue, s);
 }
 
 }  // namespace gemm_bf16
 
 // One translation unit per orientation and element type (gemm_bf16_nn/nt/tn.hip, gemm_f16_nn/nt/tn.hip).
-int gemm_bf16_launch_nn(const GemmArgs& args, int epilogue, bool big, bool exact, hipStream_t s);
-int gemm_bf16_launch_nt(const GemmArgs& args, int epilogue, bool big, bool exact, hipStream_t s);
-int gemm_bf16_launch_tn(const GemmArgs& args, int epilogue, bool big, bool exact, hipStream_t s);
-int gemm_f16_launch_nn(const GemmArgs& args, int epilogue, bool big, bool exact, hipStream_t s);
-int gemm_f16_launch_nt(const GemmArgs& args, int epilogue, bool big, bool exact, hipStream_t s);
-int gemm_f16_launch_tn(const GemmArgs& args, int epilogue, bool big, bool exact, hipStream_t s);
+int gemm_bf16_launch_nn(const GemmArgs& args, int epilogue, bool big, hipStream_t s);
+int gemm_bf16_launch_nt(const GemmArgs& args, int epilogue, bool big, hipStream_t s);
+int gemm_bf16_launch_tn(const GemmArgs& args, int epilogue, bool big, hipStream_t s);
+int gemm_f16_launch_nn(const GemmArgs& args, int epilogue, bool big, hipStream_t s);
+int gemm_f16_launch_nt(const GemmArgs& args, int epilogue, bool big, hipStream_t s);
+int gemm_f16_launch_tn(const GemmArgs& args, int epilogue, bool big, hipStream_t s);
 
 }  // namespace cw

@@ -3,8 +3,8 @@
 
 namespace cw {
 
-int gemm_bf16_launch_tn(const GemmArgs& args, int epilogue, bool big, bool exact, hipStream_t s) {
-    return gemm_bf16::launch_orientation<true, true, bf16_t>(args, epilogue, big, exact, s);
+int gemm_bf16_launch_tn(const GemmArgs& args, int epilogue, bool big, hipStream_t s) {
+    return gemm_bf16::launch_orientation<true, true, bf16_t>(args, epilogue, big, s);
 }
 
 }  // namespace cw

@@ -23,12 +23,12 @@ int gemm_prepare_args(int layout, int64_t M, int64_t N, int64_t K, int n_steps, 
 int64_t gemm_workspace_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int io_dtype);
 
 enum GemmRoute {
-    kRouteSmallRing = 0,      // 128 x 128 tiles, ring of LDS stages filled by the load unit
-    kRouteRing = 1,           // 256 x 256 tiles, the same ring
+    kRouteSmallRing = 0,      // 128 x 128 tiles
+    kRouteRing = 1,           // 256 x 256 tiles
     kRouteRingThenSmall = 2,  // whole rounds of 256 x 256 tiles (head), the mostly empty last round as 128 x 128 tiles (tail)
-    kRouteRingKTail = 3,      // ring + one short step over k in [K-32, K) for K % 32 != 0 (B stored [K, N])
-    kRouteSplitK = 4,         // ring over k slices into fp32 partials, then the reduce / epilogue launch
-    kRouteStaged = 5,         // register-staged kernel (ragged, unaligned, > 4 k-steps)
+    kRouteRingKTail = 3,      // 256 x 256 tiles with K % 32 != 0
+    kRouteSplitK = 4,         // 256 x 256 tiles over k slices into fp32 partials, then the reduce / epilogue launch
+    kRouteStaged = 5,         // whatever takes the shape without scratch
 };
 
 struct GemmPlan {
@@ -41,8 +41,44 @@ struct GemmPlan {
     int ktail_zero_rows;      // kRouteRingKTail: leading rows of the copied 32 rows of B that must be zero
 };
 
-// dma_enabled / strip_enabled: the two CW_GEMM_IMPL switches (staged / onelaunch) as the caller read them.
+// The plan of a call whose scratch is that of gemm_workspace_bytes, or none (a call with the scratch that tile_plan asks
+// for is planned by tile_plan). dma_enabled / strip_enabled: the two CW_GEMM_IMPL switches (staged / onelaunch) as the caller read them.
 GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool strip_enabled);
+
+// ---- tile kernels (gemm_tile.h) --------------------------------------------------------------------------------
+// Their configurations: wavefront tiles (block tile 64 tm x 64 tn), k extent of a trip in units of 32, ring stages, resident
+// blocks per compute unit, and what a trip costs (us; one block on the unit / two) and a block besides its trips. The
+// costs are a fit to 2000 launches over 110 shapes (products of 64 .. 8192 tokens with the model widths 768 .. 4096, in the
+// forward and weight-gradient orientations; rms error 11 %); choosing by them comes within 2 % of the best choice on average.
+struct TileConfig {
+    int tm, tn, kb, stages, resident;
+    float trip1, trip2, fixed;
+};
+constexpr TileConfig kTileConfigs[] = {
+    {4, 4, 1, 4, 1, 0.636f, 0.636f, 9.25f},  // 256 x 256: the least operand traffic per FLOP, one block per compute unit
+    {2, 4, 1, 3, 2, 0.429f, 0.897f, 5.00f},  // 128 x 256, two blocks
+    {2, 2, 1, 5, 2, 0.285f, 0.546f, 3.63f},  // 128 x 128
+    {1, 2, 2, 3, 2, 0.377f, 0.690f, 2.60f},  // 64 x 128
+    {1, 1, 2, 4, 2, 0.289f, 0.460f, 2.06f},  // 64 x 64: small outputs spread over the most compute units
+};
+constexpr int kTileConfigCount = 5;
+
+// How a product runs on the tile kernels: `full` tiles whole, the others in `slices` k slices through fp32 partial
+// sums. An operand whose rows are not 16-byte aligned is copied to rows that are, once per step (pack_a / pack_b).
+struct TilePlan {
+    int cfg;  // -1: the tile kernels do not take the shape
+    int64_t tiles;
+    int full, slices;
+    bool rotate;
+    bool pack_a, pack_b;
+    int64_t lda, ldb;             // leading dimensions the kernel sees
+    int64_t pack_a_bytes, pack_b_bytes, pack_add_bytes, partial_bytes;
+    int64_t scratch() const { return pack_a_bytes + pack_b_bytes + pack_add_bytes + partial_bytes; }
+};
+// max_scratch < 0: the choice with as much scratch as it likes; else the best one that fits. align_a / align_b: every step's
+// pointer is 16-byte aligned and the leading dimension a multiple of 8; n_pack_addends: addends of which that is not true.
+TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int64_t lda, int64_t ldb, bool align_a, bool align_b,
+                   int n_pack_addends, int64_t max_scratch);
 
 // Row slabs of the column-sum kernels for an [M, N] operand with V elements per 16 bytes: one partial row of N
 // sums per slab (vec: the vector kernel takes the shape; else the element-wise kernel).

@@ -232,6 +232,97 @@ GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool
     return plan;
 }
 
+namespace {
+
+// Time of `count` blocks of `trips` trips each, in rounds of the chip's resident blocks (us).
+double tile_rounds(const TileConfig& c, double count, double trips, double layout_factor) {
+    const double cap = 256.0 * c.resident, whole = (double)(int64_t)(count / cap), left = count - whole * cap;
+    double t = whole * (trips * c.trip2 * layout_factor + c.fixed);
+    if (left > 0) t += trips * (left > 256 ? c.trip2 : c.trip1) * layout_factor + c.fixed;
+    return t;
+}
+
+}  // namespace
+
+TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int64_t lda, int64_t ldb, bool align_a, bool align_b,
+                   int n_pack_addends, int64_t max_scratch) {
+    TilePlan best;
+    memset(&best, 0, sizeof(best));
+    best.cfg = -1;
+    const int64_t limit = (int64_t)1 << 30;
+    if (M <= 0 || N <= 0 || K <= 0 || M > limit || N > limit || K > limit || n_steps < 1 || n_steps > CW_MAX_KSTEPS) return best;
+    TilePlan p = best;
+    p.pack_a = !align_a;
+    p.pack_b = !align_b;
+    p.lda = lda;
+    p.ldb = ldb;
+    if (p.pack_a) {
+        p.lda = ((layout == CW_TN ? M : K) + 7) / 8 * 8;
+        p.pack_a_bytes = (n_steps * (layout == CW_TN ? K : M) * p.lda * 2 + 255) / 256 * 256;
+    }
+    if (p.pack_b) {
+        p.ldb = ((layout == CW_NT ? K : N) + 7) / 8 * 8;
+        p.pack_b_bytes = (n_steps * (layout == CW_NT ? N : K) * p.ldb * 2 + 255) / 256 * 256;
+    }
+    p.pack_add_bytes = (n_pack_addends * M * ((N + 7) / 8 * 8) * 2 + 255) / 256 * 256;
+    // the kernels' lane offsets: 256 rows (or 32 k rows) of either operand within 2 GB
+    if (p.lda >= ((int64_t)1 << 22) || p.ldb >= ((int64_t)1 << 22)) return best;
+    // A forward product (B stored [K, N]) that does not reduce its width, K <= N - the projections in front of an
+    // activation - sums k in ascending order whatever the tile: the 16-bit results of a row do not depend on how many rows
+    // there are, and a ReLU behind the next layer sees the same signs. Slicing gains little there anyway (the outputs have
+    // tiles enough). Two exceptions, fixed by the shape as well: whole rounds of 256 x 256 tiles start at an XCD-
+    // dependent k (memory channels, gemm_tile.h), and a few aligned tiles with a long reduction are always cut into the
+    // same slices.
+    const bool ordered = layout == CW_NN && K <= N;
+    const bool rotated = ordered && M % 256 == 0 && N % 256 == 0 && K % 32 == 0 && (M / 256) * (N / 256) >= 160;
+    const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
+    const int fixed_slices = ordered && !(tiles128 >= 192 && K * n_steps < 12288) ? gemm_bf16_split_slices(M, N, K, n_steps) : 1;
+    const double layout_factor = layout == CW_TN ? 0.9 : 1.0;  // both operands stream whole rows
+    const double bytes = 2.0 * ((double)M * K * n_steps + (double)K * N * n_steps + (double)M * N);
+    const double memory_us = bytes / 4.0e6;
+    double best_us = 0;
+    auto consider = [&](int cfg, int64_t tiles, int64_t full, int slices) {
+        const TileConfig& c = kTileConfigs[cfg];
+        const int64_t rest = tiles - full;
+        const double trips = (double)((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps;
+        TilePlan q = p;
+        q.cfg = cfg;
+        q.tiles = tiles;
+        q.full = (int)full;
+        q.slices = rest > 0 ? slices : 1;
+        q.rotate = ordered ? rotated : c.tm * c.tn == 16;
+        q.partial_bytes = rest * slices * (int64_t)(4096 * c.tm * c.tn) * 4;
+        if (max_scratch >= 0 && q.scratch() > max_scratch) return;
+        double us = tile_rounds(c, (double)full, trips, layout_factor);
+        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor) + 5.0 + 2.0 * q.partial_bytes / 6.6e6;
+        us = us > memory_us ? us + 0.1 * memory_us : memory_us + 0.1 * us;
+        if (best.cfg < 0 || us < best_us) {
+            best = q;
+            best_us = us;
+        }
+    };
+    for (int cfg = 0; cfg < kTileConfigCount; ++cfg) {
+        const TileConfig& c = kTileConfigs[cfg];
+        const int64_t tiles = ((M + 64 * c.tm - 1) / (64 * c.tm)) * ((N + 64 * c.tn - 1) / (64 * c.tn));
+        if (tiles > limit / 16 || ((rotated || fixed_slices > 1) && cfg != 0)) continue;
+        if (fixed_slices > 1) {
+            consider(cfg, tiles, 0, fixed_slices);
+            continue;
+        }
+        const int64_t trips = ((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps, cap = 256 * c.resident;
+        consider(cfg, tiles, tiles, 1);
+        // all tiles sliced, to fill the chip about once; or only those of the partial last round
+        if (ordered) continue;
+        const int64_t last = tiles % cap;
+        for (int slices = 2; slices <= 16; ++slices) {
+            if (trips / slices < 3) break;
+            if (tiles * slices <= cap) consider(cfg, tiles, 0, slices);
+            else if (tiles > cap && last > 0 && last * slices <= cap) consider(cfg, tiles, tiles - last, slices);
+        }
+    }
+    return best;
+}
+
 void colsum_plan(int64_t M, int64_t N, int V, bool vec, int64_t& slabs, int64_t& rows_per_slab) {
     if (!vec) {
         rows_per_slab = kColGenericSlabRows;

@@ -138,8 +138,10 @@ def gemm_ksteps(layout: str, A_steps: Sequence[torch.Tensor], B_steps: Sequence[
     preact = torch.empty((M, N), dtype=a0.dtype, device=a0.device) if want_preact else None
     epi = epilogue_code(bias is not None, activation)
     ta, tb, tadd = _ptr_table(A_steps), _ptr_table(B_steps), _ptr_table(addends)
-    # scratch for the split-k path (few output tiles, long reduction: the weight-gradient shape)
-    ws_bytes = lib.cw_gemm_workspace_bytes(LAYOUTS[layout], M, N, K, len(A_steps), dt)
+    # scratch for tiles cut along k and for copies of operands with unaligned rows
+    ws_bytes = lib.cw_gemm_scratch_bytes(LAYOUTS[layout], M, N, K, len(A_steps), lda, ldb, all(a.data_ptr() % 16 == 0 for a in A_steps),
+                                         all(b.data_ptr() % 16 == 0 for b in B_steps),
+                                         len(addends) if ldadd % 8 or any(t.data_ptr() % 16 for t in addends) else 0, dt)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a0.device) if ws_bytes > 0 else None
     rc = lib.cw_gemm_ksteps_ws(LAYOUTS[layout], M, N, K, len(A_steps), ta, lda, tb, ldb, _p(bias), epi, _p(out),
                                _ld(out), _p(preact), _ld(preact) if preact is not None else 0, tadd, len(addends),

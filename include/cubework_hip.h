@@ -135,6 +135,15 @@ int cw_gemm_ksteps(int layout, int64_t M, int64_t N, int64_t K, int n_steps,
  * shared by calls that may overlap on the device.
  */
 int64_t cw_gemm_workspace_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int io_dtype);
+/*
+ * Scratch with which cw_gemm_ksteps_ws runs a 16-bit product the fastest way it
+ * knows, for any shape: fp32 partial sums where the output's tiles (or those of
+ * a partly empty last round) are cut along k, and copies of operands whose rows
+ * are not 16-byte aligned (aligned_a / aligned_b: whether every step's pointer
+ * is). With less than this the call is planned for what it has, down to none.
+ */
+int64_t cw_gemm_scratch_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int64_t lda, int64_t ldb, int aligned_a,
+                              int aligned_b, int unaligned_addends, int io_dtype);
 int cw_gemm_ksteps_ws(int layout, int64_t M, int64_t N, int64_t K, int n_steps,
                       const void* const* A_steps, int64_t lda,
                       const void* const* B_steps, int64_t ldb,
