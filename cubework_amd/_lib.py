@@ -51,6 +51,10 @@ SIGNATURES = {
     "cw_embed_bwd_ids": (_int, [_i64, _i64, _ptr, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _int, _ptr]),
     "cw_attn_fwd": (_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _i64, _i64, _f32, _int, _ptr, _i64, _i64, _i64,
                            _ptr, _int, _ptr]),
+    "cw_attn_narrow_fwd": (_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _i64, _i64, _f32, _int, _ptr, _i64, _i64,
+                                  _i64, _ptr, _int, _ptr]),
+    "cw_attn_narrow_bwd": (_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr, _i64, _i64, _i64,
+                                  _ptr, _f32, _int, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _i64, _int, _ptr]),
     "cw_attn_bwd_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "cw_attn_bwd": (_int, [_i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr, _i64, _i64, _i64, _ptr,
                            _f32, _int, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr, _i64, _int, _ptr]),

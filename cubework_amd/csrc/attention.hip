@@ -1,4 +1,4 @@
-// Fused causal attention core for gfx950, head sizes 64 and 128, bf16 (or fp16: E = f16_t):
+// Fused causal attention core for gfx950, head sizes up to 128 (multiples of 8), bf16 (or fp16: E = f16_t):
 //   O = softmax(scale * Q K^T + causal mask) V        per (batch, head)
 // (benchmark/opt/opt.py:81-117 of the reference: scaled bmm, additive mask,
 // softmax, bmm). One pass over K/V per block of queries with a running
@@ -46,15 +46,18 @@ struct AttnArgs {
     int64_t sb, ss, sh;     // q/k/v strides (elements): batch, token, head
     int64_t ob, os, oh;     // output strides
     int S, H, BH, n_qblocks;
+    int D;                  // head size
     float scale_log2e;      // scale * log2(e)
     int causal;
 };
 
-// NP: head size / 64. A tile of NP x 64 columns is NP images side by side ("panels"); everything that
-// runs over the head dimension runs over NP times as many 16-wide k blocks (scores) or 32-wide output
-// blocks (O^T). Head size 64 keeps two blocks per compute unit, 128 has the registers and LDS of one.
-template <int NP, typename E>
-__global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(const AttnArgs a) {
+// HS: the head's shape (HeadShape). A tile of NP x 64 columns is NP images side by side ("panels"); everything that
+// runs over the head dimension runs over KB 16-wide k blocks (scores) or DT 32-wide output blocks (O^T). Heads up to
+// 80 columns keep two blocks per compute unit, 128 has the registers of one.
+template <typename HS, typename E>
+__global__ __launch_bounds__(kThreads, HS::NP == 1 ? 2 : 1) void attn_fwd_kernel(const AttnArgs a) {
+    constexpr int NP = HS::NP, KB = HS::KB, DT = HS::DT;
+    constexpr bool MASK = HS::MASK;
     constexpr int kStage = 2 * NP * kImage;  // K panels (row images), then V panels (transpose images)
     __shared__ __attribute__((aligned(16))) char lds_raw[2 * kStage];
     lds_char* lds = (lds_char*)lds_raw;
@@ -82,21 +85,21 @@ __global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(con
     const uint16_t* vp = a.v + b * a.sb + h * a.sh;
 
     // Q fragments (B operand): lane = query row l32 of tile qt, 8 d-values at 16 kb + 8 half
-    bf16x8_t qf[kQT][4 * NP];
+    bf16x8_t qf[kQT][KB];
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt) {
         int row = qw0 + 32 * qt + l32;
         row = row < S ? row : S - 1;
-        const uint16_t* p = qp + (int64_t)row * a.ss + 8 * half;
+        const uint16_t* p = qp + (int64_t)row * a.ss;
 #pragma unroll
-        for (int kb = 0; kb < 4 * NP; ++kb) qf[qt][kb] = __builtin_bit_cast(bf16x8_t, load_raw(p + 16 * kb));
+        for (int kb = 0; kb < KB; ++kb) qf[qt][kb] = __builtin_bit_cast(bf16x8_t, load_cols<MASK>(p, 16 * kb + 8 * half, a.D));
     }
 
-    f32x16_t oacc[kQT][2 * NP];
+    f32x16_t oacc[kQT][DT];
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt)
 #pragma unroll
-        for (int dt = 0; dt < 2 * NP; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int e = 0; e < 16; ++e) oacc[qt][dt][e] = 0.0f;
     // reference of the exponentials (scale*log2e*s units), the raw score above which it moves, this lane's share
@@ -124,8 +127,8 @@ __global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(con
     auto load_stage = [&](int row0, uint32_t stage_addr) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            dma.template load<true, false>(kp + 64 * p, a.ss, row0, S, stage_addr + p * kImage, 0);
-            dma.template load<false, true>(vp + 64 * p, a.ss, row0, S, 0, stage_addr + (NP + p) * kImage);
+            dma.template load<true, false, MASK>(kp + 64 * p, a.ss, row0, S, stage_addr + p * kImage, 0, a.D - 64 * p);
+            dma.template load<false, true, MASK>(vp + 64 * p, a.ss, row0, S, 0, stage_addr + (NP + p) * kImage, a.D - 64 * p);
         }
     };
     load_stage(0, lds_addr);
@@ -137,7 +140,7 @@ __global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(con
 #pragma unroll
     for (int qt = 0; qt < kQT; ++qt)
 #pragma unroll
-        for (int kb = 0; kb < 4 * NP; ++kb) asm volatile("" : "+v"(qf[qt][kb]));
+        for (int kb = 0; kb < KB; ++kb) asm volatile("" : "+v"(qf[qt][kb]));
 
     // One tile of 64 key rows out of LDS stage STAGE (a compile-time constant, so that every fragment read is
     // lane offset + immediate: no address arithmetic in the loop); the loop below alternates the two stages.
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(con
 #pragma unroll
                     for (int e = 0; e < 16; ++e) st[qt][e] = 0.0f;
 #pragma unroll
-                for (int kb = 0; kb < 4 * NP; ++kb) {
+                for (int kb = 0; kb < KB; ++kb) {
                     const bf16x8_t kf = read_rows<32 * kt>(ks + (kb >> 2) * kImage, ro, kb & 3);
 #pragma unroll
                     for (int qt = 0; qt < kQT; ++qt)
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(con
                         const float alpha = __builtin_amdgcn_exp2f(m_run[qt] - m_new);
                         l_run[qt] *= alpha;
 #pragma unroll
-                        for (int dt = 0; dt < 2 * NP; ++dt)
+                        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
                             for (int e = 0; e < 16; ++e) oacc[qt][dt][e] *= alpha;
                         m_run[qt] = m_new;
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(con
                 }
                 // O^T += V^T P^T over the 32 kv rows of this half tile
 #pragma unroll
-                for (int dt = 0; dt < 2 * NP; ++dt) {
+                for (int dt = 0; dt < DT; ++dt) {
                     const bf16x8_t vf0 = read_transposed<32 * kt>(vs + (dt >> 1) * kImage, ro, dt & 1);
                     const bf16x8_t vf1 = read_transposed<32 * kt + 16>(vs + (dt >> 1) * kImage, ro, dt & 1);
 #pragma unroll
@@ -254,8 +257,7 @@ __global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(con
         const float inv = l_tot > 0.0f ? __builtin_amdgcn_rcpf(l_tot) : 0.0f;
         if (qi < S) {
             uint16_t* orow = a.o + b * a.ob + (int64_t)qi * a.os + h * a.oh;
-#pragma unroll
-            for (int p = 0; p < NP; ++p) store_row_pieces<E>(orow + 64 * p, oacc[qt] + 2 * p, inv, half);
+            store_row_pieces<E, DT, MASK>(orow, oacc[qt], inv, half, a.D);
             if (half == 0 && a.lse != nullptr)
                 a.lse[(int64_t)bh * S + qi] = (m_run[qt] + __builtin_amdgcn_logf(l_tot)) * kLn2;  // natural-log LSE of scale*s
         }
@@ -267,23 +269,21 @@ __global__ __launch_bounds__(kThreads, NP == 1 ? 2 : 1) void attn_fwd_kernel(con
 
 using namespace cw;
 
-extern "C" int cw_attn_fwd(int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
-                           int64_t stride_b, int64_t stride_s, int64_t stride_h, float scale, int causal, void* out,
-                           int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h, float* lse,
-                           int io_dtype, void* stream) {
-    if (B < 0 || H < 0 || S < 0 || D <= 0) return fail(CW_ERR_INVALID, "cw_attn_fwd: bad shape B=%lld H=%lld S=%lld D=%lld", (long long)B, (long long)H, (long long)S, (long long)D);
-    if (io_dtype != CW_BF16 && io_dtype != CW_F16) return fail(CW_ERR_UNSUPPORTED, "cw_attn_fwd: only bf16 and fp16 are provided");
-    if (D != 64 && D != 128) return fail(CW_ERR_UNSUPPORTED, "cw_attn_fwd: head size %lld is not provided (64 and 128)", (long long)D);
+namespace {
+
+int attn_fwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
+             int64_t stride_b, int64_t stride_s, int64_t stride_h, float scale, int causal, void* out, int64_t out_stride_b,
+             int64_t out_stride_s, int64_t out_stride_h, float* lse, int io_dtype, void* stream) {
     if (B == 0 || H == 0 || S == 0) return CW_OK;
-    if (q == nullptr || k == nullptr || v == nullptr || out == nullptr) return fail(CW_ERR_INVALID, "cw_attn_fwd: null pointer");
+    if (q == nullptr || k == nullptr || v == nullptr || out == nullptr) return fail(CW_ERR_INVALID, "%s: null pointer", who);
     if (S > INT32_MAX / 2 || B * H > (1 << 20) || ((S + kQPerBlock - 1) / kQPerBlock) * B * H > INT32_MAX)
-        return fail(CW_ERR_INVALID, "cw_attn_fwd: S or B*H too large");
+        return fail(CW_ERR_INVALID, "%s: S or B*H too large", who);
     const bool aligned = aligned16(q) && aligned16(k) && aligned16(v) && (reinterpret_cast<uintptr_t>(out) & 7u) == 0 &&
                          stride_b % 8 == 0 && stride_s % 8 == 0 && stride_h % 8 == 0 && out_stride_b % 4 == 0 &&
                          out_stride_s % 4 == 0 && out_stride_h % 4 == 0;
-    if (!aligned) return fail(CW_ERR_ALIGNMENT, "cw_attn_fwd: q/k/v need 16-byte aligned rows, out 8-byte aligned rows");
+    if (!aligned) return fail(CW_ERR_ALIGNMENT, "%s: q/k/v need 16-byte aligned rows, out 8-byte aligned rows", who);
     if (stride_s <= 0 || stride_s >= (1 << 23))
-        return fail(CW_ERR_INVALID, "cw_attn_fwd: token stride %lld outside (0, 2^23) elements", (long long)stride_s);
+        return fail(CW_ERR_INVALID, "%s: token stride %lld outside (0, 2^23) elements", who, (long long)stride_s);
     AttnArgs a;
     a.q = (const uint16_t*)q;
     a.k = (const uint16_t*)k;
@@ -292,19 +292,41 @@ extern "C" int cw_attn_fwd(int64_t B, int64_t H, int64_t S, int64_t D, const voi
     a.lse = lse;
     a.sb = stride_b; a.ss = stride_s; a.sh = stride_h;
     a.ob = out_stride_b; a.os = out_stride_s; a.oh = out_stride_h;
-    a.S = (int)S; a.H = (int)H; a.BH = (int)(B * H);
+    a.S = (int)S; a.H = (int)H; a.BH = (int)(B * H); a.D = (int)D;
     a.scale_log2e = scale * kLog2e;
     a.causal = causal ? 1 : 0;
     a.n_qblocks = (int)((S + kQPerBlock - 1) / kQPerBlock);
     const dim3 grid((unsigned)(a.n_qblocks * B * H));
-    if (const int drc = require_gfx950("cw_attn_fwd"); drc != CW_OK) return drc;
+    if (const int drc = require_gfx950(who); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
-    if (io_dtype == CW_F16) {
-        if (D == 64) hipLaunchKernelGGL((attn_fwd_kernel<1, f16_t>), grid, dim3(kThreads), 0, s, a);
-        else hipLaunchKernelGGL((attn_fwd_kernel<2, f16_t>), grid, dim3(kThreads), 0, s, a);
-    } else {
-        if (D == 64) hipLaunchKernelGGL((attn_fwd_kernel<1, bf16_t>), grid, dim3(kThreads), 0, s, a);
-        else hipLaunchKernelGGL((attn_fwd_kernel<2, bf16_t>), grid, dim3(kThreads), 0, s, a);
-    }
-    return check_launch("attn_fwd_kernel");
+    return with_head_shape(D, [&](auto hs) {
+        using HS = decltype(hs);
+        if (io_dtype == CW_F16) hipLaunchKernelGGL((attn_fwd_kernel<HS, f16_t>), grid, dim3(kThreads), 0, s, a);
+        else hipLaunchKernelGGL((attn_fwd_kernel<HS, bf16_t>), grid, dim3(kThreads), 0, s, a);
+        return check_launch("attn_fwd_kernel");
+    });
+}
+
+}  // namespace
+
+extern "C" int cw_attn_fwd(int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
+                           int64_t stride_b, int64_t stride_s, int64_t stride_h, float scale, int causal, void* out,
+                           int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h, float* lse,
+                           int io_dtype, void* stream) {
+    if (B < 0 || H < 0 || S < 0 || D <= 0) return fail(CW_ERR_INVALID, "cw_attn_fwd: bad shape B=%lld H=%lld S=%lld D=%lld", (long long)B, (long long)H, (long long)S, (long long)D);
+    if (io_dtype != CW_BF16 && io_dtype != CW_F16) return fail(CW_ERR_UNSUPPORTED, "cw_attn_fwd: only bf16 and fp16 are provided");
+    if (D != 64 && D != 128) return fail(CW_ERR_UNSUPPORTED, "cw_attn_fwd: head size %lld is not provided (64 and 128)", (long long)D);
+    return attn_fwd("cw_attn_fwd", B, H, S, D, q, k, v, stride_b, stride_s, stride_h, scale, causal, out, out_stride_b,
+                    out_stride_s, out_stride_h, lse, io_dtype, stream);
+}
+
+extern "C" int cw_attn_narrow_fwd(int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
+                                  int64_t stride_b, int64_t stride_s, int64_t stride_h, float scale, int causal, void* out,
+                                  int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h, float* lse,
+                                  int io_dtype, void* stream) {
+    if (B < 0 || H < 0 || S < 0 || D <= 0) return fail(CW_ERR_INVALID, "cw_attn_narrow_fwd: bad shape B=%lld H=%lld S=%lld D=%lld", (long long)B, (long long)H, (long long)S, (long long)D);
+    if (io_dtype != CW_BF16 && io_dtype != CW_F16) return fail(CW_ERR_UNSUPPORTED, "cw_attn_narrow_fwd: only bf16 and fp16 are provided");
+    if (D % 8 != 0 || D > 128) return fail(CW_ERR_UNSUPPORTED, "cw_attn_narrow_fwd: head size %lld is not provided (multiples of 8 up to 128)", (long long)D);
+    return attn_fwd("cw_attn_narrow_fwd", B, H, S, D, q, k, v, stride_b, stride_s, stride_h, scale, causal, out, out_stride_b,
+                    out_stride_s, out_stride_h, lse, io_dtype, stream);
 }

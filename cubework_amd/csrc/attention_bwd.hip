@@ -1,4 +1,4 @@
-// Backward of the fused attention core for gfx950 (head sizes 64 and 128; bf16, or fp16 with E = f16_t):
+// Backward of the fused attention core for gfx950 (head sizes up to 128, multiples of 8; bf16, or fp16 with E = f16_t):
 // given Q, K, V, O, dO and the forward's log-sum-exp L (natural log),
 //   P_ij  = exp(scale q_i.k_j - L_i)              (recomputed, never stored)
 //   D_i   = sum_d dO_id O_id
@@ -41,6 +41,10 @@ constexpr int kRowsPerBlock = kWaves * kRowsPerWave;
 // and ran the same phase at the same time (302 -> 291 us for the whole backward at batch 4 x 32 heads x 2048
 // tokens). At head size 128 a wavefront needs more than 256 registers and a unit holds one workgroup. Two groups
 // of 32 keys per wavefront (every LDS operand read feeding two MFMAs, 510 registers) ran 278 us against 190 us.
+// Heads of 65 to 80 columns also leave room for one workgroup only (130 KB of LDS), but need no more than 256 registers:
+// 8 wavefronts then share the workgroup's tiles, two per SIMD. Whole backward at 32 heads of 80, 4 against 8
+// wavefronts: 4 x 1500 tokens 344 -> 290 us, 8 x 200 tokens 48 -> 42 us, 2 x 777 tokens 80 and 81 us. At head size 128
+// the same would spill (4 x 512 tokens 81 -> 100 us).
 constexpr int kDkdvWaves = 4;
 
 struct BwdArgs {
@@ -58,15 +62,17 @@ struct BwdArgs {
     int64_t ob, os, oh;  // o / dO strides
     int64_t gb, gs, gh;  // dq/dk/dv strides
     int S, H, BH, n_blocks;  // n_blocks: query blocks of the dQ kernel
-    int D;                   // head size (64 or 128)
+    int D;                   // head size
     float scale, scale_log2e;
     int causal;
 };
 
 // ---- dQ ---------------------------------------------------------------------
-// LDS per stage: K row images, K transpose images, V row images (NP = head size / 64 panels of each).
-template <int NP, typename E>
+// LDS per stage: K row images, K transpose images, V row images (NP panels of 64 columns of each).
+template <typename HS, typename E>
 __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
+    constexpr int NP = HS::NP, KB = HS::KB, DT = HS::DT;
+    constexpr bool MASK = HS::MASK;
     constexpr int kStage = 3 * NP * kImage;
     __shared__ __attribute__((aligned(16))) char lds_raw[2 * kStage];
     lds_char* lds = (lds_char*)lds_raw;
@@ -84,21 +90,21 @@ __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
     // the lane's query row: Q and dO fragments (B operands), L*log2e and D
     const int qi = qw0 + l32;
     const int qrow = qi < S ? qi : S - 1;
-    bf16x8_t qf[4 * NP], dof[4 * NP];
+    bf16x8_t qf[KB], dof[KB];
     // D of the lane's row, from the dO pieces it holds anyway and the same pieces of O: the two lanes of a row
     // (half 0 and 1) add their parts. The dK/dV launch, which follows on the stream, reads it from a.delta.
     float dlt_ld = 0.0f;
     {
-        const uint16_t* p = a.q + b * a.sb + (int64_t)qrow * a.ss + h * a.sh + 8 * half;
-        const uint16_t* g = a.d_o + b * a.ob + (int64_t)qrow * a.os + h * a.oh + 8 * half;
-        const uint16_t* o = a.o + b * a.ob + (int64_t)qrow * a.os + h * a.oh + 8 * half;
+        const uint16_t* p = a.q + b * a.sb + (int64_t)qrow * a.ss + h * a.sh;
+        const uint16_t* g = a.d_o + b * a.ob + (int64_t)qrow * a.os + h * a.oh;
+        const uint16_t* o = a.o + b * a.ob + (int64_t)qrow * a.os + h * a.oh;
 #pragma unroll
-        for (int kb = 0; kb < 4 * NP; ++kb) {
-            qf[kb] = __builtin_bit_cast(bf16x8_t, load_raw(p + 16 * kb));
-            const raw16_t graw = load_raw(g + 16 * kb);
+        for (int kb = 0; kb < KB; ++kb) {
+            qf[kb] = __builtin_bit_cast(bf16x8_t, load_cols<MASK>(p, 16 * kb + 8 * half, a.D));
+            const raw16_t graw = load_cols<MASK>(g, 16 * kb + 8 * half, a.D);
             dof[kb] = __builtin_bit_cast(bf16x8_t, graw);
             float x[8], y[8];
-            unpack_raw(load_raw(o + 16 * kb), x, (const E*)nullptr);
+            unpack_raw(load_cols<MASK>(o, 16 * kb + 8 * half, a.D), x, (const E*)nullptr);
             unpack_raw(graw, y, (const E*)nullptr);
 #pragma unroll
             for (int e = 0; e < 8; ++e) dlt_ld = __builtin_fmaf(x[e], y[e], dlt_ld);
@@ -107,9 +113,9 @@ __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
         if (half == 0 && qi < S) a.delta[(int64_t)bh * S + qi] = dlt_ld;
     }
     const float lse2_ld = a.lse[(int64_t)bh * S + qrow] * kLog2e;
-    f32x16_t dq[2 * NP];
+    f32x16_t dq[DT];
 #pragma unroll
-    for (int dt = 0; dt < 2 * NP; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) dq[dt][e] = 0.0f;
 
@@ -127,8 +133,8 @@ __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
     auto load_stage = [&](int row0, uint32_t st) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            dma.template load<true, true>(kp + 64 * p, a.ss, row0, S, st + p * kImage, st + (NP + p) * kImage);
-            dma.template load<true, false>(vp + 64 * p, a.ss, row0, S, st + (2 * NP + p) * kImage, 0);
+            dma.template load<true, true, MASK>(kp + 64 * p, a.ss, row0, S, st + p * kImage, st + (NP + p) * kImage, a.D - 64 * p);
+            dma.template load<true, false, MASK>(vp + 64 * p, a.ss, row0, S, st + (2 * NP + p) * kImage, 0, a.D - 64 * p);
         }
     };
     load_stage(0, lds_addr);
@@ -139,7 +145,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
     float lse2 = lse2_ld, dlt = dlt_ld;
     asm volatile("" : "+v"(lse2), "+v"(dlt));
 #pragma unroll
-    for (int kb = 0; kb < 4 * NP; ++kb) asm volatile("" : "+v"(qf[kb]), "+v"(dof[kb]));
+    for (int kb = 0; kb < KB; ++kb) asm volatile("" : "+v"(qf[kb]), "+v"(dof[kb]));
 
     // One tile of 64 key rows out of LDS stage STAGE, a compile-time constant so that every fragment read is lane
     // offset + immediate (no address arithmetic in the loop); the loop below alternates the two stages.
@@ -168,7 +174,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
                     dpt[e] = 0.0f;
                 }
 #pragma unroll
-                for (int kb = 0; kb < 4 * NP; ++kb) {
+                for (int kb = 0; kb < KB; ++kb) {
                     st = mfma16<E>(read_rows<32 * kt>(k_rows + (kb >> 2) * kImage, ro, kb & 3), qf[kb], st);
                     dpt = mfma16<E>(read_rows<32 * kt>(v_rows + (kb >> 2) * kImage, ro, kb & 3), dof[kb], dpt);
                 }
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
                 }
                 const bf16x8_t dsb0 = pack_slots<E>(ds, 0), dsb1 = pack_slots<E>(ds, 1);
 #pragma unroll
-                for (int dt = 0; dt < 2 * NP; ++dt) {
+                for (int dt = 0; dt < DT; ++dt) {
                     lds_char* kt_img = k_tr + (dt >> 1) * kImage;
                     dq[dt] = mfma16<E>(read_transposed<32 * kt>(kt_img, ro, dt & 1), dsb0, dq[dt]);
                     dq[dt] = mfma16<E>(read_transposed<32 * kt + 16>(kt_img, ro, dt & 1), dsb1, dq[dt]);
@@ -208,21 +214,22 @@ __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
     }
     if (qi < S) {
         uint16_t* grow = a.dq + b * a.gb + (int64_t)qi * a.gs + h * a.gh;
-#pragma unroll
-        for (int p = 0; p < NP; ++p) store_row_pieces<E>(grow + 64 * p, dq + 2 * p, a.scale, half);
+        store_row_pieces<E, DT, MASK>(grow, dq, a.scale, half, a.D);
     }
 }
 
 // ---- dK, dV -----------------------------------------------------------------
-// LDS per stage: Q row images, Q transpose images, dO row images, dO transpose images (NP = head size / 64
-// panels of each), L*log2e and -D of the 64 rows. NW wavefronts of 32 key rows.
+// LDS per stage: Q row images, Q transpose images, dO row images, dO transpose images (NP panels of 64 columns
+// of each), L*log2e and -D of the 64 rows. NW wavefronts of 32 key rows.
 template <int NP>
 constexpr int dkdv_stage_bytes() { return 4 * NP * kImage + 2 * kTile * 4; }
 
 // KG: groups of 32 key rows per wavefront. With two, every A operand read from LDS (Q, dO, their
 // transposes) feeds two MFMAs instead of one.
-template <int NP, int NW, int KG, typename E>
-__global__ __launch_bounds__(NW * 64, NP == 1 ? 2 : 1) void attn_dkdv_kernel(const BwdArgs a) {
+template <typename HS, int NW, int KG, typename E>
+__global__ __launch_bounds__(NW * 64, HS::NP == 1 ? 2 : 1) void attn_dkdv_kernel(const BwdArgs a) {
+    constexpr int NP = HS::NP, KB = HS::KB, DT = HS::DT;
+    constexpr bool MASK = HS::MASK;
     constexpr int kKeysPerWave = KG * kRowsPerWave;
     constexpr int kDkdvStage = dkdv_stage_bytes<NP>();
     constexpr int kStatsAt = 4 * NP * kImage;
@@ -242,24 +249,24 @@ __global__ __launch_bounds__(NW * 64, NP == 1 ? 2 : 1) void attn_dkdv_kernel(con
     const float* dltp = a.delta + (int64_t)bh * S;
 
     // the lane's key rows (one per group): K and V fragments (B operands)
-    bf16x8_t kf[KG][4 * NP], vf[KG][4 * NP];
+    bf16x8_t kf[KG][KB], vf[KG][KB];
 #pragma unroll
     for (int kg = 0; kg < KG; ++kg) {
         const int kvi = kw0 + 32 * kg + l32;
         const int kvrow = kvi < S ? kvi : S - 1;
-        const uint16_t* pk = a.k + b * a.sb + (int64_t)kvrow * a.ss + h * a.sh + 8 * half;
-        const uint16_t* pv = a.v + b * a.sb + (int64_t)kvrow * a.ss + h * a.sh + 8 * half;
+        const uint16_t* pk = a.k + b * a.sb + (int64_t)kvrow * a.ss + h * a.sh;
+        const uint16_t* pv = a.v + b * a.sb + (int64_t)kvrow * a.ss + h * a.sh;
 #pragma unroll
-        for (int kb = 0; kb < 4 * NP; ++kb) {
-            kf[kg][kb] = __builtin_bit_cast(bf16x8_t, load_raw(pk + 16 * kb));
-            vf[kg][kb] = __builtin_bit_cast(bf16x8_t, load_raw(pv + 16 * kb));
+        for (int kb = 0; kb < KB; ++kb) {
+            kf[kg][kb] = __builtin_bit_cast(bf16x8_t, load_cols<MASK>(pk, 16 * kb + 8 * half, a.D));
+            vf[kg][kb] = __builtin_bit_cast(bf16x8_t, load_cols<MASK>(pv, 16 * kb + 8 * half, a.D));
         }
     }
-    f32x16_t dk[KG][2 * NP], dv[KG][2 * NP];
+    f32x16_t dk[KG][DT], dv[KG][DT];
 #pragma unroll
     for (int kg = 0; kg < KG; ++kg)
 #pragma unroll
-        for (int dt = 0; dt < 2 * NP; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 dk[kg][dt][e] = 0.0f;
@@ -293,8 +300,9 @@ __global__ __launch_bounds__(NW * 64, NP == 1 ? 2 : 1) void attn_dkdv_kernel(con
     auto load_stage = [&](int row0, uint32_t st) {
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
-            dma.template load<true, true>(qp + 64 * p, a.ss, row0, S, st + p * kImage, st + (NP + p) * kImage);
-            dma.template load<true, true>(gp + 64 * p, a.os, row0, S, st + (2 * NP + p) * kImage, st + (3 * NP + p) * kImage);
+            dma.template load<true, true, MASK>(qp + 64 * p, a.ss, row0, S, st + p * kImage, st + (NP + p) * kImage, a.D - 64 * p);
+            dma.template load<true, true, MASK>(gp + 64 * p, a.os, row0, S, st + (2 * NP + p) * kImage, st + (3 * NP + p) * kImage,
+                                                a.D - 64 * p);
         }
     };
     load_stage(first_tile * kTile, lds_addr);
@@ -305,7 +313,7 @@ __global__ __launch_bounds__(NW * 64, NP == 1 ? 2 : 1) void attn_dkdv_kernel(con
 #pragma unroll
     for (int kg = 0; kg < KG; ++kg)
 #pragma unroll
-        for (int kb = 0; kb < 4 * NP; ++kb) asm volatile("" : "+v"(kf[kg][kb]), "+v"(vf[kg][kb]));  // arrived before the loop
+        for (int kb = 0; kb < KB; ++kb) asm volatile("" : "+v"(kf[kg][kb]), "+v"(vf[kg][kb]));  // arrived before the loop
 
     // One tile of 64 query rows out of LDS stage STAGE (compile-time: fragment reads are lane offset + immediate)
     auto tile_step = [&](int t, auto stage_c) {
@@ -348,7 +356,7 @@ __global__ __launch_bounds__(NW * 64, NP == 1 ? 2 : 1) void attn_dkdv_kernel(con
                     }
                 }
 #pragma unroll
-                for (int kb = 0; kb < 4 * NP; ++kb) {
+                for (int kb = 0; kb < KB; ++kb) {
                     const bf16x8_t qa = read_rows<32 * qt>(q_rows + (kb >> 2) * kImage, ro, kb & 3);
                     const bf16x8_t ga = read_rows<32 * qt>(g_rows + (kb >> 2) * kImage, ro, kb & 3);
 #pragma unroll
@@ -390,7 +398,7 @@ __global__ __launch_bounds__(NW * 64, NP == 1 ? 2 : 1) void attn_dkdv_kernel(con
 #pragma unroll
                 for (int sl = 0; sl < 2; ++sl) {
 #pragma unroll
-                    for (int dt = 0; dt < 2 * NP; ++dt) {
+                    for (int dt = 0; dt < DT; ++dt) {
                         lds_char* gi = g_tr + (dt >> 1) * kImage;
                         lds_char* qi_img = q_tr + (dt >> 1) * kImage;
                         const bf16x8_t gt = sl == 0 ? read_transposed<32 * qt>(gi, ro, dt & 1) : read_transposed<32 * qt + 16>(gi, ro, dt & 1);
@@ -424,36 +432,28 @@ __global__ __launch_bounds__(NW * 64, NP == 1 ? 2 : 1) void attn_dkdv_kernel(con
         if (kvi < S) {
             uint16_t* dkrow = a.dk + b * a.gb + (int64_t)kvi * a.gs + h * a.gh;
             uint16_t* dvrow = a.dv + b * a.gb + (int64_t)kvi * a.gs + h * a.gh;
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                store_row_pieces<E>(dkrow + 64 * p, dk[kg] + 2 * p, a.scale, half);
-                store_row_pieces<E>(dvrow + 64 * p, dv[kg] + 2 * p, 1.0f, half);
-            }
+            store_row_pieces<E, DT, MASK>(dkrow, dk[kg], a.scale, half, a.D);
+            store_row_pieces<E, DT, MASK>(dvrow, dv[kg], 1.0f, half, a.D);
         }
     }
 }
 
-// The three launches of the backward for element type E.
+// The two launches of the backward for element type E.
 template <typename E>
 int launch_bwd(const BwdArgs& a, int64_t B, int64_t H, int64_t S, int64_t D, int64_t nblk, hipStream_t s) {
-    if (D == 64) hipLaunchKernelGGL((attn_dq_kernel<1, E>), dim3((unsigned)(nblk * B * H)), dim3(kThreads), 0, s, a);
-    else hipLaunchKernelGGL((attn_dq_kernel<2, E>), dim3((unsigned)(nblk * B * H)), dim3(kThreads), 0, s, a);
-    if (const int rc = check_launch("attn_dq_kernel"); rc != CW_OK) return rc;
-    // both head sizes: 4 wavefronts (128 keys) per workgroup
-    const int64_t nkv = (S + kDkdvWaves * kRowsPerWave - 1) / (kDkdvWaves * kRowsPerWave);
-    if (nkv * B * H > INT32_MAX) return fail(CW_ERR_INVALID, "cw_attn_bwd: S or B*H too large");
-    if (D == 64) {
-        constexpr int lds_bytes = 2 * dkdv_stage_bytes<1>();
-        auto kern = attn_dkdv_kernel<1, kDkdvWaves, 1, E>;
+    return with_head_shape(D, [&](auto hs) {
+        using HS = decltype(hs);
+        hipLaunchKernelGGL((attn_dq_kernel<HS, E>), dim3((unsigned)(nblk * B * H)), dim3(kThreads), 0, s, a);
+        if (const int rc = check_launch("attn_dq_kernel"); rc != CW_OK) return rc;
+        constexpr int NW = HS::KB == 5 ? 2 * kDkdvWaves : kDkdvWaves;
+        const int64_t nkv = (S + NW * kRowsPerWave - 1) / (NW * kRowsPerWave);
+        if (nkv * B * H > INT32_MAX) return fail(CW_ERR_INVALID, "cw_attn_bwd: S or B*H too large");
+        constexpr int lds_bytes = 2 * dkdv_stage_bytes<HS::NP>();
+        auto kern = attn_dkdv_kernel<HS, NW, 1, E>;
         if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)(lds_bytes), "attn_dkdv_kernel"); lrc != CW_OK) return lrc;
-        hipLaunchKernelGGL(kern, dim3((unsigned)(nkv * B * H)), dim3(kDkdvWaves * 64), lds_bytes, s, a);
-    } else {
-        constexpr int lds_bytes = 2 * dkdv_stage_bytes<2>();
-        auto kern = attn_dkdv_kernel<2, kDkdvWaves, 1, E>;
-        if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)(lds_bytes), "attn_dkdv_kernel"); lrc != CW_OK) return lrc;
-        hipLaunchKernelGGL(kern, dim3((unsigned)(nkv * B * H)), dim3(kDkdvWaves * 64), lds_bytes, s, a);
-    }
-    return check_launch("attn_dkdv_kernel");
+        hipLaunchKernelGGL(kern, dim3((unsigned)(nkv * B * H)), dim3(NW * 64), lds_bytes, s, a);
+        return check_launch("attn_dkdv_kernel");
+    });
 }
 
 }  // namespace
@@ -466,34 +466,32 @@ extern "C" int64_t cw_attn_bwd_workspace_bytes(int64_t B, int64_t H, int64_t S) 
     return B * H * S * (int64_t)sizeof(float);
 }
 
-extern "C" int cw_attn_bwd(int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
-                           int64_t stride_b, int64_t stride_s, int64_t stride_h, const void* out, const void* d_out,
-                           int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h, const float* lse,
-                           float scale, int causal, void* dq, void* dk, void* dv, int64_t grad_stride_b,
-                           int64_t grad_stride_s, int64_t grad_stride_h, void* workspace, int64_t workspace_bytes,
-                           int io_dtype, void* stream) {
-    if (B < 0 || H < 0 || S < 0 || D <= 0)
-        return fail(CW_ERR_INVALID, "cw_attn_bwd: bad shape B=%lld H=%lld S=%lld D=%lld", (long long)B, (long long)H, (long long)S, (long long)D);
-    if (io_dtype != CW_BF16 && io_dtype != CW_F16) return fail(CW_ERR_UNSUPPORTED, "cw_attn_bwd: only bf16 and fp16 are provided");
-    if (D != 64 && D != 128) return fail(CW_ERR_UNSUPPORTED, "cw_attn_bwd: head size %lld is not provided (64 and 128)", (long long)D);
+namespace {
+
+int attn_bwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
+             int64_t stride_b, int64_t stride_s, int64_t stride_h, const void* out, const void* d_out,
+             int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h, const float* lse,
+             float scale, int causal, void* dq, void* dk, void* dv, int64_t grad_stride_b,
+             int64_t grad_stride_s, int64_t grad_stride_h, void* workspace, int64_t workspace_bytes,
+             int io_dtype, void* stream) {
     if (B == 0 || H == 0 || S == 0) return CW_OK;
     if (q == nullptr || k == nullptr || v == nullptr || out == nullptr || d_out == nullptr || lse == nullptr ||
         dq == nullptr || dk == nullptr || dv == nullptr || workspace == nullptr)
-        return fail(CW_ERR_INVALID, "cw_attn_bwd: null pointer");
+        return fail(CW_ERR_INVALID, "%s: null pointer", who);
     if (workspace_bytes < cw_attn_bwd_workspace_bytes(B, H, S))
-        return fail(CW_ERR_INVALID, "cw_attn_bwd: workspace too small (%lld bytes)", (long long)workspace_bytes);
+        return fail(CW_ERR_INVALID, "%s: workspace too small (%lld bytes)", who, (long long)workspace_bytes);
     const int64_t nblk = (S + kRowsPerBlock - 1) / kRowsPerBlock;
     if (S > INT32_MAX / 2 || B * H > (1 << 20) || nblk * B * H > INT32_MAX)
-        return fail(CW_ERR_INVALID, "cw_attn_bwd: S or B*H too large");
+        return fail(CW_ERR_INVALID, "%s: S or B*H too large", who);
     const bool aligned = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) && aligned16(d_out) &&
                          stride_b % 8 == 0 && stride_s % 8 == 0 && stride_h % 8 == 0 && out_stride_b % 8 == 0 &&
                          out_stride_s % 8 == 0 && out_stride_h % 8 == 0 &&
                          ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk) | reinterpret_cast<uintptr_t>(dv)) & 7u) == 0 &&
                          grad_stride_b % 4 == 0 && grad_stride_s % 4 == 0 && grad_stride_h % 4 == 0 &&
                          (reinterpret_cast<uintptr_t>(workspace) & 3u) == 0;
-    if (!aligned) return fail(CW_ERR_ALIGNMENT, "cw_attn_bwd: inputs need 16-byte aligned rows, gradients 8-byte aligned rows");
+    if (!aligned) return fail(CW_ERR_ALIGNMENT, "%s: inputs need 16-byte aligned rows, gradients 8-byte aligned rows", who);
     if (stride_s <= 0 || stride_s >= (1 << 23) || out_stride_s <= 0 || out_stride_s >= (1 << 23))
-        return fail(CW_ERR_INVALID, "cw_attn_bwd: token strides %lld / %lld outside (0, 2^23) elements", (long long)stride_s,
+        return fail(CW_ERR_INVALID, "%s: token strides %lld / %lld outside (0, 2^23) elements", who, (long long)stride_s,
                     (long long)out_stride_s);
     BwdArgs a;
     a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v;
@@ -507,7 +505,39 @@ extern "C" int cw_attn_bwd(int64_t B, int64_t H, int64_t S, int64_t D, const voi
     a.scale = scale; a.scale_log2e = scale * kLog2e;
     a.causal = causal ? 1 : 0;
     a.D = (int)D;
-    if (const int drc = require_gfx950("cw_attn_bwd"); drc != CW_OK) return drc;
+    if (const int drc = require_gfx950(who); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
     return io_dtype == CW_F16 ? launch_bwd<f16_t>(a, B, H, S, D, nblk, s) : launch_bwd<bf16_t>(a, B, H, S, D, nblk, s);
+}
+
+}  // namespace
+
+extern "C" int cw_attn_bwd(int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
+                           int64_t stride_b, int64_t stride_s, int64_t stride_h, const void* out, const void* d_out,
+                           int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h, const float* lse,
+                           float scale, int causal, void* dq, void* dk, void* dv, int64_t grad_stride_b,
+                           int64_t grad_stride_s, int64_t grad_stride_h, void* workspace, int64_t workspace_bytes,
+                           int io_dtype, void* stream) {
+    if (B < 0 || H < 0 || S < 0 || D <= 0)
+        return fail(CW_ERR_INVALID, "cw_attn_bwd: bad shape B=%lld H=%lld S=%lld D=%lld", (long long)B, (long long)H, (long long)S, (long long)D);
+    if (io_dtype != CW_BF16 && io_dtype != CW_F16) return fail(CW_ERR_UNSUPPORTED, "cw_attn_bwd: only bf16 and fp16 are provided");
+    if (D != 64 && D != 128) return fail(CW_ERR_UNSUPPORTED, "cw_attn_bwd: head size %lld is not provided (64 and 128)", (long long)D);
+    return attn_bwd("cw_attn_bwd", B, H, S, D, q, k, v, stride_b, stride_s, stride_h, out, d_out, out_stride_b, out_stride_s,
+                    out_stride_h, lse, scale, causal, dq, dk, dv, grad_stride_b, grad_stride_s, grad_stride_h, workspace,
+                    workspace_bytes, io_dtype, stream);
+}
+
+extern "C" int cw_attn_narrow_bwd(int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
+                                  int64_t stride_b, int64_t stride_s, int64_t stride_h, const void* out, const void* d_out,
+                                  int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h, const float* lse,
+                                  float scale, int causal, void* dq, void* dk, void* dv, int64_t grad_stride_b,
+                                  int64_t grad_stride_s, int64_t grad_stride_h, void* workspace, int64_t workspace_bytes,
+                                  int io_dtype, void* stream) {
+    if (B < 0 || H < 0 || S < 0 || D <= 0)
+        return fail(CW_ERR_INVALID, "cw_attn_narrow_bwd: bad shape B=%lld H=%lld S=%lld D=%lld", (long long)B, (long long)H, (long long)S, (long long)D);
+    if (io_dtype != CW_BF16 && io_dtype != CW_F16) return fail(CW_ERR_UNSUPPORTED, "cw_attn_narrow_bwd: only bf16 and fp16 are provided");
+    if (D % 8 != 0 || D > 128) return fail(CW_ERR_UNSUPPORTED, "cw_attn_narrow_bwd: head size %lld is not provided (multiples of 8 up to 128)", (long long)D);
+    return attn_bwd("cw_attn_narrow_bwd", B, H, S, D, q, k, v, stride_b, stride_s, stride_h, out, d_out, out_stride_b, out_stride_s,
+                    out_stride_h, lse, scale, causal, dq, dk, dv, grad_stride_b, grad_stride_s, grad_stride_h, workspace,
+                    workspace_bytes, io_dtype, stream);
 }

@@ -110,14 +110,15 @@ __device__ __forceinline__ float sum_slots(bf16x8_t v, float acc) {
     return acc;
 }
 
-// Lane (row = lane % 32, half = lane / 32) holds, of a transposed 64 x 32 result, the values
-// d = 32 dt + 8 (e / 4) + 4 half + e % 4 of its row: write them, times `mul`, as E.
-template <typename E>
-__device__ __forceinline__ void store_row_pieces(uint16_t* rowp, const f32x16_t* acc, float mul, int half) {
+// Lane (row = lane % 32, half = lane / 32) holds, of a transposed 32 DT x 32 result, the values
+// d = 32 dt + 8 (e / 4) + 4 half + e % 4 of its row: write those below D (MASK; all without), times `mul`, as E.
+template <typename E, int DT, bool MASK>
+__device__ __forceinline__ void store_row_pieces(uint16_t* rowp, const f32x16_t* acc, float mul, int half, int D) {
 #pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
+            if (MASK && 32 * dt + 8 * g >= D) continue;
             const uint2 w = make_uint2(half_conv<E>::pack2(acc[dt][4 * g] * mul, acc[dt][4 * g + 1] * mul),
                                        half_conv<E>::pack2(acc[dt][4 * g + 2] * mul, acc[dt][4 * g + 3] * mul));
             *reinterpret_cast<uint2*>(rowp + 32 * dt + 8 * g + 4 * half) = w;
@@ -169,27 +170,62 @@ struct TileDma {
             wave_off[u] = (uint32_t)__builtin_amdgcn_readfirstlane((p >> 6) * 1024);
         }
     }
-    // Tile rows row0 .. row0+63 of the [S, 64] bf16 matrix at `base` (row stride in elements); rows past
+    // Tile rows row0 .. row0+63 of the [S, cols] 16-bit matrix at `base` (row stride in elements); rows past
     // S read row S-1. row_img / tr_img: LDS byte addresses of the images to fill (ROW_IMAGE / TR_IMAGE
-    // say which are wanted).
-    template <bool ROW_IMAGE, bool TR_IMAGE>
+    // say which are wanted). MASK: columns from `cols` on (a multiple of 8, possibly below 64) are filled with zeros.
+    template <bool ROW_IMAGE, bool TR_IMAGE, bool MASK>
     __device__ __forceinline__ void load(const uint16_t* base, int64_t row_stride, int row0, int S, uint32_t row_img,
-                                         uint32_t tr_img) const {
+                                         uint32_t tr_img, int cols) const {
         const char* g = reinterpret_cast<const char*>(base + (int64_t)row0 * row_stride);
         const int last = S - 1 - row0;
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
             if (ROW_IMAGE) {
                 const int r = row_r[u] < last ? row_r[u] : last;
-                dma16(g, (uint32_t)((r * (int)row_stride + row_c[u] * 8) * 2), row_img + wave_off[u]);
+                const uint32_t voff = (uint32_t)((r * (int)row_stride + row_c[u] * 8) * 2);
+                if constexpr (MASK) dma16_buffer(g, row_c[u] * 8 < cols ? voff : kDmaRange, row_img + wave_off[u]);
+                else dma16(g, voff, row_img + wave_off[u]);
             }
             if (TR_IMAGE) {
                 const int r = tr_r[u] < last ? tr_r[u] : last;
-                dma16(g, (uint32_t)((r * (int)row_stride + tr_c[u] * 8) * 2), tr_img + wave_off[u]);
+                const uint32_t voff = (uint32_t)((r * (int)row_stride + tr_c[u] * 8) * 2);
+                if constexpr (MASK) dma16_buffer(g, tr_c[u] * 8 < cols ? voff : kDmaRange, tr_img + wave_off[u]);
+                else dma16(g, voff, tr_img + wave_off[u]);
             }
         }
     }
 };
+
+// The 8 elements of a row of D that start at column c (a multiple of 8), zeros past D (MASK).
+template <bool MASK>
+__device__ __forceinline__ raw16_t load_cols(const uint16_t* rowp, int c, int D) {
+    if constexpr (!MASK) return load_raw(rowp + c);
+    const raw16_t v = load_raw(rowp + (c < D ? c : 0));
+    const raw16_t zero = {0u, 0u, 0u, 0u};
+    return c < D ? v : zero;
+}
+
+// The kernels' shapes, chosen by head size D (a multiple of 8 up to 128): KB blocks of 16 columns in the products over
+// the head, DT blocks of 32 columns in the results, NP = (KB + 3) / 4 LDS panels of 64 columns. MASK: D is below 64 NP,
+// the tile loader fills the missing columns with zeros and the stores leave them out. Heads of 65 to 80 columns run 5
+// and 3 blocks instead of the 8 and 4 that 128 columns take, those up to 48 run 3 and 2 instead of 4 and 2. Against the
+// zero-padded copies that such heads went through before (and still do in rows that are not 16-byte aligned): 2 x 777
+// tokens, 32 heads of 80: kernels 132 -> 110 us and 46 us of copies gone; 1 x 128 tokens, 16 heads of 48: kernels
+// 27 us both, 20 us of copies and 6 launches gone.
+template <int KB_, int DT_, bool MASK_>
+struct HeadShape {
+    static constexpr int KB = KB_, DT = DT_, NP = (KB_ + 3) / 4;
+    static constexpr bool MASK = MASK_;
+};
+template <typename F>
+int with_head_shape(int64_t D, F&& f) {
+    if (D <= 48) return f(HeadShape<3, 2, true>{});
+    if (D < 64) return f(HeadShape<4, 2, true>{});
+    if (D == 64) return f(HeadShape<4, 2, false>{});
+    if (D <= 80) return f(HeadShape<5, 3, true>{});
+    if (D < 128) return f(HeadShape<8, 4, true>{});
+    return f(HeadShape<8, 4, false>{});
+}
 
 }  // namespace attn
 }  // namespace cw

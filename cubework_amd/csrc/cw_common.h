@@ -217,6 +217,14 @@ __device__ __forceinline__ raw16_t pack_raw(const float (&v)[4], const float*) {
 __device__ __forceinline__ void dma16(const char* gbase, uint32_t voff, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(gbase) : "memory", "m0");
 }
+// The same through a buffer of kDmaRange bytes at `base`: a lane whose offset is kDmaRange itself fetches nothing and the
+// load unit writes 16 zero bytes for it.
+constexpr uint32_t kDmaRange = 0x80000000u;
+__device__ __forceinline__ void dma16_buffer(const char* base, uint32_t voff, uint32_t lds_addr) {
+    const uint64_t b = reinterpret_cast<uint64_t>(base);
+    const raw16_t rsrc = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, kDmaRange, 0x00020000u};
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
+}
 template <int N>
 __device__ __forceinline__ void dma_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");

@@ -10,7 +10,7 @@
 // 1 1/3 rounds of the 768 that fit).
 //
 // Large aligned problems (at least 128 tiles of 256x256) take gemm_f32_ring_kernel instead: the ring of LDS
-// stages filled by the load unit that the 16-bit kernel uses (gemm_bf16_dma.h), with a k extent of 16 per
+// stages filled by the load unit that the 16-bit kernels use (gemm_tile.h), with a k extent of 16 per
 // stage. There is no register staging, no LDS write instruction and no fragment read right behind the
 // barrier, so a wavefront arrives at the one barrier per stage with the next products' operands already
 // in registers.

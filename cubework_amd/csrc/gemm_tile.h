@@ -2,7 +2,7 @@
 //
 //   - BM x BN tile of C per 256-thread block (4 wavefronts, 2x2; a wavefront owns TM x TN MFMA tiles of 32x32, BM = 64 TM,
 //     BN = 64 TN); k tiles of 32 in a ring of NS LDS stages filled by the load unit, one barrier per k tile in the
-//     middle of its MFMAs, fragments read one k step ahead: the pipeline of the large-tile kernel (gemm_bf16_dma.h).
+//     middle of its MFMAs, fragments read one k step ahead: a wavefront arrives at the barrier with the next products' operands in registers.
 //   - Operands are fetched with buffer_load_dwordx4 ... lds. The lane's byte offset goes through the buffer's range
 //     check, and a lane whose 16-byte chunk lies outside the operand (row >= M or N, k >= K) is handed an offset
 //     beyond the range: the load unit writes zeros for it. So edges cost no branch, no second kernel and no memory
@@ -12,7 +12,7 @@
 //     (partial sums through scratch in accumulator order, finished by tile_reduce_kernel): the last, partly empty
 //     round of tiles, or a problem with few tiles and a long reduction, is spread over the whole chip.
 //
-// LDS images per stage as in gemm_bf16_dma.h: k-contiguous operand [BM rows][32 k], chunk c of row r at c ^ ((r >> 2) & 3);
+// LDS images per stage: k-contiguous operand [BM rows][32 k], chunk c of row r at c ^ ((r >> 2) & 3);
 // k-slow operand [32 k][BM rows], chunk c of k row k at c ^ ((k & 3) << 2). Both read conflict free.
 #pragma once
 #include <cstddef>
@@ -53,14 +53,7 @@ typedef __attribute__((address_space(3))) uint16_t lds_u16;
 
 constexpr int kBK = 32;
 constexpr int kThreads = 256;
-constexpr uint32_t kRange = 0x80000000u;  // bytes a lane offset may reach; an offset of kRange itself is out of range
-
-// 64 lanes x 16 bytes of the buffer at `base` (range kRange) into LDS at lds_addr + 16 lane; counted by dma_wait.
-__device__ __forceinline__ void dma16_buffer(const char* base, uint32_t voff, uint32_t lds_addr) {
-    const uint64_t b = reinterpret_cast<uint64_t>(base);
-    const u32x4_t rsrc = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, kRange, 0x00020000u};
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
-}
+constexpr uint32_t kRange = kDmaRange;  // bytes a lane offset may reach; an offset of kRange itself is out of range
 
 constexpr int kTabA = 0, kTabB = CW_MAX_KSTEPS, kTabAddend = 2 * CW_MAX_KSTEPS;  // entries before each table
 static_assert(offsetof(TileArgs, A) == 0 && offsetof(TileArgs, B) == 8 * kTabB && offsetof(TileArgs, addend) == 8 * kTabAddend,

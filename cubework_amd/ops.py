@@ -482,9 +482,10 @@ def _bshd_strides(t: torch.Tensor):
 
 
 def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[float] = None, causal: bool = True,
-             want_lse: bool = False):
+             want_lse: bool = False, narrow: bool = False):
     """softmax(scale q k^T + causal mask) v for [b, s, h, d] views (e.g. slices of the qkv projection's
-    output); returns [b, s, h*d] (and the [b, h, s] log-sum-exp). See cw_attn_fwd."""
+    output); returns [b, s, h*d] (and the [b, h, s] log-sum-exp). See cw_attn_fwd (head sizes 64 and 128) and,
+    with narrow = True, cw_attn_narrow_fwd (multiples of 8 up to 128)."""
     lib = _lib.load()
     _require_device(q, k, v)
     if q.shape != k.shape or q.shape != v.shape or q.dtype != k.dtype or q.dtype != v.dtype:
@@ -496,17 +497,18 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: Optional[
     scale = D ** -0.5 if scale is None else float(scale)
     out = torch.empty((B, S, H, D), dtype=q.dtype, device=q.device)
     lse = torch.empty((B, H, S), dtype=torch.float32, device=q.device) if want_lse else None
-    rc = lib.cw_attn_fwd(B, H, S, D, _p(q), _p(k), _p(v), strides[0], strides[1], strides[2], scale, 1 if causal else 0,
-                         _p(out), out.stride(0), out.stride(1), out.stride(2), _p(lse), _dtype_code(q), _stream())
-    _lib.check(rc, "cw_attn_fwd")
+    name, fn = ("cw_attn_narrow_fwd", lib.cw_attn_narrow_fwd) if narrow else ("cw_attn_fwd", lib.cw_attn_fwd)
+    rc = fn(B, H, S, D, _p(q), _p(k), _p(v), strides[0], strides[1], strides[2], scale, 1 if causal else 0,
+            _p(out), out.stride(0), out.stride(1), out.stride(2), _p(lse), _dtype_code(q), _stream())
+    _lib.check(rc, name)
     out = out.view(B, S, H * D)
     return (out, lse) if want_lse else out
 
 
 def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor, d_out: torch.Tensor,
              lse: torch.Tensor, dq: torch.Tensor, dk: torch.Tensor, dv: torch.Tensor,
-             scale: Optional[float] = None, causal: bool = True) -> None:
-    """Gradients of attn_fwd into the [b, s, h, d] views dq, dk, dv (e.g. slices of one buffer shaped like
+             scale: Optional[float] = None, causal: bool = True, narrow: bool = False) -> None:
+    """Gradients of attn_fwd (narrow as there) into the [b, s, h, d] views dq, dk, dv (e.g. slices of one buffer shaped like
     the qkv projection's output). out / d_out: [b, s, h*d] or [b, s, h, d]. See cw_attn_bwd."""
     lib = _lib.load()
     _require_device(q, k, v, out, d_out, lse, dq, dk, dv)
@@ -525,16 +527,16 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tenso
     scale = D ** -0.5 if scale is None else float(scale)
     ws_bytes = lib.cw_attn_bwd_workspace_bytes(B, H, S)
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
-    rc = lib.cw_attn_bwd(B, H, S, D, _p(q), _p(k), _p(v), strides[0], strides[1], strides[2], _p(out4), _p(dout4),
-                         ostr[0], ostr[1], ostr[2], _p(lse), scale, 1 if causal else 0, _p(dq), _p(dk), _p(dv),
-                         gstrides[0], gstrides[1], gstrides[2], _p(ws), ws.numel(), _dtype_code(q), _stream())
-    _lib.check(rc, "cw_attn_bwd")
+    name, fn = ("cw_attn_narrow_bwd", lib.cw_attn_narrow_bwd) if narrow else ("cw_attn_bwd", lib.cw_attn_bwd)
+    rc = fn(B, H, S, D, _p(q), _p(k), _p(v), strides[0], strides[1], strides[2], _p(out4), _p(dout4),
+            ostr[0], ostr[1], ostr[2], _p(lse), scale, 1 if causal else 0, _p(dq), _p(dk), _p(dv),
+            gstrides[0], gstrides[1], gstrides[2], _p(ws), ws.numel(), _dtype_code(q), _stream())
+    _lib.check(rc, name)
 
 
 def _attn_padded_head(d: int) -> int:
-    """Head size the kernels run at for a model head size d: 64 and 128 are native; smaller ones and those in
-    between (the reference's opt_125m has 768 / 16 = 48, opt_2_7b and opt_13b have 80, benchmark/opt/opt.py:419-495)
-    are zero-padded up - zero columns add nothing to q.k, and the matching output and gradient columns are dropped."""
+    """Head size that a model head size d is zero-padded to where it is padded (see _attn_native) - zero columns add
+    nothing to q.k, and the matching output and gradient columns are dropped; 64 and 128 stay."""
     if d in (64, 128):
         return d
     if 0 < d < 64:
@@ -542,6 +544,14 @@ def _attn_padded_head(d: int) -> int:
     if 64 < d < 128:
         return 128
     raise NotImplementedError("attention_core: head size %d (the kernels cover head sizes up to 128)" % d)
+
+
+def _attn_native(t: torch.Tensor, d: int) -> bool:
+    """Whether the kernels read heads of d columns as they lie in t [b, s, heads, 3*d]: multiples of 8 (the reference's
+    opt_125m has 768 / 16 = 48, opt_2_7b and opt_13b have 80, benchmark/opt/opt.py:419-495) in 16-byte aligned rows.
+    Other sizes below 128 go through a zero-padded copy. 64 and 128 have no other path."""
+    return d in (64, 128) or (d % 8 == 0 and d < 128 and t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0
+                              and t.stride(1) % 8 == 0 and 0 < t.stride(1) < 1 << 23)
 
 
 def _pad_last(t: torch.Tensor, d: int, dp: int) -> torch.Tensor:
@@ -560,13 +570,15 @@ class _AttentionCore(torch.autograd.Function):
         b, s, w = qkv.shape
         d = w // (3 * heads)
         dp = _attn_padded_head(d)
+        qkv = qkv if qkv.stride(-1) == 1 else qkv.contiguous()
+        if _attn_native(qkv, d):
+            dp = d
         if dp != d:
             scale = d ** -0.5 if scale is None else scale  # of the model's head size, not the padded one
             qkv = _pad_last(qkv, d, dp)
-        qkv = qkv if qkv.stride(-1) == 1 else qkv.contiguous()
         t = qkv.view(b, s, heads, 3 * dp) if qkv.is_contiguous() else qkv.reshape(b, s, heads, 3 * dp)
         q, k, v = t[..., :dp], t[..., dp:2 * dp], t[..., 2 * dp:]
-        out, lse = attn_fwd(q, k, v, scale, causal, want_lse=True)
+        out, lse = attn_fwd(q, k, v, scale, causal, want_lse=True, narrow=dp not in (64, 128))
         ctx.save_for_backward(t, out, lse)
         ctx.meta = (heads, d, dp, scale, causal)
         if dp != d:
@@ -580,8 +592,11 @@ class _AttentionCore(torch.autograd.Function):
         b, s = t.shape[0], t.shape[1]
         q, k, v = t[..., :dp], t[..., dp:2 * dp], t[..., 2 * dp:]
         g = torch.empty((b, s, heads, 3 * dp), dtype=t.dtype, device=t.device)
+        narrow = dp not in (64, 128)
         d_out = d_out.contiguous() if dp == d else _pad_last(d_out, d, dp)
-        attn_bwd(q, k, v, out, d_out, lse, g[..., :dp], g[..., dp:2 * dp], g[..., 2 * dp:], scale, causal)
+        if narrow and d_out.data_ptr() % 16 != 0:
+            d_out = d_out.clone()
+        attn_bwd(q, k, v, out, d_out, lse, g[..., :dp], g[..., dp:2 * dp], g[..., 2 * dp:], scale, causal, narrow)
         if dp != d:
             return g.view(b, s, heads, 3, dp)[..., :d].reshape(b, s, heads * 3 * d), None, None, None
         return g.view(b, s, heads * 3 * d), None, None, None

@@ -8,8 +8,8 @@ causal attention -> out Linear -> residual -> LayerNorm -> fc1 -> activation ->
 fc2 -> residual. The four Linears and two LayerNorms are cubework_amd.module
 layers (HIP path). The attention core (scaled QK^T, causal mask, softmax, PV:
 benchmark/opt/opt.py:84-117) is the fused HIP kernel pair cw_attn_fwd /
-cw_attn_bwd for 16-bit inputs and head sizes up to 128 (64 and 128 natively, the 48 of
-opt_125m and the 80 of opt_2_7b / opt_13b zero-padded, benchmark/opt/opt.py:419-495); fp32
+cw_attn_bwd for 16-bit inputs and head sizes up to 128 (multiples of 8, as
+the 48 of opt_125m and the 80 of opt_2_7b / opt_13b, benchmark/opt/opt.py:419-495; others zero-padded); fp32
 inputs or larger heads use torch's scaled_dot_product_attention, as model code would.
 """
 

@@ -496,6 +496,27 @@ int cw_attn_bwd(int64_t B, int64_t H, int64_t S, int64_t D,
                 int64_t grad_stride_b, int64_t grad_stride_s, int64_t grad_stride_h,
                 void* workspace, int64_t workspace_bytes, int io_dtype, void* stream);
 
+/*
+ * cw_attn_fwd / cw_attn_bwd for every head size D that is a multiple of 8 up to 128, at its own width: the reference's
+ * opt_125m has heads of 48, opt_2_7b and opt_13b of 80 (benchmark/opt/opt.py:419-495). Same arguments, alignment and
+ * workspace; scale has to be given as for D itself.
+ */
+int cw_attn_narrow_fwd(int64_t B, int64_t H, int64_t S, int64_t D,
+                       const void* q, const void* k, const void* v,
+                       int64_t stride_b, int64_t stride_s, int64_t stride_h,
+                       float scale, int causal,
+                       void* out, int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h,
+                       float* lse, int io_dtype, void* stream);
+int cw_attn_narrow_bwd(int64_t B, int64_t H, int64_t S, int64_t D,
+                       const void* q, const void* k, const void* v,
+                       int64_t stride_b, int64_t stride_s, int64_t stride_h,
+                       const void* out, const void* d_out,
+                       int64_t out_stride_b, int64_t out_stride_s, int64_t out_stride_h,
+                       const float* lse, float scale, int causal,
+                       void* dq, void* dk, void* dv,
+                       int64_t grad_stride_b, int64_t grad_stride_s, int64_t grad_stride_h,
+                       void* workspace, int64_t workspace_bytes, int io_dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
