@@ -160,6 +160,14 @@ __device__ __forceinline__ raw16_t load_raw_stream(const void* p) {
 __device__ __forceinline__ void store_raw_stream(void* p, raw16_t u) {
     __builtin_nontemporal_store(u, reinterpret_cast<raw16_t*>(p));
 }
+// The same at the alignment of the elements only (global accesses need no more).
+typedef uint32_t raw16_any_t __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ raw16_t load_raw_stream_any(const void* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const raw16_any_t*>(p));
+}
+__device__ __forceinline__ void store_raw_stream_any(void* p, raw16_t u) {
+    __builtin_nontemporal_store(u, reinterpret_cast<raw16_any_t*>(p));
+}
 __device__ __forceinline__ void unpack_raw(raw16_t u, float (&v)[8], const bf16_t*) {
     v[0] = __uint_as_float(u.x << 16);
     v[1] = __uint_as_float(u.x & 0xffff0000u);

@@ -4,6 +4,9 @@
 // the bit-exact target mask / shifted index / gather. backward: recomputes the
 // softmax from the logits and the global (max, sum) and writes the gradient;
 // the logits are never modified.
+// Both are bound by memory. 16-byte accesses serve rows of any alignment (an odd vocabulary puts every row at another
+// offset): 1023 x 50257 bf16, forward 27 us where single elements took 75, backward 41 us for 44; aligned rows
+// (8192 x 12568 bf16, 33 and 69 us, 6 TB/s) run as they did with loads that assumed their alignment.
 #include <type_traits>
 
 #include "cw_common.h"
@@ -90,8 +93,7 @@ __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int6
                                                             const T* __restrict__ logits, int64_t ld,
                                                             const int64_t* __restrict__ targets, int64_t vocab_start,
                                                             float* __restrict__ out_max, float* __restrict__ out_sumexp,
-                                                            float* __restrict__ out_pred, uint8_t* __restrict__ out_mask,
-                                                            int vec_ok) {
+                                                            float* __restrict__ out_pred, uint8_t* __restrict__ out_mask) {
     constexpr int V = elem<T>::kVec;
     __shared__ float red_m[kCeBlock / 64];
     __shared__ float red_s[kCeBlock / 64];
@@ -101,28 +103,24 @@ __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int6
     for (int64_t row = blockIdx.x; row < T_rows; row += gridDim.x) {
         const T* xr = logits + row * ld;
         OnlineLse st{kNegInf, 0.0f, 0.0f};
-        if (vec_ok) {
-            const int64_t nvec = V_cols / V;
-            int64_t i = tid;
-            // kCeUnroll independent 16-byte streaming loads in flight per trip
-            for (; i + (kCeUnroll - 1) * kCeBlock < nvec; i += kCeUnroll * kCeBlock) {
-                raw16_t raw[kCeUnroll];
+        const int64_t nvec = V_cols / V;
+        int64_t i = tid;
+        // kCeUnroll independent 16-byte streaming loads in flight per trip
+        for (; i + (kCeUnroll - 1) * kCeBlock < nvec; i += kCeUnroll * kCeBlock) {
+            raw16_t raw[kCeUnroll];
 #pragma unroll
-                for (int u = 0; u < kCeUnroll; ++u) raw[u] = load_raw_stream(xr + (i + u * kCeBlock) * V);
-                float v[kCeUnroll][V];
+            for (int u = 0; u < kCeUnroll; ++u) raw[u] = load_raw_stream_any(xr + (i + u * kCeBlock) * V);
+            float v[kCeUnroll][V];
 #pragma unroll
-                for (int u = 0; u < kCeUnroll; ++u) unpack_raw(raw[u], v[u], (const T*)nullptr);
-                lse_add_chunks<V, kCeUnroll>(st, v);
-            }
-            for (; i < nvec; i += kCeBlock) {
-                float v0[V];
-                unpack_raw(load_raw_stream(xr + i * V), v0, (const T*)nullptr);
-                lse_add_chunk<V>(st, v0);
-            }
-            for (int64_t c = nvec * V + tid; c < V_cols; c += kCeBlock) lse_add_one(st, load_elem(xr + c));
-        } else {
-            for (int64_t c = tid; c < V_cols; c += kCeBlock) lse_add_one(st, load_elem(xr + c));
+            for (int u = 0; u < kCeUnroll; ++u) unpack_raw(raw[u], v[u], (const T*)nullptr);
+            lse_add_chunks<V, kCeUnroll>(st, v);
         }
+        for (; i < nvec; i += kCeBlock) {
+            float v0[V];
+            unpack_raw(load_raw_stream_any(xr + i * V), v0, (const T*)nullptr);
+            lse_add_chunk<V>(st, v0);
+        }
+        for (int64_t c = nvec * V + tid; c < V_cols; c += kCeBlock) lse_add_one(st, load_elem(xr + c));
         // wavefront, then block
         float m = st.m, s = st.s;
 #pragma unroll
@@ -180,19 +178,19 @@ __global__ __launch_bounds__(256) void vpce_finalize_kernel(int64_t T_rows, int 
 template <int V>
 __device__ __forceinline__ void store_grad(bf16_t* p, const float (&v)[V]) {
     static_assert(V == 8, "bf16 gradients are written 8 at a time");
-    store_raw_stream(p, pack_raw(v, (const bf16_t*)nullptr));
+    store_raw_stream_any(p, pack_raw(v, (const bf16_t*)nullptr));
 }
 template <int V>
 __device__ __forceinline__ void store_grad(f16_t* p, const float (&v)[V]) {
     static_assert(V == 8, "fp16 gradients are written 8 at a time");
-    store_raw_stream(p, pack_raw(v, (const f16_t*)nullptr));
+    store_raw_stream_any(p, pack_raw(v, (const f16_t*)nullptr));
 }
 template <int V>
 __device__ __forceinline__ void store_grad(float* p, const float (&v)[V]) {
 #pragma unroll
     for (int e = 0; e < V; e += 4) {
         const float q[4] = {v[e], v[e + 1], v[e + 2], v[e + 3]};
-        store_raw_stream(p + e, pack_raw(q, (const float*)nullptr));
+        store_raw_stream_any(p + e, pack_raw(q, (const float*)nullptr));
     }
 }
 
@@ -217,6 +215,7 @@ __device__ __forceinline__ void grad_vector(raw16_t raw, int64_t i, int64_t tcol
 // stores of one instruction cover one contiguous 1 KB span. With 16-byte loads a lane would write 32
 // bytes in two stores that each leave every other 16 bytes to the next instruction.
 typedef uint32_t raw8_t __attribute__((ext_vector_type(2)));
+typedef uint32_t raw8_any_t __attribute__((ext_vector_type(2), aligned(2)));
 template <typename T>
 __device__ __forceinline__ void grad_quad(raw8_t raw, int64_t i, int64_t tcol, float m2, float scale, float dl,
                                           float* __restrict__ gr) {
@@ -229,7 +228,7 @@ __device__ __forceinline__ void grad_quad(raw8_t raw, int64_t i, int64_t tcol, f
         for (int e = 0; e < 4; ++e)
             if (e == rel) v[e] -= dl;
     }
-    store_raw_stream(gr + i * 4, pack_raw(v, (const float*)nullptr));
+    store_raw_stream_any(gr + i * 4, pack_raw(v, (const float*)nullptr));
 }
 
 // Per-row scalars of the backward: fetched after the row's first loads have been issued.
@@ -258,7 +257,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                                                                const float* __restrict__ gmax,
                                                                const float* __restrict__ gsum,
                                                                const float* __restrict__ dloss_rows, float dloss_scale,
-                                                               G* __restrict__ grad, int64_t ld_grad, int vec_ok) {
+                                                               G* __restrict__ grad, int64_t ld_grad) {
     constexpr int V = elem<T>::kVec;
     constexpr int B = kCeBwdBlock;
     const int tid = threadIdx.x;
@@ -266,7 +265,6 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
         const T* xr = logits + row * ld;
         G* gr = grad + row * ld_grad;
         if constexpr (sizeof(T) == 2 && std::is_same<G, float>::value) {
-          if (vec_ok) {
             // fp32 gradient of 16-bit logits: batches of U quads (8 bytes in, 16 out) per thread, all requested
             // before the first is worked on; a position past the end of the row re-reads the last quad (no
             // load under a branch) and stores nothing
@@ -280,7 +278,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const int64_t i = base + (int64_t)u * B;
-                    raw[u] = __builtin_nontemporal_load(reinterpret_cast<const raw8_t*>(xb + (i < nq ? i : nq - 1) * 4));
+                    raw[u] = __builtin_nontemporal_load(reinterpret_cast<const raw8_any_t*>(xb + (i < nq ? i : nq - 1) * 4));
                 }
                 if (base == tid) rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
 #pragma unroll
@@ -297,10 +295,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                     store_elem(gr + c, y);
                 }
             }
-            continue;
-          }
-        }
-        if (vec_ok) {
+        } else {
             const int64_t nvec = V_cols / V;
             CeRowScalars rs;
             if constexpr (sizeof(T) == 2) {
@@ -308,7 +303,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                 // per compute unit keep enough loads in flight; batching loads per thread measured slower here.
                 rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
                 for (int64_t i = tid; i < nvec; i += B)
-                    grad_vector<T, G, V>(load_raw_stream(xr + i * V), i, rs.tcol, rs.m2, rs.scale, rs.dl, gr);
+                    grad_vector<T, G, V>(load_raw_stream_any(xr + i * V), i, rs.tcol, rs.m2, rs.scale, rs.dl, gr);
             } else {
                 constexpr int U = 4;  // 16-byte vectors per thread and batch
                 for (int64_t base = tid; base < nvec; base += (int64_t)U * B) {
@@ -316,7 +311,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
                         const int64_t i = base + (int64_t)u * B;
-                        raw[u] = load_raw_stream(xr + (i < nvec ? i : nvec - 1) * V);
+                        raw[u] = load_raw_stream_any(xr + (i < nvec ? i : nvec - 1) * V);
                     }
                     if (base == tid) rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
 #pragma unroll
@@ -334,13 +329,6 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                     store_elem(gr + c, y);
                 }
             }
-        } else {
-            const CeRowScalars rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
-            for (int64_t c = tid; c < V_cols; c += B) {
-                float y = __builtin_amdgcn_exp2f(__builtin_fmaf(load_elem(xr + c), kLog2e, -rs.m2)) * rs.scale;
-                if (c == rs.tcol) y -= rs.dl;
-                store_elem(gr + c, y);
-            }
         }
     }
 }
@@ -354,11 +342,9 @@ template <typename T, typename G>
 int bwd_impl(int64_t T_rows, int64_t V_cols, const void* logits, int64_t ld, const int64_t* targets,
              int64_t vocab_start, const float* gmax, const float* gsum, const float* dloss_rows, float dloss_scale,
              void* grad, int64_t ld_grad, hipStream_t s) {
-    const int vec_ok = aligned16(logits) && (ld % elem<T>::kVec) == 0 && aligned16(grad) &&
-                       (ld_grad % (16 / (int)sizeof(G))) == 0;
     hipLaunchKernelGGL((vpce_bwd_kernel<T, G>), dim3(ce_grid(T_rows)), dim3(kCeBwdBlock), 0, s, T_rows, V_cols,
                        (const T*)logits, ld, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale, (G*)grad,
-                       ld_grad, vec_ok);
+                       ld_grad);
     return check_launch("vpce_bwd_kernel");
 }
 
@@ -380,23 +366,12 @@ extern "C" int cw_vpce_fwd_local(int64_t T, int64_t V, const void* logits, int64
         return fail(CW_ERR_INVALID, "cw_vpce_fwd_local: null pointer or ld < V");
     if (const int drc = require_gfx950("cw_vpce_fwd_local"); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
-    if (io_dtype == CW_BF16) {
-        const int vec_ok = aligned16(logits) && (ld % 8) == 0;
-        hipLaunchKernelGGL(vpce_fwd_kernel<bf16_t>, dim3(ce_grid(T)), dim3(kCeBlock), 0, s, T, V,
-                           (const bf16_t*)logits, ld, targets, vocab_start, out_max, out_sumexp, out_pred, out_mask,
-                           vec_ok);
-    } else if (io_dtype == CW_F16) {
-        const int vec_ok = aligned16(logits) && (ld % 8) == 0;
-        hipLaunchKernelGGL(vpce_fwd_kernel<f16_t>, dim3(ce_grid(T)), dim3(kCeBlock), 0, s, T, V,
-                           (const f16_t*)logits, ld, targets, vocab_start, out_max, out_sumexp, out_pred, out_mask,
-                           vec_ok);
-    } else {
-        const int vec_ok = aligned16(logits) && (ld % 4) == 0;
-        hipLaunchKernelGGL(vpce_fwd_kernel<float>, dim3(ce_grid(T)), dim3(kCeBlock), 0, s, T, V,
-                           (const float*)logits, ld, targets, vocab_start, out_max, out_sumexp, out_pred, out_mask,
-                           vec_ok);
-    }
-    return check_launch("vpce_fwd_kernel");
+    return with_elem_type(io_dtype, [&](auto* tag) {
+        using E = std::remove_pointer_t<decltype(tag)>;
+        hipLaunchKernelGGL(vpce_fwd_kernel<E>, dim3(ce_grid(T)), dim3(kCeBlock), 0, s, T, V, (const E*)logits, ld, targets,
+                           vocab_start, out_max, out_sumexp, out_pred, out_mask);
+        return check_launch("vpce_fwd_kernel");
+    });
 }
 
 extern "C" int cw_vpce_finalize(int64_t T, int n_ranks, const float* max_all, const float* sumexp_all,

@@ -33,15 +33,19 @@ class _VocabParallelCrossEntropy(torch.autograd.Function):
             stacked = [torch.cat([s.unsqueeze(0), p.to(s.dtype).reshape(-1, s.numel())]) for s, p in zip(local, peers)]
         loss, gmax, gsum = ops.vpce_finalize(*stacked)
         ctx.save_for_backward(logits_2d, targets.reshape(-1), gmax, gsum)
-        ctx.meta = (vocab_start, logits.shape)
+        # Logits that a layer made: their gradient goes to that layer's two products, which read 16-byte aligned rows in
+        # place and copy others first (1023 x 50257 bf16: 2 x 33 us). The gradient of a leaf stays contiguous, as
+        # autograd would otherwise copy it into the leaf's layout.
+        ctx.meta = (vocab_start, logits.shape, logits.grad_fn is not None)
         return loss.reshape(targets.shape)
 
     @staticmethod
     @bwd()
     def backward(ctx, output_grad):
         logits_2d, targets, gmax, gsum = ctx.saved_tensors
-        vocab_start, shape = ctx.meta
-        grad = ops.vpce_bwd(logits_2d, targets, vocab_start, gmax, gsum, output_grad.reshape(-1).float(), 1.0)
+        vocab_start, shape, aligned_rows = ctx.meta
+        grad = ops.vpce_bwd(logits_2d, targets, vocab_start, gmax, gsum, output_grad.reshape(-1).float(), 1.0,
+                            aligned_rows=aligned_rows)
         return grad.reshape(shape), None, None
 
 

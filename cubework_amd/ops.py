@@ -454,7 +454,9 @@ def vpce_finalize(max_all: torch.Tensor, sumexp_all: torch.Tensor, pred_all: tor
 
 def vpce_bwd(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, gmax: torch.Tensor, gsum: torch.Tensor,
              dloss_rows: Optional[torch.Tensor] = None, dloss_scale: float = 1.0,
-             grad_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+             grad_dtype: Optional[torch.dtype] = None, aligned_rows: bool = False) -> torch.Tensor:
+    """Gradient of the logits slice, contiguous; with aligned_rows = True its rows begin at multiples of 16 bytes whatever
+    their length (a view of a buffer with longer rows), as the GEMMs read them without a copy."""
     lib = _lib.load()
     shape = logits.shape
     logits = _rows(logits)
@@ -462,7 +464,10 @@ def vpce_bwd(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, gmax
     T, V = logits.shape
     targets = targets.reshape(-1).to(torch.int64).contiguous()
     grad_dtype = grad_dtype or logits.dtype
-    grad = torch.empty((T, V), dtype=grad_dtype, device=logits.device)
+    ld = -(-V * grad_dtype.itemsize // 16) * 16 // grad_dtype.itemsize if aligned_rows else V
+    grad = torch.empty((T, ld), dtype=grad_dtype, device=logits.device)
+    if ld != V:
+        grad = grad[:, :V]
     if dloss_rows is not None:
         dloss_rows = dloss_rows.reshape(-1).to(torch.float32).contiguous()
     rc = lib.cw_vpce_bwd(T, V, _p(logits), _ld(logits), _p(targets), vocab_start, _p(gmax), _p(gsum), _p(dloss_rows),

@@ -1,0 +1,74 @@
+"""Vocab-parallel cross-entropy over rows of any alignment: row lengths around the vector and batch sizes, pitches and
+start addresses that put every row at another offset, gradients with padded rows; against the oracle in float64."""
+import pytest
+import torch
+
+from tests.util import assert_parity, randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _place(t, pitch, start):
+    """t [T, V] on the device with the given row pitch, `start` elements into its buffer, NaN around it."""
+    T, V = t.shape
+    buf = torch.full((start + T * pitch,), float("nan"), dtype=t.dtype, device=DEV)
+    view = buf[start:].view(T, pitch)[:, :V]
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("V", [1, 3, 7, 8, 9, 250, 2047, 6145, 8195, 12571])
+@pytest.mark.parametrize("dtype,grad_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
+                                              (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("extra,start", [(0, 0), (1, 0), (0, 1), (2, 3)])
+def test_rows_of_any_alignment(V, dtype, grad_dtype, extra, start):
+    import oracle
+    from cubework_amd import ops
+
+    T = 5
+    x = randn((T, V), dtype, seed=V, std=2.0)
+    t = torch.tensor([V, V + V - 1, 0, V + V // 2, 2 * V])  # first, last, before, inside, past the slice
+    dl = torch.linspace(0.5, 1.5, T)
+    view = _place(x, V + extra, start)
+    got = ops.vpce_fwd_local(view, t.to(DEV), V)
+    loss, gmax, gsum = ops.vpce_finalize(*(g.unsqueeze(0) for g in got))
+    grads = [ops.vpce_bwd(view, t.to(DEV), V, gmax, gsum, dl.to(DEV), 1.0, grad_dtype=grad_dtype, aligned_rows=a) for a in (False, True)]
+    with oracle.precision(torch.float64):
+        want = oracle.vpce_fwd_local(x, t, V)
+        want_grad = oracle.vpce_bwd(x, t, V, gmax.cpu(), gsum.cpu(), dl)
+    what = "V=%d %s extra=%d start=%d" % (V, dtype, extra, start)
+    assert torch.equal(got[0].cpu(), want[0].float()) and torch.equal(got[2].cpu(), want[2].float())
+    assert torch.equal(got[3].cpu(), want[3])
+    assert_parity(got[1], want[1], torch.float32, "sum exp " + what)
+    assert grads[0].is_contiguous() and torch.equal(grads[0], grads[1])
+    assert T == 1 or grads[1].stride(0) * grads[1].element_size() % 16 == 0
+    assert_parity(grads[0], want_grad, grad_dtype, "gradient " + what)
+
+
+@pytest.mark.parametrize("V", [1001, 1000])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_head_gradients_with_padded_rows(V, dtype):
+    """The classifier's two gradient products read the loss's gradient with padded rows: against a contiguous copy."""
+    from cubework_amd.distributed import initialize
+    from cubework_amd.module.loss import VocabParallelCrossEntropyLoss1D
+    from cubework_amd.module.parallel_1d import VocabParallelClassifier1D
+
+    initialize("1d", 1)
+    with torch.device(DEV):
+        layer = VocabParallelClassifier1D(96, V, bias=True).to(dtype)
+    loss_fn = VocabParallelCrossEntropyLoss1D()
+    targets = torch.randint(0, V, (2, 61), generator=torch.Generator().manual_seed(1)).to(DEV)
+    results = []
+    for contiguous in (False, True):
+        x = randn((2, 61, 96), dtype, seed=2).to(DEV).requires_grad_(True)
+        layer.zero_grad()
+        logits = layer(x)
+        if contiguous:
+            logits.register_hook(lambda g: g.contiguous())
+        loss_fn(logits, targets).backward()
+        results.append([x.grad] + [p.grad.clone() for p in layer.parameters()])
+    for got, want in zip(*results):
+        # the same products from other addresses: the 16-bit kernel copies unaligned rows and multiplies the same values,
+        # the fp32 one may take another kernel and so another order of its sums
+        assert_parity(got, want.cpu(), dtype, "head gradient V=%d" % V)
