@@ -26,6 +26,7 @@ CPU path (torch, gloo, world size 1) restated by oracle/ on the host cores, on
 a bounded sample of the same workload.
 """
 import argparse
+import ctypes
 import json
 import os
 import sys
@@ -679,12 +680,17 @@ def bench_other_configs(device, sets):
     timer = AbiCallTimer(real_lib)
     passes = 5
     _cw_lib._lib = timer
+    # the native operator calls reach the timer through callbacks
+    host = _cw_lib.host()
+    callbacks = {n: ctypes.CFUNCTYPE(_cw_lib.SIGNATURES[n][0], *_cw_lib.SIGNATURES[n][1])(getattr(timer, n)) for n in _cw_lib.HOST_ENTRIES}
+    _cw_lib.bind_host(host, callbacks)
     try:
         for _ in range(passes):
             block_step()
         torch.cuda.synchronize()
     finally:
         _cw_lib._lib = real_lib
+        _cw_lib.bind_host(host, {n: getattr(real_lib, n) for n in _cw_lib.HOST_ENTRIES})
     per_kernel = timer.table(passes, us)
     in_calls = sum(r["us_per_step"] for r in per_kernel)
     per_kernel.append({"entry_point": "(torch kernels and gaps between the calls)", "shape": "", "calls_per_step": None,

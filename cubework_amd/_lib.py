@@ -83,6 +83,9 @@ SIGNATURES = {
 _lib = None
 
 
+_host = None
+
+
 class CubeworkHipError(RuntimeError):
     """A C-ABI call returned a non-zero status."""
 
@@ -103,6 +106,32 @@ def load():
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+#: entry points that the native operator calls (csrc/host_ops.cpp) use
+HOST_ENTRIES = ("cw_gemm_scratch_bytes", "cw_gemm_ksteps_ws", "cw_colsum_workspace_bytes", "cw_colsum", "cw_act_bwd_colsum",
+                "cw_ln_partial_stats", "cw_ln_normalize", "cw_ln_forward_fused", "cw_ln_backward_fused",
+                "cw_ln_bwd_partials_open", "cw_ln_bwd_dx_close")
+
+
+def host():
+    """The native operator calls, bound to the loaded library (once)."""
+    global _host
+    if _host is None:
+        lib = load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise ImportError("cubework_amd/_host.so is not built or does not load (%s). Run `python -m cubework_amd.build`; "
+                              "there is no fallback." % e) from e
+        bind_host(module, {name: getattr(lib, name) for name in HOST_ENTRIES})
+        _host = module
+    return _host
+
+
+def bind_host(module, functions):
+    """Have the native operator calls use these ctypes functions (or callbacks) for the entry points."""
+    module.bind({name: ctypes.cast(fn, ctypes.c_void_p).value for name, fn in functions.items()})
 
 
 def check(status, what):

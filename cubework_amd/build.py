@@ -1,7 +1,7 @@
-"""Build libcubework_hip.so (the gfx950 kernels + C ABI) and libcubework_diag.so (measurement aids that only
-bench.py and their tests load) in-tree with hipcc.
+"""Build libcubework_hip.so (the gfx950 kernels + C ABI), libcubework_diag.so (measurement aids that only
+bench.py and their tests load) with hipcc and _host.so (the operators' native host side) with g++, in-tree.
 
-    python -m cubework_amd.build          # compile every source, link both
+    python -m cubework_amd.build          # compile every source, link all three
 
 hipcc cross-compiles for gfx950 without a GPU. The libraries are written next to
 this file so that they travel with the source tree.
@@ -25,6 +25,10 @@ SOURCES = TILE_OBJECTS + [  # slowest first
 # the measurement library: its own kernels plus the runtime services (error text, device check), nothing else
 DIAG_SOURCES = ["diag_gemm.hip", "diag.hip"]
 DIAG_LIB_PATH = os.path.join(HERE, "libcubework_diag.so")
+
+# the operators' native host side: a Python extension on torch's C++ API
+HOST_SOURCE = "host_ops.cpp"
+HOST_PATH = os.path.join(HERE, "_host.so")
 
 # Packed-fp32 VALU forms are kept off: plain float code only.
 HIPCC_FLAGS = [
@@ -56,6 +60,28 @@ def _compile(src, extra=(), obj_dir=None):
     return obj
 
 
+def build_host(verbose=True):
+    """Compile and link the host extension (host compiler only; it holds no device code)."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    include = [os.path.join(os.path.dirname(HERE), "include"), os.path.join(root, "include"),
+               os.path.join(root, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    tmp = HOST_PATH + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_host",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, *["-I" + d for d in include],
+           os.path.join(CSRC, HOST_SOURCE), "-o", tmp, "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+           "-ltorch_python"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("host extension failed:\n%s\n%s" % (proc.stdout, proc.stderr))
+    os.replace(tmp, HOST_PATH)
+    if verbose:
+        print("built", HOST_PATH, os.path.getsize(HOST_PATH), "bytes")
+
+
 def build(verbose=True, extra_flags=(), lib_path=None, obj_dir=None):
     """Compile every HIP source for gfx950 and link the shared library.
     extra_flags / lib_path / obj_dir build a variant beside the default one."""
@@ -63,7 +89,10 @@ def build(verbose=True, extra_flags=(), lib_path=None, obj_dir=None):
     obj_dir = obj_dir or OBJ_DIR
     os.makedirs(obj_dir, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+        host = pool.submit(build_host, verbose) if lib_path == LIB_PATH else None
         objs = list(pool.map(lambda src: _compile(src, extra_flags, obj_dir), SOURCES + DIAG_SOURCES))
+    if host is not None:
+        host.result()
     by_src = dict(zip(SOURCES + DIAG_SOURCES, objs))
 
     def link(members, path):

@@ -89,64 +89,10 @@ def gemm_ksteps(layout: str, A_steps: Sequence[torch.Tensor], B_steps: Sequence[
     layout "NN": A_i [M,K], B_i [K,N];  "NT": A_i [M,K], B_i [N,K];  "TN": A_i [K,M], B_i [K,N].
     Returns C, or (C, preact) when want_preact.
     """
-    lib = _lib.load()
-    if len(A_steps) != len(B_steps) or len(A_steps) == 0:
-        raise ValueError("need the same, non-zero number of A and B step operands")
-    A_steps = [_rows(a) for a in A_steps]
-    B_steps = [_rows(b) for b in B_steps]
-    _require_device(*A_steps, *B_steps, bias, *addends)
-    a0, b0 = A_steps[0], B_steps[0]
-    dt = _dtype_code(a0)
-    if layout == "NN":
-        M, K, N, Kb = a0.shape[0], a0.shape[1], b0.shape[1], b0.shape[0]
-    elif layout == "NT":
-        M, K, N, Kb = a0.shape[0], a0.shape[1], b0.shape[0], b0.shape[1]
-    elif layout == "TN":
-        M, K, N, Kb = a0.shape[1], a0.shape[0], b0.shape[1], b0.shape[0]
-    else:
+    if layout not in LAYOUTS:
         raise ValueError("layout must be NN, NT or TN")
-    if K != Kb:
-        raise ValueError("reduction sizes differ: A %s, B %s for %s" % (tuple(a0.shape), tuple(b0.shape), layout))
-    for t in list(A_steps) + list(B_steps):
-        if t.dtype != a0.dtype:
-            raise TypeError("all GEMM operands must share one dtype")
-    lda, ldb = _ld(a0), _ld(b0)
-    for a in A_steps:
-        if a.shape != a0.shape or _ld(a) != lda:
-            raise ValueError("A step operands must share shape and leading dimension")
-    for b in B_steps:
-        if b.shape != b0.shape or _ld(b) != ldb:
-            raise ValueError("B step operands must share shape and leading dimension")
-    if bias is not None:
-        if bias.numel() != N:
-            raise ValueError("bias has %d elements, output width is %d" % (bias.numel(), N))
-        bias = bias.to(a0.dtype).contiguous()
-    addends = [_rows(t) for t in addends]
-    for t in addends:
-        if tuple(t.shape) != (M, N) or t.dtype != a0.dtype:
-            raise ValueError("addends must be [M,N] of the operand dtype")
-    ldadd = _ld(addends[0]) if addends else 0
-    # the C ABI takes one leading dimension for all addends: copy those that are laid out differently
-    addends = [t if _ld(t) == ldadd else t.contiguous() for t in addends]
-    if any(_ld(t) != ldadd for t in addends):
-        ldadd = N
-        addends = [t.contiguous() for t in addends]
-    if out is None:
-        out = torch.empty((M, N), dtype=a0.dtype, device=a0.device)
-    elif tuple(out.shape) != (M, N) or out.dtype != a0.dtype or out.stride(1) != 1:
-        raise ValueError("out must be a row-major [M,N] tensor of the operand dtype")
-    preact = torch.empty((M, N), dtype=a0.dtype, device=a0.device) if want_preact else None
-    epi = epilogue_code(bias is not None, activation)
-    ta, tb, tadd = _ptr_table(A_steps), _ptr_table(B_steps), _ptr_table(addends)
-    # scratch for tiles cut along k and for copies of operands with unaligned rows
-    ws_bytes = lib.cw_gemm_scratch_bytes(LAYOUTS[layout], M, N, K, len(A_steps), lda, ldb, all(a.data_ptr() % 16 == 0 for a in A_steps),
-                                         all(b.data_ptr() % 16 == 0 for b in B_steps),
-                                         len(addends) if ldadd % 8 or any(t.data_ptr() % 16 for t in addends) else 0, dt)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a0.device) if ws_bytes > 0 else None
-    rc = lib.cw_gemm_ksteps_ws(LAYOUTS[layout], M, N, K, len(A_steps), ta, lda, tb, ldb, _p(bias), epi, _p(out),
-                               _ld(out), _p(preact), _ld(preact) if preact is not None else 0, tadd, len(addends),
-                               ldadd, _p(ws), ws_bytes, dt, _stream())
-    _lib.check(rc, "cw_gemm_ksteps_ws")
+    out, preact = _lib.host().gemm_ksteps(LAYOUTS[layout], A_steps, B_steps, bias, epilogue_code(bias is not None, activation),
+                                          addends, want_preact, out)
     return (out, preact) if want_preact else out
 
 
@@ -188,37 +134,13 @@ _TORCH_CODE = {torch.float32: CW_F32, torch.bfloat16: CW_BF16, torch.float16: CW
 
 def colsum(dy: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """Column sums of a [M,N] tensor (bias gradient): fp32 sums, stored as out_dtype (default float32)."""
-    lib = _lib.load()
-    dy = _rows(dy)
-    _require_device(dy)
-    M, N = dy.shape
-    out_dtype = _out_dtype(out_dtype)
-    out = torch.empty(N, dtype=out_dtype, device=dy.device)
-    ws = _workspace(M, N, dy.device)
-    rc = lib.cw_colsum(M, N, _p(dy), _ld(dy), _p(out), _TORCH_CODE[out_dtype], _p(ws), ws.numel(), _dtype_code(dy),
-                       _stream())
-    _lib.check(rc, "cw_colsum")
-    return out
+    return _lib.host().colsum(dy, out_dtype)
 
 
 def act_bwd_colsum(activation: Optional[str], dy: torch.Tensor, preact: torch.Tensor, want_dbias: bool = True,
                    out_dtype: Optional[torch.dtype] = None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """dPre = dy * act'(preact) and (optionally) its column sums (fp32 sums stored as out_dtype, default float32)."""
-    lib = _lib.load()
-    dy, preact = _rows(dy), _rows(preact)
-    _require_device(dy, preact)
-    if dy.shape != preact.shape or dy.dtype != preact.dtype:
-        raise ValueError("dy and preact must agree in shape and dtype")
-    M, N = dy.shape
-    dpre = torch.empty((M, N), dtype=dy.dtype, device=dy.device)
-    out_dtype = _out_dtype(out_dtype)
-    dbias = torch.empty(N, dtype=out_dtype, device=dy.device) if want_dbias else None
-    ws = _workspace(M, N, dy.device) if want_dbias else None
-    rc = lib.cw_act_bwd_colsum(ACTIVATIONS[activation], M, N, _p(dy), _ld(dy), _p(preact), _ld(preact), _p(dpre),
-                               _ld(dpre), _p(dbias), _TORCH_CODE[out_dtype], _p(ws), ws.numel() if ws is not None else 0,
-                               _dtype_code(dy), _stream())
-    _lib.check(rc, "cw_act_bwd_colsum")
-    return dpre, dbias
+    return _lib.host().act_bwd_colsum(ACTIVATIONS[activation], dy, preact, want_dbias, out_dtype)
 
 
 # --------------------------------------------------------------------------
@@ -226,59 +148,20 @@ def act_bwd_colsum(activation: Optional[str], dy: torch.Tensor, preact: torch.Te
 # --------------------------------------------------------------------------
 def ln_partial_stats(x: torch.Tensor, mode: int = CW_LN_ONE_PASS, mean: Optional[torch.Tensor] = None) -> torch.Tensor:
     """[R,2] fp32 partial statistics of the local columns of x [R,C]."""
-    lib = _lib.load()
-    x = _rows(x)
-    _require_device(x, mean)
-    R, C = x.shape
-    stats = torch.empty((R, 2), dtype=torch.float32, device=x.device)
-    if mean is not None:
-        mean = mean.reshape(-1).to(torch.float32).contiguous()
-        if mean.numel() != R:
-            raise ValueError("mean must have one entry per row")
-    rc = lib.cw_ln_partial_stats(R, C, _p(x), _ld(x), mode, _p(mean), _p(stats), _dtype_code(x), _stream())
-    _lib.check(rc, "cw_ln_partial_stats")
-    return stats
+    return _lib.host().ln_partial_stats(x, mode, mean)
 
 
 def ln_normalize(x: torch.Tensor, stats: torch.Tensor, hidden: int, eps: float,
                  gamma: Optional[torch.Tensor] = None, beta: Optional[torch.Tensor] = None,
                  mode: int = CW_LN_ONE_PASS, save_mean_rstd: bool = True):
     """y = gamma*(x-mean)*rstd+beta from whole-hidden-size stats; returns (y, mean_rstd)."""
-    lib = _lib.load()
-    shape = x.shape
-    x = _rows(x)
-    _require_device(x, stats, gamma, beta)
-    R, C = x.shape
-    stats = stats.reshape(R, 2).to(torch.float32).contiguous()
-    gamma = None if gamma is None else gamma.to(x.dtype).contiguous()
-    beta = None if beta is None else beta.to(x.dtype).contiguous()
-    for v in (gamma, beta):
-        if v is not None and v.numel() != C:
-            raise ValueError("gamma/beta must have C elements")
-    y = torch.empty((R, C), dtype=x.dtype, device=x.device)
-    mr = torch.empty((R, 2), dtype=torch.float32, device=x.device) if save_mean_rstd else None
-    rc = lib.cw_ln_normalize(R, C, _p(x), _ld(x), _p(stats), mode, hidden, eps, _p(gamma), _p(beta), _p(y), _ld(y),
-                             _p(mr), _dtype_code(x), _stream())
-    _lib.check(rc, "cw_ln_normalize")
-    return y.reshape(shape), mr
+    return _lib.host().ln_forward(x, stats, hidden, eps, gamma, beta, mode, save_mean_rstd)
 
 
 def ln_forward_fused(x: torch.Tensor, eps: float, gamma: Optional[torch.Tensor] = None,
                      beta: Optional[torch.Tensor] = None, mode: int = CW_LN_ONE_PASS, save_mean_rstd: bool = True):
     """LayerNorm over the last dimension when this rank holds the whole hidden size."""
-    lib = _lib.load()
-    shape = x.shape
-    x = _rows(x)
-    _require_device(x, gamma, beta)
-    R, C = x.shape
-    gamma = None if gamma is None else gamma.to(x.dtype).contiguous()
-    beta = None if beta is None else beta.to(x.dtype).contiguous()
-    y = torch.empty((R, C), dtype=x.dtype, device=x.device)
-    mr = torch.empty((R, 2), dtype=torch.float32, device=x.device) if save_mean_rstd else None
-    rc = lib.cw_ln_forward_fused(R, C, _p(x), _ld(x), mode, eps, _p(gamma), _p(beta), _p(y), _ld(y), _p(mr),
-                                 _dtype_code(x), _stream())
-    _lib.check(rc, "cw_ln_forward_fused")
-    return y.reshape(shape), mr
+    return _lib.host().ln_forward(x, None, 0, eps, gamma, beta, mode, save_mean_rstd)
 
 
 def ln_bwd_partials(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor,
@@ -327,44 +210,16 @@ def ln_bwd_partials_open(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Ten
                          gamma: Optional[torch.Tensor] = None):
     """Row sums [R,2] fp32 now, the parameter gradients later: returns (row_sums, pending), where `pending`
     goes to ln_bwd_dx_close after the row sums have been summed over the ranks. See cw_ln_bwd_partials_open."""
-    lib = _lib.load()
-    dy, x = _rows(dy), _rows(x)
-    _require_device(dy, x, mean_rstd, gamma)
-    if dy.shape != x.shape or dy.dtype != x.dtype:
-        raise ValueError("dy and x must agree in shape and dtype")
-    R, C = x.shape
-    gamma = None if gamma is None else gamma.to(x.dtype).contiguous()
-    row_sums = torch.empty((R, 2), dtype=torch.float32, device=x.device)
-    ws = _workspace(R, C, x.device)
-    n_parts = ctypes.c_int64(0)
-    rc = lib.cw_ln_bwd_partials_open(R, C, _p(dy), _ld(dy), _p(x), _ld(x), _p(mean_rstd), _p(gamma), _p(row_sums), _p(ws),
-                                     ws.numel(), ctypes.cast(ctypes.byref(n_parts), ctypes.c_void_p), _dtype_code(x),
-                                     _stream())
-    _lib.check(rc, "cw_ln_bwd_partials_open")
-    return row_sums, (ws, n_parts.value)
+    row_sums, ws, n_parts = _lib.host().ln_bwd_partials_open(dy, x, mean_rstd, gamma)
+    return row_sums, (ws, n_parts)
 
 
 def ln_bwd_dx_close(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor, row_sums: torch.Tensor, hidden: int,
                     pending, gamma: Optional[torch.Tensor] = None, param_dtype: Optional[torch.dtype] = None):
     """(dx, dgamma [C], dbeta [C]): ln_bwd_dx whose launch also finishes the column sums that
     ln_bwd_partials_open left pending (stored as param_dtype, default float32). See cw_ln_bwd_dx_close."""
-    lib = _lib.load()
-    shape = x.shape
-    dy, x = _rows(dy), _rows(x)
-    _require_device(dy, x, mean_rstd, row_sums, gamma)
-    R, C = x.shape
     ws, n_parts = pending
-    gamma = None if gamma is None else gamma.to(x.dtype).contiguous()
-    row_sums = row_sums.reshape(R, 2).to(torch.float32).contiguous()
-    dx = torch.empty((R, C), dtype=x.dtype, device=x.device)
-    param_dtype = _out_dtype(param_dtype)
-    dgamma = torch.empty(C, dtype=param_dtype, device=x.device)
-    dbeta = torch.empty(C, dtype=param_dtype, device=x.device)
-    rc = lib.cw_ln_bwd_dx_close(R, C, _p(dy), _ld(dy), _p(x), _ld(x), _p(mean_rstd), _p(gamma), _p(row_sums), hidden,
-                                _p(dx), _ld(dx), _p(ws), n_parts, _p(dgamma), _p(dbeta), _TORCH_CODE[param_dtype],
-                                _dtype_code(x), _stream())
-    _lib.check(rc, "cw_ln_bwd_dx_close")
-    return dx.reshape(shape), dgamma, dbeta
+    return _lib.host().ln_bwd_dx_close(dy, x, mean_rstd, row_sums, hidden, ws, n_parts, gamma, param_dtype)
 
 
 def ln_backward_fused(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor,
@@ -374,42 +229,7 @@ def ln_backward_fused(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor
     one pass over dy and x; the parameter gradients are fp32 sums stored as param_dtype (default float32).
     dx_addend: the gradient reaching x along a residual branch, added to dx in the same pass where the kernel
     offers it (else by a separate addition here). See cw_ln_backward_fused."""
-    lib = _lib.load()
-    shape = x.shape
-    dy, x = _rows(dy), _rows(x)
-    _require_device(dy, x, mean_rstd, gamma)
-    if dy.shape != x.shape or dy.dtype != x.dtype:
-        raise ValueError("dy and x must agree in shape and dtype")
-    R, C = x.shape
-    gamma = None if gamma is None else gamma.to(x.dtype).contiguous()
-    row_sums = torch.empty((R, 2), dtype=torch.float32, device=x.device)
-    dx = torch.empty((R, C), dtype=x.dtype, device=x.device)
-    dgamma = dbeta = ws = None
-    param_dtype = _out_dtype(param_dtype)
-    if want_param_grads:
-        dgamma = torch.empty(C, dtype=param_dtype, device=x.device)
-        dbeta = torch.empty(C, dtype=param_dtype, device=x.device)
-        ws = _workspace(R, C, x.device)
-    add = None
-    if dx_addend is not None:
-        add = _rows(dx_addend)
-        if add.shape != x.shape or add.dtype != x.dtype:
-            raise ValueError("dx_addend must agree with x in shape and dtype")
-        _require_device(add)
-
-    def call(a):
-        return lib.cw_ln_backward_fused(R, C, _p(dy), _ld(dy), _p(x), _ld(x), _p(mean_rstd), _p(gamma), _p(row_sums), _p(dx),
-                                        _ld(dx), _p(a), _ld(a) if a is not None else 0, _p(dgamma), _p(dbeta),
-                                        _TORCH_CODE[param_dtype], _p(ws), ws.numel() if ws is not None else 0,
-                                        _dtype_code(x), _stream())
-    rc = call(add)
-    if rc == _lib.CW_ERR_UNSUPPORTED and add is not None:   # a shape of the two-kernel path: add separately
-        rc = call(None)
-        _lib.check(rc, "cw_ln_backward_fused")
-        dx = dx + add
-        return dx.reshape(shape), dgamma, dbeta
-    _lib.check(rc, "cw_ln_backward_fused")
-    return dx.reshape(shape), dgamma, dbeta
+    return _lib.host().ln_backward_fused(dy, x, mean_rstd, gamma, want_param_grads, param_dtype, dx_addend)
 
 
 # --------------------------------------------------------------------------
