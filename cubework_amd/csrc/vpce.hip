@@ -151,24 +151,32 @@ __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int6
     }
 }
 
-__global__ __launch_bounds__(256) void vpce_finalize_kernel(int64_t T_rows, int n_ranks,
-                                                            const float* __restrict__ max_all,
-                                                            const float* __restrict__ sumexp_all,
-                                                            const float* __restrict__ pred_all,
-                                                            const uint8_t* __restrict__ mask_all,
+// One slice's statistics, [T] each; for the peers' [n_peers, T].
+struct CeStats {
+    const float* max;
+    const float* sumexp;
+    const float* pred;
+    const uint8_t* mask;
+};
+// This rank's statistics and the peers' as they arrived, combined in that order: stacking them first took four launches
+// (14 us of the GPU at 8192 rows of 4 ranks, and as much of the host) in front of this one (5 us): the loss, forward and
+// backward, 173 -> 144 us.
+__global__ __launch_bounds__(256) void vpce_finalize_kernel(int64_t T_rows, int n_peers, const CeStats own, const CeStats peers,
                                                             float* __restrict__ loss, float* __restrict__ gmax,
                                                             float* __restrict__ gsum) {
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (t >= T_rows) return;
-    float m = max_all[t];
-    for (int r = 1; r < n_ranks; ++r) m = fmaxf(m, max_all[(int64_t)r * T_rows + t]);
+    float m = own.max[t];
+    for (int r = 0; r < n_peers; ++r) m = fmaxf(m, peers.max[(int64_t)r * T_rows + t]);
     float s = 0.0f, p = 0.0f;
-    for (int r = 0; r < n_ranks; ++r) {
-        const float mr = max_all[(int64_t)r * T_rows + t];
+    auto add = [&](const CeStats& st, int64_t i) {
+        const float mr = st.max[i];
         const float f = (mr == kNegInf) ? 0.0f : expf(mr - m);
-        s += sumexp_all[(int64_t)r * T_rows + t] * f;
-        if (mask_all[(int64_t)r * T_rows + t] == 0) p += pred_all[(int64_t)r * T_rows + t] - m;
-    }
+        s += st.sumexp[i] * f;
+        if (st.mask[i] == 0) p += st.pred[i] - m;
+    };
+    add(own, t);
+    for (int r = 0; r < n_peers; ++r) add(peers, (int64_t)r * T_rows + t);
     loss[t] = logf(s) - p;
     if (gmax != nullptr) gmax[t] = m;
     if (gsum != nullptr) gsum[t] = s;
@@ -381,9 +389,22 @@ extern "C" int cw_vpce_finalize(int64_t T, int n_ranks, const float* max_all, co
     if (T == 0) return CW_OK;
     if (max_all == nullptr || sumexp_all == nullptr || pred_all == nullptr || mask_all == nullptr || loss == nullptr)
         return fail(CW_ERR_INVALID, "cw_vpce_finalize: null pointer");
-    if (const int drc = require_gfx950("cw_vpce_finalize"); drc != CW_OK) return drc;
-    hipLaunchKernelGGL(vpce_finalize_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, (hipStream_t)stream, T,
-                       n_ranks, max_all, sumexp_all, pred_all, mask_all, loss, gmax, gsum);
+    return cw_vpce_finalize_peers(T, n_ranks - 1, max_all, sumexp_all, pred_all, mask_all, max_all + T, sumexp_all + T,
+                                  pred_all + T, mask_all + T, loss, gmax, gsum, stream);
+}
+
+extern "C" int cw_vpce_finalize_peers(int64_t T, int n_peers, const float* max, const float* sumexp, const float* pred,
+                                      const uint8_t* mask, const float* max_peers, const float* sumexp_peers,
+                                      const float* pred_peers, const uint8_t* mask_peers, float* loss, float* gmax,
+                                      float* gsum, void* stream) {
+    if (T < 0 || n_peers < 0) return fail(CW_ERR_INVALID, "cw_vpce_finalize_peers: bad T=%lld or n_peers=%d", (long long)T, n_peers);
+    if (T == 0) return CW_OK;
+    if (max == nullptr || sumexp == nullptr || pred == nullptr || mask == nullptr || loss == nullptr ||
+        (n_peers > 0 && (max_peers == nullptr || sumexp_peers == nullptr || pred_peers == nullptr || mask_peers == nullptr)))
+        return fail(CW_ERR_INVALID, "cw_vpce_finalize_peers: null pointer");
+    if (const int drc = require_gfx950("cw_vpce_finalize_peers"); drc != CW_OK) return drc;
+    hipLaunchKernelGGL(vpce_finalize_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, (hipStream_t)stream, T, n_peers,
+                       (CeStats{max, sumexp, pred, mask}), (CeStats{max_peers, sumexp_peers, pred_peers, mask_peers}), loss, gmax, gsum);
     return check_launch("vpce_finalize_kernel");
 }
 

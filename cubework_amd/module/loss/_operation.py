@@ -26,12 +26,10 @@ class _VocabParallelCrossEntropy(torch.autograd.Function):
         logits_2d = logits.reshape(-1, vocab)
         local = ops.vpce_fwd_local(logits_2d, targets.reshape(-1), vocab_start)
         if parallel_mode.world_size == 1:
-            stacked = [s.unsqueeze(0) for s in local]
+            loss, gmax, gsum = ops.vpce_finalize(*(s.unsqueeze(0) for s in local))
         else:
             # peers' (max, sumexp, pred, mask), each [world_size - 1, tokens]
-            peers = parallel_mode.take("vpce_stats")
-            stacked = [torch.cat([s.unsqueeze(0), p.to(s.dtype).reshape(-1, s.numel())]) for s, p in zip(local, peers)]
-        loss, gmax, gsum = ops.vpce_finalize(*stacked)
+            loss, gmax, gsum = ops.vpce_finalize_peers(local, parallel_mode.take("vpce_stats"))
         ctx.save_for_backward(logits_2d, targets.reshape(-1), gmax, gsum)
         # Logits that a layer made: their gradient goes to that layer's two products, which read 16-byte aligned rows in
         # place and copy others first (1023 x 50257 bf16: 2 x 33 us). The gradient of a leaf stays contiguous, as

@@ -272,6 +272,22 @@ def vpce_finalize(max_all: torch.Tensor, sumexp_all: torch.Tensor, pred_all: tor
     return loss, gmax, gsum
 
 
+def vpce_finalize_peers(local: Sequence[torch.Tensor], peers: Sequence[torch.Tensor]):
+    """vpce_finalize of this rank's (max, sumexp, pred, mask), [T] each as vpce_fwd_local returns them, and its peers',
+    [n_ranks - 1, T] each; returns (loss, gmax, gsum), each [T] fp32."""
+    lib = _lib.load()
+    T = local[0].numel()
+    peers = [p.to(s.dtype).reshape(-1, T).contiguous() for s, p in zip(local, peers)]
+    _require_device(*local, *peers)
+    n = peers[0].shape[0]
+    if len(peers) != 4 or any(p.shape[0] != n for p in peers):
+        raise ValueError("the peers' max, sumexp, pred and mask must come from the same ranks")
+    loss, gmax, gsum = (torch.empty(T, dtype=torch.float32, device=local[0].device) for _ in range(3))
+    rc = lib.cw_vpce_finalize_peers(T, n, *map(_p, local), *map(_p, peers), _p(loss), _p(gmax), _p(gsum), _stream())
+    _lib.check(rc, "cw_vpce_finalize_peers")
+    return loss, gmax, gsum
+
+
 def vpce_bwd(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, gmax: torch.Tensor, gsum: torch.Tensor,
              dloss_rows: Optional[torch.Tensor] = None, dloss_scale: float = 1.0,
              grad_dtype: Optional[torch.dtype] = None, aligned_rows: bool = False) -> torch.Tensor:

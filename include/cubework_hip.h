@@ -323,6 +323,11 @@ int cw_vpce_fwd_local(int64_t T, int64_t V, const void* logits, int64_t ld,
 int cw_vpce_finalize(int64_t T, int n_ranks, const float* max_all, const float* sumexp_all,
                      const float* pred_all, const uint8_t* mask_all,
                      float* loss, float* gmax, float* gsum, void* stream);
+/* The same from this rank's statistics ([T] each) and its peers' ([n_peers][T]) as they arrived. */
+int cw_vpce_finalize_peers(int64_t T, int n_peers, const float* max, const float* sumexp, const float* pred,
+                           const uint8_t* mask, const float* max_peers, const float* sumexp_peers,
+                           const float* pred_peers, const uint8_t* mask_peers, float* loss, float* gmax,
+                           float* gsum, void* stream);
 
 /*
  * grad[t,c] = (exp(logits[t,c]-gmax[t]) / gsum[t] - [c == target column, in slice]) * dloss

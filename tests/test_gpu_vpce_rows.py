@@ -72,3 +72,22 @@ def test_head_gradients_with_padded_rows(V, dtype):
         # the same products from other addresses: the 16-bit kernel copies unaligned rows and multiplies the same values,
         # the fp32 one may take another kernel and so another order of its sums
         assert_parity(got, want.cpu(), dtype, "head gradient V=%d" % V)
+
+
+@pytest.mark.parametrize("T", [1, 255, 257, 8192])
+@pytest.mark.parametrize("n_peers", [0, 1, 3])
+def test_finalize_from_the_peers_as_they_arrived(T, n_peers):
+    """The same combination as of the stacked statistics, in the same order: the same bits. A rank without a finite logit
+    and peers of another type are among them."""
+    from cubework_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(T + n_peers)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device=DEV)  # noqa: E731
+    stats = [rnd(n_peers + 1, T) * 3, rnd(n_peers + 1, T).abs() + 1, rnd(n_peers + 1, T), torch.ones(n_peers + 1, T, dtype=torch.uint8, device=DEV)]
+    stats[0][-1, 0], stats[1][-1, 0] = float("-inf"), 0.0
+    stats[3][torch.arange(T, device=DEV) % (n_peers + 1), torch.arange(T, device=DEV)] = 0
+    want = ops.vpce_finalize(*stats)
+    peers = [s[1:].double() if k < 3 else s[1:].bool() for k, s in enumerate(stats)]
+    got = ops.vpce_finalize_peers([s[0].contiguous() for s in stats], peers)
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
