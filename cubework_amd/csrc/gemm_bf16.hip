@@ -70,12 +70,14 @@ static int pack_rows(const void* const* src, int n, int64_t ld, int64_t rows, in
     return CW_OK;
 }
 
-static TileArgs to_tile_args(const GemmArgs& g) {
+// One instantiation serves CW_EPI_NONE and CW_EPI_BIAS: without an epilogue there is no bias, whatever the caller passes.
+static TileArgs to_tile_args(const GemmArgs& g, int epilogue) {
     TileArgs a;
     memcpy(a.A, g.A, sizeof(a.A));
     memcpy(a.B, g.B, sizeof(a.B));
     memcpy(a.addend, g.addend, sizeof(a.addend));
-    a.bias = g.bias; a.C = g.C; a.preact = g.preact;
+    a.bias = epilogue == CW_EPI_NONE ? nullptr : g.bias;
+    a.C = g.C; a.preact = g.preact;
     a.lda = g.lda; a.ldb = g.ldb; a.ldc = g.ldc; a.ldp = g.ldp; a.ldadd = g.ldadd;
     a.M = g.M; a.N = g.N; a.K = g.K; a.n_steps = g.n_steps; a.n_addends = g.n_addends;
     a.vec_out = g.vec_c && (g.preact == nullptr || g.vec_p);
@@ -87,7 +89,7 @@ static TileArgs to_tile_args(const GemmArgs& g) {
 }
 
 static int tile_launch(const GemmArgs& g, const TilePlan& plan, int layout, int epilogue, bool f16, hipStream_t s) {
-    TileArgs a = to_tile_args(g);
+    TileArgs a = to_tile_args(g, epilogue);
     char* ws = reinterpret_cast<char*>(g.workspace);
     if (plan.pack_a) {
         const bool tn = layout == CW_TN;

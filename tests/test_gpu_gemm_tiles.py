@@ -72,3 +72,45 @@ def test_forward_rows_do_not_depend_on_the_batch():
     whole = ops.gemm_ksteps("NN", [a], [b])
     for rows in (1, 65, 300):
         assert torch.equal(ops.gemm_ksteps("NN", [a[:rows]], [b]), whole[:rows])
+
+
+def _abi_gemm(layout, A, B, bias, epilogue, scratch, addend=None):
+    """cw_gemm_ksteps_ws as a C caller makes it, with `scratch` bytes of scratch."""
+    import ctypes
+
+    from cubework_amd import _lib
+    from cubework_amd.ops import LAYOUTS, _dtype_code, _ld, _p, _ptr_table, _stream
+
+    M, K = A.shape[::-1] if layout == "TN" else A.shape
+    N = B.shape[0] if layout == "NT" else B.shape[1]
+    C = torch.full((M, N), float("nan"), dtype=A.dtype, device=A.device)
+    ws = torch.empty(max(scratch, 16), dtype=torch.uint8, device=A.device)
+    add = [] if addend is None else [addend]
+    rc = _lib.load().cw_gemm_ksteps_ws(LAYOUTS[layout], M, N, K, 1, _ptr_table([A]), _ld(A), _ptr_table([B]), _ld(B), _p(bias), epilogue, _p(C),
+                                       _ld(C), ctypes.c_void_p(0), 0, _ptr_table(add), len(add), N, _p(ws) if scratch else None, scratch,
+                                       _dtype_code(A), _stream())
+    _lib.check(rc, "cw_gemm_ksteps_ws")
+    return C
+
+
+# whole tiles; every tile sliced (a long reduction over few tiles); unaligned rows without scratch for their copy (the
+# register-staged kernel); the two fp32 kernels
+@pytest.mark.parametrize("layout,M,N,K,dtype,pad,sliced", [
+    ("NN", 300, 264, 64, torch.bfloat16, 0, False), ("NT", 64, 768, 3072, torch.float16, 0, True),
+    ("NN", 130, 70, 50, torch.bfloat16, 3, False), ("NN", 130, 72, 40, torch.float32, 0, False),
+    ("NN", 4096, 2048, 64, torch.float32, 0, False)])
+def test_no_epilogue_ignores_a_bias_pointer(layout, M, N, K, dtype, pad, sliced):
+    """CW_EPI_NONE is acc (+ addends) whatever the bias argument holds: the same bits as without a bias."""
+    from cubework_amd import _lib
+    from cubework_amd.ops import LAYOUTS, _dtype_code, _ld
+
+    a = randn((M, K + pad), dtype, 1).cuda()[:, :K]
+    b = randn((N, K + pad) if layout == "NT" else (K, N), dtype, 2, 0.05).cuda()[:, :K if layout == "NT" else N]
+    bias, add = torch.full((N,), 1000.0, dtype=dtype, device="cuda"), randn((M, N), dtype, 3).cuda()
+    scratch = 0 if pad else _lib.load().cw_gemm_scratch_bytes(LAYOUTS[layout], M, N, K, 1, _ld(a), _ld(b), 1, 1, 0, _dtype_code(a))
+    assert (scratch > 0) == sliced
+    for addend in (None, add):
+        with_bias = _abi_gemm(layout, a, b, bias, _lib.CW_EPI_NONE, scratch, addend)
+        assert torch.equal(with_bias, _abi_gemm(layout, a, b, None, _lib.CW_EPI_NONE, scratch, addend))
+        want = a.double().cpu() @ (b.double().cpu().t() if layout == "NT" else b.double().cpu()) + (0 if addend is None else addend.double().cpu())
+        assert_parity(with_bias, want, dtype, "no epilogue beside a bias pointer")
