@@ -31,19 +31,15 @@ class _VocabParallelCrossEntropy(torch.autograd.Function):
             # peers' (max, sumexp, pred, mask), each [world_size - 1, tokens]
             loss, gmax, gsum = ops.vpce_finalize_peers(local, parallel_mode.take("vpce_stats"))
         ctx.save_for_backward(logits_2d, targets.reshape(-1), gmax, gsum)
-        # Logits that a layer made: their gradient goes to that layer's two products, which read 16-byte aligned rows in
-        # place and copy others first (1023 x 50257 bf16: 2 x 33 us). The gradient of a leaf stays contiguous, as
-        # autograd would otherwise copy it into the leaf's layout.
-        ctx.meta = (vocab_start, logits.shape, logits.grad_fn is not None)
+        ctx.meta = (vocab_start, logits.shape)
         return loss.reshape(targets.shape)
 
     @staticmethod
     @bwd()
     def backward(ctx, output_grad):
         logits_2d, targets, gmax, gsum = ctx.saved_tensors
-        vocab_start, shape, aligned_rows = ctx.meta
-        grad = ops.vpce_bwd(logits_2d, targets, vocab_start, gmax, gsum, output_grad.reshape(-1).float(), 1.0,
-                            aligned_rows=aligned_rows)
+        vocab_start, shape = ctx.meta
+        grad = ops.vpce_bwd(logits_2d, targets, vocab_start, gmax, gsum, output_grad.reshape(-1).float(), 1.0)
         return grad.reshape(shape), None, None
 
 

@@ -52,6 +52,8 @@ class _LinearNT(torch.autograd.Function):
                 g, dbias = ops.act_bwd_colsum(activation, g, pre, want_dbias=has_bias, out_dtype=bias_dtype)
             elif has_bias:
                 dbias = ops.colsum(g, out_dtype=bias_dtype)   # fp32 sums stored in the parameter's dtype: no cast launch
+            if all(ctx.needs_input_grad[:2]):
+                g = ops.aligned_rows(g)
             dx = ops.gemm_ksteps("NN", [g], [weight]).reshape(in_shape) if ctx.needs_input_grad[0] else None
             dw = ops.gemm_ksteps("TN", [g], [x2]) if ctx.needs_input_grad[1] else None
         return dx, dw, dbias, None

@@ -60,6 +60,16 @@ def _ld(t: torch.Tensor) -> int:
     return t.stride(0) if t.shape[0] > 1 else max(t.shape[1], 1)
 
 
+def aligned_rows(t: torch.Tensor) -> torch.Tensor:
+    """A 16-bit [rows, cols] operand of two products with rows that begin at multiples of 16 bytes: itself, or one copy that
+    both read in place, where each would make its own (1023 x 50257 bf16: one copy 43 us, the products' two 66 us)."""
+    t = _rows(t)
+    if t.element_size() != 2 or t.shape[0] < 2 or (t.data_ptr() % 16 == 0 and _ld(t) % 8 == 0):
+        return t
+    out = t.new_empty((t.shape[0], -(-t.shape[1] // 8) * 8))[:, :t.shape[1]]
+    return out.copy_(t)
+
+
 def _stream() -> ctypes.c_void_p:
     # the raw handle of torch's current stream on the current device; torch.cuda.current_stream() builds a
     # Stream object for the same value and costs ten times as much per call

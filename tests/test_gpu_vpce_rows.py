@@ -49,7 +49,7 @@ def test_rows_of_any_alignment(V, dtype, grad_dtype, extra, start):
 @pytest.mark.parametrize("V", [1001, 1000])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_head_gradients_with_padded_rows(V, dtype):
-    """The classifier's two gradient products read the loss's gradient with padded rows: against a contiguous copy."""
+    """The classifier's two gradient products from the loss's contiguous gradient and from one that a hook returns with padded rows."""
     from cubework_amd.distributed import initialize
     from cubework_amd.module.loss import VocabParallelCrossEntropyLoss1D
     from cubework_amd.module.parallel_1d import VocabParallelClassifier1D
@@ -60,12 +60,17 @@ def test_head_gradients_with_padded_rows(V, dtype):
     loss_fn = VocabParallelCrossEntropyLoss1D()
     targets = torch.randint(0, V, (2, 61), generator=torch.Generator().manual_seed(1)).to(DEV)
     results = []
+
+    def padded(g):
+        out = torch.full(g.shape[:-1] + (V + 15,), float("nan"), dtype=dtype, device=DEV)[..., :V]
+        return out.copy_(g)
+
     for contiguous in (False, True):
         x = randn((2, 61, 96), dtype, seed=2).to(DEV).requires_grad_(True)
         layer.zero_grad()
         logits = layer(x)
-        if contiguous:
-            logits.register_hook(lambda g: g.contiguous())
+        if not contiguous:
+            logits.register_hook(padded)
         loss_fn(logits, targets).backward()
         results.append([x.grad] + [p.grad.clone() for p in layer.parameters()])
     for got, want in zip(*results):
@@ -91,3 +96,22 @@ def test_finalize_from_the_peers_as_they_arrived(T, n_peers):
     got = ops.vpce_finalize_peers([s[0].contiguous() for s in stats], peers)
     for a, b in zip(got, want):
         assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("V", [1001, 1000])
+def test_logits_gradient_is_contiguous(V):
+    """Hooks on the logits and retain_grad see a dense gradient for every vocabulary, as any operator's."""
+    from cubework_amd.distributed import initialize
+    from cubework_amd.module.loss import VocabParallelCrossEntropyLoss1D
+    from cubework_amd.module.parallel_1d import VocabParallelClassifier1D
+
+    initialize("1d", 1)
+    with torch.device(DEV):
+        layer = VocabParallelClassifier1D(96, V, bias=False).to(torch.bfloat16)
+    x = randn((2, 61, 96), torch.bfloat16, seed=2).to(DEV).requires_grad_(True)
+    logits = layer(x)
+    seen = []
+    logits.register_hook(lambda g: seen.append(g.view(-1).numel()))
+    logits.retain_grad()
+    VocabParallelCrossEntropyLoss1D()(logits, torch.zeros((2, 61), dtype=torch.int64, device=DEV)).backward()
+    assert seen == [2 * 61 * V] and logits.grad.is_contiguous() and logits.grad.untyped_storage().nbytes() == 2 * 61 * V * 2
