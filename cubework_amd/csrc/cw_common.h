@@ -221,9 +221,10 @@ __device__ __forceinline__ raw16_t pack_raw(const float (&v)[4], const float*) {
 // unit writes them at LDS address lds_addr + 16 l (M0 holds lds_addr): no staging registers, no LDS write
 // instructions. The compiler does not see these loads (inline asm); a kernel that uses them counts them and
 // waits with dma_wait<N> (at most N of this thread's loads still in flight; loads complete in issue order)
-// before the barrier that publishes the data.
+// before the barrier that publishes the data. s_nop: the load reads M0, and a write of M0 by the instruction in front of it
+// needs one wait state, which the compiler inserts between its own instructions but not inside inline asm.
 __device__ __forceinline__ void dma16(const char* gbase, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(gbase) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(gbase) : "memory", "m0");
 }
 // The same through a buffer of kDmaRange bytes at `base`: a lane whose offset is kDmaRange itself fetches nothing and the
 // load unit writes 16 zero bytes for it.
@@ -231,7 +232,7 @@ constexpr uint32_t kDmaRange = 0x80000000u;
 __device__ __forceinline__ void dma16_buffer(const char* base, uint32_t voff, uint32_t lds_addr) {
     const uint64_t b = reinterpret_cast<uint64_t>(base);
     const raw16_t rsrc = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, kDmaRange, 0x00020000u};
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc) : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void dma_wait() {
