@@ -101,8 +101,9 @@ def gemm_ksteps(layout: str, A_steps: Sequence[torch.Tensor], B_steps: Sequence[
     """
     if layout not in LAYOUTS:
         raise ValueError("layout must be NN, NT or TN")
-    out, preact = _lib.host().gemm_ksteps(LAYOUTS[layout], A_steps, B_steps, bias, epilogue_code(bias is not None, activation),
-                                          addends, want_preact, out)
+    # tuple: a stacked tensor is a sequence of its slices here, but none that the native call takes
+    out, preact = _lib.host().gemm_ksteps(LAYOUTS[layout], tuple(A_steps), tuple(B_steps), bias,
+                                          epilogue_code(bias is not None, activation), tuple(addends), want_preact, out)
     return (out, preact) if want_preact else out
 
 

@@ -13,6 +13,9 @@ def _t(*shape, dtype=torch.float32):
     (lambda o: o.gemm_ksteps("NN", [_t(2, 3)], []), ValueError),
     (lambda o: o.gemm_ksteps("XX", [_t(2, 3)], [_t(3, 2)]), ValueError),
     (lambda o: o.gemm_ksteps("NN", [_t(2, 3)], [_t(3, 2)]), RuntimeError),
+    # step operands and addends may be one stacked tensor, as any sequence: it gets as far as the device check
+    (lambda o: o.gemm_ksteps("NN", _t(2, 2, 3), _t(2, 3, 2)), RuntimeError),
+    (lambda o: o.gemm_ksteps("NN", [_t(2, 3)], [_t(3, 2)], addends=_t(1, 2, 2)), RuntimeError),
     (lambda o: o.gemm_ksteps("NN", [3], [_t(3, 2)]), TypeError),
     (lambda o: o.gemm_ksteps("NN", [_t(2, 3)], [_t(3, 2)], _t(2), "swish"), KeyError),
     (lambda o: o.colsum(_t(2, 3)), RuntimeError),
