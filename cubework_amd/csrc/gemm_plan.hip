@@ -242,6 +242,9 @@ double tile_rounds(const TileConfig& c, double count, double trips, double layou
     return t;
 }
 
+// Whole tiles of a launch: 256 work-items each, fewer than 2^32 together (as the reduction's, which are fewer).
+constexpr int64_t kTileLaunchMax = ((int64_t)1 << 24) - 8;
+
 }  // namespace
 
 TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int64_t lda, int64_t ldb, bool align_a, bool align_b,
@@ -256,15 +259,22 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     p.pack_b = !align_b;
     p.lda = lda;
     p.ldb = ldb;
+    // A copy is one launch of a work-item per 8 elements, and a launch has fewer than 2^32 of them: larger operands are not
+    // copied.
+    auto copy_ld = [](int64_t cols) { return (cols + 7) / 8 * 8; };
+    auto copied = [&](int64_t rows, int64_t cols) { return rows <= (((int64_t)1 << 32) - 256) * 8 / copy_ld(cols); };
+    auto copy_bytes = [&](int64_t n, int64_t rows, int64_t cols) { return (n * rows * copy_ld(cols) * 2 + 255) / 256 * 256; };
+    const int64_t a_rows = layout == CW_TN ? K : M, a_cols = layout == CW_TN ? M : K, b_rows = layout == CW_NT ? N : K, b_cols = layout == CW_NT ? K : N;
+    if ((p.pack_a && !copied(a_rows, a_cols)) || (p.pack_b && !copied(b_rows, b_cols)) || (n_pack_addends > 0 && !copied(M, N))) return best;
     if (p.pack_a) {
-        p.lda = ((layout == CW_TN ? M : K) + 7) / 8 * 8;
-        p.pack_a_bytes = (n_steps * (layout == CW_TN ? K : M) * p.lda * 2 + 255) / 256 * 256;
+        p.lda = copy_ld(a_cols);
+        p.pack_a_bytes = copy_bytes(n_steps, a_rows, a_cols);
     }
     if (p.pack_b) {
-        p.ldb = ((layout == CW_NT ? K : N) + 7) / 8 * 8;
-        p.pack_b_bytes = (n_steps * (layout == CW_NT ? N : K) * p.ldb * 2 + 255) / 256 * 256;
+        p.ldb = copy_ld(b_cols);
+        p.pack_b_bytes = copy_bytes(n_steps, b_rows, b_cols);
     }
-    p.pack_add_bytes = (n_pack_addends * M * ((N + 7) / 8 * 8) * 2 + 255) / 256 * 256;
+    if (n_pack_addends > 0) p.pack_add_bytes = copy_bytes(n_pack_addends, M, N);
     // the kernels' lane offsets: 256 rows (or 32 k rows) of either operand within 2 GB
     if (p.lda >= ((int64_t)1 << 22) || p.ldb >= ((int64_t)1 << 22)) return best;
     // A forward product (B stored [K, N]) that does not reduce its width, K <= N - the projections in front of an
@@ -304,7 +314,7 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     for (int cfg = 0; cfg < kTileConfigCount; ++cfg) {
         const TileConfig& c = kTileConfigs[cfg];
         const int64_t tiles = ((M + 64 * c.tm - 1) / (64 * c.tm)) * ((N + 64 * c.tn - 1) / (64 * c.tn));
-        if (tiles > limit / 16 || ((rotated || fixed_slices > 1) && cfg != 0)) continue;
+        if (tiles > kTileLaunchMax || ((rotated || fixed_slices > 1) && cfg != 0)) continue;
         if (fixed_slices > 1) {
             consider(cfg, tiles, 0, fixed_slices);
             continue;

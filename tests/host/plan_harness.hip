@@ -8,6 +8,8 @@
 //   * the short extra step of a ragged reduction: starts at K - 32, its A part lies inside A, the scratch
 //     copy of B's last rows fits the workspace that cw_gemm_workspace_bytes asked for;
 //   * split k: slices divide K into multiples of 64, the partial sums fit the workspace;
+//   * the tile kernels' plans (tile_plan): scratch within its bound, whole and sliced tiles, copies and partial sums that
+//     add up, lane offsets below 2 GiB, launches below 2^32 work-items;
 //   * column sums: the slabs cover the rows exactly once and their partial rows fit cw_colsum_workspace_bytes'
 //     promise of at most 512 (or ceil(M / 64)) rows.
 // Prints "ok <checks> routes <how often each kernel route was planned>" and exits 0, or the first violated invariant and exits 1.
@@ -24,6 +26,7 @@ namespace {
 
 long g_checked = 0;
 long g_routes[6] = {0, 0, 0, 0, 0, 0};
+long g_tile_plans[3] = {0, 0, 0};  // whole tiles, every tile sliced, the last round sliced
 
 #define REQUIRE(cond, ...)                                    \
     do {                                                      \
@@ -190,6 +193,86 @@ void sweep_gemm() {
                 }
 }
 
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// What one plan of the tile kernels promises: it fits the scratch it was given, its tiles, slices and sub-buffers add up
+// as the launches use them (gemm_bf16.hip's tile_launch, gemm_tile.h's launch_cfg), and no offset or grid leaves its type.
+void check_tile_plan(int layout, int64_t M, int64_t N, int64_t K, int steps, int64_t lda, int64_t ldb, bool al_a, bool al_b, int n_pack,
+                     int64_t max_scratch, bool must_plan) {
+    const TilePlan p = tile_plan(layout, M, N, K, steps, lda, ldb, al_a, al_b, n_pack, max_scratch);
+    ++g_checked;
+#define PLAN_REQUIRE(cond)                                                                                                        \
+    REQUIRE(cond, "layout %d M=%lld N=%lld K=%lld steps %d lda=%lld ldb=%lld aligned %d %d addends %d scratch %lld: cfg %d full %d slices %d", \
+            layout, (long long)M, (long long)N, (long long)K, steps, (long long)lda, (long long)ldb, al_a, al_b, n_pack,         \
+            (long long)max_scratch, p.cfg, p.full, p.slices)
+    PLAN_REQUIRE(p.cfg >= -1 && p.cfg < kTileConfigCount);
+    PLAN_REQUIRE(!must_plan || p.cfg >= 0);
+    if (p.cfg < 0) return;
+    ++g_tile_plans[p.full == p.tiles ? 0 : (p.full == 0 ? 1 : 2)];
+    const TileConfig& c = kTileConfigs[p.cfg];
+    const int64_t bm = 64 * c.tm, bn = 64 * c.tn;
+    PLAN_REQUIRE(p.tiles == ceil_div(M, bm) * ceil_div(N, bn));
+    PLAN_REQUIRE(p.full >= 0 && p.full <= p.tiles && p.slices >= 1 && (p.full < p.tiles || p.slices == 1));
+    const int64_t rest = p.tiles - p.full, trips = ceil_div(K, 32 * c.kb) * steps;
+    PLAN_REQUIRE(p.slices <= trips);
+    // the partial sums of every (tile, slice), behind the copies, all at 16-byte boundaries and within the scratch
+    PLAN_REQUIRE(p.partial_bytes == rest * (p.slices > 1 || rest > 0 ? p.slices : 0) * bm * bn * 4);
+    PLAN_REQUIRE(p.pack_a_bytes % 16 == 0 && p.pack_b_bytes % 16 == 0 && p.pack_add_bytes % 16 == 0);
+    PLAN_REQUIRE(max_scratch < 0 || p.scratch() <= max_scratch);
+    // copies: every step's rows at an aligned pitch that holds them; operands that are not copied keep theirs
+    const int64_t a_rows = layout == CW_TN ? K : M, a_cols = layout == CW_TN ? M : K, b_rows = layout == CW_NT ? N : K, b_cols = layout == CW_NT ? K : N;
+    PLAN_REQUIRE(p.pack_a == !al_a && p.pack_b == !al_b);
+    if (p.pack_a) PLAN_REQUIRE(p.lda % 8 == 0 && p.lda >= a_cols && p.pack_a_bytes >= steps * a_rows * p.lda * 2);
+    else PLAN_REQUIRE(p.lda == lda && p.pack_a_bytes == 0);
+    if (p.pack_b) PLAN_REQUIRE(p.ldb % 8 == 0 && p.ldb >= b_cols && p.pack_b_bytes >= steps * b_rows * p.ldb * 2);
+    else PLAN_REQUIRE(p.ldb == ldb && p.pack_b_bytes == 0);
+    PLAN_REQUIRE(p.pack_add_bytes >= n_pack * M * ceil_div(N, 8) * 16);
+    // a lane's byte offset (the block's rows, or 32 rows of k) stays inside the buffer's 2 GiB
+    const int64_t reach = (int64_t)1 << 31;
+    PLAN_REQUIRE((layout == CW_TN ? 31 * p.lda + bm : (bm - 1) * p.lda + 32) * 2 < reach);
+    PLAN_REQUIRE((layout == CW_NT ? (bn - 1) * p.ldb + 32 : 31 * p.ldb + bn) * 2 < reach);
+    // every launch is at most 2^32 - 1 work-items: the tiles and slices, their reduction, the copies (16 bytes each)
+    const int64_t items = ((int64_t)1 << 32) - 1;
+    PLAN_REQUIRE((ceil_div(p.full, 8) + ceil_div(rest * p.slices, 8)) * 8 * 256 <= items);
+    PLAN_REQUIRE(rest * c.tm * 256 <= items);
+    for (const int64_t bytes : {p.pack_a_bytes / steps, p.pack_b_bytes / steps, n_pack > 0 ? p.pack_add_bytes / n_pack : 0})
+        PLAN_REQUIRE(ceil_div(bytes, 16 * 256) * 256 <= items);
+#undef PLAN_REQUIRE
+}
+
+void sweep_tile_plan() {
+    const int64_t dims[] = {1, 7, 63, 64, 65, 128, 250, 256, 264, 777, 2048, 2056, 4376, 8192, 12568, 50257, 1 << 20, 3 << 20, 1 << 28, 1 << 30};
+    const int64_t ks[] = {1, 8, 31, 32, 72, 1003, 2048, 4096, 12568, 50257, 1 << 20, 1 << 30};
+    for (int layout = 0; layout < 3; ++layout)
+        for (int64_t M : dims)
+            for (int64_t N : dims)
+                for (int64_t K : ks)
+                    for (int variant = 0; variant < 6; ++variant) {
+                        const int steps = variant == 3 ? 4 : (variant == 4 ? CW_MAX_KSTEPS : 1), n_pack = variant == 2 ? 1 : (variant == 4 ? CW_MAX_ADDENDS : 0);
+                        const int64_t pad = variant == 1 ? 8 : (variant == 5 ? (int64_t)1 << 22 : 0);
+                        const int64_t lda = ((layout == CW_TN ? M : K) + 7) / 8 * 8 + pad + (variant == 2 ? 3 : 0);
+                        const int64_t ldb = ((layout == CW_NT ? K : N) + 7) / 8 * 8 + pad + (variant == 4 ? 1 : 0);
+                        const bool al_a = variant != 2, al_b = variant != 4;
+                        // operands and output that a 288 GB device holds, in rows the lane offsets reach: there is a plan
+                        const double bytes = 2.0 * ((double)M * K * steps * (al_a ? 1 : 2) + (double)N * K * steps * (al_b ? 1 : 2) + (double)M * N * (1 + 2 * n_pack));
+                        const int64_t limit = (int64_t)1 << 22;
+                        const bool wide = lda >= limit || ldb >= limit;
+                        auto too_big = [](int64_t rows, int64_t cols) { return (double)rows * (double)ceil_div(cols, 8) >= 4294967040.0; };
+                        const bool big_copy = (!al_a && (layout == CW_TN ? too_big(K, M) : too_big(M, K))) ||
+                                              (!al_b && (layout == CW_NT ? too_big(N, K) : too_big(K, N))) || (n_pack > 0 && too_big(M, N));
+                        check_tile_plan(layout, M, N, K, steps, lda, ldb, al_a, al_b, n_pack, -1, bytes < 2.9e11 && !wide && !big_copy);
+                        for (const int64_t scratch : {(int64_t)0, (int64_t)4096, (int64_t)1 << 22, (int64_t)1 << 26, (int64_t)1 << 33})
+                            check_tile_plan(layout, M, N, K, steps, lda, ldb, al_a, al_b, n_pack, scratch, false);
+                    }
+    REQUIRE(g_tile_plans[0] > 0 && g_tile_plans[1] > 0 && g_tile_plans[2] > 0, "plans: %ld whole, %ld sliced, %ld with a sliced last round",
+            g_tile_plans[0], g_tile_plans[1], g_tile_plans[2]);
+    for (int64_t bad : {(int64_t)0, (int64_t)-1, ((int64_t)1 << 30) + 1}) {
+        REQUIRE(tile_plan(CW_NN, bad, 8, 8, 1, 8, 8, true, true, 0, -1).cfg == -1 && tile_plan(CW_NN, 8, bad, 8, 1, 8, 8, true, true, 0, -1).cfg == -1 &&
+                    tile_plan(CW_NN, 8, 8, bad, 1, 8, 8, true, true, 0, -1).cfg == -1, "a plan for a size of %lld", (long long)bad);
+    }
+    REQUIRE(tile_plan(CW_NN, 8, 8, 8, 0, 8, 8, true, true, 0, -1).cfg == -1 && tile_plan(CW_NN, 8, 8, 8, CW_MAX_KSTEPS + 1, 8, 8, true, true, 0, -1).cfg == -1, "bad step counts");
+}
+
 void check_refusals() {
     GemmArgs args;
     bool nothing = false;
@@ -242,6 +325,7 @@ int main() {
     check_refusals();
     sweep_colsum();
     sweep_gemm();
+    sweep_tile_plan();
     printf("ok %ld routes small_ring=%ld ring=%ld ring_then_small=%ld ring_ktail=%ld split_k=%ld staged=%ld\n", g_checked, g_routes[0],
            g_routes[1], g_routes[2], g_routes[3], g_routes[4], g_routes[5]);
     return 0;
