@@ -570,7 +570,7 @@ int launch(const GemmArgs& g, int epilogue, hipStream_t s) {
     r.bias = g.bias; r.C = g.C; r.preact = g.preact;
     r.lda = g.lda; r.ldb = g.ldb; r.ldc = g.ldc; r.ldp = g.ldp; r.ldadd = g.ldadd;
     r.M = g.M; r.N = g.N; r.K = g.K; r.n_steps = g.n_steps; r.n_addends = g.n_addends;
-    r.vec_bias = 1; r.vec_add = 1; r.k_tail = 0; r.partial = nullptr;
+    r.vec_bias = 1; r.vec_add = 1;
     auto kern = gemm_f32_ring_kernel<TI, TJ, AS, BS>;
     constexpr int stages = kStages * (oper_bytes(TI) + oper_bytes(TJ));
     constexpr int patches = 4 * 32 * kPatchPitch * 4;

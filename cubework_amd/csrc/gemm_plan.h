@@ -1,6 +1,6 @@
 // Host-side planning of the block GEMM and of the column sums: argument validation, which kernel takes a
-// shape, how a product is cut into launches (a strip of tile rows / columns for the small-tile kernel, the
-// short extra step that finishes a ragged reduction, k slices) and how much scratch that needs. Pure integer
+// shape, how a product is cut into launches (whole and sliced tiles, a strip of tile rows / columns for the small
+// tiles) and how much scratch that needs (partial sums, copies of unaligned operands). Pure integer
 // and pointer arithmetic with no HIP call, so that the same functions the entry points run can be driven on a
 // machine without a GPU under the address and undefined-behaviour sanitizers (tests/host/plan_harness.hip):
 // this is the arithmetic where an off-by-one becomes an out-of-bounds access on the device.
@@ -19,26 +19,24 @@ int gemm_prepare_args(int layout, int64_t M, int64_t N, int64_t K, int n_steps, 
                       void* preact, int64_t ldp, const void* const* addends, int n_addends, int64_t ldadd, void* workspace,
                       int64_t workspace_bytes, int io_dtype, GemmArgs* out, bool* nothing_to_do);
 
-// Scratch that enables the split-k launch or the ragged-reduction step for a 16-bit product (0: neither).
+// Scratch of the split-k launch of a 16-bit product (0: not split). For a large product over a ragged K it is 32 rows of B,
+// which no launch reads any more: the size stays for callers that allocate by it.
 int64_t gemm_workspace_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int io_dtype);
 
 enum GemmRoute {
     kRouteSmallRing = 0,      // 128 x 128 tiles
     kRouteRing = 1,           // 256 x 256 tiles
     kRouteRingThenSmall = 2,  // whole rounds of 256 x 256 tiles (head), the mostly empty last round as 128 x 128 tiles (tail)
-    kRouteRingKTail = 3,      // 256 x 256 tiles with K % 32 != 0
-    kRouteSplitK = 4,         // 256 x 256 tiles over k slices into fp32 partials, then the reduce / epilogue launch
-    kRouteStaged = 5,         // whatever takes the shape without scratch
+    kRouteSplitK = 3,         // 256 x 256 tiles over k slices into fp32 partials, then the reduce / epilogue launch
+    kRouteOther = 4,          // the best tile_plan for the scratch there is, or the register-staged kernel
 };
 
 struct GemmPlan {
     int route;
-    GemmArgs head;            // the launch of every route (kRouteRingKTail: K already shortened to a multiple of 32)
+    GemmArgs head;            // the launch of every route
     GemmArgs tail;            // kRouteRingThenSmall only: the strip
     int slices;               // kRouteSplitK
-    bool big, exact;          // kRouteStaged: 256 x 256 tiles / unguarded instantiation
-    const void* ktail_a;      // kRouteRingKTail: A's part of the extra step (inside A[0])
-    int ktail_zero_rows;      // kRouteRingKTail: leading rows of the copied 32 rows of B that must be zero
+    bool big;                 // register-staged kernel: 256 x 256 tiles
 };
 
 // The plan of a call whose scratch is that of gemm_workspace_bytes, or none (a call with the scratch that tile_plan asks

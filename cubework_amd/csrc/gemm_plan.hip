@@ -16,7 +16,7 @@ int gemm_bf16_split_slices(int64_t M, int64_t N, int64_t K, int n_steps) {
     return slices;
 }
 
-int64_t gemm_bf16_ktail_workspace_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_steps) {
+static int64_t ragged_k_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_steps) {
     if (layout == CW_NT || n_steps != 1 || K < 64 || (K % 32) == 0 || (K % 8) != 0) return 0;
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
     if (tiles < 128 || M < 256 || N < 256 || (N % 8) != 0) return 0;
@@ -34,7 +34,7 @@ int64_t gemm_workspace_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_
         if (tiles128 >= 192 && K * n_steps < 12288) return 0;
         return (int64_t)slices * M * N * (int64_t)sizeof(float);
     }
-    return gemm_bf16_ktail_workspace_bytes(layout, M, N, K, n_steps);
+    return ragged_k_bytes(layout, M, N, K, n_steps);
 }
 
 int gemm_prepare_args(int layout, int64_t M, int64_t N, int64_t K, int n_steps, const void* const* A_steps, int64_t lda,
@@ -132,15 +132,10 @@ GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool
                          (args.bias == nullptr || args.vec_bias) && (args.n_addends == 0 || args.vec_add);
     const int64_t tiles256 = (int64_t)((args.M + 255) / 256) * ((args.N + 255) / 256);
     const bool big = tiles256 >= 128;
-    const int tile = big ? 256 : 128;
-    const bool exact = all_vec && (args.M % tile) == 0 && (args.N % tile) == 0 && (args.K % gemm_bf16::kBK) == 0;
     plan.big = big;
-    plan.exact = exact;
     const bool ring_ok = args.n_steps > 0 && args.n_steps <= kRingMaxSteps && args.n_addends <= kRingMaxAddends && dma_enabled;
-    // The LDS-DMA kernel takes M and N that are not tile multiples (its last tiles overlap their
-    // neighbours): a vocabulary slice of 12568 columns is 50 tiles instead of 49.1. What it needs is one
-    // full tile in each direction and 16-byte steps wherever a tile origin moves along a contiguous
-    // dimension (N always: the output and a [K, N] operand; M for a [K, M] operand).
+    // 256 x 256 tiles also for M and N that are not tile multiples (a vocabulary slice of 12568 columns is 50 tiles instead
+    // of 49.1), from one full tile in each direction on.
     const bool edges_ok = args.M >= 256 && args.N >= 256 && (args.N % 8) == 0 && (layout != CW_TN || (args.M % 8) == 0);
     // Fewer than 160 tiles of 256 x 256 (at 128 .. 159 of them the large tiles leave 40 % of the compute units
     // idle, and four times as many small tiles fill them): the ring kernel with 128 x 128 tiles, unless a long
@@ -207,28 +202,12 @@ GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool
         plan.route = kRouteRing;
         return plan;
     }
-    // A reduction length that is not a multiple of the k tile (a vocabulary slice as K: 12568 = 392 x 32 +
-    // 24), with B stored [K, N]: the regular step covers the first K - K % 32 columns, one more step of 32
-    // covers [K-32, K) with a copy of B's last 32 rows whose overlapping rows are zero. The copy (64 bytes
-    // per column) lives in the caller's scratch and has B's row pitch, which the steps share.
-    if (big && all_vec && ring_ok && edges_ok && layout != CW_NT && args.n_steps == 1 && args.K >= 64 &&
-        (args.K % 32) != 0 && (args.K % 8) == 0 && args.workspace != nullptr && aligned16(args.workspace) &&
-        args.workspace_bytes >= 32 * args.ldb * (int64_t)sizeof(uint16_t)) {
-        const int kr = args.K % 32;
-        // A's part of the step: columns (NN, A is [M, K]) or rows (TN, A is [K, M]) K-32 .. K-1, in place
-        const uint16_t* a0 = reinterpret_cast<const uint16_t*>(args.A[0]);
-        plan.ktail_a = layout == CW_TN ? a0 + (int64_t)(args.K - 32) * args.lda : a0 + (args.K - 32);
-        plan.ktail_zero_rows = 32 - kr;
-        plan.head.K = args.K - kr;
-        plan.route = kRouteRingKTail;
-        return plan;
-    }
     if (splits && all_vec && args.n_addends <= kRingMaxAddends && dma_enabled) {
         plan.slices = slices;
         plan.route = kRouteSplitK;
         return plan;
     }
-    plan.route = kRouteStaged;
+    plan.route = kRouteOther;
     return plan;
 }
 

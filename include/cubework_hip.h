@@ -124,15 +124,12 @@ int cw_gemm_ksteps(int layout, int64_t M, int64_t N, int64_t K, int n_steps,
  * step is split over several workgroups per tile, whose fp32 partial sums go
  * through `workspace` and are added in a fixed order (bit-reproducible; the
  * reference leaves this choice, and its scratch, to the BLAS library inside
- * torch.matmul). The scratch also serves a large product whose reduction
- * length is not a multiple of the kernel's k tile and whose B is stored [K, N]
- * (the input gradient dC W of the vocabulary-slice classifiers,
- * parallel_2d/_operation.py:408, parallel_1d/module.py:209: K = 12568): 32 rows
- * of B are copied there, zero-padded, for one short extra k step.
- * cw_gemm_workspace_bytes gives the size that enables either (0 when the shape
- * uses neither); with workspace NULL or smaller the call behaves exactly like
- * cw_gemm_ksteps (same results, a slower kernel). The scratch must not be
- * shared by calls that may overlap on the device.
+ * torch.matmul). cw_gemm_workspace_bytes gives the size of that split over
+ * 256 x 256 tiles (0 when the shape does not use it). For a large product whose
+ * reduction length is no multiple of 32 and whose B is stored [K, N] it still
+ * gives 32 rows of B, which nothing reads: callers may leave it out. With
+ * workspace NULL or smaller the call is planned for what it has. The scratch must
+ * not be shared by calls that may overlap on the device.
  */
 int64_t cw_gemm_workspace_bytes(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int io_dtype);
 /*

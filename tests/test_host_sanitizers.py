@@ -1,6 +1,6 @@
 """The library's host-side planning and validation code under the address and undefined-behaviour sanitizers, on
 the CPU: tests/host/plan_harness.hip drives cubework_amd/csrc/gemm_plan.hip (argument checks of cw_gemm_ksteps,
-the choice of kernel, strip / k-tail / split-k cuts, scratch sizes, the column sums' slabs) over ragged, huge,
+the choice of kernel, whole, sliced and strip tiles, scratch sizes, the column sums' slabs) over ragged, huge,
 zero and misaligned shapes and checks that every launch a plan describes stays inside the caller's buffers.
 No GPU call is made. hipcc compiles the three small translation units in a few seconds."""
 import os
