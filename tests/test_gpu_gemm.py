@@ -235,14 +235,31 @@ def test_kstep_sum_equals_concatenated_gemm():
 
 @pytest.mark.parametrize("layout", LAYOUTS)
 def test_bf16_split_k_long_reduction(layout):
-    # 2 x 3 output tiles of 256x256 and k = 2 x 1024: few tiles, long reduction -> the k range of every
-    # step is split over several workgroups per tile (cw_gemm_workspace_bytes > 0)
+    # a small output over k = 2 x 4096: every tile is cut along k (TN: the tile kernels take it without an activation only)
+    for M, N, K, steps in ((512, 768, 1024, 2), (256, 512, 4096, 2)):
+        if K == 4096:
+            assert 0 < _sliced_scratch(layout, M, N, K, steps, torch.bfloat16)
+        _run(layout, M, N, K, steps, torch.bfloat16, act="gelu_tanh", n_add=1, preact=True, seed=5)
+        _run(layout, M, N, K, steps, torch.bfloat16, act=None, bias=False, seed=6)
+        _run(layout, M, N, K, steps, torch.bfloat16, act=None, n_add=2, preact=True, seed=8)
+
+
+def _sliced_scratch(layout, M, N, K, steps, dtype):
+    """Bytes of fp32 partial sums of the launch that the operators make for aligned operands: 0 if no tile is cut along k."""
     from cubework_amd import _lib
     from cubework_amd.ops import LAYOUTS as CODES
 
-    assert _lib.load().cw_gemm_workspace_bytes(CODES[layout], 512, 768, 1024, 2, 0) > 0
-    _run(layout, 512, 768, 1024, 2, torch.bfloat16, act="gelu_tanh", n_add=1, preact=True, seed=5)
-    _run(layout, 512, 768, 1024, 2, torch.bfloat16, act=None, bias=False, seed=6)
+    code = _lib.CW_F16 if dtype == torch.float16 else _lib.CW_BF16
+    return _lib.load().cw_gemm_scratch_bytes(CODES[layout], M, N, K, steps, M if layout == "TN" else K, K if layout == "NT" else N, 1, 1, 0, code)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout,act", [("NT", "gelu_tanh"), ("TN", None)])
+def test_split_k_of_the_last_round_only(layout, act, dtype):
+    """525 tiles in rounds of 512: 512 whole ones and 13 cut along k, with every operand of the epilogue on both."""
+    M, N, K = 2600, 6160, 1032
+    assert 0 < _sliced_scratch(layout, M, N, K, 1, dtype) < 4 * M * N
+    _run(layout, M, N, K, 1, dtype, act=act, n_add=2, preact=True, seed=9)
 
 
 def test_split_k_matches_unsplit_call():
@@ -309,7 +326,7 @@ def test_ring_kernel_order_of_summation_is_fixed_per_shape_and_bounded_across_sh
     of the range per XCD), and only where M and N are tile multiples. So: (1) the same call twice gives the same
     bits; (2) the same logical product reached another way - as rows of a product whose M is not a tile multiple
     (no rotated start), or with CW_GEMM_IMPL=onelaunch in a fresh process for a shape whose last round of tiles
-    is otherwise peeled off into a second launch - may differ in the last bits, by no more than fp32
+    is otherwise cut along k - may differ in the last bits, by no more than fp32
     reassociation of the K-term sums allows: here at most one bf16 step of the largest magnitude, in few
     elements."""
     import os
@@ -328,16 +345,17 @@ def test_ring_kernel_order_of_summation_is_fixed_per_shape_and_bounded_across_sh
     diff = (c1.float() - ragged.float()).abs()
     assert diff.max().item() <= step
     assert (diff > 0).float().mean().item() < 0.05
-    # the second launch for a mostly empty last round, against the one launch (read once per process: a fresh one)
-    Ms, Ns, Ks = 4096, 4376, 128
+    # a mostly empty last round cut along k, against whole tiles in one launch (read once per process: a fresh one)
+    Ms, Ns, Ks = 2600, 6160, 1032
+    assert 0 < _sliced_scratch("NT", Ms, Ns, Ks, 1, torch.bfloat16) < 4 * Ms * Ns
     a2 = randn((Ms, Ks), torch.bfloat16, 73)
-    b2 = randn((Ks, Ns), torch.bfloat16, 74, 0.05)
-    here = ops.gemm_ksteps("NN", [a2.to(DEV)], [b2.to(DEV)]).cpu()
+    b2 = randn((Ns, Ks), torch.bfloat16, 74, 0.05)
+    here = ops.gemm_ksteps("NT", [a2.to(DEV)], [b2.to(DEV)]).cpu()
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     code = ("import sys, torch; sys.path.insert(0, %r)\n"
             "from tests.util import randn\nfrom cubework_amd import ops\n"
             "a = randn((%d, %d), torch.bfloat16, 73).to('cuda:0'); b = randn((%d, %d), torch.bfloat16, 74, 0.05).to('cuda:0')\n"
-            "torch.save(ops.gemm_ksteps('NN', [a], [b]).cpu(), sys.argv[1])\n" % (root, Ms, Ks, Ks, Ns))
+            "torch.save(ops.gemm_ksteps('NT', [a], [b]).cpu(), sys.argv[1])\n" % (root, Ms, Ks, Ns, Ks))
     import tempfile
     with tempfile.TemporaryDirectory() as tmp:
         path = os.path.join(tmp, "c.pt")
@@ -347,5 +365,6 @@ def test_ring_kernel_order_of_summation_is_fixed_per_shape_and_bounded_across_sh
         other = torch.load(path, weights_only=True)
     step = here.float().abs().max().item() * 2.0 ** -8
     diff = (here.float() - other.float()).abs()
+    assert diff.max().item() > 0  # the two launches do sum in another order
     assert diff.max().item() <= step
     assert (diff > 0).float().mean().item() < 0.05

@@ -8,7 +8,7 @@ float16), the rtol of the reference's own tests (tests/test_2d/check_2d_modules.
 import pytest
 import torch
 
-from tests.test_gpu_gemm import LAYOUTS, _run
+from tests.test_gpu_gemm import LAYOUTS, _run, _sliced_scratch
 from tests.util import assert_parity, rand_uniform, randn
 
 pytestmark = pytest.mark.gpu
@@ -54,11 +54,9 @@ def test_f16_epilogues_with_preact_and_addends(act):
 
 @pytest.mark.parametrize("layout", LAYOUTS)
 def test_f16_split_k_long_reduction(layout):
-    from cubework_amd import _lib
-    from cubework_amd.ops import LAYOUTS as CODES
-
-    assert _lib.load().cw_gemm_workspace_bytes(CODES[layout], 512, 768, 1024, 2, _lib.CW_F16) > 0
     _run(layout, 512, 768, 1024, 2, F16, act="gelu_tanh", n_add=1, preact=True, seed=5)
+    assert 0 < _sliced_scratch(layout, 256, 512, 4096, 2, F16)     # every tile is cut along k
+    _run(layout, 256, 512, 4096, 2, F16, act=None if layout == "TN" else "gelu_tanh", n_add=1, preact=True, seed=5)
 
 
 def test_f16_differs_from_bf16_reading_of_the_same_bits():

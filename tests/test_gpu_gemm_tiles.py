@@ -114,3 +114,28 @@ def test_no_epilogue_ignores_a_bias_pointer(layout, M, N, K, dtype, pad, sliced)
         assert torch.equal(with_bias, _abi_gemm(layout, a, b, None, _lib.CW_EPI_NONE, scratch, addend))
         want = a.double().cpu() @ (b.double().cpu().t() if layout == "NT" else b.double().cpu()) + (0 if addend is None else addend.double().cpu())
         assert_parity(with_bias, want, dtype, "no epilogue beside a bias pointer")
+
+
+# Calls whose scratch is less than the best plan's: none, or cw_gemm_workspace_bytes
+@pytest.mark.parametrize("layout,M,N,K,workspace", [
+    ("NN", 256, 512, 8192, False),     # 128 x 128 tiles
+    ("NT", 2600, 6160, 1024, False),   # 256 x 256 tiles
+    ("NT", 4352, 4096, 1024, False),   # 256 x 256 tiles and a strip of 256 rows
+    ("TN", 256, 256, 16384, True),     # 256 x 256 tiles in eight slices
+    ("NT", 2600, 6160, 1032, False),   # the best plan without scratch
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_calls_with_less_scratch(layout, M, N, K, workspace, dtype):
+    from cubework_amd import _lib
+    from cubework_amd.ops import LAYOUTS, _dtype_code, _ld
+
+    a = randn((K, M) if layout == "TN" else (M, K), dtype, 1)
+    b = randn((N, K) if layout == "NT" else (K, N), dtype, 2, 0.05)
+    bias, add = randn((N,), dtype, 3), randn((M, N), dtype, 4)
+    lib, code = _lib.load(), LAYOUTS[layout]
+    scratch = lib.cw_gemm_workspace_bytes(code, M, N, K, 1, _dtype_code(a)) if workspace else 0
+    assert scratch < lib.cw_gemm_scratch_bytes(code, M, N, K, 1, _ld(a), _ld(b), 1, 1, 0, _dtype_code(a))
+    assert (scratch > 0) == workspace
+    got = _abi_gemm(layout, a.cuda(), b.cuda(), bias.cuda(), _lib.CW_EPI_BIAS, scratch, add.cuda())
+    want = (a.float().t() if layout == "TN" else a.float()) @ (b.float().t() if layout == "NT" else b.float()) + bias.float() + add.float()
+    assert_parity(got, want, dtype, "%s %dx%dx%d with %d bytes of scratch" % (layout, M, N, K, scratch))
