@@ -139,3 +139,18 @@ def test_calls_with_less_scratch(layout, M, N, K, workspace, dtype):
     got = _abi_gemm(layout, a.cuda(), b.cuda(), bias.cuda(), _lib.CW_EPI_BIAS, scratch, add.cuda())
     want = (a.float().t() if layout == "TN" else a.float()) @ (b.float().t() if layout == "NT" else b.float()) + bias.float() + add.float()
     assert_parity(got, want, dtype, "%s %dx%dx%d with %d bytes of scratch" % (layout, M, N, K, scratch))
+
+
+@pytest.mark.parametrize("M,N,K,steps", [(1992, 2040, 4099, 1), (1992, 2040, 1030, 2), (2048, 2048, 8192, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_weight_gradient_of_one_block_per_unit(M, N, K, steps, dtype):
+    """At most one block per compute unit: ragged tiles, a reduction that ends inside a trip, a seam of two steps."""
+    import oracle
+    from cubework_amd import ops
+
+    A = [randn((K, M), dtype, 3 * i) for i in range(steps)]
+    B = [randn((K, N), dtype, 3 * i + 1, std=0.05) for i in range(steps)]
+    add = [randn((M, N), dtype, 91)]
+    want = oracle.gemm_ksteps("TN", A, B, None, None, add)
+    got = ops.gemm_ksteps("TN", [a.cuda() for a in A], [b.cuda() for b in B], None, None, [t.cuda() for t in add])
+    assert_parity(got, want, dtype, "TN %dx%dx%d steps=%d" % (M, N, K, steps))
