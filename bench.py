@@ -1270,8 +1270,8 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": measured_traffic(),
                      "traffic_source": "profiles/gemm_bf16_dma_kernel_linear2d_q2_counters.txt (committed counter runs of "
-                                       "this script, not measured in this run)",
-                     "kernel": "the launch cw_gemm_ksteps makes for this shape (gemm_bf16_dma_kernel, 256x256 tiles; "
+                                       "this script on the kernel's predecessor, same tiles; not measured in this run)",
+                     "kernel": "the launch cw_gemm_ksteps makes for this shape (gemm_tile_kernel, 256x256 tiles; "
                                "name as the kernel trace of this command shows it)",
                      "avg_launch_us": round(kernel_us, 2), "launches": args.sustained if args.sustained > 0 else args.steps,
                      "timed_steps": {"avg_launch_us": round(steps_us, 2),

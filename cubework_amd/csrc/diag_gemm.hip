@@ -1,6 +1,6 @@
 // Measurement aid (libcubework_diag.so, loaded by bench.py only): the 256 x 256 tile kernel of the block GEMM with one part
 // taken out, so that the part's share of a launch - in time and, through the socket's energy counter, in joules -
-// can be read as a difference against the whole kernel. Same source as the library's kernel (gemm_bf16_dma.h),
+// can be read as a difference against the whole kernel. Same source as the library's kernel (gemm_tile.h),
 // another value of its ABL template parameter:
 //   part 0  the whole kernel (the instantiation the library launches for this shape)
 //   part 1  the k loop issues no operand loads: the four LDS stages are filled once and re-used

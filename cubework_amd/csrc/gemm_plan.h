@@ -48,6 +48,7 @@ GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool
 // blocks per compute unit, and what a trip costs (us; one block on the unit / two) and a block besides its trips. The
 // costs are a fit to 2000 launches over 110 shapes (products of 64 .. 8192 tokens with the model widths 768 .. 4096, in the
 // forward and weight-gradient orientations; rms error 11 %); choosing by them comes within 2 % of the best choice on average.
+// (The launches' times are not kept in this tree: a change of the kernels' speed means measuring and fitting again.)
 struct TileConfig {
     int tm, tn, kb, stages, resident;
     float trip1, trip2, fixed;

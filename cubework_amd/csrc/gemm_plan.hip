@@ -256,12 +256,15 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     if (n_pack_addends > 0) p.pack_add_bytes = copy_bytes(n_pack_addends, M, N);
     // the kernels' lane offsets: 256 rows (or 32 k rows) of either operand within 2 GB
     if (p.lda >= ((int64_t)1 << 22) || p.ldb >= ((int64_t)1 << 22)) return best;
-    // A forward product (B stored [K, N]) that does not reduce its width, K <= N - the projections in front of an
-    // activation - sums k in ascending order whatever the tile: the 16-bit results of a row do not depend on how many rows
-    // there are, and a ReLU behind the next layer sees the same signs. Slicing gains little there anyway (the outputs have
-    // tiles enough). Two exceptions, fixed by the shape as well: whole rounds of 256 x 256 tiles start at an XCD-
-    // dependent k (memory channels, gemm_tile.h), and a few aligned tiles with a long reduction are always cut into the
-    // same slices.
+    // An NN product (B stored [K, N]) that does not reduce its width, K <= N, sums k in ascending order whatever the tile: the
+    // 16-bit results of a row do not depend on how many rows there are, and a ReLU behind the next layer sees the same signs.
+    // That is the forward of the 2D and 3D layers' projections in front of an activation; by the same rule the 1D layers' input
+    // gradient, which is NN too, while their forward is NT and is cut like any other product. Slicing gains little there
+    // anyway (the outputs have tiles enough). Two exceptions, fixed by the shape, where a row's sums are taken in another order
+    // than those of a batch off the multiples of 256: whole rounds of 256 x 256 tiles start at an XCD-dependent k (memory
+    // channels, gemm_tile.h), and M and N multiples of 256 with few tiles and K x steps >= 2048 are always cut as
+    // gemm_bf16_split_slices says. The second keeps the bits that these shapes have had, at a price: by the cost model below
+    // 512 x 2048 x 2048 (M x K x N) takes 30 us, and 12 us on unsliced 64 x 64 tiles.
     const bool ordered = layout == CW_NN && K <= N;
     const bool rotated = ordered && M % 256 == 0 && N % 256 == 0 && K % 32 == 0 && (M / 256) * (N / 256) >= 160;
     const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);

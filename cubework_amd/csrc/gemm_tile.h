@@ -157,9 +157,12 @@ __device__ __forceinline__ void tile_origin(int tile, int tiles_m, int tiles_n, 
     tn = in_group / gsz;
 }
 
-// gelu(x) = x/2 erfc(-x / sqrt 2) without branches (erff has some, and see Epilogue::stage): erfc(z) = t exp(-z^2 + q(t)),
-// t = 1 / (1 + z/2), for z >= 0, with q a least-squares fit of degree 9 in Chebyshev points of log(erfc(z) e^(z^2) / t);
-// relative error below 2e-6, where the result is rounded to 2^-9 or 2^-12.
+// gelu(x) = x/2 erfc(-x / sqrt 2) without branches (erff has some, and see Epilogue::stage). erfc(z) = t exp(-z^2 + q(t)),
+// t = 1 / (1 + z/2), z >= 0, is the form that "Numerical Recipes" gives for erfc; q here is a least-squares fit of degree 9 of
+// its own, in Chebyshev points of log(erfc(z) e^(z^2) / t). In float32 against float64: relative error 5e-7 for |x| < 1
+// (x/2 (1 + erf) has 2e-7 there), 1.3e-6 for -3 < x < -1, 2e-6 for -4 < x < -3 and, growing with the exponent's rounding,
+// 3e-6, 7e-6 and 2e-5 down to x = -5.5, -8 and -13 (x/2 (1 + erf) cancels there: 5e-4 at -4, all digits below -5.5). The
+// result is rounded to 2^-9 or 2^-12. The register-staged kernel and the backward use erff.
 __device__ __forceinline__ float gelu_erf_smooth(float x) {
     const float z = fabsf(x) * 0.7071067811865476f;
     const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.5f, z, 1.0f));
