@@ -1014,7 +1014,7 @@ def energy_table(device, sets, bias, outs, seconds):
         return call
 
     runs = {}
-    for name, part, rotate in (("whole_kernel_operands_from_hbm", 0, True), ("whole_kernel_operands_cache_resident", 0, False),
+    for name, part, rotate in (("whole_kernel_operands_from_hbm", 4, True), ("whole_kernel_operands_cache_resident", 4, False),
                                ("no_operand_loads_in_the_k_loop", 1, False), ("no_lds_fragment_reads_in_the_k_loop", 3, False),
                                ("no_epilogue", 2, False)):
         fn = make(part, rotate)

@@ -1,14 +1,14 @@
-// Measurement aid (libcubework_diag.so, loaded by bench.py only): the 256 x 256 tile kernel of the block GEMM with one part
-// taken out, so that the part's share of a launch - in time and, through the socket's energy counter, in joules -
-// can be read as a difference against the whole kernel. Same source as the library's kernel (gemm_tile.h),
-// another value of its ABL template parameter:
-//   part 0  the whole kernel (the instantiation the library launches for this shape)
+// Measurement aid (libcubework_diag.so, loaded by bench.py only): the block GEMM's launch for the headline shape, and a
+// 256 x 256 tile kernel with one part taken out, so that the part's share of a launch - in time and, through the socket's
+// energy counter, in joules - can be read as a difference against the same kernel whole:
+//   part 0  the library's launch for this shape (gemm_wide.h)
+//   part 4  the kernel of 4 wavefronts and 32x32x16 matrix instructions (gemm_tile.h's template on 4 x 4 tiles), whole; of it
 //   part 1  the k loop issues no operand loads: the four LDS stages are filled once and re-used
 //   part 2  no epilogue: no bias / activation arithmetic, nothing stored
 //   part 3  the k loop reads no fragments from LDS: the first tile's stay in the registers
 // NN layout, bf16, bias + GeLU(tanh) epilogue, tile-aligned shapes with at least 128 tiles, 1 to 4 k-steps:
 // the headline shape of the benchmark. Results of parts 1 to 3 are meaningless as numbers.
-#include "gemm_tile.h"
+#include "gemm_wide.h"
 
 namespace cw {
 namespace {
@@ -33,10 +33,10 @@ using namespace cw;
 extern "C" int cw_diag_gemm_part(int part, int64_t M, int64_t N, int64_t K, int n_steps, const void* const* A_steps,
                                  int64_t lda, const void* const* B_steps, int64_t ldb, const void* bias, void* C,
                                  int64_t ldc, void* stream) {
-    if (part < 0 || part > 3) return fail(CW_ERR_INVALID, "cw_diag_gemm_part: part %d outside [0, 3]", part);
+    if (part < 0 || part > 4) return fail(CW_ERR_INVALID, "cw_diag_gemm_part: part %d outside [0, 4]", part);
     if (n_steps < 1 || n_steps > kMaxSteps || A_steps == nullptr || B_steps == nullptr || bias == nullptr || C == nullptr)
         return fail(CW_ERR_INVALID, "cw_diag_gemm_part: 1 to %d k-steps, operands, bias and C are needed", kMaxSteps);
-    if (M < 256 || N < 256 || K < 128 || (M % 256) != 0 || (N % 256) != 0 || (K % 64) != 0 || (M / 256) * (N / 256) < 128 ||
+    if (M < 256 || N < 256 || K < 192 || (M % 256) != 0 || (N % 256) != 0 || (K % 64) != 0 || (M / 256) * (N / 256) < 128 ||
         M > (1 << 24) || N > (1 << 24) || K > (1 << 24))
         return fail(CW_ERR_UNSUPPORTED, "cw_diag_gemm_part: tile-aligned shapes with at least 128 tiles of 256 x 256 only");
     if (lda < K || ldb < N || ldc < N || (lda % 8) != 0 || (ldb % 8) != 0 || (ldc % 8) != 0)
@@ -66,9 +66,10 @@ extern "C" int cw_diag_gemm_part(int part, int64_t M, int64_t N, int64_t K, int 
     args.rotate = 1;
     hipStream_t s = (hipStream_t)stream;
     switch (part) {
-        case 0: return launch_part<0>(args, s);
+        case 0: return gemm_wide::launch_rows<false, true, 8, CW_EPI_BIAS_GELU_TANH, bf16_t>(args, s);
         case 1: return launch_part<1>(args, s);
         case 2: return launch_part<2>(args, s);
-        default: return launch_part<3>(args, s);
+        case 3: return launch_part<3>(args, s);
+        default: return launch_part<0>(args, s);
     }
 }

@@ -15,13 +15,17 @@
 
 namespace cw {
 
-#define CW_TILE_CFGS(e, l) {gemm_tile_##e##_##l##_0, gemm_tile_##e##_##l##_1, gemm_tile_##e##_##l##_2, gemm_tile_##e##_##l##_3, gemm_tile_##e##_##l##_4}
+#define CW_TILE_CFGS(e, l) {gemm_tile_##e##_##l##_1, gemm_tile_##e##_##l##_2, gemm_tile_##e##_##l##_3, gemm_tile_##e##_##l##_4}
+#define CW_WIDE_ROWS(e, l) {gemm_wide_##e##_##l##_160, gemm_wide_##e##_##l##_192, gemm_wide_##e##_##l##_224, gemm_wide_##e##_##l##_256}
 #define CW_TILE_DECL(e, l)                                              \
-    int gemm_tile_##e##_##l##_0(const TileArgs&, int, hipStream_t);     \
     int gemm_tile_##e##_##l##_1(const TileArgs&, int, hipStream_t);     \
     int gemm_tile_##e##_##l##_2(const TileArgs&, int, hipStream_t);     \
     int gemm_tile_##e##_##l##_3(const TileArgs&, int, hipStream_t);     \
-    int gemm_tile_##e##_##l##_4(const TileArgs&, int, hipStream_t);
+    int gemm_tile_##e##_##l##_4(const TileArgs&, int, hipStream_t);     \
+    int gemm_wide_##e##_##l##_160(const TileArgs&, int, hipStream_t);   \
+    int gemm_wide_##e##_##l##_192(const TileArgs&, int, hipStream_t);   \
+    int gemm_wide_##e##_##l##_224(const TileArgs&, int, hipStream_t);   \
+    int gemm_wide_##e##_##l##_256(const TileArgs&, int, hipStream_t);
 CW_TILE_DECL(bf16_t, NN)
 CW_TILE_DECL(bf16_t, NT)
 CW_TILE_DECL(bf16_t, TN)
@@ -30,9 +34,13 @@ CW_TILE_DECL(f16_t, NT)
 CW_TILE_DECL(f16_t, TN)
 
 using TileLaunch = int (*)(const TileArgs&, int, hipStream_t);
-static constexpr TileLaunch kTileLaunch[2][3][kTileConfigCount] = {
+static constexpr TileLaunch kTileLaunch[2][3][kTileConfigCount - 1] = {
     {CW_TILE_CFGS(bf16_t, NN), CW_TILE_CFGS(bf16_t, NT), CW_TILE_CFGS(bf16_t, TN)},
     {CW_TILE_CFGS(f16_t, NN), CW_TILE_CFGS(f16_t, NT), CW_TILE_CFGS(f16_t, TN)},
+};
+static constexpr TileLaunch kWideLaunch[2][3][4] = {
+    {CW_WIDE_ROWS(bf16_t, NN), CW_WIDE_ROWS(bf16_t, NT), CW_WIDE_ROWS(bf16_t, TN)},
+    {CW_WIDE_ROWS(f16_t, NN), CW_WIDE_ROWS(f16_t, NT), CW_WIDE_ROWS(f16_t, TN)},
 };
 static_assert(CW_NN == 0 && CW_NT == 1 && CW_TN == 2, "kTileLaunch is indexed by layout");
 
@@ -111,7 +119,8 @@ static int tile_launch(const GemmArgs& g, const TilePlan& plan, int layout, int 
     a.slices = plan.slices;
     a.rotate = plan.rotate ? 1 : 0;
     a.partial = reinterpret_cast<float*>(ws + plan.pack_a_bytes + plan.pack_b_bytes + plan.pack_add_bytes);
-    return kTileLaunch[f16 ? 1 : 0][layout][plan.cfg](a, epilogue, s);
+    if (plan.cfg == 0) return kWideLaunch[f16 ? 1 : 0][layout][(plan.rows - 160) / 32](a, epilogue, s);
+    return kTileLaunch[f16 ? 1 : 0][layout][plan.cfg - 1](a, epilogue, s);
 }
 
 // A plan of one configuration without scratch for operand copies (slices > 1: every tile sliced, partial sums in g.workspace).
@@ -119,6 +128,7 @@ static TilePlan tile_plan_of(const GemmArgs& g, int cfg, int slices = 1) {
     TilePlan p = {};
     const int bm = 64 * kTileConfigs[cfg].tm, bn = 64 * kTileConfigs[cfg].tn;
     p.cfg = cfg;
+    p.rows = cfg == 0 ? wide_rows(g.M) : bm;
     p.tiles = (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn);
     p.full = slices > 1 ? 0 : (int)p.tiles;
     p.slices = slices;
@@ -169,9 +179,10 @@ int gemm_half_launch(const GemmArgs& args, int layout, int epilogue, bool f16, h
     const GemmPlan plan = gemm_half_plan(args, layout, tiles_ok, strip_split_enabled());
     switch (plan.route) {
         case kRouteSmallRing: return tile_launch(args, tile_plan_of(args, 2), layout, epilogue, f16, s);
-        case kRouteRing: return tile_launch(args, tile_plan_of(args, 0), layout, epilogue, f16, s);
+        case kRouteRing: return tile_launch(args, tile_plan_of(args, wide_takes(layout, args.K, args.n_steps, false, false) ? 0 : 1), layout, epilogue, f16, s);
         case kRouteRingThenSmall: {
-            if (const int rc = tile_launch(plan.head, tile_plan_of(plan.head, 0), layout, epilogue, f16, s); rc != CW_OK) return rc;
+            const int head = wide_takes(layout, args.K, args.n_steps, false, false) ? 0 : 1;
+            if (const int rc = tile_launch(plan.head, tile_plan_of(plan.head, head), layout, epilogue, f16, s); rc != CW_OK) return rc;
             return tile_launch(plan.tail, tile_plan_of(plan.tail, 2), layout, epilogue, f16, s);
         }
         case kRouteSplitK: return tile_launch(args, tile_plan_of(args, 0, plan.slices), layout, epilogue, f16, s);

@@ -226,6 +226,17 @@ constexpr int64_t kTileLaunchMax = ((int64_t)1 << 24) - 8;
 
 }  // namespace
 
+bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b) {
+    const bool a_ok = layout == CW_TN || K % 8 == 0 || pack_a, b_ok = layout != CW_NT || K % 8 == 0 || pack_b;
+    return a_ok && b_ok && (K + 63) / 64 * n_steps >= 3;
+}
+
+int wide_rows(int64_t M) {
+    for (int rows : {160, 192, 224})
+        if ((M + rows - 1) / rows == (M + 255) / 256) return rows;
+    return 256;
+}
+
 TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int64_t lda, int64_t ldb, bool align_a, bool align_b,
                    int n_pack_addends, int64_t max_scratch) {
     TilePlan best;
@@ -260,33 +271,33 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     // 16-bit results of a row do not depend on how many rows there are, and a ReLU behind the next layer sees the same signs.
     // That is the forward of the 2D and 3D layers' projections in front of an activation; by the same rule the 1D layers' input
     // gradient, which is NN too, while their forward is NT and is cut like any other product. Slicing gains little there
-    // anyway (the outputs have tiles enough). Two exceptions, fixed by the shape, where a row's sums are taken in another order
+    // anyway (the outputs have tiles enough). One exception, fixed by the shape, where a row's sums are taken in another order
     // than those of a batch off the multiples of 256: whole rounds of 256 x 256 tiles start at an XCD-dependent k (memory
-    // channels, gemm_tile.h), and M and N multiples of 256 with few tiles and K x steps >= 2048 are always cut as
-    // gemm_bf16_split_slices says. The second keeps the bits that these shapes have had, at a price: by the cost model below
-    // 512 x 2048 x 2048 (M x K x N) takes 30 us, and 12 us on unsliced 64 x 64 tiles.
+    // channels, gemm_tile.h). (The 16x16x32 instruction of configuration 0 and the 32x32x16 one of the others give the same bits.)
     const bool ordered = layout == CW_NN && K <= N;
     const bool rotated = ordered && M % 256 == 0 && N % 256 == 0 && K % 32 == 0 && (M / 256) * (N / 256) >= 160;
-    const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
-    const int fixed_slices = ordered && !(tiles128 >= 192 && K * n_steps < 12288) ? gemm_bf16_split_slices(M, N, K, n_steps) : 1;
-    const double layout_factor = layout == CW_TN ? 0.9 : 1.0;  // both operands stream whole rows
+    const double small_factor = layout == CW_TN ? 0.9 : 1.0;  // gemm_tile.h: k-contiguous operands move as pieces of 64 bytes
     const double bytes = 2.0 * ((double)M * K * n_steps + (double)K * N * n_steps + (double)M * N);
     const double memory_us = bytes / 4.0e6;
     double best_us = 0;
     auto consider = [&](int cfg, int64_t tiles, int64_t full, int slices) {
         const TileConfig& c = kTileConfigs[cfg];
         const int64_t rest = tiles - full;
-        const double trips = (double)((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps;
+        double trips = (double)((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps;
         TilePlan q = p;
         q.cfg = cfg;
+        q.rows = cfg == 0 ? wide_rows(M) : 64 * c.tm;
         q.tiles = tiles;
         q.full = (int)full;
         q.slices = rest > 0 ? slices : 1;
-        q.rotate = ordered ? rotated : c.tm * c.tn == 16;
+        q.rotate = cfg == 0 && (!ordered || rotated);
         q.partial_bytes = rest * slices * (int64_t)(4096 * c.tm * c.tn) * 4;
         if (max_scratch >= 0 && q.scratch() > max_scratch) return;
-        double us = tile_rounds(c, (double)full, trips, layout_factor);
-        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor) + 5.0 + 2.0 * q.partial_bytes / 6.6e6;
+        const double layout_factor = cfg == 0 ? 1.0 : small_factor;
+        if (cfg == 0) trips *= 0.2 + 0.8 / 256 * q.rows;  // a lower tile's trips are shorter
+        // configuration 0: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's
+        double us = tile_rounds(c, (double)full, trips, layout_factor) + (cfg == 0 ? 3.0 : 0.0);
+        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor) + 5.0 + 2.0 * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
         us = us > memory_us ? us + 0.1 * memory_us : memory_us + 0.1 * us;
         if (best.cfg < 0 || us < best_us) {
             best = q;
@@ -296,11 +307,7 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     for (int cfg = 0; cfg < kTileConfigCount; ++cfg) {
         const TileConfig& c = kTileConfigs[cfg];
         const int64_t tiles = ((M + 64 * c.tm - 1) / (64 * c.tm)) * ((N + 64 * c.tn - 1) / (64 * c.tn));
-        if (tiles > kTileLaunchMax || ((rotated || fixed_slices > 1) && cfg != 0)) continue;
-        if (fixed_slices > 1) {
-            consider(cfg, tiles, 0, fixed_slices);
-            continue;
-        }
+        if (tiles > kTileLaunchMax || (cfg == 0 && !wide_takes(layout, K, n_steps, p.pack_a, p.pack_b))) continue;
         const int64_t trips = ((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps, cap = 256 * c.resident;
         consider(cfg, tiles, tiles, 1);
         // all tiles sliced, to fill the chip about once; or only those of the partial last round

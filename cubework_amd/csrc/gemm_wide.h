@@ -1,0 +1,592 @@
+// 16-bit block GEMM on tiles of up to 256 x 256 (gfx950): the kernel of every product with enough tiles.
+//
+//   - One block of 8 wavefronts (2 x 4) per compute unit walks through its tiles (grid: at most the 256 units). A wavefront
+//     owns 16 TM x 64 of the tile as TM x 4 accumulators of v_mfma_f32_16x16x32, two wavefronts share a SIMD. The loads run
+//     ahead over the seams of steps and of tiles, so that only the first tile of a block waits for memory, and a tile's stores
+//     drain under the next tile's products.
+//   - Operands go to LDS by buffer_load_dwordx4 ... lds in stages of 64 k, three stages of A and two of B: all 160 KB. Rows of 64
+//     k are whole 128-byte lines: with stages of 32 k a load instruction fetched 16 pieces of 64 bytes, and the load unit takes
+//     35 cycles for those against 17 (measured from L2, a compute unit: 29 and 61 bytes a cycle, where a tile needs 31).
+//   - One barrier per stage, behind the second row of MFMAs of its second k step: there this wavefront's fragments of the stage
+//     are all read, which frees the stage's LDS, and the next stage's first fragments are read under the remaining rows. LDS
+//     reads and loads stand singly between MFMAs.
+//   - 16x16x32 and not 32x32x16: the same FLOP with half of the accumulator traffic. On random operands, where the board's
+//     power cap sets the clock, 8192^3 NT took 784 us against 858 with everything else alike, and the same time on zeros. Both
+//     instructions give the same bits.
+//
+// What bounds it: matrix cores and the power cap. 8192 x 8192 x 2048 (M x N x K) in us, random bf16 from HBM, NT / NN / TN:
+// 199 / 203 / 206, the kernel of 4 wavefronts and 32x32x16 that it replaced 240 / 241 / 217; 8192 x 2048 x 2048: 53 / 54,
+// before 62 / 62 (a launch of one round: 6 of the 53 us are its epilogue, whose stores nothing hides).
+//
+// Whole 256-row tiles whose rows are mostly beyond M are wasted products: BM is 32 TM, the least of 160, 192, 224 and 256 that
+// covers M with as many tiles (gemm_plan.hip).
+#pragma once
+#include <cstddef>
+
+#include "gemm_tile.h"
+
+namespace cw {
+namespace gemm_wide {
+
+using gemm_bf16::bf16x8_t;
+using gemm_bf16::f32x16_t;
+using gemm_bf16::static_for;
+using gemm_bf16::u32x2_t;
+using gemm_bf16::u32x4_t;
+using gemm_tile::kRange;
+using gemm_tile::kTabA;
+using gemm_tile::kTabAddend;
+using gemm_tile::kTabB;
+using gemm_tile::lds_char;
+using gemm_tile::lds_u16;
+using gemm_tile::s16x4_t;
+using gemm_tile::s16x8_t;
+using gemm_tile::step_ptr;
+
+constexpr int kBK = 64;
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+template <typename E>
+__device__ __forceinline__ f32x4_t mfma_16x16x32(bf16x8_t a, bf16x8_t b, f32x4_t acc) {
+    if constexpr (std::is_same<E, f16_t>::value)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gemm_bf16::f16x8_t, a), __builtin_bit_cast(gemm_bf16::f16x8_t, b), acc, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+}
+
+// 16-byte chunks by which k row k of a k-slow image is rotated (xor)
+__device__ __forceinline__ int kslow_swizzle(int k) { return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1); }
+
+// Loader of one operand: ROWS operand rows x 64 k, 1 KB per load instruction, PER instructions per wavefront and stage.
+// k-contiguous image [ROWS][64 k]: chunk c of row r at c ^ ((r >> 1) & 7); k-slow image [64 k][ROWS]: chunk c of k row k
+// at c ^ kslow_swizzle(k).
+template <bool TRANS, int ROWS, int NW>
+struct Loader {
+    static constexpr int kBytes = ROWS * kBK * 2;
+    static constexpr int PER = ROWS / 8 / NW;
+    static constexpr int CPR = ROWS / 8;  // TRANS: 16-byte chunks per k row
+    static_assert(ROWS % (8 * NW) == 0 && (!TRANS || (ROWS & (ROWS - 1)) == 0), "whole instructions per wavefront");
+    uint32_t voff[PER];
+    // k position of the lane's chunk in instruction i (k row for TRANS)
+    static __device__ __forceinline__ int kpos(int lane, int wave, int i) {
+        const int j = wave * PER + i;
+        if constexpr (!TRANS) return ((lane & 7) ^ ((4 * j + (lane >> 4)) & 7)) * 8;
+        else return (j * 64 + lane) / CPR;
+    }
+    __device__ __forceinline__ void init(int lane, int wave, int64_t ld, int row0, int rmax) {
+        asm volatile("" : "+v"(lane));  // opaque: nothing of this is kept in registers between tiles
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int j = wave * PER + i, k = kpos(lane, wave, i);
+            if constexpr (!TRANS) {
+                const int r = 8 * j + (lane >> 3);
+                voff[i] = row0 + r < rmax ? (uint32_t)(((int64_t)r * ld + k) * 2) : kRange;
+            } else {
+                const int c = ((j * 64 + lane) % CPR) ^ kslow_swizzle(k);
+                voff[i] = row0 + c * 8 < rmax ? (uint32_t)(((int64_t)k * ld + c * 8) * 2) : kRange;
+            }
+        }
+    }
+    template <int I>
+    __device__ __forceinline__ void issue(const char* base, uint32_t lds_oper) const {
+        dma16_buffer(base, voff[I], lds_oper + I * 1024);
+    }
+    // the lane's chunks at k positions from k_rem on are not fetched (until the next init)
+    __device__ __forceinline__ void mask(int lane, int wave, int k_rem) {
+        asm volatile("" : "+v"(lane));
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (kpos(lane, wave, i) >= k_rem) voff[i] = kRange;
+    }
+};
+
+// Fragment reads of one operand: W MFMA tiles of 16 rows x 32 k per wavefront from operand row wrow on.
+template <bool TRANS, int ROWS, int W>
+struct Frags {
+    uint32_t off[TRANS ? W : 2];
+    __device__ __forceinline__ void init(int lane, int wrow) {
+        const int i = lane & 15, q = lane >> 4;
+        if constexpr (!TRANS) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) off[ks] = (uint32_t)((wrow + i) * 128 + (((4 * ks + q) ^ ((i >> 1) & 7)) << 4));
+        } else {
+            const int k = 8 * q + (i >> 2);
+#pragma unroll
+            for (int t = 0; t < W; ++t) off[t] = (uint32_t)(k * (ROWS * 2) + (((wrow / 8 + 2 * t + ((i & 3) >> 1)) ^ kslow_swizzle(k)) << 4) + 8 * (i & 1));
+        }
+    }
+    template <int T, int KS>
+    __device__ __forceinline__ bf16x8_t read(lds_char* oper) const {
+        if constexpr (!TRANS) {
+            return *(__attribute__((address_space(3))) const bf16x8_t*)(oper + off[KS] + T * 16 * 128);
+        } else {
+            lds_char* p = oper + off[T] + KS * 32 * (ROWS * 2);
+            const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)p);
+            const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + 4 * (ROWS * 2)));
+            const s16x8_t v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            return __builtin_bit_cast(bf16x8_t, v);
+        }
+    }
+};
+
+// What follows the sums: a wavefront's accumulators go through 4 KB of LDS of its own, one row of MFMA tiles (16 x 64 fp32)
+// at a time, and come back as 8 columns of a row per lane: bias, addends and results move as 16 bytes per lane, whole
+// 128-byte lines per 8 lanes, edges are a matter of one lane, and no accumulator is copied to another register.
+// Chunk c (4 columns) of row r stands at c ^ r: both directions are conflict free.
+constexpr int kPatch = 4096;
+template <int EPI, typename E>
+struct Out {
+    lds_char *wr, *rd;  // the lane's addresses in the wavefront's patch
+    int row, col, M, N;  // of the lane's piece in half 0 of row 0 of the tiles
+    bool whole;
+    u32x4_t bias;
+    __device__ __forceinline__ Out(const TileArgs& a, lds_char* patch, int row0, int col0, bool whole_tile, int lane) {
+        asm volatile("" : "+v"(lane));  // opaque: nothing of this is kept in registers between tiles
+        const int r = lane & 15, q = lane >> 4, rr = lane >> 3, c = lane & 7;
+        wr = patch + r * 256 + ((q ^ r) << 4);
+        rd = patch + rr * 256 + (((2 * c) ^ rr) << 4);
+        row = row0 + rr;
+        col = col0 + 8 * c;
+        M = a.M;
+        N = a.N;
+        whole = whole_tile;
+        bias = u32x4_t{0u, 0u, 0u, 0u};
+        if (a.bias != nullptr) {
+            const uint16_t* b = reinterpret_cast<const uint16_t*>(a.bias) + col;
+            if (whole && ((uintptr_t)a.bias & 15) == 0) {
+                bias = *reinterpret_cast<const u32x4_t*>(b);
+            } else {
+                uint32_t w[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) w[e] = col + e < N ? b[e] : 0u;
+                bias = u32x4_t{w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16};
+            }
+        }
+    }
+    static __device__ __forceinline__ lds_char* flip(lds_char* p, uint32_t bits) { return (lds_char*)(uintptr_t)((uint32_t)(uintptr_t)p ^ bits); }
+    __device__ __forceinline__ void put(const f32x4_t (&acc)[4]) const {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *(__attribute__((address_space(3))) f32x4_t*)flip(wr, 64 * j) = acc[j];
+    }
+    // half H (8 rows) of the row of tiles in the patch
+    template <int H>
+    __device__ __forceinline__ void get(float (&v)[8]) const {
+        lds_char* p = flip(rd, H * 128) + H * 2048;
+        const f32x4_t lo = *(__attribute__((address_space(3))) const f32x4_t*)p;
+        const f32x4_t hi = *(__attribute__((address_space(3))) const f32x4_t*)flip(p, 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = lo[e];
+            v[4 + e] = hi[e];
+        }
+    }
+    // an addend's piece of row r (16-byte aligned rows: the host copies others, so the last group of eight is whole memory)
+    __device__ __forceinline__ u32x4_t addend(const TileArgs& a, int k, int r) const {
+        const int last = (N - 1) & ~7;
+        const uint16_t* p = reinterpret_cast<const uint16_t*>(step_ptr(kTabAddend, k)) + (int64_t)(r < M ? r : M - 1) * a.ldadd;
+        return *reinterpret_cast<const u32x4_t*>(p + (col < last ? col : last));
+    }
+    static __device__ __forceinline__ void add(float (&v)[8], const u32x4_t& raw) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            v[2 * d] += half_conv<E>::lo(raw[d]);
+            v[2 * d + 1] += half_conv<E>::hi(raw[d]);
+        }
+    }
+    __device__ __forceinline__ void store(const float (&v)[8], void* dst, int64_t ld, int r) const {
+        u32x4_t o;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) o[d] = half_conv<E>::pack2(v[2 * d], v[2 * d + 1]);
+        uint16_t* out = reinterpret_cast<uint16_t*>(dst) + (int64_t)r * ld + col;
+        if (whole) {
+            *reinterpret_cast<u32x4_t*>(out) = o;
+        } else if (r < M) {
+            const int left = N - col;
+            if (left >= 8) {
+                __builtin_memcpy(out, &o, 16);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 7; ++e)
+                    if (e < left) out[e] = (uint16_t)(o[e >> 1] >> ((e & 1) * 16));
+            }
+        }
+    }
+    __device__ __forceinline__ void finish(float (&v)[8], const TileArgs& a, int r) const {
+        if (a.preact != nullptr) store(v, a.preact, a.ldp, r);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = gemm_tile::tile_act<EPI>(v[e]);
+        store(v, a.C, a.ldc, r);
+    }
+    template <int TM>
+    __device__ __forceinline__ void rows(const f32x4_t (&acc)[TM][4], const TileArgs& a) const {
+        put(acc[0]);
+        if (a.n_addends == 0) {
+            static_for<TM>([&](auto i) {
+                float v[2][8];
+                get<0>(v[0]);
+                get<1>(v[1]);
+                if constexpr (i.value + 1 < TM) put(acc[i.value + 1]);
+                add(v[0], bias);
+                add(v[1], bias);
+                int r = row + 16 * i.value;
+                asm volatile("" : "+v"(r));  // opaque: the addresses of a row are formed here and not for all rows at once
+                finish(v[0], a, r);
+                finish(v[1], a, r + 8);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        } else {
+            constexpr int G = TM < 2 ? 1 : 2;  // rows of tiles whose pieces of the first addend are requested together
+            u32x4_t raw[G][2];
+            static_for<TM>([&](auto i) {
+                if constexpr (i.value % G == 0) {
+#pragma unroll
+                    for (int g = 0; g < G && i.value + g < TM; ++g) {
+                        int r = row + 16 * (i.value + g);
+                        asm volatile("" : "+v"(r));
+                        raw[g][0] = addend(a, 0, r);
+                        raw[g][1] = addend(a, 0, r + 8);
+                    }
+                }
+                float v[2][8];
+                get<0>(v[0]);
+                get<1>(v[1]);
+                if constexpr (i.value + 1 < TM) put(acc[i.value + 1]);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    int r = row + 16 * i.value + 8 * h;
+                    asm volatile("" : "+v"(r));
+                    add(v[h], bias);
+                    add(v[h], raw[i.value % G][h]);
+                    for (int k = 1; k < a.n_addends; ++k) add(v[h], addend(a, k, r));
+                    finish(v[h], a, r);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        }
+    }
+};
+
+constexpr int WM = 2, WN = 4, NW = WM * WN, TN = 4;  // wavefronts; MFMA tiles of a wavefront along N
+constexpr int kThreads = 64 * NW, kUnits = 256;
+constexpr int kRows = 256;  // rows of either operand's LDS image (of A, BM of them are fetched)
+constexpr int BN = 16 * WN * TN;
+static_assert(BN == kRows, "");
+constexpr int kStagesA = 3, kStagesB = 2;
+constexpr size_t kLdsBytes = (size_t)(kStagesA + kStagesB) * kRows * kBK * 2;
+static_assert(kLdsBytes == 160 * 1024 && kRows * kBK * 2 >= NW * kPatch, "one block per compute unit; the epilogue's patches in a free stage of A");
+
+template <bool TRANS_A, bool TRANS_B, int TM, int EPI, typename E>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_wide_kernel(const TileArgs args) {
+    constexpr int BM = 16 * WM * TM;
+    using LA = Loader<TRANS_A, kRows, NW>;
+    using LB = Loader<TRANS_B, kRows, NW>;
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+    lds_char* lds_base = (lds_char*)lds;
+    const uint32_t lds_a = (uint32_t)(uintptr_t)lds_base, lds_b = lds_a + kStagesA * LA::kBytes;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    const int M = args.M, N = args.N, K = args.K;
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const int kps = (K + kBK - 1) / kBK;
+    const int total = kps * args.n_steps;  // at least 3
+    const int full_grid = (args.full + 7) & ~7;
+    const int rest = tiles_m * tiles_n - args.full, units = rest * args.slices, per_xcd = (units + 7) >> 3;
+    const int pids = full_grid + 8 * per_xcd;
+
+    struct Unit {
+        int m0, n0, step, k, len, unit;
+    };
+    // the first unit at or after pid, which moves behind it; false (and a unit of no length) behind the last
+    auto next_unit = [&](int& pid, Unit& u) -> bool {
+        for (; pid < pids; pid += gridDim.x) {
+            int tile, beg = 0;
+            if (pid < full_grid) {
+                tile = (pid & 7) * (full_grid >> 3) + (pid >> 3);
+                if (tile >= args.full) continue;
+                if (args.rotate) beg = (int)(((unsigned)total * (unsigned)(pid & 7)) >> 3);
+                u.len = total;
+                u.unit = -1;
+            } else {
+                const int p = pid - full_grid;
+                u.unit = (p & 7) * per_xcd + (p >> 3);
+                if (u.unit >= units) continue;
+                const int z = (int)((unsigned)u.unit / (unsigned)rest), per = (int)((unsigned)total / (unsigned)args.slices), more = total - per * args.slices;
+                tile = args.full + u.unit - z * rest;
+                beg = z * per + (z < more ? z : more);
+                u.len = per + (z < more ? 1 : 0);
+            }
+            const unsigned per_group = 8u * (unsigned)tiles_n, group = (unsigned)tile / per_group, in_group = (unsigned)tile - group * per_group;
+            const unsigned first_m = group * 8u, gsz = (unsigned)tiles_m - first_m < 8u ? (unsigned)tiles_m - first_m : 8u;
+            const unsigned tn = gsz == 8u ? in_group >> 3 : in_group / gsz;
+            u.m0 = __builtin_amdgcn_readfirstlane((int)(first_m + in_group - tn * gsz)) * BM;
+            u.n0 = __builtin_amdgcn_readfirstlane((int)tn) * BN;
+            u.step = beg == 0 ? 0 : __builtin_amdgcn_readfirstlane((int)((unsigned)beg / (unsigned)kps));
+            u.k = __builtin_amdgcn_readfirstlane(beg - u.step * kps);
+            u.len = __builtin_amdgcn_readfirstlane(u.len);
+            u.unit = __builtin_amdgcn_readfirstlane(u.unit);
+            pid += gridDim.x;
+            return true;
+        }
+        u.len = 0;
+        return false;
+    };
+
+    LA la;
+    LB lb;
+    Frags<TRANS_A, kRows, TM> fa;
+    Frags<TRANS_B, kRows, TN> fb;
+    fa.init(lane, wm * 16 * TM);
+    fb.init(lane, wn * 16 * TN);
+    const int64_t a_adv = TRANS_A ? args.lda * (2 * kBK) : 2 * kBK, b_adv = TRANS_B ? args.ldb * (2 * kBK) : 2 * kBK;
+
+    // ---- what is requested next of either operand: `cnt` stages from p on, then `part` (the stage in which a step's K ends
+    // inside 64), then the next of the unit's `left` stages, then the next unit
+    struct Walk {
+        const char* p;
+        int cnt, part, left, step, m0;
+    };
+    Unit cur, nxt;
+    Walk wa, wb;
+    auto walk_step = [&](Walk& w, auto is_a, int k) {
+        const int64_t org = is_a.value ? (TRANS_A ? (int64_t)w.m0 * 2 : (int64_t)w.m0 * args.lda * 2) : (TRANS_B ? (int64_t)w.m0 * 2 : (int64_t)w.m0 * args.ldb * 2);
+        w.p = step_ptr(is_a.value ? kTabA : kTabB, w.step) + org + k * (is_a.value ? a_adv : b_adv);
+        const int take = kps - k < w.left ? kps - k : w.left;
+        w.part = (K % kBK) != 0 && take == kps - k ? 1 : 0;
+        w.cnt = take - w.part;
+        w.left -= take;
+        if constexpr (is_a.value) la.init(lane, wave, args.lda, w.m0, w.m0 + BM < M ? w.m0 + BM : M);
+        else lb.init(lane, wave, args.ldb, w.m0, N);
+    };
+    auto walk_unit = [&](Walk& w, auto is_a, const Unit& u) {
+        w.m0 = is_a.value ? u.m0 : u.n0;
+        w.left = u.len;
+        w.step = u.step;
+        walk_step(w, is_a, u.k);
+    };
+    auto walk_event = [&](Walk& w, auto is_a) {  // cnt is 0
+        if (w.part == 0) {
+            if (w.left > 0) {
+                w.step = w.step + 1 == args.n_steps ? 0 : w.step + 1;
+                walk_step(w, is_a, 0);
+            } else if (nxt.len > 0) {
+                walk_unit(w, is_a, nxt);
+            } else {  // nothing is left: the instructions go on and fetch nothing
+                w.cnt = INT32_MAX;
+                if constexpr (is_a.value) la.mask(lane, wave, -1);
+                else lb.mask(lane, wave, -1);
+            }
+        }
+        if (w.cnt == 0) {
+            w.part = 0;
+            w.cnt = 1;
+            if constexpr (is_a.value) la.mask(lane, wave, K % kBK);
+            else lb.mask(lane, wave, K % kBK);
+        }
+    };
+    auto walk_on = [&](Walk& w, auto is_a) {
+        w.p += is_a.value ? a_adv : b_adv;
+        if (--w.cnt == 0) walk_event(w, is_a);
+    };
+    constexpr std::true_type kA{};
+    constexpr std::false_type kB{};
+    constexpr uint32_t kRingA = kStagesA * LA::kBytes, kRingB = kStagesB * LB::kBytes;
+    const uint32_t lds_wa = lds_a + wave * (LA::PER * 1024), lds_wb = lds_b + wave * (LB::PER * 1024);
+    uint32_t wr_a = 0, wr_b = 0;  // ring positions written and read next
+    uint32_t rd_a = 0, rd_b = 0;
+    auto ring_on = [](uint32_t& pos, uint32_t bytes, uint32_t ring) { pos = pos + bytes == ring ? 0 : pos + bytes; };
+    auto issue_a = [&](auto op) { la.template issue<op.value>(wa.p, lds_wa + wr_a); };
+    auto issue_b = [&](auto op) { lb.template issue<op.value>(wb.p, lds_wb + wr_b); };
+
+    int pid = blockIdx.x;
+    if (!next_unit(pid, cur)) return;
+    nxt.len = 0;
+    walk_unit(wa, kA, cur);
+    walk_unit(wb, kB, cur);
+    if (wa.cnt == 0) walk_event(wa, kA);
+    if (wb.cnt == 0) walk_event(wb, kB);
+    for (int p = 0; p < 2; ++p) {
+        static_for<LA::PER>(issue_a);
+        static_for<LB::PER>(issue_b);
+        ring_on(wr_a, LA::kBytes, kRingA);
+        ring_on(wr_b, LB::kBytes, kRingB);
+        walk_on(wa, kA);
+        walk_on(wb, kB);
+    }
+    auto publish = [&]() {
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    f32x4_t acc[TM][TN];
+    bf16x8_t af[TM], bfr[2][TN];
+    lds_char *pa = lds_base, *pb = lds_base + kRingA;
+    dma_wait<LA::PER + LB::PER>();
+    publish();
+
+    auto read_first = [&]() {
+        static_for<TN>([&](auto t) { bfr[0][t.value] = fb.template read<t.value, 0>(pb); });
+        static_for<TM>([&](auto t) { af[t.value] = fa.template read<t.value, 0>(pa); });
+    };
+    read_first();
+
+    constexpr int kStores = TM * 2;  // of a wavefront and whole tile: 16 bytes a lane each
+    constexpr int kBarRow = 1;  // the row of k step 1 behind which the barrier stands
+    bool stored_fast = false;
+    // One k step: TM x TN MFMAs in serpentine order; what else there is to do is dealt out behind single MFMAs, so that no more
+    // instructions than fit under an MFMA stand between two.
+    auto k_step = [&](auto set, auto zero, auto&& behind) {
+        static_for<TM>([&](auto row) {
+            static_for<TN>([&](auto jc) {
+                constexpr int I = row.value, J = (I & 1) ? TN - 1 - jc.value : jc.value;
+                const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
+                acc[I][J] = mfma_16x16x32<E>(bfr[set.value][J], af[I], zero.value ? z : acc[I][J]);
+                behind(row, jc);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+    };
+    auto stage = [&](auto first) {
+        constexpr std::integral_constant<int, 0> k0{};
+        constexpr std::integral_constant<int, 1> k1{};
+        __builtin_amdgcn_sched_barrier(0);
+        k_step(k0, first, [&](auto row, auto jc) {
+            constexpr int R = row.value, P = jc.value, NB = TM - 2, H = TN / 2;
+            if constexpr (P == 0 && R > 0) af[R - 1] = fa.template read<R - 1, 1>(pa);
+            if constexpr (P % H == 1 % H && R < NB) {
+                constexpr int T = R * TN / NB + P / H;
+                if constexpr (T < (R + 1) * TN / NB) bfr[1][T] = fb.template read<T, 1>(pb);
+            }
+            static_for<LA::PER>([&](auto d) {
+                if constexpr (d.value * TM / LA::PER == R && P == (2 + (d.value & 1) * H * (LA::PER > TM ? 1 : 0)) % TN) issue_a(d);
+            });
+            if constexpr (R == TM - 1 && P == TN - 1) {
+                ring_on(wr_a, LA::kBytes, kRingA);
+                walk_on(wa, kA);
+            }
+        });
+        af[TM - 1] = fa.template read<TM - 1, 1>(pa);
+        k_step(k1, std::false_type{}, [&](auto row, auto jc) {
+            constexpr int R = row.value - kBarRow - 1, P = jc.value, NR = TM - 1 - kBarRow, H = TN / 2;
+            if constexpr (R == -1 && P == TN - 1) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (decltype(first)::value && stored_fast) dma_wait<LA::PER + kStores>();
+                else dma_wait<LA::PER>();
+                publish();
+                ring_on(rd_a, LA::kBytes, kRingA);
+                ring_on(rd_b, LB::kBytes, kRingB);
+                pa = lds_base + rd_a;
+                pb = lds_base + kRingA + rd_b;
+            }
+            if constexpr (R >= 0) {
+                if constexpr ((P == 0 || P == TN - 1)) {
+                    constexpr int T = R * (TM - 1) / NR + (P == 0 ? 0 : 1);
+                    static_assert(T >= (R + 1) * (TM - 1) / NR || T < row.value, "a fragment is replaced behind its last use");
+                    if constexpr (T < (R + 1) * (TM - 1) / NR) af[T] = fa.template read<T, 0>(pa);
+                }
+                if constexpr (P % H == 1 % H && R < NR - 1) {
+                    constexpr int T = R * TN / (NR - 1) + P / H;
+                    if constexpr (T < (R + 1) * TN / (NR - 1)) bfr[0][T] = fb.template read<T, 0>(pb);
+                }
+                static_for<LB::PER>([&](auto d) {
+                    constexpr int D = d.value * NR / LB::PER, FIRST = (D * LB::PER + NR - 1) / NR;
+                    if constexpr (D == R && P == (2 + (d.value - FIRST) * H) % TN) issue_b(d);
+                });
+                if constexpr (row.value == TM - 1 && P == TN - 1) {
+                    ring_on(wr_b, LB::kBytes, kRingB);
+                    walk_on(wb, kB);
+                }
+            }
+        });
+        af[TM - 1] = fa.template read<TM - 1, 0>(pa);
+    };
+
+    for (;;) {
+        const bool more = next_unit(pid, nxt);
+        stage(std::true_type{});
+        for (int kt = cur.len - 1; kt > 0; --kt) stage(std::false_type{});
+        stored_fast = false;
+        if (cur.unit >= 0) {
+            // accumulator order: [TM][TN][threads] x 4 floats
+            float* part = args.partial + (int64_t)cur.unit * (BM * BN) + tid * 4;
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4_t*>(part + (i * TN + j) * (kThreads * 4)) = acc[i][j];
+        } else {
+            const bool whole = args.vec_out != 0 && cur.m0 + BM <= M && cur.n0 + BN <= N;
+            stored_fast = whole && args.preact == nullptr;
+            // the slot of A that is free until the next stage's loads, which wait for the barrier below
+            const Out<EPI, E> out(args, lds_base + wr_a + wave * kPatch, cur.m0 + wm * (16 * TM), cur.n0 + wn * (16 * TN), whole, lane);
+            out.rows(acc, args);
+        }
+        if (!more) break;
+        cur = nxt;
+        __builtin_amdgcn_s_barrier();
+        // the next stage's first fragments once more: kept through the epilogue, they would be spilled
+        asm volatile("" ::: "memory");
+        read_first();
+    }
+    dma_wait<0>();
+}
+
+// Finishes the sliced tiles: block (tile, row of MFMA tiles) adds the slices' partial sums in slice order and runs the epilogue.
+template <int TM, int EPI, typename E>
+__global__ __launch_bounds__(kThreads) void wide_reduce_kernel(const TileArgs args) {
+    constexpr int BM = 16 * WM * TM;
+    __shared__ __attribute__((aligned(1024))) char lds[NW * kPatch];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles_m = (args.M + BM - 1) / BM, tiles_n = (args.N + BN - 1) / BN;
+    const int rest = tiles_m * tiles_n - args.full;
+    const int r = blockIdx.x / TM, i = blockIdx.x % TM;
+    int tm, tn;
+    gemm_tile::tile_origin(args.full + r, tiles_m, tiles_n, tm, tn);
+    f32x4_t acc[1][TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[0][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const float* part = args.partial + (int64_t)r * (BM * BN) + i * (TN * kThreads * 4) + tid * 4;
+    for (int z = 0; z < args.slices; ++z, part += (int64_t)rest * (BM * BN)) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const raw16_t u = load_raw_stream(part + j * (kThreads * 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[0][j][e] += __uint_as_float(u[e]);
+        }
+    }
+    const int m0 = tm * BM, n0 = tn * BN;
+    const bool whole = args.vec_out != 0 && m0 + BM <= args.M && n0 + BN <= args.N;
+    const Out<EPI, E> out(args, (lds_char*)lds + wave * kPatch, m0 + (wave / WN * TM + i) * 16, n0 + wave % WN * (16 * TN), whole, lane);
+    out.rows(acc, args);
+}
+
+template <bool TA, bool TB, int TM, int EPI, typename E>
+int launch_rows(const TileArgs& args, hipStream_t s) {
+    constexpr int BM = 16 * WM * TM;
+    auto kern = gemm_wide_kernel<TA, TB, TM, EPI, E>;
+    if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)kLdsBytes, "gemm_wide"); lrc != CW_OK) return lrc;
+    const int64_t tiles = (int64_t)((args.M + BM - 1) / BM) * ((args.N + BN - 1) / BN), rest = tiles - args.full;
+    const int64_t pids = ((args.full + 7) & ~7) + ((rest * args.slices + 7) & ~(int64_t)7);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(pids < kUnits ? pids : kUnits)), dim3(kThreads), kLdsBytes, s, args);
+    if (const int rc = check_launch("gemm_wide_kernel"); rc != CW_OK || rest == 0) return rc;
+    hipLaunchKernelGGL((wide_reduce_kernel<TM, EPI, E>), dim3((unsigned)(rest * TM)), dim3(kThreads), 0, s, args);
+    return check_launch("wide_reduce_kernel");
+}
+
+// PLAIN_ONLY: no activations (the weight-gradient orientation, which nothing asks to be activated).
+template <bool TA, bool TB, bool PLAIN_ONLY, int TM, typename E>
+int launch_epi(const TileArgs& args, int epilogue, hipStream_t s) {
+    if constexpr (!PLAIN_ONLY) {
+        switch (epilogue) {
+            case CW_EPI_BIAS_GELU_TANH: return launch_rows<TA, TB, TM, CW_EPI_BIAS_GELU_TANH, E>(args, s);
+            case CW_EPI_BIAS_GELU_ERF: return launch_rows<TA, TB, TM, CW_EPI_BIAS_GELU_ERF, E>(args, s);
+            case CW_EPI_BIAS_RELU: return launch_rows<TA, TB, TM, CW_EPI_BIAS_RELU, E>(args, s);
+            default: break;
+        }
+    }
+    if (epilogue != CW_EPI_NONE && epilogue != CW_EPI_BIAS) return fail(CW_ERR_INVALID, "cw_gemm_ksteps: bad epilogue %d", epilogue);
+    return launch_rows<TA, TB, TM, CW_EPI_BIAS, E>(args, s);
+}
+
+}  // namespace gemm_wide
+}  // namespace cw

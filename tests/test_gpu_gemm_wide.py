@@ -1,0 +1,58 @@
+"""GPU parity of the block GEMM's kernel of 256-column tiles (configuration 0 of the planner) against float64 where it can go
+wrong: every tile height, edges of M and N, steps whose K ends inside a stage, the shortest reductions it takes, seams of steps
+and of tiles, sliced tiles, unaligned output rows, every operand of the epilogue."""
+import pytest
+import torch
+
+from tests.util import assert_parity, randn
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K, steps), which the planner gives to this kernel: heights 160, 192, 224 and 256 with ragged edges, K of a part of a stage
+# behind whole ones, three steps (rotated starts in NT), three tiles a block, a last row and column of tiles with few elements, an
+# odd last column
+SHAPES = [(300, 32768, 1016, 1), (376, 32760, 1000, 1), (1552, 7672, 1352, 1), (8184, 2040, 328, 3), (8184, 6136, 520, 1),
+          (7000, 4600, 1000, 1), (1024, 25003, 768, 1), (8192, 2048, 512, 2)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tiles_of_256_columns(layout, shape, dtype):
+    from cubework_amd import ops
+
+    M, N, K, steps = shape
+    pad = -N % 8  # B's rows are 16-byte aligned (an odd N has an odd output alone)
+    a_shape, b_shape = ((K, M) if layout == "TN" else (M, K)), ((N, K) if layout == "NT" else (K, N + pad))
+    A = [randn(a_shape, dtype, 3 * i).cuda() for i in range(steps)]
+    B = [randn(b_shape, dtype, 3 * i + 1, std=0.05).cuda()[:, :K if layout == "NT" else N] for i in range(steps)]
+    bias, add = randn((N,), dtype, 90).cuda(), randn((M, N + pad), dtype, 91).cuda()[:, :N]
+    act = None if layout == "TN" else "relu"
+    got = ops.gemm_ksteps(layout, A, B, bias, act, [add], want_preact=True)
+    rows = torch.cat([torch.arange(0, min(M, 48)), torch.arange(max(M // 2 - 24, 0), M // 2 + 24), torch.arange(max(M - 48, 0), M)]).unique().cuda()
+    want = add[rows].double() + bias.double()
+    for a, b in zip(A, B):
+        a64 = a[:, rows].double().t().contiguous() if layout == "TN" else a[rows].double()
+        want += a64 @ (b.double().t().contiguous() if layout == "NT" else b.double())
+    # fp32 sums rounded once: the storage type's bar
+    assert_parity(got[1][rows], want, dtype, "preact %s %s %s" % (layout, shape, dtype))
+    assert_parity(got[0][rows], want if act is None else want.clamp_min(0), dtype, "out %s %s %s" % (layout, shape, dtype))
+    plain = ops.gemm_ksteps(layout, A, B)  # whole tiles' stores are counted, not waited for
+    assert_parity(plain[rows], want - add[rows].double() - bias.double(), dtype, "plain %s %s %s" % (layout, shape, dtype))
+
+
+@pytest.mark.parametrize("layout,M,N,K", [("NN", 300, 4096, 16384), ("NT", 1554, 2560, 7680), ("TN", 2040, 2296, 8200), ("NT", 4352, 4096, 1024)])
+def test_sliced_tiles(layout, M, N, K):
+    """Every tile, or the last round's, cut along k; bias, addend and pre-activation behind the reduction."""
+    from cubework_amd import _lib, ops
+
+    a = randn((K, M) if layout == "TN" else (M, K), torch.bfloat16, 1).cuda()
+    b = randn((N, K) if layout == "NT" else (K, N), torch.bfloat16, 2, 0.05).cuda()
+    bias, add = randn((N,), torch.bfloat16, 3).cuda(), randn((M, N), torch.bfloat16, 4).cuda()
+    assert _lib.load().cw_gemm_scratch_bytes(ops.LAYOUTS[layout], M, N, K, 1, a.stride(0), b.stride(0), 1, 1, 0, _lib.CW_BF16) > 0
+    act = None if layout == "TN" else "gelu_tanh"
+    out, pre = ops.gemm_ksteps(layout, [a], [b], bias, act, [add], want_preact=True)
+    want = (a.double().t().contiguous() if layout == "TN" else a.double()) @ (b.double().t().contiguous() if layout == "NT" else b.double())
+    want += bias.double() + add.double()
+    assert_parity(pre, want, torch.bfloat16, "sliced preact")
+    assert_parity(out, want if act is None else torch.nn.functional.gelu(want, approximate="tanh"), torch.bfloat16, "sliced out")
