@@ -16,12 +16,13 @@
 namespace cw {
 
 #define CW_TILE_CFGS(e, l) {gemm_tile_##e##_##l##_1, gemm_tile_##e##_##l##_2, gemm_tile_##e##_##l##_3, gemm_tile_##e##_##l##_4}
-#define CW_WIDE_ROWS(e, l) {gemm_wide_##e##_##l##_160, gemm_wide_##e##_##l##_192, gemm_wide_##e##_##l##_224, gemm_wide_##e##_##l##_256}
+#define CW_WIDE_ROWS(e, l) {gemm_wide_##e##_##l##_128, gemm_wide_##e##_##l##_160, gemm_wide_##e##_##l##_192, gemm_wide_##e##_##l##_224, gemm_wide_##e##_##l##_256}
 #define CW_TILE_DECL(e, l)                                              \
     int gemm_tile_##e##_##l##_1(const TileArgs&, int, hipStream_t);     \
     int gemm_tile_##e##_##l##_2(const TileArgs&, int, hipStream_t);     \
     int gemm_tile_##e##_##l##_3(const TileArgs&, int, hipStream_t);     \
     int gemm_tile_##e##_##l##_4(const TileArgs&, int, hipStream_t);     \
+    int gemm_wide_##e##_##l##_128(const TileArgs&, int, hipStream_t);   \
     int gemm_wide_##e##_##l##_160(const TileArgs&, int, hipStream_t);   \
     int gemm_wide_##e##_##l##_192(const TileArgs&, int, hipStream_t);   \
     int gemm_wide_##e##_##l##_224(const TileArgs&, int, hipStream_t);   \
@@ -34,11 +35,11 @@ CW_TILE_DECL(f16_t, NT)
 CW_TILE_DECL(f16_t, TN)
 
 using TileLaunch = int (*)(const TileArgs&, int, hipStream_t);
-static constexpr TileLaunch kTileLaunch[2][3][kTileConfigCount - 1] = {
+static constexpr TileLaunch kTileLaunch[2][3][4] = {
     {CW_TILE_CFGS(bf16_t, NN), CW_TILE_CFGS(bf16_t, NT), CW_TILE_CFGS(bf16_t, TN)},
     {CW_TILE_CFGS(f16_t, NN), CW_TILE_CFGS(f16_t, NT), CW_TILE_CFGS(f16_t, TN)},
 };
-static constexpr TileLaunch kWideLaunch[2][3][4] = {
+static constexpr TileLaunch kWideLaunch[2][3][5] = {
     {CW_WIDE_ROWS(bf16_t, NN), CW_WIDE_ROWS(bf16_t, NT), CW_WIDE_ROWS(bf16_t, TN)},
     {CW_WIDE_ROWS(f16_t, NN), CW_WIDE_ROWS(f16_t, NT), CW_WIDE_ROWS(f16_t, TN)},
 };
@@ -119,7 +120,7 @@ static int tile_launch(const GemmArgs& g, const TilePlan& plan, int layout, int 
     a.slices = plan.slices;
     a.rotate = plan.rotate ? 1 : 0;
     a.partial = reinterpret_cast<float*>(ws + plan.pack_a_bytes + plan.pack_b_bytes + plan.pack_add_bytes);
-    if (plan.cfg == 0) return kWideLaunch[f16 ? 1 : 0][layout][(plan.rows - 160) / 32](a, epilogue, s);
+    if (plan.cfg == 0 || plan.cfg == kPairedConfig) return kWideLaunch[f16 ? 1 : 0][layout][(plan.rows - 128) / 32](a, epilogue, s);
     return kTileLaunch[f16 ? 1 : 0][layout][plan.cfg - 1](a, epilogue, s);
 }
 

@@ -43,12 +43,13 @@ struct GemmPlan {
 // for is planned by tile_plan). dma_enabled / strip_enabled: the two CW_GEMM_IMPL switches (staged / onelaunch) as the caller read them.
 GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool strip_enabled);
 
-// ---- tile kernels (gemm_wide.h: configuration 0; gemm_tile.h: the others) ---------------------------------------
+// ---- tile kernels (gemm_wide.h: configurations 0 and 5; gemm_tile.h: the others) ---------------------------------------
 // Their configurations: block tile 64 tm x 64 tn, k extent of a trip in units of 32, ring stages, resident
 // blocks per compute unit, and what a trip costs (us; one block on the unit / two) and a block besides its trips. The
 // costs are a fit to 2000 launches over 110 shapes (products of 64 .. 8192 tokens with the model widths 768 .. 4096, in the
 // forward and weight-gradient orientations; rms error 11 %); choosing by them comes within 2 % of the best choice on average.
-// (The launches' times are not kept in this tree: a change of the kernels' speed means measuring and fitting again.)
+// (The launches' times are not kept in this tree: a change of the kernels' speed means measuring and fitting again. Configurations
+// 0 and 5, and what cutting along k costs them, are a fit to 250 launches over 30 of these shapes.)
 struct TileConfig {
     int tm, tn, kb, stages, resident;
     float trip1, trip2, fixed;
@@ -56,11 +57,12 @@ struct TileConfig {
 constexpr TileConfig kTileConfigs[] = {
     {4, 4, 2, 2, 1, 1.43f, 1.43f, 4.00f},    // up to 256 x 256: the least operand traffic per FLOP, one block per compute unit
     {2, 4, 1, 3, 2, 0.480f, 0.897f, 5.00f},  // 128 x 256, two blocks
-    {2, 2, 1, 5, 2, 0.285f, 0.546f, 3.63f},  // 128 x 128
-    {1, 2, 2, 3, 2, 0.377f, 0.690f, 2.60f},  // 64 x 128
+    {2, 2, 1, 5, 2, 0.285f, 0.546f, 4.50f},  // 128 x 128
+    {1, 2, 2, 3, 2, 0.440f, 0.800f, 2.60f},  // 64 x 128
     {1, 1, 2, 4, 2, 0.289f, 0.460f, 2.06f},  // 64 x 64: small outputs spread over the most compute units
+    {2, 2, 4, 2, 1, 0.78f, 0.78f, 4.50f},    // 128 x 128, one block of two groups of wavefronts along k (gemm_wide.h)
 };
-constexpr int kTileConfigCount = 5;
+constexpr int kTileConfigCount = 6, kPairedConfig = 5;
 
 // How a product runs on the tile kernels: `full` tiles whole, the others in `slices` k slices through fp32 partial
 // sums. An operand whose rows are not 16-byte aligned is copied to rows that are, once per step (pack_a / pack_b).
@@ -76,9 +78,9 @@ struct TilePlan {
     int64_t pack_a_bytes, pack_b_bytes, pack_add_bytes, partial_bytes;
     int64_t scratch() const { return pack_a_bytes + pack_b_bytes + pack_add_bytes + partial_bytes; }
 };
-// Whether the kernel of configuration 0 takes such a product: at least three stages of 64 k, and k-contiguous rows whose last 16
+// Whether the kernel of configuration 0 (stage: 64) or 5 (128) takes such a product: at least three stages, and k-contiguous rows whose last 16
 // bytes hold nothing behind K (multiples of 8, or copied rows, whose padding is zeros).
-bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b);
+bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b, int stage = 64);
 int wide_rows(int64_t M);
 // max_scratch < 0: the choice with as much scratch as it likes; else the best one that fits. align_a / align_b: every step's
 // pointer is 16-byte aligned and the leading dimension a multiple of 8; n_pack_addends: addends of which that is not true.

@@ -226,9 +226,9 @@ constexpr int64_t kTileLaunchMax = ((int64_t)1 << 24) - 8;
 
 }  // namespace
 
-bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b) {
+bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b, int stage) {
     const bool a_ok = layout == CW_TN || K % 8 == 0 || pack_a, b_ok = layout != CW_NT || K % 8 == 0 || pack_b;
-    return a_ok && b_ok && (K + 63) / 64 * n_steps >= 3;
+    return a_ok && b_ok && (K + stage - 1) / stage * n_steps >= 3;
 }
 
 int wide_rows(int64_t M) {
@@ -276,7 +276,6 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     // channels, gemm_tile.h). (The 16x16x32 instruction of configuration 0 and the 32x32x16 one of the others give the same bits.)
     const bool ordered = layout == CW_NN && K <= N;
     const bool rotated = ordered && M % 256 == 0 && N % 256 == 0 && K % 32 == 0 && (M / 256) * (N / 256) >= 160;
-    const double small_factor = layout == CW_TN ? 0.9 : 1.0;  // gemm_tile.h: k-contiguous operands move as pieces of 64 bytes
     const double bytes = 2.0 * ((double)M * K * n_steps + (double)K * N * n_steps + (double)M * N);
     const double memory_us = bytes / 4.0e6;
     double best_us = 0;
@@ -290,14 +289,19 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         q.tiles = tiles;
         q.full = (int)full;
         q.slices = rest > 0 ? slices : 1;
-        q.rotate = cfg == 0 && (!ordered || rotated);
+        q.rotate = cfg == kPairedConfig || (cfg == 0 && (!ordered || rotated));
         q.partial_bytes = rest * slices * (int64_t)(4096 * c.tm * c.tn) * 4;
         if (max_scratch >= 0 && q.scratch() > max_scratch) return;
-        const double layout_factor = cfg == 0 ? 1.0 : small_factor;
+        // TN on the kernels of gemm_tile.h: k-contiguous operands move as pieces of 64 bytes, k-slow ones as whole lines. On the
+        // paired one: the two groups' transposing reads take more LDS cycles than their products.
+        const double layout_factor = cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9;
         if (cfg == 0) trips *= 0.2 + 0.8 / 256 * q.rows;  // a lower tile's trips are shorter
-        // configuration 0: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's
-        double us = tile_rounds(c, (double)full, trips, layout_factor) + (cfg == 0 ? 3.0 : 0.0);
-        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor) + 5.0 + 2.0 * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
+        // the kernels of gemm_wide.h: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's
+        // (the reduction waits about 0.9 us a slice whatever its size, and its bytes come from the cache)
+        const bool walks = cfg == 0 || cfg == kPairedConfig;
+        double us = tile_rounds(c, (double)full, trips, layout_factor) + (walks && full > 0 ? 3.0 : 0.0);
+        const double reduce_us = (walks ? 2.0 + 0.9 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
+        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor) + reduce_us;
         us = us > memory_us ? us + 0.1 * memory_us : memory_us + 0.1 * us;
         if (best.cfg < 0 || us < best_us) {
             best = q;
@@ -307,7 +311,8 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     for (int cfg = 0; cfg < kTileConfigCount; ++cfg) {
         const TileConfig& c = kTileConfigs[cfg];
         const int64_t tiles = ((M + 64 * c.tm - 1) / (64 * c.tm)) * ((N + 64 * c.tn - 1) / (64 * c.tn));
-        if (tiles > kTileLaunchMax || (cfg == 0 && !wide_takes(layout, K, n_steps, p.pack_a, p.pack_b))) continue;
+        if (tiles > kTileLaunchMax || ((cfg == 0 || cfg == kPairedConfig) && !wide_takes(layout, K, n_steps, p.pack_a, p.pack_b, 32 * c.kb))) continue;
+        if (cfg == kPairedConfig && ordered) continue;  // it sums k in another order than the other tiles do
         const int64_t trips = ((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps, cap = 256 * c.resident;
         consider(cfg, tiles, tiles, 1);
         // all tiles sliced, to fill the chip about once; or only those of the partial last round

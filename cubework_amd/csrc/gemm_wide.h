@@ -20,6 +20,15 @@
 //
 // Whole 256-row tiles whose rows are mostly beyond M are wasted products: BM is 32 TM, the least of 160, 192, 224 and 256 that
 // covers M with as many tiles (gemm_plan.hip).
+//
+// KG = 2: tiles of 128 x 128 for outputs of about 256 of them (a weight gradient of 2048 x 2048, 4096 tokens by a hidden size of
+// 1024). A block of 4 wavefronts leaves one per SIMD, which waits at every barrier and for every fragment, and stages of 32 k
+// run the load unit at half rate. Here two groups of 4 wavefronts own the tile together and each takes one 64 k half of a 128 k
+// stage: the stage has the bytes of the 256 x 256 tile's, so the ring and its waits are the same. Their sums meet in LDS behind
+// the last stage, in one order (a group's sum each, then the two added). us against 128 x 128 tiles of 4 wavefronts, NT / TN
+// (M x N x K): 4096 x 1024 x 4096 42 -> 33, 2048 x 2048 x 8192 TN 79 -> 66, 1024 x 4096 x 4096 TN 41 -> 36; below about 1300 of k
+// the smaller blocks' epilogue is the cheaper one (4096 x 1024 x 1024: 15 and 14). Bound by L2 -> LDS: 62 bytes a cycle and
+// compute unit at the full matrix rate, where the load unit reaches 61; TN by the transposing LDS reads.
 #pragma once
 #include <cstddef>
 
@@ -57,20 +66,20 @@ __device__ __forceinline__ f32x4_t mfma_16x16x32(bf16x8_t a, bf16x8_t b, f32x4_t
 // 16-byte chunks by which k row k of a k-slow image is rotated (xor)
 __device__ __forceinline__ int kslow_swizzle(int k) { return ((k & 3) << 2) ^ (((k >> 3) & 1) << 1); }
 
-// Loader of one operand: ROWS operand rows x 64 k, 1 KB per load instruction, PER instructions per wavefront and stage.
-// k-contiguous image [ROWS][64 k]: chunk c of row r at c ^ ((r >> 1) & 7); k-slow image [64 k][ROWS]: chunk c of k row k
+// Loader of one operand: ROWS operand rows x KG images of 64 k, 1 KB per load instruction, PER instructions per wavefront and
+// stage. k-contiguous image [ROWS][64 k]: chunk c of row r at c ^ ((r >> 1) & 7); k-slow image [64 k][ROWS]: chunk c of k row k
 // at c ^ kslow_swizzle(k).
-template <bool TRANS, int ROWS, int NW>
+template <bool TRANS, int ROWS, int KG, int NW>
 struct Loader {
-    static constexpr int kBytes = ROWS * kBK * 2;
-    static constexpr int PER = ROWS / 8 / NW;
+    static constexpr int kBytes = ROWS * KG * kBK * 2;
+    static constexpr int PER = ROWS * KG / 8 / NW;
     static constexpr int CPR = ROWS / 8;  // TRANS: 16-byte chunks per k row
-    static_assert(ROWS % (8 * NW) == 0 && (!TRANS || (ROWS & (ROWS - 1)) == 0), "whole instructions per wavefront");
+    static_assert(ROWS * KG % (8 * NW) == 0 && ROWS % 16 == 0 && (!TRANS || (ROWS & (ROWS - 1)) == 0), "whole instructions per wavefront");
     uint32_t voff[PER];
     // k position of the lane's chunk in instruction i (k row for TRANS)
     static __device__ __forceinline__ int kpos(int lane, int wave, int i) {
         const int j = wave * PER + i;
-        if constexpr (!TRANS) return ((lane & 7) ^ ((4 * j + (lane >> 4)) & 7)) * 8;
+        if constexpr (!TRANS) return ((lane & 7) ^ ((4 * j + (lane >> 4)) & 7)) * 8 + 8 * j / ROWS * kBK;
         else return (j * 64 + lane) / CPR;
     }
     __device__ __forceinline__ void init(int lane, int wave, int64_t ld, int row0, int rmax) {
@@ -79,7 +88,7 @@ struct Loader {
         for (int i = 0; i < PER; ++i) {
             const int j = wave * PER + i, k = kpos(lane, wave, i);
             if constexpr (!TRANS) {
-                const int r = 8 * j + (lane >> 3);
+                const int r = 8 * j % ROWS + (lane >> 3);
                 voff[i] = row0 + r < rmax ? (uint32_t)(((int64_t)r * ld + k) * 2) : kRange;
             } else {
                 const int c = ((j * 64 + lane) % CPR) ^ kslow_swizzle(k);
@@ -100,19 +109,20 @@ struct Loader {
     }
 };
 
-// Fragment reads of one operand: W MFMA tiles of 16 rows x 32 k per wavefront from operand row wrow on.
+// Fragment reads of one operand: W MFMA tiles of 16 rows x 32 k per wavefront from operand row wrow of a 64 k image on, which
+// begins `image` bytes behind the operand.
 template <bool TRANS, int ROWS, int W>
 struct Frags {
     uint32_t off[TRANS ? W : 2];
-    __device__ __forceinline__ void init(int lane, int wrow) {
+    __device__ __forceinline__ void init(int lane, int wrow, uint32_t image) {
         const int i = lane & 15, q = lane >> 4;
         if constexpr (!TRANS) {
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) off[ks] = (uint32_t)((wrow + i) * 128 + (((4 * ks + q) ^ ((i >> 1) & 7)) << 4));
+            for (int ks = 0; ks < 2; ++ks) off[ks] = image + (uint32_t)((wrow + i) * 128 + (((4 * ks + q) ^ ((i >> 1) & 7)) << 4));
         } else {
             const int k = 8 * q + (i >> 2);
 #pragma unroll
-            for (int t = 0; t < W; ++t) off[t] = (uint32_t)(k * (ROWS * 2) + (((wrow / 8 + 2 * t + ((i & 3) >> 1)) ^ kslow_swizzle(k)) << 4) + 8 * (i & 1));
+            for (int t = 0; t < W; ++t) off[t] = image + (uint32_t)(k * (ROWS * 2) + (((wrow / 8 + 2 * t + ((i & 3) >> 1)) ^ kslow_swizzle(k)) << 4) + 8 * (i & 1));
         }
     }
     template <int T, int KS>
@@ -266,30 +276,44 @@ struct Out {
     }
 };
 
-constexpr int WM = 2, WN = 4, NW = WM * WN, TN = 4;  // wavefronts; MFMA tiles of a wavefront along N
+constexpr int NW = 8, WM = 2, TN = 4;  // wavefronts of a block, along M; MFMA tiles of a wavefront along N
 constexpr int kThreads = 64 * NW, kUnits = 256;
-constexpr int kRows = 256;  // rows of either operand's LDS image (of A, BM of them are fetched)
-constexpr int BN = 16 * WN * TN;
-static_assert(BN == kRows, "");
 constexpr int kStagesA = 3, kStagesB = 2;
-constexpr size_t kLdsBytes = (size_t)(kStagesA + kStagesB) * kRows * kBK * 2;
-static_assert(kLdsBytes == 160 * 1024 && kRows * kBK * 2 >= NW * kPatch, "one block per compute unit; the epilogue's patches in a free stage of A");
+constexpr int kImage = 32 * 1024;  // LDS bytes of an operand's stage
+constexpr size_t kLdsBytes = (size_t)(kStagesA + kStagesB) * kImage;
+static_assert(kLdsBytes == 160 * 1024 && kImage >= NW * kPatch, "one block per compute unit; the epilogue's patches in a free stage of A");
 
-template <bool TRANS_A, bool TRANS_B, int TM, int EPI, typename E>
+// KG = 1: the wavefronts are 2 x 4, each of 16 TM x 64 of the tile. KG = 2: two groups of 2 x 2, each of which owns the whole tile
+// and takes one half of a stage's 128 k; behind the last stage they exchange halves of their sums.
+template <int TM, int KG>
+struct Shape {
+    static constexpr int WN = 4 / KG, kRows = 256 / KG;  // kRows: rows of either operand's LDS image (of A, BM of them are fetched)
+    static constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN, kStage = KG * kBK;
+    static constexpr int kOutTM = TM / KG;  // rows of MFMA tiles that a wavefront finishes
+    static_assert(BN == kRows && BM <= kRows && TM % KG == 0, "");
+    static __device__ __forceinline__ int group(int wave) { return wave / (WM * WN); }
+    static __device__ __forceinline__ int wm(int wave) { return wave / WN % WM; }
+    static __device__ __forceinline__ int wn(int wave) { return wave % WN; }
+    static __device__ __forceinline__ int out_row(int wave) { return wm(wave) * 16 * TM + group(wave) * 16 * kOutTM; }
+    static __device__ __forceinline__ int out_col(int wave) { return wn(wave) * 16 * TN; }
+};
+
+template <bool TRANS_A, bool TRANS_B, int TM, int KG, int EPI, typename E>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_wide_kernel(const TileArgs args) {
-    constexpr int BM = 16 * WM * TM;
-    using LA = Loader<TRANS_A, kRows, NW>;
-    using LB = Loader<TRANS_B, kRows, NW>;
+    using S = Shape<TM, KG>;
+    constexpr int BM = S::BM, BN = S::BN, kStage = S::kStage;
+    using LA = Loader<TRANS_A, S::kRows, KG, NW>;
+    using LB = Loader<TRANS_B, S::kRows, KG, NW>;
+    static_assert(LA::kBytes == kImage && LB::kBytes == kImage, "");
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     lds_char* lds_base = (lds_char*)lds;
     const uint32_t lds_a = (uint32_t)(uintptr_t)lds_base, lds_b = lds_a + kStagesA * LA::kBytes;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
     const int M = args.M, N = args.N, K = args.K;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-    const int kps = (K + kBK - 1) / kBK;
+    const int kps = (K + kStage - 1) / kStage;
     const int total = kps * args.n_steps;  // at least 3
     const int full_grid = (args.full + 7) & ~7;
     const int rest = tiles_m * tiles_n - args.full, units = rest * args.slices, per_xcd = (units + 7) >> 3;
@@ -335,14 +359,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     LA la;
     LB lb;
-    Frags<TRANS_A, kRows, TM> fa;
-    Frags<TRANS_B, kRows, TN> fb;
-    fa.init(lane, wm * 16 * TM);
-    fb.init(lane, wn * 16 * TN);
-    const int64_t a_adv = TRANS_A ? args.lda * (2 * kBK) : 2 * kBK, b_adv = TRANS_B ? args.ldb * (2 * kBK) : 2 * kBK;
+    Frags<TRANS_A, S::kRows, TM> fa;
+    Frags<TRANS_B, S::kRows, TN> fb;
+    fa.init(lane, S::wm(wave) * 16 * TM, S::group(wave) * (kImage / KG));
+    fb.init(lane, S::wn(wave) * 16 * TN, S::group(wave) * (kImage / KG));
+    const int64_t a_adv = TRANS_A ? args.lda * (2 * kStage) : 2 * kStage, b_adv = TRANS_B ? args.ldb * (2 * kStage) : 2 * kStage;
 
     // ---- what is requested next of either operand: `cnt` stages from p on, then `part` (the stage in which a step's K ends
-    // inside 64), then the next of the unit's `left` stages, then the next unit
+    // inside a stage), then the next of the unit's `left` stages, then the next unit
     struct Walk {
         const char* p;
         int cnt, part, left, step, m0;
@@ -353,7 +377,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int64_t org = is_a.value ? (TRANS_A ? (int64_t)w.m0 * 2 : (int64_t)w.m0 * args.lda * 2) : (TRANS_B ? (int64_t)w.m0 * 2 : (int64_t)w.m0 * args.ldb * 2);
         w.p = step_ptr(is_a.value ? kTabA : kTabB, w.step) + org + k * (is_a.value ? a_adv : b_adv);
         const int take = kps - k < w.left ? kps - k : w.left;
-        w.part = (K % kBK) != 0 && take == kps - k ? 1 : 0;
+        w.part = (K % kStage) != 0 && take == kps - k ? 1 : 0;
         w.cnt = take - w.part;
         w.left -= take;
         if constexpr (is_a.value) la.init(lane, wave, args.lda, w.m0, w.m0 + BM < M ? w.m0 + BM : M);
@@ -381,8 +405,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         if (w.cnt == 0) {
             w.part = 0;
             w.cnt = 1;
-            if constexpr (is_a.value) la.mask(lane, wave, K % kBK);
-            else lb.mask(lane, wave, K % kBK);
+            if constexpr (is_a.value) la.mask(lane, wave, K % kStage);
+            else lb.mask(lane, wave, K % kStage);
         }
     };
     auto walk_on = [&](Walk& w, auto is_a) {
@@ -431,8 +455,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     };
     read_first();
 
-    constexpr int kStores = TM * 2;  // of a wavefront and whole tile: 16 bytes a lane each
-    constexpr int kBarRow = 1;  // the row of k step 1 behind which the barrier stands
+    constexpr int kStores = S::kOutTM * 2;  // of a wavefront and whole tile: 16 bytes a lane each
+    constexpr int kBarRow = TM > 4 ? 1 : 0;  // the row of k step 1 behind which the barrier stands
     bool stored_fast = false;
     // One k step: TM x TN MFMAs in serpentine order; what else there is to do is dealt out behind single MFMAs, so that no more
     // instructions than fit under an MFMA stand between two.
@@ -507,19 +531,40 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         stage(std::true_type{});
         for (int kt = cur.len - 1; kt > 0; --kt) stage(std::false_type{});
         stored_fast = false;
-        if (cur.unit >= 0) {
-            // accumulator order: [TM][TN][threads] x 4 floats
-            float* part = args.partial + (int64_t)cur.unit * (BM * BN) + tid * 4;
+        // the slot of A that is free until the next stage's loads, which wait for the barrier below
+        lds_char* patch = lds_base + wr_a;
+        auto finish = [&](const auto& sum) {
+            if (cur.unit >= 0) {
+                // accumulator order: [kOutTM][TN][threads] x 4 floats
+                float* part = args.partial + (int64_t)cur.unit * (BM * BN) + tid * 4;
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+                for (int i = 0; i < S::kOutTM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4_t*>(part + (i * TN + j) * (kThreads * 4)) = acc[i][j];
+                    for (int j = 0; j < TN; ++j) *reinterpret_cast<f32x4_t*>(part + (i * TN + j) * (kThreads * 4)) = sum[i][j];
+            } else {
+                const bool whole = args.vec_out != 0 && cur.m0 + BM <= M && cur.n0 + BN <= N;
+                stored_fast = whole && args.preact == nullptr;
+                const Out<EPI, E> out(args, patch + wave * kPatch, cur.m0 + S::out_row(wave), cur.n0 + S::out_col(wave), whole, lane);
+                out.rows(sum, args);
+            }
+        };
+        if constexpr (KG == 1) {
+            finish(acc);
         } else {
-            const bool whole = args.vec_out != 0 && cur.m0 + BM <= M && cur.n0 + BN <= N;
-            stored_fast = whole && args.preact == nullptr;
-            // the slot of A that is free until the next stage's loads, which wait for the barrier below
-            const Out<EPI, E> out(args, lds_base + wr_a + wave * kPatch, cur.m0 + wm * (16 * TM), cur.n0 + wn * (16 * TN), whole, lane);
-            out.rows(acc, args);
+            // group g finishes the g-th half of its wavefronts' rows of tiles; of the others, a row at a time goes to its peer
+            const bool second = S::group(wave) != 0;
+            f32x4_t sum[S::kOutTM][TN];
+#pragma unroll
+            for (int i = 0; i < S::kOutTM; ++i) {
+                auto slot = [&](int w, int j) { return (__attribute__((address_space(3))) f32x4_t*)(patch + w * kPatch + j * 1024 + lane * 16); };
+#pragma unroll
+                for (int j = 0; j < TN; ++j) *slot(wave, j) = second ? acc[i][j] : acc[S::kOutTM + i][j];
+                publish();
+#pragma unroll
+                for (int j = 0; j < TN; ++j) sum[i][j] = (second ? acc[S::kOutTM + i][j] : acc[i][j]) + *slot(wave ^ (NW / 2), j);
+                publish();
+            }
+            finish(sum);
         }
         if (!more) break;
         cur = nxt;
@@ -532,60 +577,73 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // Finishes the sliced tiles: block (tile, row of MFMA tiles) adds the slices' partial sums in slice order and runs the epilogue.
-template <int TM, int EPI, typename E>
+template <int TM, int KG, int EPI, typename E>
 __global__ __launch_bounds__(kThreads) void wide_reduce_kernel(const TileArgs args) {
-    constexpr int BM = 16 * WM * TM;
+    using S = Shape<TM, KG>;
+    constexpr int BM = S::BM, BN = S::BN;
     __shared__ __attribute__((aligned(1024))) char lds[NW * kPatch];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tiles_m = (args.M + BM - 1) / BM, tiles_n = (args.N + BN - 1) / BN;
     const int rest = tiles_m * tiles_n - args.full;
-    const int r = blockIdx.x / TM, i = blockIdx.x % TM;
+    const int r = blockIdx.x / S::kOutTM, i = blockIdx.x % S::kOutTM;
     int tm, tn;
     gemm_tile::tile_origin(args.full + r, tiles_m, tiles_n, tm, tn);
     f32x4_t acc[1][TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[0][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const float* part = args.partial + (int64_t)r * (BM * BN) + i * (TN * kThreads * 4) + tid * 4;
-    for (int z = 0; z < args.slices; ++z, part += (int64_t)rest * (BM * BN)) {
+    // four slices' pieces requested together: a launch of a few tiles waits for memory alone
+    constexpr int kAhead = 4;
+    for (int z = 0; z < args.slices; z += kAhead, part += (int64_t)rest * (kAhead * BM * BN)) {
+        raw16_t u[kAhead][TN];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const raw16_t u = load_raw_stream(part + j * (kThreads * 4));
+        for (int a = 0; a < kAhead; ++a) {
+            const float* p = part + (z + a < args.slices ? a : 0) * ((int64_t)rest * (BM * BN));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[0][j][e] += __uint_as_float(u[e]);
+            for (int j = 0; j < TN; ++j) u[a][j] = load_raw_stream(p + j * (kThreads * 4));
         }
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a)
+            if (z + a < args.slices) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[0][j][e] += __uint_as_float(u[a][j][e]);
+            }
     }
     const int m0 = tm * BM, n0 = tn * BN;
     const bool whole = args.vec_out != 0 && m0 + BM <= args.M && n0 + BN <= args.N;
-    const Out<EPI, E> out(args, (lds_char*)lds + wave * kPatch, m0 + (wave / WN * TM + i) * 16, n0 + wave % WN * (16 * TN), whole, lane);
+    const Out<EPI, E> out(args, (lds_char*)lds + wave * kPatch, m0 + S::out_row(wave) + i * 16, n0 + S::out_col(wave), whole, lane);
     out.rows(acc, args);
 }
 
-template <bool TA, bool TB, int TM, int EPI, typename E>
+template <bool TA, bool TB, int TM, int KG, int EPI, typename E>
 int launch_rows(const TileArgs& args, hipStream_t s) {
-    constexpr int BM = 16 * WM * TM;
-    auto kern = gemm_wide_kernel<TA, TB, TM, EPI, E>;
+    using S = Shape<TM, KG>;
+    constexpr int BM = S::BM, BN = S::BN;
+    auto kern = gemm_wide_kernel<TA, TB, TM, KG, EPI, E>;
     if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)kLdsBytes, "gemm_wide"); lrc != CW_OK) return lrc;
     const int64_t tiles = (int64_t)((args.M + BM - 1) / BM) * ((args.N + BN - 1) / BN), rest = tiles - args.full;
     const int64_t pids = ((args.full + 7) & ~7) + ((rest * args.slices + 7) & ~(int64_t)7);
     hipLaunchKernelGGL(kern, dim3((unsigned)(pids < kUnits ? pids : kUnits)), dim3(kThreads), kLdsBytes, s, args);
     if (const int rc = check_launch("gemm_wide_kernel"); rc != CW_OK || rest == 0) return rc;
-    hipLaunchKernelGGL((wide_reduce_kernel<TM, EPI, E>), dim3((unsigned)(rest * TM)), dim3(kThreads), 0, s, args);
+    hipLaunchKernelGGL((wide_reduce_kernel<TM, KG, EPI, E>), dim3((unsigned)(rest * S::kOutTM)), dim3(kThreads), 0, s, args);
     return check_launch("wide_reduce_kernel");
 }
 
 // PLAIN_ONLY: no activations (the weight-gradient orientation, which nothing asks to be activated).
-template <bool TA, bool TB, bool PLAIN_ONLY, int TM, typename E>
+template <bool TA, bool TB, bool PLAIN_ONLY, int TM, int KG, typename E>
 int launch_epi(const TileArgs& args, int epilogue, hipStream_t s) {
     if constexpr (!PLAIN_ONLY) {
         switch (epilogue) {
-            case CW_EPI_BIAS_GELU_TANH: return launch_rows<TA, TB, TM, CW_EPI_BIAS_GELU_TANH, E>(args, s);
-            case CW_EPI_BIAS_GELU_ERF: return launch_rows<TA, TB, TM, CW_EPI_BIAS_GELU_ERF, E>(args, s);
-            case CW_EPI_BIAS_RELU: return launch_rows<TA, TB, TM, CW_EPI_BIAS_RELU, E>(args, s);
+            case CW_EPI_BIAS_GELU_TANH: return launch_rows<TA, TB, TM, KG, CW_EPI_BIAS_GELU_TANH, E>(args, s);
+            case CW_EPI_BIAS_GELU_ERF: return launch_rows<TA, TB, TM, KG, CW_EPI_BIAS_GELU_ERF, E>(args, s);
+            case CW_EPI_BIAS_RELU: return launch_rows<TA, TB, TM, KG, CW_EPI_BIAS_RELU, E>(args, s);
             default: break;
         }
     }
     if (epilogue != CW_EPI_NONE && epilogue != CW_EPI_BIAS) return fail(CW_ERR_INVALID, "cw_gemm_ksteps: bad epilogue %d", epilogue);
-    return launch_rows<TA, TB, TM, CW_EPI_BIAS, E>(args, s);
+    return launch_rows<TA, TB, TM, KG, CW_EPI_BIAS, E>(args, s);
 }
 
 }  // namespace gemm_wide

@@ -1,5 +1,5 @@
-"""GPU parity of the block GEMM's kernel of 256-column tiles (configuration 0 of the planner) against float64 where it can go
-wrong: every tile height, edges of M and N, steps whose K ends inside a stage, the shortest reductions it takes, seams of steps
+"""GPU parity of the block GEMM's kernels of 8 wavefronts (256-column tiles, and 128 x 128 tiles with two groups of wavefronts
+along k: configurations 0 and 5 of the planner) against float64 where they can go wrong: every tile height, edges of M and N, steps whose K ends inside a stage, the shortest reductions it takes, seams of steps
 and of tiles, sliced tiles, unaligned output rows, every operand of the epilogue."""
 import pytest
 import torch
@@ -14,8 +14,13 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(300, 32768, 1016, 1), (376, 32760, 1000, 1), (1552, 7672, 1352, 1), (8184, 2040, 328, 3), (8184, 6136, 520, 1),
           (7000, 4600, 1000, 1), (1024, 25003, 768, 1), (8192, 2048, 512, 2)]
 
+# shapes that the planner gives to 128 x 128 tiles: ragged last tiles of either direction, K that ends in the first and in the
+# second half of a stage, several steps, the shortest reduction it takes (in NT), an odd last column, every tile cut along k
+PAIRED = [(2040, 2040, 8200, 1), (4001, 1000, 1032, 3), (2040, 2040, 1416, 1), (4001, 1000, 4200, 1), (2040, 2047, 4200, 1),
+          (1016, 768, 5000, 1), (300, 2048, 8192, 1), (4096, 1024, 4096, 1)]
 
-@pytest.mark.parametrize("shape", SHAPES, ids=str)
+
+@pytest.mark.parametrize("shape", SHAPES + PAIRED, ids=str)
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_tiles_of_256_columns(layout, shape, dtype):
@@ -41,7 +46,8 @@ def test_tiles_of_256_columns(layout, shape, dtype):
     assert_parity(plain[rows], want - add[rows].double() - bias.double(), dtype, "plain %s %s %s" % (layout, shape, dtype))
 
 
-@pytest.mark.parametrize("layout,M,N,K", [("NN", 300, 4096, 16384), ("NT", 1554, 2560, 7680), ("TN", 2040, 2296, 8200), ("NT", 4352, 4096, 1024)])
+@pytest.mark.parametrize("layout,M,N,K", [("NN", 300, 4096, 16384), ("NT", 1554, 2560, 7680), ("TN", 2040, 2296, 8200), ("NT", 4352, 4096, 1024),
+                                          ("NN", 300, 2048, 8192), ("NT", 1552, 2560, 10240)])
 def test_sliced_tiles(layout, M, N, K):
     """Every tile, or the last round's, cut along k; bias, addend and pre-activation behind the reduction."""
     from cubework_amd import _lib, ops
