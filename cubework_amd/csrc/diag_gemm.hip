@@ -66,7 +66,7 @@ extern "C" int cw_diag_gemm_part(int part, int64_t M, int64_t N, int64_t K, int 
     args.rotate = 1;
     hipStream_t s = (hipStream_t)stream;
     switch (part) {
-        case 0: return gemm_wide::launch_rows<false, true, 8, 1, CW_EPI_BIAS_GELU_TANH, bf16_t>(args, s);
+        case 0: return gemm_wide::launch_rows<false, true, 8, 4, 1, CW_EPI_BIAS_GELU_TANH, bf16_t>(args, s);
         case 1: return launch_part<1>(args, s);
         case 2: return launch_part<2>(args, s);
         case 3: return launch_part<3>(args, s);

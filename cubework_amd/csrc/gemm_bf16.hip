@@ -17,6 +17,11 @@ namespace cw {
 
 #define CW_TILE_CFGS(e, l) {gemm_tile_##e##_##l##_1, gemm_tile_##e##_##l##_2, gemm_tile_##e##_##l##_3, gemm_tile_##e##_##l##_4}
 #define CW_WIDE_ROWS(e, l) {gemm_wide_##e##_##l##_128, gemm_wide_##e##_##l##_160, gemm_wide_##e##_##l##_192, gemm_wide_##e##_##l##_224, gemm_wide_##e##_##l##_256}
+#define CW_NARROW_ROWS(e, l) {gemm_wide_##e##_##l##_2128, gemm_wide_##e##_##l##_2160, gemm_wide_##e##_##l##_2192}
+#define CW_NARROW_DECL(e, l)                                            \
+    int gemm_wide_##e##_##l##_2128(const TileArgs&, int, hipStream_t);  \
+    int gemm_wide_##e##_##l##_2160(const TileArgs&, int, hipStream_t);  \
+    int gemm_wide_##e##_##l##_2192(const TileArgs&, int, hipStream_t);
 #define CW_TILE_DECL(e, l)                                              \
     int gemm_tile_##e##_##l##_1(const TileArgs&, int, hipStream_t);     \
     int gemm_tile_##e##_##l##_2(const TileArgs&, int, hipStream_t);     \
@@ -33,6 +38,10 @@ CW_TILE_DECL(bf16_t, TN)
 CW_TILE_DECL(f16_t, NN)
 CW_TILE_DECL(f16_t, NT)
 CW_TILE_DECL(f16_t, TN)
+CW_NARROW_DECL(bf16_t, NN)
+CW_NARROW_DECL(bf16_t, NT)
+CW_NARROW_DECL(f16_t, NN)
+CW_NARROW_DECL(f16_t, NT)
 
 using TileLaunch = int (*)(const TileArgs&, int, hipStream_t);
 static constexpr TileLaunch kTileLaunch[2][3][4] = {
@@ -42,6 +51,10 @@ static constexpr TileLaunch kTileLaunch[2][3][4] = {
 static constexpr TileLaunch kWideLaunch[2][3][5] = {
     {CW_WIDE_ROWS(bf16_t, NN), CW_WIDE_ROWS(bf16_t, NT), CW_WIDE_ROWS(bf16_t, TN)},
     {CW_WIDE_ROWS(f16_t, NN), CW_WIDE_ROWS(f16_t, NT), CW_WIDE_ROWS(f16_t, TN)},
+};
+static constexpr TileLaunch kNarrowLaunch[2][2][3] = {
+    {CW_NARROW_ROWS(bf16_t, NN), CW_NARROW_ROWS(bf16_t, NT)},
+    {CW_NARROW_ROWS(f16_t, NN), CW_NARROW_ROWS(f16_t, NT)},
 };
 static_assert(CW_NN == 0 && CW_NT == 1 && CW_TN == 2, "kTileLaunch is indexed by layout");
 
@@ -121,6 +134,7 @@ static int tile_launch(const GemmArgs& g, const TilePlan& plan, int layout, int 
     a.rotate = plan.rotate ? 1 : 0;
     a.partial = reinterpret_cast<float*>(ws + plan.pack_a_bytes + plan.pack_b_bytes + plan.pack_add_bytes);
     if (plan.cfg == 0 || plan.cfg == kPairedConfig) return kWideLaunch[f16 ? 1 : 0][layout][(plan.rows - 128) / 32](a, epilogue, s);
+    if (plan.cfg >= kNarrowConfig) return kNarrowLaunch[f16 ? 1 : 0][layout][(plan.rows - 128) / 32](a, epilogue, s);
     return kTileLaunch[f16 ? 1 : 0][layout][plan.cfg - 1](a, epilogue, s);
 }
 

@@ -43,7 +43,7 @@ struct GemmPlan {
 // for is planned by tile_plan). dma_enabled / strip_enabled: the two CW_GEMM_IMPL switches (staged / onelaunch) as the caller read them.
 GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool strip_enabled);
 
-// ---- tile kernels (gemm_wide.h: configurations 0 and 5; gemm_tile.h: the others) ---------------------------------------
+// ---- tile kernels (gemm_wide.h: configurations 0 and 5 to 7; gemm_tile.h: the others) ---------------------------------------
 // Their configurations: block tile 64 tm x 64 tn, k extent of a trip in units of 32, ring stages, resident
 // blocks per compute unit, and what a trip costs (us; one block on the unit / two) and a block besides its trips. The
 // costs are a fit to 2000 launches over 110 shapes (products of 64 .. 8192 tokens with the model widths 768 .. 4096, in the
@@ -61,15 +61,17 @@ constexpr TileConfig kTileConfigs[] = {
     {1, 2, 2, 3, 2, 0.440f, 0.800f, 2.60f},  // 64 x 128
     {1, 1, 2, 4, 2, 0.289f, 0.460f, 2.06f},  // 64 x 64: small outputs spread over the most compute units
     {2, 2, 4, 2, 1, 0.78f, 0.78f, 4.50f},    // 128 x 128, one block of two groups of wavefronts along k (gemm_wide.h)
+    {3, 2, 2, 3, 1, 0.62f, 0.62f, 4.00f},    // up to 192 x 128, 8 wavefronts (gemm_wide.h), not for TN
+    {2, 2, 2, 4, 1, 0.46f, 0.46f, 4.00f},    // 128 x 128, 8 wavefronts (gemm_wide.h), not for TN
 };
-constexpr int kTileConfigCount = 6, kPairedConfig = 5;
+constexpr int kTileConfigCount = 8, kPairedConfig = 5, kNarrowConfig = 6;  // kNarrowConfig and the one behind it
 
 // How a product runs on the tile kernels: `full` tiles whole, the others in `slices` k slices through fp32 partial
 // sums. An operand whose rows are not 16-byte aligned is copied to rows that are, once per step (pack_a / pack_b).
 struct TilePlan {
     int cfg;   // -1: the tile kernels do not take the shape
     int rows;  // tile height: that of the configuration, or less (configuration 0: the least of 160, 192, 224 and 256 that covers
-               // M with as many tiles)
+               // M with as many tiles; configuration 6: of 160 and 192)
     int64_t tiles;
     int full, slices;
     bool rotate;
@@ -78,10 +80,11 @@ struct TilePlan {
     int64_t pack_a_bytes, pack_b_bytes, pack_add_bytes, partial_bytes;
     int64_t scratch() const { return pack_a_bytes + pack_b_bytes + pack_add_bytes + partial_bytes; }
 };
-// Whether the kernel of configuration 0 (stage: 64) or 5 (128) takes such a product: at least three stages, and k-contiguous rows whose last 16
+// Whether a kernel of gemm_wide.h takes such a product: at least `stages` stages of `stage` k (the loads run ahead by one less), and k-contiguous rows whose last 16
 // bytes hold nothing behind K (multiples of 8, or copied rows, whose padding is zeros).
-bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b, int stage = 64);
+bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b, int stage = 64, int stages = 3);
 int wide_rows(int64_t M);
+int narrow_rows(int64_t M);
 // max_scratch < 0: the choice with as much scratch as it likes; else the best one that fits. align_a / align_b: every step's
 // pointer is 16-byte aligned and the leading dimension a multiple of 8; n_pack_addends: addends of which that is not true.
 TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int64_t lda, int64_t ldb, bool align_a, bool align_b,

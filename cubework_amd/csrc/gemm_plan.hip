@@ -226,9 +226,9 @@ constexpr int64_t kTileLaunchMax = ((int64_t)1 << 24) - 8;
 
 }  // namespace
 
-bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b, int stage) {
+bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b, int stage, int stages) {
     const bool a_ok = layout == CW_TN || K % 8 == 0 || pack_a, b_ok = layout != CW_NT || K % 8 == 0 || pack_b;
-    return a_ok && b_ok && (K + stage - 1) / stage * n_steps >= 3;
+    return a_ok && b_ok && (K + stage - 1) / stage * n_steps >= stages;
 }
 
 int wide_rows(int64_t M) {
@@ -236,6 +236,8 @@ int wide_rows(int64_t M) {
         if ((M + rows - 1) / rows == (M + 255) / 256) return rows;
     return 256;
 }
+
+int narrow_rows(int64_t M) { return (M + 159) / 160 == (M + 191) / 192 ? 160 : 192; }
 
 TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int64_t lda, int64_t ldb, bool align_a, bool align_b,
                    int n_pack_addends, int64_t max_scratch) {
@@ -279,50 +281,59 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     const double bytes = 2.0 * ((double)M * K * n_steps + (double)K * N * n_steps + (double)M * N);
     const double memory_us = bytes / 4.0e6;
     double best_us = 0;
-    auto consider = [&](int cfg, int64_t tiles, int64_t full, int slices) {
+    auto consider = [&](int cfg, int rows, int64_t tiles, int64_t full, int slices) {
         const TileConfig& c = kTileConfigs[cfg];
         const int64_t rest = tiles - full;
         double trips = (double)((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps;
         TilePlan q = p;
         q.cfg = cfg;
-        q.rows = cfg == 0 ? wide_rows(M) : 64 * c.tm;
+        q.rows = rows;
         q.tiles = tiles;
         q.full = (int)full;
         q.slices = rest > 0 ? slices : 1;
-        q.rotate = cfg == kPairedConfig || (cfg == 0 && (!ordered || rotated));
+        q.rotate = cfg == 0 ? !ordered || rotated : cfg >= kPairedConfig && !ordered;
         q.partial_bytes = rest * slices * (int64_t)(4096 * c.tm * c.tn) * 4;
         if (max_scratch >= 0 && q.scratch() > max_scratch) return;
         // TN on the kernels of gemm_tile.h: k-contiguous operands move as pieces of 64 bytes, k-slow ones as whole lines. On the
         // paired one: the two groups' transposing reads take more LDS cycles than their products.
         const double layout_factor = cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9;
-        if (cfg == 0) trips *= 0.2 + 0.8 / 256 * q.rows;  // a lower tile's trips are shorter
+        if (rows != 64 * c.tm) trips *= 0.2 + 0.8 * rows / (64 * c.tm);  // a lower tile's trips are shorter
         // the kernels of gemm_wide.h: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's
         // (the reduction waits about 0.9 us a slice whatever its size, and its bytes come from the cache)
-        const bool walks = cfg == 0 || cfg == kPairedConfig;
+        const bool walks = cfg == 0 || cfg >= kPairedConfig;
         double us = tile_rounds(c, (double)full, trips, layout_factor) + (walks && full > 0 ? 3.0 : 0.0);
         const double reduce_us = (walks ? 2.0 + 0.9 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
         if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor) + reduce_us;
+        // behind whole tiles: the slices start under the last tile's stores, and nothing hides theirs
+        if (cfg == 0 && rest > 0 && full > 0) us += 1.2 * q.partial_bytes / 6.6e6 - 8.0;
         us = us > memory_us ? us + 0.1 * memory_us : memory_us + 0.1 * us;
         if (best.cfg < 0 || us < best_us) {
             best = q;
             best_us = us;
         }
     };
-    for (int cfg = 0; cfg < kTileConfigCount; ++cfg) {
+    auto consider_rows = [&](int cfg, int rows) {
         const TileConfig& c = kTileConfigs[cfg];
+        // k ranges of the kernels of gemm_wide.h: more stages than their loads run ahead
+        const int least = cfg >= kNarrowConfig ? 5 : 3;
         const int64_t tiles = ((M + 64 * c.tm - 1) / (64 * c.tm)) * ((N + 64 * c.tn - 1) / (64 * c.tn));
-        if (tiles > kTileLaunchMax || ((cfg == 0 || cfg == kPairedConfig) && !wide_takes(layout, K, n_steps, p.pack_a, p.pack_b, 32 * c.kb))) continue;
-        if (cfg == kPairedConfig && ordered) continue;  // it sums k in another order than the other tiles do
+        if (tiles > kTileLaunchMax) return;
+        if ((cfg == 0 || cfg >= kPairedConfig) && !wide_takes(layout, K, n_steps, p.pack_a, p.pack_b, 32 * c.kb, least)) return;
         const int64_t trips = ((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps, cap = 256 * c.resident;
-        consider(cfg, tiles, tiles, 1);
+        consider(cfg, rows, tiles, tiles, 1);
         // all tiles sliced, to fill the chip about once; or only those of the partial last round
-        if (ordered) continue;
+        if (ordered) return;
         const int64_t last = tiles % cap;
         for (int slices = 2; slices <= 16; ++slices) {
-            if (trips / slices < 3) break;
-            if (tiles * slices <= cap) consider(cfg, tiles, 0, slices);
-            else if (tiles > cap && last > 0 && last * slices <= cap) consider(cfg, tiles, tiles - last, slices);
+            if (trips / slices < least) break;
+            if (tiles * slices <= cap) consider(cfg, rows, tiles, 0, slices);
+            else if (tiles > cap && last > 0 && last * slices <= cap) consider(cfg, rows, tiles, tiles - last, slices);
         }
+    };
+    for (int cfg = 0; cfg < kTileConfigCount; ++cfg) {
+        if (cfg == kPairedConfig && ordered) continue;  // it sums k in another order than the other tiles do
+        if (cfg >= kNarrowConfig && layout == CW_TN) continue;  // not built
+        consider_rows(cfg, cfg == 0 ? wide_rows(M) : cfg == kNarrowConfig ? narrow_rows(M) : 64 * kTileConfigs[cfg].tm);
     }
     return best;
 }

@@ -29,6 +29,13 @@
 // (M x N x K): 4096 x 1024 x 4096 42 -> 33, 2048 x 2048 x 8192 TN 79 -> 66, 1024 x 4096 x 4096 TN 41 -> 36; below about 1300 of k
 // the smaller blocks' epilogue is the cheaper one (4096 x 1024 x 1024: 15 and 14). Bound by L2 -> LDS: 62 bytes a cycle and
 // compute unit at the full matrix rate, where the load unit reaches 61; TN by the transposing LDS reads.
+//
+// TN = 2: tiles of 128 columns by 128, 160 or 192 rows for few rows (an evaluation of 300) and for NN products whose order of sums
+// is fixed, which the planner does not slice. 300 rows by 256 columns are 64 tiles for a projection of 16384, and 64 or 128 x 256
+// ones on blocks of 4 wavefronts fetch every weight three to five times; here 256 tiles of 160 x 128 take it in one round. The
+// stages are half as long, so the loads run three (128 rows: four) ahead instead of two: weights come from HBM once and are waited
+// for. us (M x N x K): 300 x 16384 x 4096 66 -> 47, 300 x 12288 x 4096 57 -> 45, 1554 x 2560 x 2560 33 -> 29 (NT 38 -> 29),
+// 500 x 8192 x 2048 25 -> 22. LDS-read bound at the full matrix rate (7 fragments for 10 MFMAs), memory-bound below 160 rows.
 #pragma once
 #include <cstddef>
 
@@ -139,22 +146,24 @@ struct Frags {
     }
 };
 
-// What follows the sums: a wavefront's accumulators go through 4 KB of LDS of its own, one row of MFMA tiles (16 x 64 fp32)
-// at a time, and come back as 8 columns of a row per lane: bias, addends and results move as 16 bytes per lane, whole
-// 128-byte lines per 8 lanes, edges are a matter of one lane, and no accumulator is copied to another register.
-// Chunk c (4 columns) of row r stands at c ^ r: both directions are conflict free.
-constexpr int kPatch = 4096;
-template <int EPI, typename E>
+// What follows the sums: a wavefront's accumulators go through LDS of its own, one row of TN MFMA tiles (16 x 16 TN fp32)
+// at a time, and come back as 8 columns of a row per lane: bias, addends and results move as 16 bytes per lane, 128-byte
+// lines per 8 lanes (TN = 2: 64 bytes per 4), edges are a matter of one lane, and no accumulator is copied to another register.
+// Chunk c (4 columns) of row r stands at c ^ r.
+template <int TN, int EPI, typename E>
 struct Out {
+    static constexpr int kPitch = 64 * TN, kPatch = 16 * kPitch;  // bytes of a row, of the wavefront's patch
+    static constexpr int LPR = 2 * TN, kHalves = TN / 2, kHalfRows = 64 / LPR;  // lanes of a row, passes, rows of a pass
+    static_assert(TN == 2 || TN == 4, "");
     lds_char *wr, *rd;  // the lane's addresses in the wavefront's patch
     int row, col, M, N;  // of the lane's piece in half 0 of row 0 of the tiles
     bool whole;
     u32x4_t bias;
     __device__ __forceinline__ Out(const TileArgs& a, lds_char* patch, int row0, int col0, bool whole_tile, int lane) {
         asm volatile("" : "+v"(lane));  // opaque: nothing of this is kept in registers between tiles
-        const int r = lane & 15, q = lane >> 4, rr = lane >> 3, c = lane & 7;
-        wr = patch + r * 256 + ((q ^ r) << 4);
-        rd = patch + rr * 256 + (((2 * c) ^ rr) << 4);
+        const int r = lane & 15, q = lane >> 4, rr = lane / LPR, c = lane % LPR, m = 4 * TN - 1;
+        wr = patch + r * kPitch + ((q ^ (r & m)) << 4);
+        rd = patch + rr * kPitch + (((2 * c) ^ (rr & m)) << 4);
         row = row0 + rr;
         col = col0 + 8 * c;
         M = a.M;
@@ -174,11 +183,11 @@ struct Out {
         }
     }
     static __device__ __forceinline__ lds_char* flip(lds_char* p, uint32_t bits) { return (lds_char*)(uintptr_t)((uint32_t)(uintptr_t)p ^ bits); }
-    __device__ __forceinline__ void put(const f32x4_t (&acc)[4]) const {
+    __device__ __forceinline__ void put(const f32x4_t (&acc)[TN]) const {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) *(__attribute__((address_space(3))) f32x4_t*)flip(wr, 64 * j) = acc[j];
+        for (int j = 0; j < TN; ++j) *(__attribute__((address_space(3))) f32x4_t*)flip(wr, 64 * j) = acc[j];
     }
-    // half H (8 rows) of the row of tiles in the patch
+    // pass H of the row of tiles in the patch (TN = 4: 8 rows each)
     template <int H>
     __device__ __forceinline__ void get(float (&v)[8]) const {
         lds_char* p = flip(rd, H * 128) + H * 2048;
@@ -228,42 +237,40 @@ struct Out {
         store(v, a.C, a.ldc, r);
     }
     template <int TM>
-    __device__ __forceinline__ void rows(const f32x4_t (&acc)[TM][4], const TileArgs& a) const {
+    __device__ __forceinline__ void rows(const f32x4_t (&acc)[TM][TN], const TileArgs& a) const {
         put(acc[0]);
         if (a.n_addends == 0) {
             static_for<TM>([&](auto i) {
-                float v[2][8];
-                get<0>(v[0]);
-                get<1>(v[1]);
+                float v[kHalves][8];
+                static_for<kHalves>([&](auto h) { get<h.value>(v[h.value]); });
                 if constexpr (i.value + 1 < TM) put(acc[i.value + 1]);
-                add(v[0], bias);
-                add(v[1], bias);
+#pragma unroll
+                for (int h = 0; h < kHalves; ++h) add(v[h], bias);
                 int r = row + 16 * i.value;
                 asm volatile("" : "+v"(r));  // opaque: the addresses of a row are formed here and not for all rows at once
-                finish(v[0], a, r);
-                finish(v[1], a, r + 8);
+#pragma unroll
+                for (int h = 0; h < kHalves; ++h) finish(v[h], a, r + kHalfRows * h);
                 __builtin_amdgcn_sched_barrier(0);
             });
         } else {
             constexpr int G = TM < 2 ? 1 : 2;  // rows of tiles whose pieces of the first addend are requested together
-            u32x4_t raw[G][2];
+            u32x4_t raw[G][kHalves];
             static_for<TM>([&](auto i) {
                 if constexpr (i.value % G == 0) {
 #pragma unroll
                     for (int g = 0; g < G && i.value + g < TM; ++g) {
                         int r = row + 16 * (i.value + g);
                         asm volatile("" : "+v"(r));
-                        raw[g][0] = addend(a, 0, r);
-                        raw[g][1] = addend(a, 0, r + 8);
+#pragma unroll
+                        for (int h = 0; h < kHalves; ++h) raw[g][h] = addend(a, 0, r + kHalfRows * h);
                     }
                 }
-                float v[2][8];
-                get<0>(v[0]);
-                get<1>(v[1]);
+                float v[kHalves][8];
+                static_for<kHalves>([&](auto h) { get<h.value>(v[h.value]); });
                 if constexpr (i.value + 1 < TM) put(acc[i.value + 1]);
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    int r = row + 16 * i.value + 8 * h;
+                for (int h = 0; h < kHalves; ++h) {
+                    int r = row + 16 * i.value + kHalfRows * h;
                     asm volatile("" : "+v"(r));
                     add(v[h], bias);
                     add(v[h], raw[i.value % G][h]);
@@ -276,21 +283,22 @@ struct Out {
     }
 };
 
-constexpr int NW = 8, WM = 2, TN = 4;  // wavefronts of a block, along M; MFMA tiles of a wavefront along N
+constexpr int NW = 8, WM = 2;  // wavefronts of a block, along M
 constexpr int kThreads = 64 * NW, kUnits = 256;
-constexpr int kStagesA = 3, kStagesB = 2;
-constexpr int kImage = 32 * 1024;  // LDS bytes of an operand's stage
-constexpr size_t kLdsBytes = (size_t)(kStagesA + kStagesB) * kImage;
-static_assert(kLdsBytes == 160 * 1024 && kImage >= NW * kPatch, "one block per compute unit; the epilogue's patches in a free stage of A");
 
-// KG = 1: the wavefronts are 2 x 4, each of 16 TM x 64 of the tile. KG = 2: two groups of 2 x 2, each of which owns the whole tile
-// and takes one half of a stage's 128 k; behind the last stage they exchange halves of their sums.
-template <int TM, int KG>
+// TN = 4, KG = 1: the wavefronts are 2 x 4, each of 16 TM x 64 of the tile. TN = 2: each of 16 TM x 32. KG = 2: two groups of 2 x 2,
+// each of which owns the whole tile and takes one half of a stage's 128 k; behind the last stage they exchange halves of their sums.
+template <int TM, int TN, int KG>
 struct Shape {
-    static constexpr int WN = 4 / KG, kRows = 256 / KG;  // kRows: rows of either operand's LDS image (of A, BM of them are fetched)
-    static constexpr int BM = 16 * WM * TM, BN = 16 * WN * TN, kStage = KG * kBK;
+    static constexpr int WN = 4 / KG, BM = 16 * WM * TM, BN = 16 * WN * TN, kStage = KG * kBK;
+    // rows of the operands' LDS images (of A, BM of them are fetched)
+    static constexpr int kRowsA = TN == 4 ? 256 / KG : (BM + 63) / 64 * 64, kRowsB = BN;
+    // stages that the loads run ahead: what 160 KB of LDS hold
+    static constexpr int kAhead = TN == 4 ? 2 : TM == 4 ? 4 : 3, kStagesA = kAhead + 1, kStagesB = kAhead;
+    static constexpr size_t kLdsBytes = (size_t)(kStagesA * kRowsA + kStagesB * kRowsB) * kStage * 2;
     static constexpr int kOutTM = TM / KG;  // rows of MFMA tiles that a wavefront finishes
-    static_assert(BN == kRows && BM <= kRows && TM % KG == 0, "");
+    static_assert(BM <= kRowsA && TM % KG == 0 && (KG == 1 || TN == 4), "");
+    static_assert(kLdsBytes <= 160 * 1024 && kRowsA * kStage * 2 >= NW * 1024 * TN, "one block per compute unit; the epilogue's patches in a free stage of A");
     static __device__ __forceinline__ int group(int wave) { return wave / (WM * WN); }
     static __device__ __forceinline__ int wm(int wave) { return wave / WN % WM; }
     static __device__ __forceinline__ int wn(int wave) { return wave % WN; }
@@ -298,23 +306,23 @@ struct Shape {
     static __device__ __forceinline__ int out_col(int wave) { return wn(wave) * 16 * TN; }
 };
 
-template <bool TRANS_A, bool TRANS_B, int TM, int KG, int EPI, typename E>
+template <bool TRANS_A, bool TRANS_B, int TM, int TN, int KG, int EPI, typename E>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_wide_kernel(const TileArgs args) {
-    using S = Shape<TM, KG>;
+    using S = Shape<TM, TN, KG>;
     constexpr int BM = S::BM, BN = S::BN, kStage = S::kStage;
-    using LA = Loader<TRANS_A, S::kRows, KG, NW>;
-    using LB = Loader<TRANS_B, S::kRows, KG, NW>;
-    static_assert(LA::kBytes == kImage && LB::kBytes == kImage, "");
+    using LA = Loader<TRANS_A, S::kRowsA, KG, NW>;
+    using LB = Loader<TRANS_B, S::kRowsB, KG, NW>;
+    using Epi = Out<TN, EPI, E>;
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     lds_char* lds_base = (lds_char*)lds;
-    const uint32_t lds_a = (uint32_t)(uintptr_t)lds_base, lds_b = lds_a + kStagesA * LA::kBytes;
+    const uint32_t lds_a = (uint32_t)(uintptr_t)lds_base, lds_b = lds_a + S::kStagesA * LA::kBytes;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = args.M, N = args.N, K = args.K;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const int kps = (K + kStage - 1) / kStage;
-    const int total = kps * args.n_steps;  // at least 3
+    const int total = kps * args.n_steps;  // more than kAhead, as is the length of a slice
     const int full_grid = (args.full + 7) & ~7;
     const int rest = tiles_m * tiles_n - args.full, units = rest * args.slices, per_xcd = (units + 7) >> 3;
     const int pids = full_grid + 8 * per_xcd;
@@ -359,10 +367,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     LA la;
     LB lb;
-    Frags<TRANS_A, S::kRows, TM> fa;
-    Frags<TRANS_B, S::kRows, TN> fb;
-    fa.init(lane, S::wm(wave) * 16 * TM, S::group(wave) * (kImage / KG));
-    fb.init(lane, S::wn(wave) * 16 * TN, S::group(wave) * (kImage / KG));
+    Frags<TRANS_A, S::kRowsA, TM> fa;
+    Frags<TRANS_B, S::kRowsB, TN> fb;
+    fa.init(lane, S::wm(wave) * 16 * TM, S::group(wave) * (LA::kBytes / KG));
+    fb.init(lane, S::wn(wave) * 16 * TN, S::group(wave) * (LB::kBytes / KG));
     const int64_t a_adv = TRANS_A ? args.lda * (2 * kStage) : 2 * kStage, b_adv = TRANS_B ? args.ldb * (2 * kStage) : 2 * kStage;
 
     // ---- what is requested next of either operand: `cnt` stages from p on, then `part` (the stage in which a step's K ends
@@ -415,7 +423,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     };
     constexpr std::true_type kA{};
     constexpr std::false_type kB{};
-    constexpr uint32_t kRingA = kStagesA * LA::kBytes, kRingB = kStagesB * LB::kBytes;
+    constexpr uint32_t kRingA = S::kStagesA * LA::kBytes, kRingB = S::kStagesB * LB::kBytes;
     const uint32_t lds_wa = lds_a + wave * (LA::PER * 1024), lds_wb = lds_b + wave * (LB::PER * 1024);
     uint32_t wr_a = 0, wr_b = 0;  // ring positions written and read next
     uint32_t rd_a = 0, rd_b = 0;
@@ -430,7 +438,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     walk_unit(wb, kB, cur);
     if (wa.cnt == 0) walk_event(wa, kA);
     if (wb.cnt == 0) walk_event(wb, kB);
-    for (int p = 0; p < 2; ++p) {
+    for (int p = 0; p < S::kAhead; ++p) {
         static_for<LA::PER>(issue_a);
         static_for<LB::PER>(issue_b);
         ring_on(wr_a, LA::kBytes, kRingA);
@@ -446,7 +454,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     f32x4_t acc[TM][TN];
     bf16x8_t af[TM], bfr[2][TN];
     lds_char *pa = lds_base, *pb = lds_base + kRingA;
-    dma_wait<LA::PER + LB::PER>();
+    dma_wait<(S::kAhead - 1) * (LA::PER + LB::PER)>();
     publish();
 
     auto read_first = [&]() {
@@ -455,7 +463,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     };
     read_first();
 
-    constexpr int kStores = S::kOutTM * 2;  // of a wavefront and whole tile: 16 bytes a lane each
+    constexpr int kStores = S::kOutTM * Epi::kHalves;  // of a wavefront and whole tile: 16 bytes a lane each
+    // loads behind the next stage's last one when the barrier is reached
+    constexpr int kBehind = (S::kAhead - 1) * LA::PER + (S::kAhead - 2) * LB::PER;
     constexpr int kBarRow = TM > 4 ? 1 : 0;  // the row of k step 1 behind which the barrier stands
     bool stored_fast = false;
     // One k step: TM x TN MFMAs in serpentine order; what else there is to do is dealt out behind single MFMAs, so that no more
@@ -495,8 +505,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             constexpr int R = row.value - kBarRow - 1, P = jc.value, NR = TM - 1 - kBarRow, H = TN / 2;
             if constexpr (R == -1 && P == TN - 1) {
                 __builtin_amdgcn_sched_barrier(0);
-                if (decltype(first)::value && stored_fast) dma_wait<LA::PER + kStores>();
-                else dma_wait<LA::PER>();
+                if (decltype(first)::value && stored_fast) dma_wait<kBehind + kStores>();
+                else dma_wait<kBehind>();
                 publish();
                 ring_on(rd_a, LA::kBytes, kRingA);
                 ring_on(rd_b, LB::kBytes, kRingB);
@@ -544,7 +554,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             } else {
                 const bool whole = args.vec_out != 0 && cur.m0 + BM <= M && cur.n0 + BN <= N;
                 stored_fast = whole && args.preact == nullptr;
-                const Out<EPI, E> out(args, patch + wave * kPatch, cur.m0 + S::out_row(wave), cur.n0 + S::out_col(wave), whole, lane);
+                const Epi out(args, patch + wave * Epi::kPatch, cur.m0 + S::out_row(wave), cur.n0 + S::out_col(wave), whole, lane);
                 out.rows(sum, args);
             }
         };
@@ -556,7 +566,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             f32x4_t sum[S::kOutTM][TN];
 #pragma unroll
             for (int i = 0; i < S::kOutTM; ++i) {
-                auto slot = [&](int w, int j) { return (__attribute__((address_space(3))) f32x4_t*)(patch + w * kPatch + j * 1024 + lane * 16); };
+                auto slot = [&](int w, int j) { return (__attribute__((address_space(3))) f32x4_t*)(patch + w * Epi::kPatch + j * 1024 + lane * 16); };
 #pragma unroll
                 for (int j = 0; j < TN; ++j) *slot(wave, j) = second ? acc[i][j] : acc[S::kOutTM + i][j];
                 publish();
@@ -577,11 +587,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // Finishes the sliced tiles: block (tile, row of MFMA tiles) adds the slices' partial sums in slice order and runs the epilogue.
-template <int TM, int KG, int EPI, typename E>
+template <int TM, int TN, int KG, int EPI, typename E>
 __global__ __launch_bounds__(kThreads) void wide_reduce_kernel(const TileArgs args) {
-    using S = Shape<TM, KG>;
+    using S = Shape<TM, TN, KG>;
     constexpr int BM = S::BM, BN = S::BN;
-    __shared__ __attribute__((aligned(1024))) char lds[NW * kPatch];
+    using Epi = Out<TN, EPI, E>;
+    __shared__ __attribute__((aligned(1024))) char lds[NW * Epi::kPatch];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tiles_m = (args.M + BM - 1) / BM, tiles_n = (args.N + BN - 1) / BN;
     const int rest = tiles_m * tiles_n - args.full;
@@ -613,37 +624,40 @@ __global__ __launch_bounds__(kThreads) void wide_reduce_kernel(const TileArgs ar
     }
     const int m0 = tm * BM, n0 = tn * BN;
     const bool whole = args.vec_out != 0 && m0 + BM <= args.M && n0 + BN <= args.N;
-    const Out<EPI, E> out(args, (lds_char*)lds + wave * kPatch, m0 + S::out_row(wave) + i * 16, n0 + S::out_col(wave), whole, lane);
+    const Epi out(args, (lds_char*)lds + wave * Epi::kPatch, m0 + S::out_row(wave) + i * 16, n0 + S::out_col(wave), whole, lane);
     out.rows(acc, args);
 }
 
-template <bool TA, bool TB, int TM, int KG, int EPI, typename E>
+template <bool TA, bool TB, int TM, int TN, int KG, int EPI, typename E>
 int launch_rows(const TileArgs& args, hipStream_t s) {
-    using S = Shape<TM, KG>;
+    using S = Shape<TM, TN, KG>;
     constexpr int BM = S::BM, BN = S::BN;
-    auto kern = gemm_wide_kernel<TA, TB, TM, KG, EPI, E>;
-    if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)kLdsBytes, "gemm_wide"); lrc != CW_OK) return lrc;
+    auto kern = gemm_wide_kernel<TA, TB, TM, TN, KG, EPI, E>;
+    if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)S::kLdsBytes, "gemm_wide"); lrc != CW_OK) return lrc;
     const int64_t tiles = (int64_t)((args.M + BM - 1) / BM) * ((args.N + BN - 1) / BN), rest = tiles - args.full;
+    // a plan for other tiles than these would have the kernel write partial sums that nothing holds
+    if (rest < 0 || (rest > 0 && (args.slices < 2 || args.partial == nullptr)))
+        return fail(CW_ERR_INVALID, "gemm_wide: %d whole tiles of %lld in %d slices", args.full, (long long)tiles, args.slices);
     const int64_t pids = ((args.full + 7) & ~7) + ((rest * args.slices + 7) & ~(int64_t)7);
-    hipLaunchKernelGGL(kern, dim3((unsigned)(pids < kUnits ? pids : kUnits)), dim3(kThreads), kLdsBytes, s, args);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(pids < kUnits ? pids : kUnits)), dim3(kThreads), S::kLdsBytes, s, args);
     if (const int rc = check_launch("gemm_wide_kernel"); rc != CW_OK || rest == 0) return rc;
-    hipLaunchKernelGGL((wide_reduce_kernel<TM, KG, EPI, E>), dim3((unsigned)(rest * S::kOutTM)), dim3(kThreads), 0, s, args);
+    hipLaunchKernelGGL((wide_reduce_kernel<TM, TN, KG, EPI, E>), dim3((unsigned)(rest * S::kOutTM)), dim3(kThreads), 0, s, args);
     return check_launch("wide_reduce_kernel");
 }
 
 // PLAIN_ONLY: no activations (the weight-gradient orientation, which nothing asks to be activated).
-template <bool TA, bool TB, bool PLAIN_ONLY, int TM, int KG, typename E>
+template <bool TA, bool TB, bool PLAIN_ONLY, int TM, int TN, int KG, typename E>
 int launch_epi(const TileArgs& args, int epilogue, hipStream_t s) {
     if constexpr (!PLAIN_ONLY) {
         switch (epilogue) {
-            case CW_EPI_BIAS_GELU_TANH: return launch_rows<TA, TB, TM, KG, CW_EPI_BIAS_GELU_TANH, E>(args, s);
-            case CW_EPI_BIAS_GELU_ERF: return launch_rows<TA, TB, TM, KG, CW_EPI_BIAS_GELU_ERF, E>(args, s);
-            case CW_EPI_BIAS_RELU: return launch_rows<TA, TB, TM, KG, CW_EPI_BIAS_RELU, E>(args, s);
+            case CW_EPI_BIAS_GELU_TANH: return launch_rows<TA, TB, TM, TN, KG, CW_EPI_BIAS_GELU_TANH, E>(args, s);
+            case CW_EPI_BIAS_GELU_ERF: return launch_rows<TA, TB, TM, TN, KG, CW_EPI_BIAS_GELU_ERF, E>(args, s);
+            case CW_EPI_BIAS_RELU: return launch_rows<TA, TB, TM, TN, KG, CW_EPI_BIAS_RELU, E>(args, s);
             default: break;
         }
     }
     if (epilogue != CW_EPI_NONE && epilogue != CW_EPI_BIAS) return fail(CW_ERR_INVALID, "cw_gemm_ksteps: bad epilogue %d", epilogue);
-    return launch_rows<TA, TB, TM, KG, CW_EPI_BIAS, E>(args, s);
+    return launch_rows<TA, TB, TM, TN, KG, CW_EPI_BIAS, E>(args, s);
 }
 
 }  // namespace gemm_wide

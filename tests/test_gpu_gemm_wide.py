@@ -1,5 +1,5 @@
-"""GPU parity of the block GEMM's kernels of 8 wavefronts (256-column tiles, and 128 x 128 tiles with two groups of wavefronts
-along k: configurations 0 and 5 of the planner) against float64 where they can go wrong: every tile height, edges of M and N, steps whose K ends inside a stage, the shortest reductions it takes, seams of steps
+"""GPU parity of the block GEMM's kernels of 8 wavefronts (256-column tiles, 128 x 128 tiles with two groups of wavefronts
+along k, 128-column tiles of up to 192 rows: configurations 0 and 5 to 7 of the planner) against float64 where they can go wrong: every tile height, edges of M and N, steps whose K ends inside a stage, the shortest reductions it takes, seams of steps
 and of tiles, sliced tiles, unaligned output rows, every operand of the epilogue."""
 import pytest
 import torch
@@ -20,7 +20,11 @@ PAIRED = [(2040, 2040, 8200, 1), (4001, 1000, 1032, 3), (2040, 2040, 1416, 1), (
           (1016, 768, 5000, 1), (300, 2048, 8192, 1), (4096, 1024, 4096, 1)]
 
 
-@pytest.mark.parametrize("shape", SHAPES + PAIRED, ids=str)
+# shapes that the planner gives to 128 columns by 128, 160 or 192 rows in NN or NT: the same edges, and slices of the fewest rows
+NARROW = [(300, 16376, 2056, 1), (1554, 2559, 1000, 3), (496, 8184, 2056, 1), (300, 4090, 12296, 1), (1554, 2560, 2560, 1)]
+
+
+@pytest.mark.parametrize("shape", SHAPES + PAIRED + NARROW, ids=str)
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_tiles_of_256_columns(layout, shape, dtype):
@@ -47,7 +51,7 @@ def test_tiles_of_256_columns(layout, shape, dtype):
 
 
 @pytest.mark.parametrize("layout,M,N,K", [("NN", 300, 4096, 16384), ("NT", 1554, 2560, 7680), ("TN", 2040, 2296, 8200), ("NT", 4352, 4096, 1024),
-                                          ("NN", 300, 2048, 8192), ("NT", 1552, 2560, 10240)])
+                                          ("NN", 300, 2048, 8192), ("NT", 300, 4096, 12288), ("NT", 1552, 2560, 10240)])
 def test_sliced_tiles(layout, M, N, K):
     """Every tile, or the last round's, cut along k; bias, addend and pre-activation behind the reduction."""
     from cubework_amd import _lib, ops
