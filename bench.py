@@ -233,7 +233,7 @@ def measured_traffic():
     size); None when the summary is not there."""
     import re
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
-                        "gemm_bf16_dma_kernel_linear2d_q2_counters.txt")
+                        "gemm_wide_kernel_linear2d_q2_counters.txt")
     try:
         with open(path) as f:
             m = re.search(r"^traffic_bytes_per_launch:\s*(\d+)", f.read(), re.M)
@@ -1269,9 +1269,9 @@ def main():
                    "layout": "NN", "flop_per_step": GEMM_FLOP, "operand_sets_rotated": n_sets, "device_arch": arch},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": measured_traffic(),
-                     "traffic_source": "profiles/gemm_bf16_dma_kernel_linear2d_q2_counters.txt (committed counter runs of "
-                                       "this script on the kernel's predecessor, same tiles; not measured in this run)",
-                     "kernel": "the launch cw_gemm_ksteps makes for this shape (gemm_tile_kernel, 256x256 tiles; "
+                     "traffic_source": "profiles/gemm_wide_kernel_linear2d_q2_counters.txt (committed counter runs of "
+                                       "this script; not measured in this run)",
+                     "kernel": "the launch cw_gemm_ksteps makes for this shape (gemm_wide_kernel, 256x256 tiles; "
                                "name as the kernel trace of this command shows it)",
                      "avg_launch_us": round(kernel_us, 2), "launches": args.sustained if args.sustained > 0 else args.steps,
                      "timed_steps": {"avg_launch_us": round(steps_us, 2),
@@ -1279,7 +1279,7 @@ def main():
                                      "note": "HIP events around the K timed steps only, which follow the sustained run"}},
     }
     if smi is not None and smi.get("shader_clock_MHz"):
-        # 4096 matrix instructions of 32 cycles per SIMD and launch: the share of the launch's shader cycles in which
+        # 8192 matrix instructions of 16 cycles per SIMD and launch: the share of the launch's shader cycles in which
         # the matrix pipe is busy, at the clock the driver reports
         cycles = kernel_us * smi["shader_clock_MHz"]
         smi["mfma_busy_frac"] = round(GEMM_FLOP / (256 * 4 * 1024.0) / cycles, 4) if cycles > 0 else None
