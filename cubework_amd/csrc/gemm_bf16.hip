@@ -194,9 +194,9 @@ int gemm_half_launch(const GemmArgs& args, int layout, int epilogue, bool f16, h
     const GemmPlan plan = gemm_half_plan(args, layout, tiles_ok, strip_split_enabled());
     switch (plan.route) {
         case kRouteSmallRing: return tile_launch(args, tile_plan_of(args, 2), layout, epilogue, f16, s);
-        case kRouteRing: return tile_launch(args, tile_plan_of(args, wide_takes(layout, args.K, args.n_steps, false, false) ? 0 : 1), layout, epilogue, f16, s);
+        case kRouteRing: return tile_launch(args, tile_plan_of(args, wide_takes(args.K, args.n_steps) ? 0 : 1), layout, epilogue, f16, s);
         case kRouteRingThenSmall: {
-            const int head = wide_takes(layout, args.K, args.n_steps, false, false) ? 0 : 1;
+            const int head = wide_takes(args.K, args.n_steps) ? 0 : 1;
             if (const int rc = tile_launch(plan.head, tile_plan_of(plan.head, head), layout, epilogue, f16, s); rc != CW_OK) return rc;
             return tile_launch(plan.tail, tile_plan_of(plan.tail, 2), layout, epilogue, f16, s);
         }

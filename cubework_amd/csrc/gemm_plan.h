@@ -80,9 +80,8 @@ struct TilePlan {
     int64_t pack_a_bytes, pack_b_bytes, pack_add_bytes, partial_bytes;
     int64_t scratch() const { return pack_a_bytes + pack_b_bytes + pack_add_bytes + partial_bytes; }
 };
-// Whether a kernel of gemm_wide.h takes such a product: at least `stages` stages of `stage` k (the loads run ahead by one less), and k-contiguous rows whose last 16
-// bytes hold nothing behind K (multiples of 8, or copied rows, whose padding is zeros).
-bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b, int stage = 64, int stages = 3);
+// Whether a kernel of gemm_wide.h takes such a product: at least `stages` stages of `stage` k (the loads run ahead by one less).
+bool wide_takes(int64_t K, int n_steps, int stage = 64, int stages = 3);
 int wide_rows(int64_t M);
 int narrow_rows(int64_t M);
 // max_scratch < 0: the choice with as much scratch as it likes; else the best one that fits. align_a / align_b: every step's

@@ -226,10 +226,7 @@ constexpr int64_t kTileLaunchMax = ((int64_t)1 << 24) - 8;
 
 }  // namespace
 
-bool wide_takes(int layout, int64_t K, int n_steps, bool pack_a, bool pack_b, int stage, int stages) {
-    const bool a_ok = layout == CW_TN || K % 8 == 0 || pack_a, b_ok = layout != CW_NT || K % 8 == 0 || pack_b;
-    return a_ok && b_ok && (K + stage - 1) / stage * n_steps >= stages;
-}
+bool wide_takes(int64_t K, int n_steps, int stage, int stages) { return (K + stage - 1) / stage * n_steps >= stages; }
 
 int wide_rows(int64_t M) {
     for (int rows : {160, 192, 224})
@@ -318,7 +315,7 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         const int least = cfg >= kNarrowConfig ? 5 : 3;
         const int64_t tiles = ((M + 64 * c.tm - 1) / (64 * c.tm)) * ((N + 64 * c.tn - 1) / (64 * c.tn));
         if (tiles > kTileLaunchMax) return;
-        if ((cfg == 0 || cfg >= kPairedConfig) && !wide_takes(layout, K, n_steps, p.pack_a, p.pack_b, 32 * c.kb, least)) return;
+        if ((cfg == 0 || cfg >= kPairedConfig) && !wide_takes(K, n_steps, 32 * c.kb, least)) return;
         const int64_t trips = ((K + 32 * c.kb - 1) / (32 * c.kb)) * n_steps, cap = 256 * c.resident;
         consider(cfg, rows, tiles, tiles, 1);
         // all tiles sliced, to fill the chip about once; or only those of the partial last round

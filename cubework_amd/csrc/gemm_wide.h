@@ -114,6 +114,20 @@ struct Loader {
         for (int i = 0; i < PER; ++i)
             if (kpos(lane, wave, i) >= k_rem) voff[i] = kRange;
     }
+    // k-contiguous rows whose K is no multiple of 8: what the wavefront's chunks hold behind K, in a stage that has arrived and is
+    // not yet published, becomes zeros (`lds_oper` as in issue)
+    static __device__ __forceinline__ void zero_tail(int lane, int wave, int k_rem, lds_char* lds_oper) {
+        if constexpr (!TRANS) {
+            asm volatile("" : "+v"(lane));
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const int d = k_rem - kpos(lane, wave, i);
+                if (d <= 0 || d >= 8) continue;
+                volatile lds_u16* chunk = (volatile lds_u16*)(lds_oper + i * 1024 + lane * 16);
+                for (int e = d; e < 8; ++e) chunk[e] = 0;
+            }
+        }
+    }
 };
 
 // Fragment reads of one operand: W MFMA tiles of 16 rows x 32 k per wavefront from operand row wrow of a 64 k image on, which
@@ -433,7 +447,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     int pid = blockIdx.x;
     if (!next_unit(pid, cur)) return;
-    nxt.len = 0;
+    nxt.len = nxt.k = 0;
     walk_unit(wa, kA, cur);
     walk_unit(wb, kB, cur);
     if (wa.cnt == 0) walk_event(wa, kA);
@@ -451,10 +465,30 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    // K that ends inside a 16-byte piece of k-contiguous rows: what is behind it in a step's last stage is cleared before that stage
+    // is published, by the wavefront that fetched it: a uniform branch a stage, nothing where K is a multiple of 8. Such products ran
+    // on the kernels of 4 wavefronts before (us, M x N x K): 300 x 16384 x 4092 NT 87 -> 53, 8192 x 2048 x 12565 NN 369 -> 315,
+    // 8192 x 8192 x 2044 NT 250 -> 216, 1554 x 2560 x 2556 NT 40 -> 33. pk, pleft: the step's stage that is published next, stages of its unit from it on.
+    const bool ragged = (!TRANS_A || !TRANS_B) && K % 8 != 0;
+    int pk = cur.k, pleft = cur.len;
+    auto zero_tails = [&]() {
+        if (pk + 1 == kps) {
+            LA::zero_tail(lane, wave, K % kStage, lds_base + wave * (LA::PER * 1024) + rd_a);
+            LB::zero_tail(lane, wave, K % kStage, lds_base + kRingA + wave * (LB::PER * 1024) + rd_b);
+        }
+        ++pk;
+        if (--pleft == 0) {
+            pk = nxt.k;
+            pleft = nxt.len;
+        } else if (pk == kps) {
+            pk = 0;
+        }
+    };
     f32x4_t acc[TM][TN];
     bf16x8_t af[TM], bfr[2][TN];
     lds_char *pa = lds_base, *pb = lds_base + kRingA;
     dma_wait<(S::kAhead - 1) * (LA::PER + LB::PER)>();
+    if (ragged) zero_tails();
     publish();
 
     auto read_first = [&]() {
@@ -507,9 +541,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 __builtin_amdgcn_sched_barrier(0);
                 if (decltype(first)::value && stored_fast) dma_wait<kBehind + kStores>();
                 else dma_wait<kBehind>();
-                publish();
                 ring_on(rd_a, LA::kBytes, kRingA);
                 ring_on(rd_b, LB::kBytes, kRingB);
+                if (ragged) zero_tails();
+                publish();
                 pa = lds_base + rd_a;
                 pb = lds_base + kRingA + rd_b;
             }

@@ -66,3 +66,31 @@ def test_sliced_tiles(layout, M, N, K):
     want += bias.double() + add.double()
     assert_parity(pre, want, torch.bfloat16, "sliced preact")
     assert_parity(out, want if act is None else torch.nn.functional.gelu(want, approximate="tanh"), torch.bfloat16, "sliced out")
+
+
+# K of every remainder by 8: the piece of 16 bytes in which a row ends, whole K inside a stage, steps and slices that end there
+RAGGED_K = [(8184, 2040, 331, 3), (7000, 4600, 961, 1), (1023, 768, 12565, 1), (4001, 1000, 1039, 3), (4001, 1000, 4162, 1),
+            (300, 16376, 2059, 1), (300, 4090, 12302, 1), (1554, 2560, 2556, 1), (300, 32768, 1021, 1)]
+
+
+@pytest.mark.parametrize("shape", RAGGED_K, ids=str)
+@pytest.mark.parametrize("layout", ["NN", "NT"])
+def test_rows_that_end_inside_16_bytes(layout, shape):
+    """What stands behind K in k-contiguous rows (NaN here) does not reach the sums."""
+    from cubework_amd import ops
+
+    M, N, K, steps = shape
+
+    def rows_of_k(n, seed, std):
+        t = torch.full((n, -(-K // 8) * 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+        t[:, :K] = randn((n, K), torch.bfloat16, seed, std).cuda()
+        return t[:, :K]
+
+    A = [rows_of_k(M, 3 * i, 1.0) for i in range(steps)]
+    B = [rows_of_k(N, 3 * i + 1, 0.05) if layout == "NT" else randn((K, -(-N // 8) * 8), torch.bfloat16, 3 * i + 1, 0.05).cuda()[:, :N]
+         for i in range(steps)]
+    got = ops.gemm_ksteps(layout, A, B)
+    rows = torch.cat([torch.arange(0, min(M, 64)), torch.arange(max(M - 64, 0), M)]).unique().cuda()
+    want = sum(a[rows].double() @ (b.double().t().contiguous() if layout == "NT" else b.double()) for a, b in zip(A, B))
+    assert_parity(got[rows], want, torch.bfloat16, "%s %s" % (layout, shape))
+    assert bool(torch.isfinite(got).all())
