@@ -293,7 +293,10 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         if (max_scratch >= 0 && q.scratch() > max_scratch) return;
         // TN on the kernels of gemm_tile.h: k-contiguous operands move as pieces of 64 bytes, k-slow ones as whole lines. On the
         // paired one: the two groups' transposing reads take more LDS cycles than their products.
-        const double layout_factor = cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9;
+        // Rows that are not whole 128-byte lines cost the paired kernel's loads more the longer its blocks run (us, M x N x K, paired
+        // / 256 x 256 in slices): 4096 x 1024 x 4104 NT 41 / 44, 4000 x 1000 x 8200 NT 70 / 81, 4096 x 1024 x 12568 NN 131 / 104.
+        const double pitch_factor = cfg == kPairedConfig && trips > 80 && (p.lda % 64 != 0 || p.ldb % 64 != 0) ? 1.25 : 1.0;
+        const double layout_factor = pitch_factor * (cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9);
         if (rows != 64 * c.tm) trips *= 0.2 + 0.8 * rows / (64 * c.tm);  // a lower tile's trips are shorter
         // the kernels of gemm_wide.h: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's
         // (the reduction waits about 0.9 us a slice whatever its size, and its bytes come from the cache)

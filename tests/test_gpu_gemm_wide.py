@@ -68,9 +68,11 @@ def test_sliced_tiles(layout, M, N, K):
     assert_parity(out, want if act is None else torch.nn.functional.gelu(want, approximate="tanh"), torch.bfloat16, "sliced out")
 
 
-# K of every remainder by 8: the piece of 16 bytes in which a row ends, whole K inside a stage, steps and slices that end there
+# K of every remainder by 8: the piece of 16 bytes in which a row ends, whole K inside a stage, steps and slices that end there; both
+# sides of the planner's rule for long rows that are not whole lines
 RAGGED_K = [(8184, 2040, 331, 3), (7000, 4600, 961, 1), (1023, 768, 12565, 1), (4001, 1000, 1039, 3), (4001, 1000, 4162, 1),
-            (300, 16376, 2059, 1), (300, 4090, 12302, 1), (1554, 2560, 2556, 1), (300, 32768, 1021, 1)]
+            (300, 16376, 2059, 1), (300, 4090, 12302, 1), (1554, 2560, 2556, 1), (300, 32768, 1021, 1),
+            (4096, 1024, 12565, 1), (4096, 1024, 10235, 1)]
 
 
 @pytest.mark.parametrize("shape", RAGGED_K, ids=str)
