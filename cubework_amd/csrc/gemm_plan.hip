@@ -293,17 +293,21 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         if (max_scratch >= 0 && q.scratch() > max_scratch) return;
         // TN on the kernels of gemm_tile.h: k-contiguous operands move as pieces of 64 bytes, k-slow ones as whole lines. On the
         // paired one: the two groups' transposing reads take more LDS cycles than their products.
-        // Rows that are not whole 128-byte lines cost the paired kernel's loads more the longer its blocks run (us, M x N x K, paired
-        // / 256 x 256 in slices): 4096 x 1024 x 4104 NT 41 / 44, 4000 x 1000 x 8200 NT 70 / 81, 4096 x 1024 x 12568 NN 131 / 104.
-        const double pitch_factor = cfg == kPairedConfig && trips > 80 && (p.lda % 64 != 0 || p.ldb % 64 != 0) ? 1.25 : 1.0;
-        const double layout_factor = pitch_factor * (cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9);
+        const double layout_factor = cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9;
+        // Rows that are not whole 128-byte lines cost the paired kernel's loads more the longer a block walks along them (us, M x N x K):
+        // whole tiles, paired / 256 x 256 in slices: 4096 x 1024 x 4104 NT 41 / 44, 4000 x 1000 x 8200 NT 70 / 81, 4096 x 1024 x 12568 NN
+        // 131 / 104; the blocks of a sliced product are short, paired / 128 x 128 of one group: 1023 x 768 x 50257 NN in 5 slices 99 / 111,
+        // 251 x 2048 x 50272 NN in 8 64 / 73, 2048 x 1024 x 12568 NN in 2 65 / 72, 1632 x 768 x 12568 NN in 3 45 / 50.
+        auto pitch_factor = [&](double block_trips) {
+            return cfg == kPairedConfig && block_trips > 80 && (p.lda % 64 != 0 || p.ldb % 64 != 0) ? 1.25 : 1.0;
+        };
         if (rows != 64 * c.tm) trips *= 0.2 + 0.8 * rows / (64 * c.tm);  // a lower tile's trips are shorter
         // the kernels of gemm_wide.h: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's
         // (the reduction waits about 0.9 us a slice whatever its size, and its bytes come from the cache)
         const bool walks = cfg == 0 || cfg >= kPairedConfig;
-        double us = tile_rounds(c, (double)full, trips, layout_factor) + (walks && full > 0 ? 3.0 : 0.0);
+        double us = tile_rounds(c, (double)full, trips, layout_factor * pitch_factor(trips)) + (walks && full > 0 ? 3.0 : 0.0);
         const double reduce_us = (walks ? 2.0 + 0.9 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
-        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor) + reduce_us;
+        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor * pitch_factor(trips / slices)) + reduce_us;
         // behind whole tiles: the slices start under the last tile's stores, and nothing hides theirs
         if (cfg == 0 && rest > 0 && full > 0) us += 1.2 * q.partial_bytes / 6.6e6 - 8.0;
         us = us > memory_us ? us + 0.1 * memory_us : memory_us + 0.1 * us;
