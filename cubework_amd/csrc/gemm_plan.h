@@ -46,10 +46,14 @@ GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool
 // ---- tile kernels (gemm_wide.h: configurations 0 and 5 to 7; gemm_tile.h: the others) ---------------------------------------
 // Their configurations: block tile 64 tm x 64 tn, k extent of a trip in units of 32, ring stages, resident
 // blocks per compute unit, and what a trip costs (us; one block on the unit / two) and a block besides its trips. The
-// costs are a fit to 2000 launches over 110 shapes (products of 64 .. 8192 tokens with the model widths 768 .. 4096, in the
-// forward and weight-gradient orientations; rms error 11 %); choosing by them comes within 2 % of the best choice on average.
-// (The launches' times are not kept in this tree: a change of the kernels' speed means measuring and fitting again. Configurations
-// 0 and 5, and what cutting along k costs them, are a fit to 250 launches over 30 of these shapes.)
+// costs were a fit to 2000 launches over 110 shapes (products of 64 .. 8192 tokens with the model widths 768 .. 4096, in the
+// forward and weight-gradient orientations; rms error 11 %). Configurations 0 and 5 to 7, what cutting along k costs them, and where the
+// choice against them lies (1 and 2, the factors of TN) were fitted to some 250 later launches of 30 of these shapes; 3 and 4 to 14000
+// launches of every configuration over 1000 shapes (also layers of any width and vocabularies), the others held. Choosing by them
+// costs 1.6 % over the best launch of a shape on average. 3 and 4 at 0.440, 0.800, 2.60 and 0.289, 0.460, 2.06 (2.1 %) gave short products
+// 64 x 64 tiles in two rounds (us, M x N x K): 2394 x 576 x 1536 NT 15.8 / 12.9 on 64 x 128, 1894 x 1024 x 1024 NT 11.2 / 9.5,
+// 1280 x 1024 x 1024 NT 10.5 / 9.1, 473 x 3072 x 768 NN 9.7 / 8.8. (The launches' times are not kept in this tree: a change of the
+// kernels' speed means measuring and fitting again.)
 struct TileConfig {
     int tm, tn, kb, stages, resident;
     float trip1, trip2, fixed;
@@ -58,8 +62,8 @@ constexpr TileConfig kTileConfigs[] = {
     {4, 4, 2, 2, 1, 1.43f, 1.43f, 4.00f},    // up to 256 x 256: the least operand traffic per FLOP, one block per compute unit
     {2, 4, 1, 3, 2, 0.480f, 0.897f, 5.00f},  // 128 x 256, two blocks
     {2, 2, 1, 5, 2, 0.285f, 0.546f, 4.50f},  // 128 x 128
-    {1, 2, 2, 3, 2, 0.440f, 0.800f, 2.60f},  // 64 x 128
-    {1, 1, 2, 4, 2, 0.289f, 0.460f, 2.06f},  // 64 x 64: small outputs spread over the most compute units
+    {1, 2, 2, 3, 2, 0.420f, 0.760f, 2.50f},  // 64 x 128
+    {1, 1, 2, 4, 2, 0.260f, 0.550f, 2.00f},  // 64 x 64: small outputs spread over the most compute units
     {2, 2, 4, 2, 1, 0.78f, 0.78f, 4.50f},    // 128 x 128, one block of two groups of wavefronts along k (gemm_wide.h)
     {3, 2, 2, 3, 1, 0.62f, 0.62f, 4.00f},    // up to 192 x 128, 8 wavefronts (gemm_wide.h), not for TN
     {2, 2, 2, 4, 1, 0.46f, 0.46f, 4.00f},    // 128 x 128, 8 wavefronts (gemm_wide.h), not for TN

@@ -44,3 +44,10 @@ def test_long_rows_in_short_blocks_stay_on_the_paired_kernel(plans, layout, M, N
 def test_long_rows_in_long_blocks_leave_the_paired_kernel(plans):
     (cfg, *_), = plans([("NN", 4096, 1024, 12568, 1)])
     assert cfg != PAIRED
+
+
+@pytest.mark.parametrize("layout,M,N,K", [("NT", 2394, 576, 1536), ("NT", 1894, 1024, 1024), ("NT", 1280, 1024, 1024), ("NN", 1777, 768, 768),
+                                          ("NN", 473, 3072, 768), ("NN", 351, 3072, 1024)])
+def test_short_products_of_one_round_take_64_x_128_tiles(plans, layout, M, N, K):
+    """140 to 240 tiles of 64 x 128 are one round of the chip; as 64 x 64 they share its units in pairs (10 to 20 % slower)."""
+    assert plans([(layout, M, N, K, 1)]) == [(3, 64, -(-M // 64) * -(-N // 128), 1, 0)]
