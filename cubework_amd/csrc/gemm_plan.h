@@ -86,6 +86,13 @@ struct TilePlan {
 };
 // Whether a kernel of gemm_wide.h takes such a product: at least `stages` stages of `stage` k (the loads run ahead by one less).
 bool wide_takes(int64_t K, int n_steps, int stage = 64, int stages = 3);
+// What a launch of such a kernel rests on: `tiles` tiles of which `full` are whole, the others in slices through partial sums, and every
+// unit longer than the `ahead` stages that the loads run ahead (of a shorter one the loads behind its last stage are given up, the next
+// unit's with them: wrong sums).
+inline bool wide_units_hold(int64_t tiles, int64_t full, int slices, bool has_partial, int64_t stages, int ahead) {
+    if (full < 0 || full > tiles || stages <= ahead) return false;
+    return full == tiles || (slices >= 2 && has_partial && stages / slices > ahead);
+}
 int wide_rows(int64_t M);
 int narrow_rows(int64_t M);
 // max_scratch < 0: the choice with as much scratch as it likes; else the best one that fits. align_a / align_b: every step's

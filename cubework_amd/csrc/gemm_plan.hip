@@ -264,7 +264,7 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         p.pack_b_bytes = copy_bytes(n_steps, b_rows, b_cols);
     }
     if (n_pack_addends > 0) p.pack_add_bytes = copy_bytes(n_pack_addends, M, N);
-    // the kernels' lane offsets: 256 rows (or 32 k rows) of either operand within 2 GB
+    // the kernels' lane offsets: 256 rows of either operand (or the k rows of a trip, 128 at most) within 2 GB
     if (p.lda >= ((int64_t)1 << 22) || p.ldb >= ((int64_t)1 << 22)) return best;
     // An NN product (B stored [K, N]) that does not reduce its width, K <= N, sums k in ascending order whatever the tile: the
     // 16-bit results of a row do not depend on how many rows there are, and a ReLU behind the next layer sees the same signs.

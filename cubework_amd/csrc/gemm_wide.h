@@ -39,15 +39,14 @@
 #pragma once
 #include <cstddef>
 
+#include "gemm_plan.h"
 #include "gemm_tile.h"
 
 namespace cw {
 namespace gemm_wide {
 
 using gemm_bf16::bf16x8_t;
-using gemm_bf16::f32x16_t;
 using gemm_bf16::static_for;
-using gemm_bf16::u32x2_t;
 using gemm_bf16::u32x4_t;
 using gemm_tile::kRange;
 using gemm_tile::kTabA;
@@ -667,12 +666,13 @@ template <bool TA, bool TB, int TM, int TN, int KG, int EPI, typename E>
 int launch_rows(const TileArgs& args, hipStream_t s) {
     using S = Shape<TM, TN, KG>;
     constexpr int BM = S::BM, BN = S::BN;
+    const int64_t tiles = (int64_t)((args.M + BM - 1) / BM) * ((args.N + BN - 1) / BN), rest = tiles - args.full;
+    const int64_t stages = (int64_t)((args.K + S::kStage - 1) / S::kStage) * args.n_steps;
+    if (!wide_units_hold(tiles, args.full, args.slices, args.partial != nullptr, stages, S::kAhead))
+        return fail(CW_ERR_INVALID, "gemm_wide: %d whole tiles of %lld, the others in %d slices, of %lld stages", args.full, (long long)tiles,
+                    args.slices, (long long)stages);
     auto kern = gemm_wide_kernel<TA, TB, TM, TN, KG, EPI, E>;
     if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)S::kLdsBytes, "gemm_wide"); lrc != CW_OK) return lrc;
-    const int64_t tiles = (int64_t)((args.M + BM - 1) / BM) * ((args.N + BN - 1) / BN), rest = tiles - args.full;
-    // a plan for other tiles than these would have the kernel write partial sums that nothing holds
-    if (rest < 0 || (rest > 0 && (args.slices < 2 || args.partial == nullptr)))
-        return fail(CW_ERR_INVALID, "gemm_wide: %d whole tiles of %lld in %d slices", args.full, (long long)tiles, args.slices);
     const int64_t pids = ((args.full + 7) & ~7) + ((rest * args.slices + 7) & ~(int64_t)7);
     hipLaunchKernelGGL(kern, dim3((unsigned)(pids < kUnits ? pids : kUnits)), dim3(kThreads), S::kLdsBytes, s, args);
     if (const int rc = check_launch("gemm_wide_kernel"); rc != CW_OK || rest == 0) return rc;

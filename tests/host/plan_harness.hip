@@ -7,7 +7,8 @@
 //     pointer stays inside its operand, the strip fits one round of 128 x 128 tiles;
 //   * split k: slices divide K into multiples of 64, the partial sums fit the workspace;
 //   * the tile kernels' plans (tile_plan): scratch within its bound, whole and sliced tiles, copies and partial sums that
-//     add up, lane offsets below 2 GiB, launches below 2^32 work-items;
+//     add up, tile heights that are built, units longer than the loads run ahead, one order of sums where it is promised, lane offsets
+//     below 2 GiB, launches below 2^32 work-items;
 //   * column sums: the slabs cover the rows exactly once and their partial rows fit cw_colsum_workspace_bytes'
 //     promise of at most 512 (or ceil(M / 64)) rows.
 // Prints "ok <checks> routes <how often each kernel route was planned>" and exits 0, or the first violated invariant and exits 1.
@@ -143,6 +144,7 @@ void run_problem(const Problem& p) {
                 case kRouteSplitK:
                     REQUIRE(plan.slices >= 2 && plan.slices <= 8 && args.K % (64 * plan.slices) == 0, "slices %d of K=%d", plan.slices, args.K);
                     REQUIRE((int64_t)plan.slices * args.M * args.N * 4 <= args.workspace_bytes, "partial sums exceed the workspace");
+                    REQUIRE(wide_units_hold((int64_t)(args.M / 256) * (args.N / 256), 0, plan.slices, true, (int64_t)(args.K / 64) * args.n_steps, 2), "short slices of K=%d", args.K);
                     REQUIRE((int64_t)(args.M / 256) * (args.N / 256) * plan.slices <= 256 && args.M % 256 == 0 && args.N % 256 == 0, "split grid");
                     break;
                 default: break;
@@ -185,7 +187,7 @@ void sweep_gemm() {
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // What one plan of the tile kernels promises: it fits the scratch it was given, its tiles, slices and sub-buffers add up
-// as the launches use them (gemm_bf16.hip's tile_launch, gemm_tile.h's launch_cfg), and no offset or grid leaves its type.
+// as the launches use them (gemm_bf16.hip's tile_launch, gemm_tile.h's launch_cfg, gemm_wide.h's launch_rows), and no offset or grid leaves its type.
 void check_tile_plan(int layout, int64_t M, int64_t N, int64_t K, int steps, int64_t lda, int64_t ldb, bool al_a, bool al_b, int n_pack,
                      int64_t max_scratch, bool must_plan) {
     const TilePlan p = tile_plan(layout, M, N, K, steps, lda, ldb, al_a, al_b, n_pack, max_scratch);
@@ -204,6 +206,23 @@ void check_tile_plan(int layout, int64_t M, int64_t N, int64_t K, int steps, int
     PLAN_REQUIRE(p.full >= 0 && p.full <= p.tiles && p.slices >= 1 && (p.full < p.tiles || p.slices == 1));
     const int64_t rest = p.tiles - p.full, trips = ceil_div(K, 32 * c.kb) * steps;
     PLAN_REQUIRE(p.slices <= trips);
+    // heights that are built, with as many tiles as the configuration's own; the 128-column tiles are not built for TN
+    switch (p.cfg) {
+        case 0: PLAN_REQUIRE(p.rows == 160 || p.rows == 192 || p.rows == 224 || p.rows == 256); break;
+        case kNarrowConfig: PLAN_REQUIRE(p.rows == 160 || p.rows == 192); break;
+        default: PLAN_REQUIRE(p.rows == bm); break;
+    }
+    PLAN_REQUIRE(ceil_div(M, p.rows) == ceil_div(M, bm));
+    PLAN_REQUIRE(p.cfg < kNarrowConfig || layout != CW_TN);
+    // gemm_wide.h: every unit is longer than the loads run ahead (4 stages at most for 128 columns, 2 for the others)
+    const bool walks = p.cfg == 0 || p.cfg >= kPairedConfig;
+    if (walks) PLAN_REQUIRE(wide_units_hold(p.tiles, p.full, p.slices, p.partial_bytes > 0, trips, p.cfg >= kNarrowConfig ? 4 : 2));
+    // a product whose rows do not depend on their number sums k in one order: not cut, no two sums, rotated on aligned 256 x 256 tiles alone
+    if (layout == CW_NN && K <= N) {
+        PLAN_REQUIRE(rest == 0 && p.cfg != kPairedConfig);
+        PLAN_REQUIRE(!p.rotate || (p.cfg == 0 && M % 256 == 0 && N % 256 == 0));
+    }
+    PLAN_REQUIRE(!p.rotate || walks);
     // the partial sums of every (tile, slice), behind the copies, all at 16-byte boundaries and within the scratch
     PLAN_REQUIRE(p.partial_bytes == rest * (p.slices > 1 || rest > 0 ? p.slices : 0) * bm * bn * 4);
     PLAN_REQUIRE(p.pack_a_bytes % 16 == 0 && p.pack_b_bytes % 16 == 0 && p.pack_add_bytes % 16 == 0);
@@ -216,14 +235,15 @@ void check_tile_plan(int layout, int64_t M, int64_t N, int64_t K, int steps, int
     if (p.pack_b) PLAN_REQUIRE(p.ldb % 8 == 0 && p.ldb >= b_cols && p.pack_b_bytes >= steps * b_rows * p.ldb * 2);
     else PLAN_REQUIRE(p.ldb == ldb && p.pack_b_bytes == 0);
     PLAN_REQUIRE(p.pack_add_bytes >= n_pack * M * ceil_div(N, 8) * 16);
-    // a lane's byte offset (the block's rows, or 32 rows of k) stays inside the buffer's 2 GiB
-    const int64_t reach = (int64_t)1 << 31;
-    PLAN_REQUIRE((layout == CW_TN ? 31 * p.lda + bm : (bm - 1) * p.lda + 32) * 2 < reach);
-    PLAN_REQUIRE((layout == CW_NT ? (bn - 1) * p.ldb + 32 : 31 * p.ldb + bn) * 2 < reach);
+    // a lane's byte offset (the block's rows, or a trip's rows of k) stays inside the buffer's 2 GiB
+    const int64_t reach = (int64_t)1 << 31, kt = 32 * c.kb;
+    PLAN_REQUIRE((layout == CW_TN ? (kt - 1) * p.lda + bm : (bm - 1) * p.lda + kt) * 2 < reach);
+    PLAN_REQUIRE((layout == CW_NT ? (bn - 1) * p.ldb + kt : (kt - 1) * p.ldb + bn) * 2 < reach);
     // every launch is at most 2^32 - 1 work-items: the tiles and slices, their reduction, the copies (16 bytes each)
     const int64_t items = ((int64_t)1 << 32) - 1;
-    PLAN_REQUIRE((ceil_div(p.full, 8) + ceil_div(rest * p.slices, 8)) * 8 * 256 <= items);
-    PLAN_REQUIRE(rest * c.tm * 256 <= items);
+    const int64_t threads = walks ? 512 : 256;  // (gemm_wide.h's launches have 256 blocks at most, their reductions one for 32 rows)
+    if (!walks) PLAN_REQUIRE((ceil_div(p.full, 8) + ceil_div(rest * p.slices, 8)) * 8 * threads <= items);
+    PLAN_REQUIRE(rest * (walks ? p.rows / 32 : c.tm) * threads <= items);
     for (const int64_t bytes : {p.pack_a_bytes / steps, p.pack_b_bytes / steps, n_pack > 0 ? p.pack_add_bytes / n_pack : 0})
         PLAN_REQUIRE(ceil_div(bytes, 16 * 256) * 256 <= items);
 #undef PLAN_REQUIRE
@@ -231,7 +251,7 @@ void check_tile_plan(int layout, int64_t M, int64_t N, int64_t K, int steps, int
 
 void sweep_tile_plan() {
     const int64_t dims[] = {1, 7, 63, 64, 65, 128, 250, 256, 264, 777, 2048, 2056, 4376, 8192, 12568, 50257, 1 << 20, 3 << 20, 1 << 28, 1 << 30};
-    const int64_t ks[] = {1, 8, 31, 32, 72, 1003, 2048, 4096, 12568, 50257, 1 << 20, 1 << 30};
+    const int64_t ks[] = {1, 8, 31, 32, 40, 72, 136, 200, 264, 331, 1003, 2048, 4096, 12568, 50257, 1 << 20, 1 << 30};
     for (int layout = 0; layout < 3; ++layout)
         for (int64_t M : dims)
             for (int64_t N : dims)
@@ -259,6 +279,11 @@ void sweep_tile_plan() {
         REQUIRE(tile_plan(CW_NN, bad, 8, 8, 1, 8, 8, true, true, 0, -1).cfg == -1 && tile_plan(CW_NN, 8, bad, 8, 1, 8, 8, true, true, 0, -1).cfg == -1 &&
                     tile_plan(CW_NN, 8, 8, bad, 1, 8, 8, true, true, 0, -1).cfg == -1, "a plan for a size of %lld", (long long)bad);
     }
+    // the launches of gemm_wide.h refuse a plan for other tiles, partial sums that nothing holds, units as short as the loads run ahead
+    REQUIRE(wide_units_hold(10, 10, 1, false, 3, 2) && wide_units_hold(10, 0, 3, true, 9, 2) && wide_units_hold(10, 8, 2, true, 11, 4), "launches that hold");
+    REQUIRE(!wide_units_hold(10, 11, 1, true, 9, 2) && !wide_units_hold(10, -1, 2, true, 9, 2), "a plan for other tiles");
+    REQUIRE(!wide_units_hold(10, 8, 1, true, 9, 2) && !wide_units_hold(10, 8, 2, false, 9, 2), "partial sums that nothing holds");
+    REQUIRE(!wide_units_hold(10, 10, 1, false, 2, 2) && !wide_units_hold(10, 0, 3, true, 8, 2) && !wide_units_hold(10, 8, 2, true, 9, 4), "short units");
     REQUIRE(tile_plan(CW_NN, 8, 8, 8, 0, 8, 8, true, true, 0, -1).cfg == -1 && tile_plan(CW_NN, 8, 8, 8, CW_MAX_KSTEPS + 1, 8, 8, true, true, 0, -1).cfg == -1, "bad step counts");
 }
 
