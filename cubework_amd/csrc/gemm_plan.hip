@@ -272,7 +272,7 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
     // gradient, which is NN too, while their forward is NT and is cut like any other product. Slicing gains little there
     // anyway (the outputs have tiles enough). One exception, fixed by the shape, where a row's sums are taken in another order
     // than those of a batch off the multiples of 256: whole rounds of 256 x 256 tiles start at an XCD-dependent k (memory
-    // channels, gemm_tile.h). (The 16x16x32 instruction of configuration 0 and the 32x32x16 one of the others give the same bits.)
+    // channels, gemm_wide.h). (The 16x16x32 instruction of configurations 0, 6 and 7 and the 32x32x16 one of 1 to 4 give the same bits.)
     const bool ordered = layout == CW_NN && K <= N;
     const bool rotated = ordered && M % 256 == 0 && N % 256 == 0 && K % 32 == 0 && (M / 256) * (N / 256) >= 160;
     const double bytes = 2.0 * ((double)M * K * n_steps + (double)K * N * n_steps + (double)M * N);

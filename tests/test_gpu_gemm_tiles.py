@@ -74,6 +74,27 @@ def test_forward_rows_do_not_depend_on_the_batch():
         assert torch.equal(ops.gemm_ksteps("NN", [a[:rows]], [b]), whole[:rows])
 
 
+# (K, N, rows): the planner gives 64 x 64, 128 x 128 (8 wavefronts), 192 x 128, 128 x 256 and 224 x 256 tiles to the rows of the first,
+# 64 x 128, 128 x 128 (8 wavefronts) and 128 x 256 to those of the others (tests/test_gemm_plans.py): both matrix instructions, 32x32x16
+# and 16x16x32, trips of 32 and of 64 k
+ORDERED = [(2560, 7680, (64, 300, 600, 900, 1554)), (4096, 4096, (300, 600, 1600)), (2044, 4096, (300, 600, 1600))]
+
+
+@pytest.mark.parametrize("K,N,rows", ORDERED)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_forward_rows_do_not_depend_on_the_kernel(K, N, rows, dtype):
+    """The same across every kernel that a projection's row can meet: terms of very different size, so that sums in another order or
+    through another rounding would show."""
+    from cubework_amd import ops
+
+    M = max(rows)
+    a = (randn((M, K), torch.float32, 1) * torch.exp2(randn((M, K), torch.float32, 2))).to(dtype).cuda()
+    b = randn((K, N), dtype, 3, 0.02).cuda()
+    whole = ops.gemm_ksteps("NN", [a], [b])
+    for r in rows:
+        assert torch.equal(ops.gemm_ksteps("NN", [a[:r]], [b]), whole[:r])
+
+
 def _abi_gemm(layout, A, B, bias, epilogue, scratch, addend=None):
     """cw_gemm_ksteps_ws as a C caller makes it, with `scratch` bytes of scratch."""
     import ctypes
