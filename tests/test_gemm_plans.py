@@ -51,3 +51,50 @@ def test_long_rows_in_long_blocks_leave_the_paired_kernel(plans):
 def test_short_products_of_one_round_take_64_x_128_tiles(plans, layout, M, N, K):
     """140 to 240 tiles of 64 x 128 are one round of the chip; as 64 x 64 they share its units in pairs (10 to 20 % slower)."""
     assert plans([(layout, M, N, K, 1)]) == [(3, 64, -(-M // 64) * -(-N // 128), 1, 0)]
+
+
+# What the lists of the GPU tests are there for: configuration, tile height, and w (whole tiles), s (every tile cut along k) or m (the
+# last round's cut), in NN, NT and TN. A plan that moves takes a kernel's coverage with it: find the list another shape then.
+WIDE_PLANS = {
+    "SHAPES": {(300, 50257, 40, 3): "0x160w 0x160w 0x160w", (4100, 4090, 328, 1): "1x128w 0x256m 0x256m", (300, 32768, 1016, 1): "0x160w 0x160w 0x160w",
+               (376, 32760, 1000, 1): "0x192w 0x192w 0x192w", (1552, 7672, 1352, 1): "0x224w 0x224w 0x224w",
+               (8184, 2040, 328, 3): "0x256w 0x256w 1x128w", (8184, 6136, 520, 1): "0x256w 0x256w 0x256w",
+               (7000, 4600, 1000, 1): "0x256w 0x256w 0x256w", (1024, 25003, 768, 1): "0x256w 0x256w 0x256w", (8192, 2048, 512, 2): "0x256w 0x256w 0x256w"},
+    "PAIRED": {(4100, 2047, 4104, 2): "5x128m 5x128m 5x128m", (2040, 2040, 8200, 1): "5x128w 5x128w 5x128w",
+               (4001, 1000, 1032, 3): "5x128w 5x128w 5x128w", (2040, 2040, 1416, 1): "2x128w 5x128w 2x128w",
+               (4001, 1000, 4200, 1): "5x128w 5x128w 5x128w", (2040, 2047, 4200, 1): "5x128w 5x128w 5x128w",
+               (1016, 768, 5000, 1): "5x128s 5x128s 4x64w", (300, 2048, 8192, 1): "5x128s 5x128s 5x128s", (4096, 1024, 4096, 1): "5x128w 5x128w 5x128w"},
+    "NARROW": {(300, 16384, 40, 5): "6x160w 6x160w 1x128w", (4100, 2047, 1000, 3): "6x192w 6x192m 5x128m", (496, 2560, 520, 5): "3x64w 7x128s 3x64w",
+               (300, 16376, 2056, 1): "6x160w 6x160w 0x160s", (1554, 2559, 1000, 3): "6x192w 6x192w 3x64w",
+               (496, 8184, 2056, 1): "7x128w 5x128w 5x128w", (300, 4090, 12296, 1): "6x160s 6x160s 0x160s", (1554, 2560, 2560, 1): "6x192w 6x192w 3x64w"},
+    "RAGGED_K": {(300, 50257, 37, 3): "0x160w 0x160w", (300, 16384, 37, 5): "6x160w 6x160w", (8184, 2040, 331, 3): "0x256w 0x256w",
+                 (7000, 4600, 961, 1): "0x256w 0x256w", (1023, 768, 12565, 1): "5x128s 5x128s", (4001, 1000, 1039, 3): "5x128w 5x128w",
+                 (4001, 1000, 4162, 1): "5x128w 5x128w", (300, 16376, 2059, 1): "6x160w 6x160w", (300, 4090, 12302, 1): "6x160s 6x160s",
+                 (1554, 2560, 2556, 1): "6x192w 6x192w", (300, 32768, 1021, 1): "0x160w 0x160w", (4096, 1024, 12565, 1): "0x256s 0x256s",
+                 (4096, 1024, 10235, 1): "5x128w 5x128w"},
+}
+
+
+def _code(plan):
+    cfg, rows, full, _, rest = plan
+    return "%dx%d%s" % (cfg, rows, "w" if rest == 0 else "s" if full == 0 else "m")
+
+
+@pytest.mark.parametrize("name", sorted(WIDE_PLANS))
+def test_the_gpu_tests_reach_the_kernels_they_name(plans, name):
+    from tests import test_gpu_gemm_wide as gpu
+
+    shapes = getattr(gpu, name)
+    assert sorted(WIDE_PLANS[name]) == sorted(shapes)
+    for shape in shapes:
+        want = WIDE_PLANS[name][shape].split()
+        assert [_code(p) for p in plans([(lay, *shape) for lay in ("NN", "NT", "TN")[:len(want)]])] == want, shape
+
+
+def test_the_gpu_tests_reach_the_kernels_they_compare(plans):
+    from tests import test_gpu_gemm_tiles as tiles
+    from tests import test_gpu_gemm_wide as wide
+
+    assert [_code(p) for p in plans([("NT", *s) for s in wide.NARROW_NT])] == ["7x128w", "7x128m"]
+    ordered = [[_code(p) for p in plans([("NN", m, N, K, 1) for m in rows])] for K, N, rows in tiles.ORDERED]
+    assert ordered == [["4x64w", "7x128w", "6x160w", "1x128w", "0x224w"], ["3x64w", "7x128w", "1x128w"], ["3x64w", "7x128w", "1x128w"]]

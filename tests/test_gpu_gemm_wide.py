@@ -1,6 +1,8 @@
 """GPU parity of the block GEMM's kernels of 8 wavefronts (256-column tiles, 128 x 128 tiles with two groups of wavefronts
-along k, 128-column tiles of up to 192 rows: configurations 0 and 5 to 7 of the planner) against float64 where they can go wrong: every tile height, edges of M and N, steps whose K ends inside a stage, the shortest reductions it takes, seams of steps
-and of tiles, sliced tiles, unaligned output rows, every operand of the epilogue."""
+along k, 128-column tiles of up to 192 rows: configurations 0 and 5 to 7 of the planner) against float64 where they can go wrong:
+every tile height, edges of M and N, steps whose K ends inside a stage, units of no more stages than the kernel takes, seams of steps
+and of tiles, sliced tiles, unaligned output rows, every operand of the epilogue. Which configuration the planner gives a shape in
+which orientation is held by tests/test_gemm_plans.py."""
 import pytest
 import torch
 
@@ -8,26 +10,41 @@ from tests.util import assert_parity, randn
 
 pytestmark = pytest.mark.gpu
 
-# (M, N, K, steps), which the planner gives to this kernel: heights 160, 192, 224 and 256 with ragged edges, K of a part of a stage
-# behind whole ones, three steps (rotated starts in NT), three tiles a block, a last row and column of tiles with few elements, an
-# odd last column
-SHAPES = [(300, 32768, 1016, 1), (376, 32760, 1000, 1), (1552, 7672, 1352, 1), (8184, 2040, 328, 3), (8184, 6136, 520, 1),
+# (M, N, K, steps), which the planner gives to 256-column tiles in NN and NT and, mostly, in TN: heights 160, 192, 224 and 256 with
+# ragged edges, K of a part of a stage behind whole ones, three steps (rotated starts in NT), three tiles a block, a last row and column
+# of tiles with few elements, an odd last column; three stages to a tile, each of them a part of one (as short as the kernel
+# takes: every stage is the last of its step, every third of its tile); slices of three stages (NT and TN)
+SHAPES = [(300, 50257, 40, 3), (4100, 4090, 328, 1), (300, 32768, 1016, 1), (376, 32760, 1000, 1), (1552, 7672, 1352, 1), (8184, 2040, 328, 3), (8184, 6136, 520, 1),
           (7000, 4600, 1000, 1), (1024, 25003, 768, 1), (8192, 2048, 512, 2)]
 
-# shapes that the planner gives to 128 x 128 tiles: ragged last tiles of either direction, K that ends in the first and in the
-# second half of a stage, several steps, the shortest reduction it takes (in NT), an odd last column, every tile cut along k
-PAIRED = [(2040, 2040, 8200, 1), (4001, 1000, 1032, 3), (2040, 2040, 1416, 1), (4001, 1000, 4200, 1), (2040, 2047, 4200, 1),
+# shapes that the planner gives to 128 x 128 tiles of two groups, in one orientation at least: ragged last tiles of either direction, K
+# that ends in the first and in the second half of a stage, several steps, a short reduction, an odd last column, every tile cut along k,
+# the last round's
+PAIRED = [(4100, 2047, 4104, 2), (2040, 2040, 8200, 1), (4001, 1000, 1032, 3), (2040, 2040, 1416, 1), (4001, 1000, 4200, 1), (2040, 2047, 4200, 1),
           (1016, 768, 5000, 1), (300, 2048, 8192, 1), (4096, 1024, 4096, 1)]
 
 
-# shapes that the planner gives to 128 columns by 128, 160 or 192 rows in NN or NT: the same edges, and slices of the fewest rows
-NARROW = [(300, 16376, 2056, 1), (1554, 2559, 1000, 3), (496, 8184, 2056, 1), (300, 4090, 12296, 1), (1554, 2560, 2560, 1)]
+# shapes that the planner gives to 128 columns by 128, 160 or 192 rows in NN or NT (TN has none): the same edges, slices of the fewest
+# rows, five partial stages to a tile (as short as they take), every tile and the last round's cut along k
+NARROW = [(300, 16384, 40, 5), (4100, 2047, 1000, 3), (496, 2560, 520, 5), (300, 16376, 2056, 1), (1554, 2559, 1000, 3), (496, 8184, 2056, 1), (300, 4090, 12296, 1), (1554, 2560, 2560, 1)]
+NARROW_NT = [(620, 6000, 4104, 3), (384, 12500, 4104, 3)]
 
 
 @pytest.mark.parametrize("shape", SHAPES + PAIRED + NARROW, ids=str)
 @pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_tiles_of_256_columns(layout, shape, dtype):
+    _check(layout, shape, dtype)
+
+
+# 128 x 128 tiles of one group with k-contiguous B, whole and in a sliced last round: long reductions over several steps alone
+@pytest.mark.parametrize("shape", NARROW_NT, ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tiles_of_one_group_in_nt(shape, dtype):
+    _check("NT", shape, dtype)
+
+
+def _check(layout, shape, dtype):
     from cubework_amd import ops
 
     M, N, K, steps = shape
@@ -70,7 +87,7 @@ def test_sliced_tiles(layout, M, N, K):
 
 # K of every remainder by 8: the piece of 16 bytes in which a row ends, whole K inside a stage, steps and slices that end there; both
 # sides of the planner's rule for long rows that are not whole lines
-RAGGED_K = [(8184, 2040, 331, 3), (7000, 4600, 961, 1), (1023, 768, 12565, 1), (4001, 1000, 1039, 3), (4001, 1000, 4162, 1),
+RAGGED_K = [(300, 50257, 37, 3), (300, 16384, 37, 5), (8184, 2040, 331, 3), (7000, 4600, 961, 1), (1023, 768, 12565, 1), (4001, 1000, 1039, 3), (4001, 1000, 4162, 1),
             (300, 16376, 2059, 1), (300, 4090, 12302, 1), (1554, 2560, 2556, 1), (300, 32768, 1021, 1),
             (4096, 1024, 12565, 1), (4096, 1024, 10235, 1)]
 
