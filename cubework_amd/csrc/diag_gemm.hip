@@ -1,7 +1,7 @@
 // Measurement aid (libcubework_diag.so, loaded by bench.py only): the block GEMM's launch for the headline shape, and a
 // 256 x 256 tile kernel with one part taken out, so that the part's share of a launch - in time and, through the socket's
 // energy counter, in joules - can be read as a difference against the same kernel whole:
-//   part 0  the library's launch for this shape (gemm_wide.h)
+//   part 0  the library's launch for this shape (gemm_wide.h; part 4 for K = 128 in one step, which that kernel does not take)
 //   part 4  the kernel of 4 wavefronts and 32x32x16 matrix instructions (gemm_tile.h's template on 4 x 4 tiles), whole; of it
 //   part 1  the k loop issues no operand loads: the four LDS stages are filled once and re-used
 //   part 2  no epilogue: no bias / activation arithmetic, nothing stored
@@ -36,7 +36,7 @@ extern "C" int cw_diag_gemm_part(int part, int64_t M, int64_t N, int64_t K, int 
     if (part < 0 || part > 4) return fail(CW_ERR_INVALID, "cw_diag_gemm_part: part %d outside [0, 4]", part);
     if (n_steps < 1 || n_steps > kMaxSteps || A_steps == nullptr || B_steps == nullptr || bias == nullptr || C == nullptr)
         return fail(CW_ERR_INVALID, "cw_diag_gemm_part: 1 to %d k-steps, operands, bias and C are needed", kMaxSteps);
-    if (M < 256 || N < 256 || K < 192 || (M % 256) != 0 || (N % 256) != 0 || (K % 64) != 0 || (M / 256) * (N / 256) < 128 ||
+    if (M < 256 || N < 256 || K < 128 || (M % 256) != 0 || (N % 256) != 0 || (K % 64) != 0 || (M / 256) * (N / 256) < 128 ||
         M > (1 << 24) || N > (1 << 24) || K > (1 << 24))
         return fail(CW_ERR_UNSUPPORTED, "cw_diag_gemm_part: tile-aligned shapes with at least 128 tiles of 256 x 256 only");
     if (lda < K || ldb < N || ldc < N || (lda % 8) != 0 || (ldb % 8) != 0 || (ldc % 8) != 0)
@@ -65,6 +65,7 @@ extern "C" int cw_diag_gemm_part(int part, int64_t M, int64_t N, int64_t K, int 
     args.slices = 1;
     args.rotate = 1;
     hipStream_t s = (hipStream_t)stream;
+    if (part == 0 && !wide_takes(K, n_steps)) part = 4;
     switch (part) {
         case 0: return gemm_wide::launch_rows<false, true, 8, 4, 1, CW_EPI_BIAS_GELU_TANH, bf16_t>(args, s);
         case 1: return launch_part<1>(args, s);

@@ -85,7 +85,7 @@ struct TilePlan {
     int64_t scratch() const { return pack_a_bytes + pack_b_bytes + pack_add_bytes + partial_bytes; }
 };
 // Whether a kernel of gemm_wide.h takes such a product: at least `stages` stages of `stage` k (the loads run ahead by one less).
-bool wide_takes(int64_t K, int n_steps, int stage = 64, int stages = 3);
+inline bool wide_takes(int64_t K, int n_steps, int stage = 64, int stages = 3) { return (K + stage - 1) / stage * n_steps >= stages; }
 // What a launch of such a kernel rests on: `tiles` tiles of which `full` are whole, the others in slices through partial sums, and every
 // unit longer than the `ahead` stages that the loads run ahead (of a shorter one the loads behind its last stage are given up, the next
 // unit's with them: wrong sums).

@@ -226,8 +226,6 @@ constexpr int64_t kTileLaunchMax = ((int64_t)1 << 24) - 8;
 
 }  // namespace
 
-bool wide_takes(int64_t K, int n_steps, int stage, int stages) { return (K + stage - 1) / stage * n_steps >= stages; }
-
 int wide_rows(int64_t M) {
     for (int rows : {160, 192, 224})
         if ((M + rows - 1) / rows == (M + 255) / 256) return rows;

@@ -102,3 +102,27 @@ def test_gemm_part_diagnostic_whole_kernel_matches_the_library():
     for part in (1, 2, 3):
         assert lib.cw_diag_gemm_part(part, M, N, K, 2, ta, K, tb, N, bias.data_ptr(), out.data_ptr(), N, stream) == 0
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("steps", [1, 2])
+def test_gemm_part_diagnostic_takes_k_of_128(steps):
+    """cw_diag_gemm_part's shortest K: two stages of 64 k (one step), fewer than the library's 256 x 256 kernel takes, and four."""
+    import ctypes
+    from cubework_amd import _diag
+
+    lib = _diag.load()
+    M, N, K = 4096, 2048, 128
+    A = [randn((M, K), torch.bfloat16, 40 + i).to(DEV) for i in range(steps)]
+    B = [randn((K, N), torch.bfloat16, 50 + i, 0.05).to(DEV) for i in range(steps)]
+    bias = randn((N,), torch.bfloat16, 60, 0.1).to(DEV)
+    ta = (ctypes.c_void_p * steps)(*[t.data_ptr() for t in A])
+    tb = (ctypes.c_void_p * steps)(*[t.data_ptr() for t in B])
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    want = torch.nn.functional.gelu(sum(a.double() @ b.double() for a, b in zip(A, B)) + bias.double(), approximate="tanh")
+    for part in (0, 4):
+        out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert lib.cw_diag_gemm_part(part, M, N, K, steps, ta, K, tb, N, bias.data_ptr(), out.data_ptr(), N, stream) == 0
+        assert_parity(out, want, torch.bfloat16, "part %d, %d steps of 128" % (part, steps))
+    for part in (1, 2, 3):
+        assert lib.cw_diag_gemm_part(part, M, N, K, steps, ta, K, tb, N, bias.data_ptr(), out.data_ptr(), N, stream) == 0
+    torch.cuda.synchronize()
