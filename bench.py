@@ -987,9 +987,9 @@ def gemm_k_sweep(device):
 
 
 def energy_table(device, sets, bias, outs, seconds):
-    """Where a launch of the headline GEMM spends its energy: the ring kernel whole and with one part taken out
-    (cw_diag_gemm_part of the measurement library: the same kernel source, parts 1-3 not computing anything
-    meaningful), each run back to back for `seconds`, priced by the socket's energy counter (average power over
+    """Where a launch of the headline product on 4 wavefronts spends its energy: that kernel (cw_diag_gemm_part of the
+    measurement library, part 4; the library launches the one of 8 wavefronts) whole and with one part taken out (parts
+    1-3, which compute nothing meaningful), each run back to back for `seconds`, priced by the socket's energy counter (average power over
     whole refresh periods of the firmware's table inside the run x the event-timed launch duration). At the power
     cap time = energy / power, so the joules are what the microseconds are made of."""
     import ctypes
@@ -1054,7 +1054,7 @@ def energy_table(device, sets, bias, outs, seconds):
         if pj["random_operands_read_from_lds"]:
             out["energy_mJ_per_launch"]["cross_check_lds_reads_from_the_matrix_loops"] = round(
                 (pj["random_operands_read_from_lds"] - pj["random_operands"]) * GEMM_FLOP * 1e-9, 2)
-        out["note"] = ("each part = whole kernel minus the kernel without that part (cache-resident operands), the matrix "
+        out["note"] = ("the kernel of 4 wavefronts, not the library's of 8; each part = whole kernel minus the kernel without that part (cache-resident operands), the matrix "
                        "instructions priced by the register-only loop on random operands; the parts overlap in time, so "
                        "the differences are attributions, and the rest is what no ablation removes")
     return out
@@ -1125,7 +1125,7 @@ def main():
                          "LayerNorm / cross-entropy sizes reach on this GPU")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline")
     ap.add_argument("--energy-table", type=float, default=0.0, metavar="SECONDS",
-                    help="instead of the benchmark: run the headline GEMM kernel whole and with one part taken out "
+                    help="instead of the benchmark: run the headline GEMM on 4 wavefronts whole and with one part taken out "
                          "(operand loads, LDS fragment reads, epilogue), and the register-only matrix instruction "
                          "loops, each for SECONDS (4 or more, for the firmware's energy counter), and print where a "
                          "launch's energy goes")

@@ -12,9 +12,9 @@ it, the operators never call it, and libcubework_hip.so exports none of its symb
   cw_diag_lds_rate(iters, transposing, sink, stream), cw_diag_lds_rate_bytes(iters)
                                                  LDS read rate of a compute unit: ds_read_b128 / ds_read_b64_tr_b16
   cw_diag_gemm_part(part, M, N, K, n_steps, A_steps, lda, B_steps, ldb, bias, C, ldc, stream)
-                                                 the ring kernel of the block GEMM (NN, bf16, bias + GeLU-tanh) whole
-                                                 (part 0) or without its operand loads (1), its epilogue (2), its LDS
-                                                 fragment reads (3)
+                                                 the block GEMM (NN, bf16, bias + GeLU-tanh): the library's launch
+                                                 (part 0), or a kernel of 4 wavefronts whole (4), without its operand
+                                                 loads (1), its epilogue (2), its LDS fragment reads (3)
 """
 import ctypes
 import os

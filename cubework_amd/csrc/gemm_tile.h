@@ -1,8 +1,9 @@
 // 16-bit block GEMM for any shape (gfx950): ragged M, N and K, outputs with few tiles, partial last rounds.
 //
 //   - BM x BN tile of C per 256-thread block (4 wavefronts, 2x2; a wavefront owns TM x TN MFMA tiles of 32x32, BM = 64 TM,
-//     BN = 64 TN); k tiles of 32 in a ring of NS LDS stages filled by the load unit, one barrier per k tile in the
-//     middle of its MFMAs, fragments read one k step ahead: a wavefront arrives at the barrier with the next products' operands in registers.
+//     BN = 64 TN); trips of KB k tiles of 32 in a ring of NS LDS stages filled by the load unit, one barrier per trip, fragments read a
+//     whole trip ahead: a wavefront arrives at the barrier with the next products' operands in registers, and neither the barrier
+//     nor the LDS latency is exposed.
 //   - Operands are fetched with buffer_load_dwordx4 ... lds. The lane's byte offset goes through the buffer's range
 //     check, and a lane whose 16-byte chunk lies outside the operand (row >= M or N, k >= K) is handed an offset
 //     beyond the range: the load unit writes zeros for it. So edges cost no branch, no second kernel and no memory
@@ -35,7 +36,7 @@ struct TileArgs {
     int vec_out;    // C and preact allow 16-byte accesses at every tile column
     int full;       // tiles computed whole
     int slices;     // k slices of each of the other tiles
-    int rotate;     // the XCDs start a whole tile's reduction at different k
+    int rotate;     // the XCDs start a whole tile's reduction at different k (gemm_wide.h)
     float* partial; // slices x (tiles - full) tiles of BM x BN fp32 partial sums
 };
 
@@ -217,60 +218,50 @@ struct Epilogue {
         uint16_t* dst = buf + (wm * 32 + (lane & 31)) * CP + col_l;
         const int64_t add_row = (int64_t)(mrow < a.M ? mrow : a.M - 1) * a.ldadd;
         const int last_col = (a.N - 1) & ~3;
-        // An addend's pieces of JC column blocks are requested together, ahead of the arithmetic. Addend rows are 16-byte
+        // An addend's pieces of a column block are requested together, ahead of the arithmetic. Addend rows are 16-byte
         // aligned (the host copies others), so the last group of four is whole memory.
-        constexpr int JC = TM * TN == 16 ? TN : 1;
 #pragma unroll
-        for (int j0 = 0; j0 < TN; j0 += JC) {
-            float add[JC][4][4];
+        for (int j = 0; j < TN; ++j) {
+            float add[4][4];
 #pragma unroll
-            for (int j = 0; j < JC; ++j)
+            for (int g = 0; g < 4; ++g)
 #pragma unroll
-                for (int g = 0; g < 4; ++g)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) add[j][g][e] = 0.0f;
+                for (int e = 0; e < 4; ++e) add[g][e] = 0.0f;
 #pragma unroll 1
             for (int k = 0; k < a.n_addends; ++k) {
                 const uint16_t* ap = reinterpret_cast<const uint16_t*>(step_ptr(kTabAddend, k)) + add_row;
-                u32x2_t raw[JC][4];
-#pragma unroll
-                for (int j = 0; j < JC; ++j)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const int col = n0 + col_l + (j0 + j) * 32 + 8 * g;
-                        raw[j][g] = *reinterpret_cast<const u32x2_t*>(ap + (col < last_col ? col : last_col));
-                    }
-#pragma unroll
-                for (int j = 0; j < JC; ++j)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        add[j][g][0] += half_conv<E>::lo(raw[j][g].x);
-                        add[j][g][1] += half_conv<E>::hi(raw[j][g].x);
-                        add[j][g][2] += half_conv<E>::lo(raw[j][g].y);
-                        add[j][g][3] += half_conv<E>::hi(raw[j][g].y);
-                    }
-            }
-#pragma unroll
-            for (int j = 0; j < JC; ++j) {
+                u32x2_t raw[4];
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    // opaque: the sums are formed here and not, once for both stagings, in front of them, where all would be live at once
-                    u32x2_t b = bias[j0 + j][g];
-                    asm volatile("" : "+v"(b));
-                    float v[4];
-                    v[0] = acc[j0 + j][4 * g] + half_conv<E>::lo(b.x) + add[j][g][0];
-                    v[1] = acc[j0 + j][4 * g + 1] + half_conv<E>::hi(b.x) + add[j][g][1];
-                    v[2] = acc[j0 + j][4 * g + 2] + half_conv<E>::lo(b.y) + add[j][g][2];
-                    v[3] = acc[j0 + j][4 * g + 3] + half_conv<E>::hi(b.y) + add[j][g][3];
-                    if constexpr (ACT) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = tile_act<EPI>(v[e]);
-                    }
-                    u32x2_t p;
-                    p.x = half_conv<E>::pack2(v[0], v[1]);
-                    p.y = half_conv<E>::pack2(v[2], v[3]);
-                    *reinterpret_cast<u32x2_t*>(dst + (j0 + j) * 32 + 8 * g) = p;
+                    const int col = n0 + col_l + j * 32 + 8 * g;
+                    raw[g] = *reinterpret_cast<const u32x2_t*>(ap + (col < last_col ? col : last_col));
                 }
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    add[g][0] += half_conv<E>::lo(raw[g].x);
+                    add[g][1] += half_conv<E>::hi(raw[g].x);
+                    add[g][2] += half_conv<E>::lo(raw[g].y);
+                    add[g][3] += half_conv<E>::hi(raw[g].y);
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                // opaque: the sums are formed here and not, once for both stagings, in front of them, where all would be live at once
+                u32x2_t b = bias[j][g];
+                asm volatile("" : "+v"(b));
+                float v[4];
+                v[0] = acc[j][4 * g] + half_conv<E>::lo(b.x) + add[g][0];
+                v[1] = acc[j][4 * g + 1] + half_conv<E>::hi(b.x) + add[g][1];
+                v[2] = acc[j][4 * g + 2] + half_conv<E>::lo(b.y) + add[g][2];
+                v[3] = acc[j][4 * g + 3] + half_conv<E>::hi(b.y) + add[g][3];
+                if constexpr (ACT) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = tile_act<EPI>(v[e]);
+                }
+                u32x2_t p;
+                p.x = half_conv<E>::pack2(v[0], v[1]);
+                p.y = half_conv<E>::pack2(v[2], v[3]);
+                *reinterpret_cast<u32x2_t*>(dst + j * 32 + 8 * g) = p;
             }
         }
     }
@@ -326,12 +317,8 @@ constexpr size_t kLdsBytes = (size_t)NS * KB * 64 * (TM + TN) * kBK * 2 > kEpilo
 template <int TM, int TN, int KB, int NS>
 constexpr int kBlocksPerCU = kLdsBytes<TM, TN, KB, NS> <= 80 * 1024 ? 2 : 1;
 
-// ABL: 0 in every instantiation of the library. The measurement library instantiates the one-step-ahead loop with one
-// part taken out, to price that part (time and energy per launch against the whole kernel; such a launch's results are
-// meaningless): 1 = the k loop issues no operand loads (the stages are filled once and re-used), 2 = no epilogue
-// (nothing is stored), 3 = the k loop reads no fragments from LDS (the first trip's stay in the registers).
 // KB: k extent of a trip in units of 32 (one barrier per trip); NS: ring stages of KB k blocks.
-template <bool TRANS_A, bool TRANS_B, int TM, int TN, int KB, int NS, int EPI, typename E, int ABL = 0>
+template <bool TRANS_A, bool TRANS_B, int TM, int TN, int KB, int NS, int EPI, typename E>
 __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm_tile_kernel(const TileArgs args) {
     constexpr int BM = 64 * TM, BN = 64 * TN, BK = KB * kBK;
     using LA = Loader<TRANS_A, TM>;
@@ -339,10 +326,6 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
     constexpr int kBlock = LA::kBytes + LB::kBytes;  // one k block: A image, B image
     constexpr int kStage = KB * kBlock;
     constexpr int kPer = KB * (TM + TN);             // load instructions per wavefront and trip
-    // 4 x 4 MFMA tiles leave registers for the fragments of one k step ahead (and it needs no more: each k step is 16
-    // MFMAs); the smaller tiles read a whole trip ahead, so that neither the barrier nor the LDS latency is exposed
-    constexpr bool kWholeTrip = TM * TN < 16;
-    static_assert(kWholeTrip || (KB == 1 && TM == 4 && TN == 4), "the one-step-ahead loop is laid out for 4 x 4 MFMA tiles and one k block");
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     lds_char* lds_base = (lds_char*)lds;
     const uint32_t lds_addr0 = (uint32_t)(uintptr_t)lds_base;
@@ -363,10 +346,6 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
         if (pid < full_grid) {
             tile = (pid & 7) * (full_grid >> 3) + (pid >> 3);
             if (tile >= args.full) return;
-            // The XCDs walk the flattened (step, k) range cyclically from starting points an eighth of it apart: walking
-            // in step, all workgroups would ask memory for the same k slice at the same moment, and where it comes from
-            // HBM that concentrates the traffic on a few channels (8192 x 2048 x 2 x 2048 from memory: k loop 95 -> 78 us).
-            if (args.rotate) kt_beg = (int)(((int64_t)KT * (pid & 7)) >> 3);
         } else {
             const int rest = tiles_m * tiles_n - args.full, units = rest * args.slices;
             const int p = pid - full_grid;
@@ -450,7 +429,7 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
         if (pub_rem <= 0) pub_rem = K;
         pub_stage = (pub_stage + 1 == NS) ? 0 : pub_stage + 1;
         // this wavefront's fragment reads (of a stage that is about to be refilled) and tail writes are done
-        if (kWholeTrip || odd_tail) asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
@@ -461,109 +440,49 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
         rd_stage = (rd_stage + 1 == NS) ? 0 : rd_stage + 1;
         rd = lds_base + rd_stage * kStage;
     };
-    if constexpr (kWholeTrip) {
-        bf16x8_t af[2][2 * KB][TM], bfr[2][2 * KB][TN];
-        auto read_one = [&](auto set, auto op) {  // fragment `op` of a trip: [k step][A fragments, B fragments]
-            constexpr int KS = op.value / (TM + TN), O = op.value % (TM + TN);
-            lds_char* blk = rd + (KS / 2) * kBlock;
-            if constexpr (O < TM) af[set.value][KS][O] = fa.template read<O, KS % 2>(blk);
-            else bfr[set.value][KS][O - TM] = fb.template read<O - TM, KS % 2>(blk + LA::kBytes);
-        };
-        // prologue: trips 0 .. NS-1 requested, trip 0 published and its fragments on the way
-        for (int p = 0; p < NS; ++p) {
-            static_for<kPer>([&](auto o) { issue_one(o); });
-            issue_advance();
-        }
-        dma_wait<kPer*(NS - 1)>();
+    bf16x8_t af[2][2 * KB][TM], bfr[2][2 * KB][TN];
+    auto read_one = [&](auto set, auto op) {  // fragment `op` of a trip: [k step][A fragments, B fragments]
+        constexpr int KS = op.value / (TM + TN), O = op.value % (TM + TN);
+        lds_char* blk = rd + (KS / 2) * kBlock;
+        if constexpr (O < TM) af[set.value][KS][O] = fa.template read<O, KS % 2>(blk);
+        else bfr[set.value][KS][O - TM] = fb.template read<O - TM, KS % 2>(blk + LA::kBytes);
+    };
+    // prologue: trips 0 .. NS-1 requested, trip 0 published and its fragments on the way
+    for (int p = 0; p < NS; ++p) {
+        static_for<kPer>([&](auto o) { issue_one(o); });
+        issue_advance();
+    }
+    dma_wait<kPer*(NS - 1)>();
+    publish();
+    static_for<2 * KB * (TM + TN)>([&](auto o) { read_one(std::integral_constant<int, 0>{}, o); });
+    read_advance();
+    // Trip kt: barrier (trip kt+1 complete in LDS for everybody, the stage of trip kt free: its fragments are in
+    // registers); then the MFMAs of kt with the fragment reads of kt+1 and the loads of kt+NS placed between them.
+    constexpr int kMfma = 2 * KB * TM * TN, kReads = 2 * KB * (TM + TN), kOps = kReads + kPer;
+    auto trip = [&](auto set) {
+        constexpr int S = set.value;
+        dma_wait<kPer*(NS - 2)>();
         publish();
-        static_for<2 * KB * (TM + TN)>([&](auto o) { read_one(std::integral_constant<int, 0>{}, o); });
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<kMfma>([&](auto q) {
+            constexpr int KS = q.value / (TM * TN), R = q.value % (TM * TN), I = R / TN, J = R % TN, JS = (I & 1) ? TN - 1 - J : J;
+            acc[I][JS] = gemm_bf16::mfma_32x32x16<E>(bfr[S][KS][JS], af[S][KS][I], acc[I][JS]);
+            constexpr int O0 = q.value * kOps / kMfma, O1 = (q.value + 1) * kOps / kMfma;
+            static_for<O1 - O0>([&](auto o) {
+                constexpr int OP = O0 + o.value;
+                if constexpr (OP < kReads) read_one(std::integral_constant<int, 1 - S>{}, std::integral_constant<int, OP>{});
+                else issue_one(std::integral_constant<int, OP - kReads>{});
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
         read_advance();
-        // Trip kt: barrier (trip kt+1 complete in LDS for everybody, the stage of trip kt free: its fragments are in
-        // registers); then the MFMAs of kt with the fragment reads of kt+1 and the loads of kt+NS placed between them.
-        constexpr int kMfma = 2 * KB * TM * TN, kReads = 2 * KB * (TM + TN), kOps = kReads + kPer;
-        auto trip = [&](auto set) {
-            constexpr int S = set.value;
-            dma_wait<kPer*(NS - 2)>();
-            publish();
-            __builtin_amdgcn_sched_barrier(0);
-            static_for<kMfma>([&](auto q) {
-                constexpr int KS = q.value / (TM * TN), R = q.value % (TM * TN), I = R / TN, J = R % TN, JS = (I & 1) ? TN - 1 - J : J;
-                acc[I][JS] = gemm_bf16::mfma_32x32x16<E>(bfr[S][KS][JS], af[S][KS][I], acc[I][JS]);
-                constexpr int O0 = q.value * kOps / kMfma, O1 = (q.value + 1) * kOps / kMfma;
-                static_for<O1 - O0>([&](auto o) {
-                    constexpr int OP = O0 + o.value;
-                    if constexpr (OP < kReads) read_one(std::integral_constant<int, 1 - S>{}, std::integral_constant<int, OP>{});
-                    else issue_one(std::integral_constant<int, OP - kReads>{});
-                });
-                __builtin_amdgcn_sched_barrier(0);
-            });
-            read_advance();
-            issue_advance();
-        };
-        for (int kt = 0;;) {
-            trip(std::integral_constant<int, 0>{});
-            if (++kt >= KT) break;
-            trip(std::integral_constant<int, 1>{});
-            if (++kt >= KT) break;
-        }
-    } else {
-        // prologue: trips 0 .. NS-3 requested and the A part of trip NS-2
-        for (int p = 0; p < (ABL == 1 ? NS : NS - 2); ++p) {
-            static_for<kPer>([&](auto o) { issue_one(o); });
-            issue_advance();
-        }
-        if constexpr (ABL == 1) {
-            dma_wait<0>();
-        } else {
-            static_for<TM>([&](auto o) { issue_one(o); });
-            dma_wait<kPer*(NS - 3) + TM>();
-        }
-        publish();
-        bf16x8_t af[2][TM], bfr[2][TN];
-        static_for<TM>([&](auto t) { af[0][t.value] = fa.template read<t.value, 0>(rd); });
-        static_for<TN>([&](auto t) { bfr[0][t.value] = fb.template read<t.value, 0>(rd + LA::kBytes); });
-        if constexpr (ABL == 3) {
-            static_for<TM>([&](auto t) { af[1][t.value] = fa.template read<t.value, 1>(rd); });
-            static_for<TN>([&](auto t) { bfr[1][t.value] = fb.template read<t.value, 1>(rd + LA::kBytes); });
-        }
-        constexpr int kMfma = TM * TN;
-        for (int kt = 0; kt < KT; ++kt) {
-            __builtin_amdgcn_sched_barrier(0);
-            // k step 0; reads of k step 1; the B part of the trip whose A part went out in the previous one
-            static_for<kMfma>([&](auto q) {
-                constexpr int I = q.value / TN, J = q.value % TN, JS = (I & 1) ? TN - 1 - J : J;
-                acc[I][JS] = gemm_bf16::mfma_32x32x16<E>(bfr[0][JS], af[0][I], acc[I][JS]);
-                // fragment reads behind the first half of the MFMAs (their latency passes under the second), loads behind it
-                if constexpr (q.value < TM + TN) {
-                    if constexpr (ABL != 3) {
-                        if constexpr (q.value < TM) af[1][q.value] = fa.template read<q.value, 1>(rd);
-                        else bfr[1][q.value - TM] = fb.template read<q.value - TM, 1>(rd + LA::kBytes);
-                    }
-                } else if constexpr ((q.value - TM) % 2 == 0 && ABL != 1) {
-                    issue_one(std::integral_constant<int, TM + (q.value - TM - TN) / 2>{});
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            });
-            issue_advance();
-            read_advance();
-            // trip kt+1 complete for everybody, the stage of trip kt-1 free
-            dma_wait<kPer*(NS - 3)>();
-            publish();
-            __builtin_amdgcn_sched_barrier(0);
-            static_for<kMfma>([&](auto q) {
-                constexpr int I = q.value / TN, J = q.value % TN, JS = (I & 1) ? TN - 1 - J : J;
-                acc[I][JS] = gemm_bf16::mfma_32x32x16<E>(bfr[1][JS], af[1][I], acc[I][JS]);
-                if constexpr (q.value < TM + TN) {
-                    if constexpr (ABL != 3) {
-                        if constexpr (q.value < TM) af[0][q.value] = fa.template read<q.value, 0>(rd);
-                        else bfr[0][q.value - TM] = fb.template read<q.value - TM, 0>(rd + LA::kBytes);
-                    }
-                } else if constexpr ((q.value - TM) % 2 == 0 && ABL != 1) {
-                    issue_one(std::integral_constant<int, (q.value - TM - TN) / 2>{});
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            });
-        }
+        issue_advance();
+    };
+    for (int kt = 0;;) {
+        trip(std::integral_constant<int, 0>{});
+        if (++kt >= KT) break;
+        trip(std::integral_constant<int, 1>{});
+        if (++kt >= KT) break;
     }
     dma_wait<0>();
     __syncthreads();
@@ -583,8 +502,6 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
                 }
         return;
     }
-    // measurement build without an epilogue: never true, and keeps the products alive
-    if (ABL == 2 && args.n_steps >= 0) return;
     using Epi = Epilogue<TM, TN, EPI, E>;
     lds[2 * Epi::BUF + tid] = (uint16_t)bias_bits;
     __syncthreads();

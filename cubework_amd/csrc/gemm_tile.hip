@@ -1,6 +1,6 @@
-// 16-bit block GEMM, tile kernels (gemm_tile.h): one object per element type, orientation and configuration of
+// 16-bit block GEMM, tile kernels (gemm_tile.h): one object per element type, orientation and configuration 1 to 4 of
 // kTileConfigs (gemm_plan.h), compiled from this file with CW_TILE_E (bf16_t, f16_t), CW_TILE_LAYOUT (NN, NT, TN) and
-// CW_TILE_CFG (1 .. kTileConfigCount-1).
+// CW_TILE_CFG (1 .. 4).
 #include "gemm_plan.h"
 #include "gemm_tile.h"
 

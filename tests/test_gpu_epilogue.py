@@ -81,8 +81,8 @@ def test_mfma_rate_diagnostic_runs_in_every_mode():
 
 
 def test_gemm_part_diagnostic_whole_kernel_matches_the_library():
-    """cw_diag_gemm_part with part 0 is the library's ring kernel for the benchmark's shape: bit-equal to
-    cw_gemm_ksteps; parts 1 to 3 (no operand loads / no epilogue / no LDS reads in the k loop) run and return."""
+    """cw_diag_gemm_part with part 0 is the library's launch for the benchmark's shape: bit-equal to cw_gemm_ksteps; parts 1 to 3
+    (4 wavefronts; no operand loads / no epilogue / no LDS reads in the k loop) run and return."""
     import ctypes
     from cubework_amd import _diag, ops
 
