@@ -299,14 +299,15 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         auto pitch_factor = [&](double block_trips) {
             return cfg == kPairedConfig && block_trips > 80 && (p.lda % 64 != 0 || p.ldb % 64 != 0) ? 1.25 : 1.0;
         };
-        if (rows != 64 * c.tm) trips *= 0.2 + 0.8 * rows / (64 * c.tm);  // a lower tile's trips are shorter
-        // the kernels of gemm_wide.h: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's
-        // (the reduction waits about 0.9 us a slice whatever its size, and its bytes come from the cache)
+        // a lower tile's trips are shorter (160 rows are still priced some 15 % above what they take)
+        if (rows != 64 * c.tm) trips *= 0.2 + 0.8 * rows / (64 * c.tm);
+        // The kernels of gemm_wide.h: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's. Their
+        // reduction waits about 0.9 us a slice whatever its size, and its bytes come from the cache.
         const bool walks = cfg == 0 || cfg >= kPairedConfig;
         double us = tile_rounds(c, (double)full, trips, layout_factor * pitch_factor(trips)) + (walks && full > 0 ? 3.0 : 0.0);
         const double reduce_us = (walks ? 2.0 + 0.9 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
         if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor * pitch_factor(trips / slices)) + reduce_us;
-        // behind whole tiles: the slices start under the last tile's stores, and nothing hides theirs
+        // behind whole tiles: the slices start under the last tile's stores, and nothing hides theirs (146 launches: 3 us too high in the median)
         if (cfg == 0 && rest > 0 && full > 0) us += 1.2 * q.partial_bytes / 6.6e6 - 8.0;
         us = us > memory_us ? us + 0.1 * memory_us : memory_us + 0.1 * us;
         if (best.cfg < 0 || us < best_us) {

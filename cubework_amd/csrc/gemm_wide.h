@@ -16,7 +16,9 @@
 //
 // What bounds it: matrix cores and the power cap. 8192 x 8192 x 2048 (M x N x K) in us, random bf16 from HBM, NT / NN / TN:
 // 199 / 203 / 206, the kernel of 4 wavefronts and 32x32x16 that it replaced 240 / 241 / 217; 8192 x 2048 x 2048: 53 / 54,
-// before 62 / 62 (a launch of one round: 6 of the 53 us are its epilogue, whose stores nothing hides).
+// before 62 / 62 (a launch of one round: 6 of the 53 us are its epilogue, whose stores nothing hides). 128 accumulators, 80 fragment
+// registers and the loaders' offsets fill the 256 registers of a wavefront: at 256 rows the compiler spills 11 (NT), 17 (NN) or 24 (TN)
+// vector registers a lane (the headline writes 1.5 MiB more than its result a launch), at 224 rows 0 or 2.
 //
 // Whole 256-row tiles whose rows are mostly beyond M are wasted products: BM is 32 TM, the least of 160, 192, 224 and 256 that
 // covers M with as many tiles (gemm_plan.hip).
