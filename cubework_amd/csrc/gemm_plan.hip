@@ -305,7 +305,11 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         // reduction waits about 0.9 us a slice whatever its size, and its bytes come from the cache.
         const bool walks = cfg == 0 || cfg >= kPairedConfig;
         double us = tile_rounds(c, (double)full, trips, layout_factor * pitch_factor(trips)) + (walks && full > 0 ? 3.0 : 0.0);
-        const double reduce_us = (walks ? 2.0 + 0.9 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
+        double reduce_us = (walks ? 2.0 + 0.9 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
+        // Weight gradients cut in many slices of 256 x 256 tiles: all blocks write their partial sums at once and have walked little besides
+        // (us, M x N x K, TN, on such slices / as chosen now): 768 x 3072 x 4416 42.7 / 35.2, 3072 x 768 x 5295 46.4 / 38.4, 1024 x 3072 x
+        // 6080 53.4 / 43.5; from some 11000 of k on both are alike. Not so with k-contiguous A: 660 x 4096 x 12288 NT 71 / 78.
+        if (layout == CW_TN && cfg == 0 && full == 0 && slices > 3) reduce_us += 3.0 - 0.48 * slices + 0.37 * q.partial_bytes / 6.6e6 * q.rows / 256;
         if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor * pitch_factor(trips / slices)) + reduce_us;
         // behind whole tiles: the slices start under the last tile's stores, and nothing hides theirs (146 launches: 3 us too high in the median)
         if (cfg == 0 && rest > 0 && full > 0) us += 1.2 * q.partial_bytes / 6.6e6 - 8.0;

@@ -53,6 +53,13 @@ def test_short_products_of_one_round_take_64_x_128_tiles(plans, layout, M, N, K)
     assert plans([(layout, M, N, K, 1)]) == [(3, 64, -(-M // 64) * -(-N // 128), 1, 0)]
 
 
+@pytest.mark.parametrize("M,N,K", [(768, 3072, 4416), (3072, 768, 5295), (3072, 768, 6528), (1024, 3072, 6080)])
+def test_weight_gradients_are_not_cut_into_many_slices_of_large_tiles(plans, M, N, K):
+    """Six or seven slices of 36 tiles of 256 x 256 took 20 % longer than three of 128 x 256 or whole 128 x 128 tiles."""
+    (cfg, _, full, slices, _), = plans([("TN", M, N, K, 1)])
+    assert cfg != 0 or full > 0 or slices <= 3
+
+
 # What the lists of the GPU tests are there for: configuration, tile height, and w (whole tiles), s (every tile cut along k) or m (the
 # last round's cut), in NN, NT and TN. A plan that moves takes a kernel's coverage with it: find the list another shape then.
 WIDE_PLANS = {
