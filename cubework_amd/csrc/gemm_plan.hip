@@ -311,6 +311,10 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         // 6080 53.4 / 43.5; from some 11000 of k on both are alike. Not so with k-contiguous A: 660 x 4096 x 12288 NT 71 / 78.
         if (layout == CW_TN && cfg == 0 && full == 0 && slices > 3) reduce_us += 3.0 - 0.48 * slices + 0.37 * q.partial_bytes / 6.6e6 * q.rows / 256;
         if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor * pitch_factor(trips / slices)) + reduce_us;
+        // Weight gradients of so few tokens that a 256 x 256 tile has fewer than 7 stages: its stores do not drain under the next one's products,
+        // and where the last round is a quarter full or less the smaller tiles' finer rounds are the faster ones (us, M x N x K, TN, 256 x
+        // 256 / 128 x 256): 50257 x 1024 x 166 44.4 / 38.1, 50272 x 2048 x 188 76 / 67; fuller last rounds: 50257 x 2560 x 250 98 / 104.
+        if (layout == CW_TN && cfg == 0 && trips < 7 && tiles % 256 > 0 && tiles % 256 <= 64) us += (double)((full + 255) / 256);
         // behind whole tiles: the slices start under the last tile's stores, and nothing hides theirs (146 launches: 3 us too high in the median)
         if (cfg == 0 && rest > 0 && full > 0) us += 1.2 * q.partial_bytes / 6.6e6 - 8.0;
         us = us > memory_us ? us + 0.1 * memory_us : memory_us + 0.1 * us;

@@ -60,10 +60,16 @@ def test_weight_gradients_are_not_cut_into_many_slices_of_large_tiles(plans, M, 
     assert cfg != 0 or full > 0 or slices <= 3
 
 
+@pytest.mark.parametrize("M,N,K,cfg", [(50257, 1024, 166, 1), (50272, 2048, 188, 1), (50272, 1024, 250, 1), (50257, 2560, 250, 0)])
+def test_vocabulary_gradients_of_few_tokens(plans, M, N, K, cfg):
+    """Four stages of k: 256 x 256 tiles only where their last round is fuller than a quarter."""
+    assert plans([("TN", M, N, K, 1)])[0][0] == cfg
+
+
 # What the lists of the GPU tests are there for: configuration, tile height, and w (whole tiles), s (every tile cut along k) or m (the
 # last round's cut), in NN, NT and TN. A plan that moves takes a kernel's coverage with it: find the list another shape then.
 WIDE_PLANS = {
-    "SHAPES": {(300, 50257, 40, 3): "0x160w 0x160w 0x160w", (4100, 4090, 328, 1): "1x128w 0x256m 0x256m", (300, 32768, 1016, 1): "0x160w 0x160w 0x160w",
+    "SHAPES": {(300, 50257, 40, 3): "0x160w 0x160w 0x160w", (4100, 4090, 392, 1): "1x128w 0x256m 0x256m", (300, 32768, 1016, 1): "0x160w 0x160w 0x160w",
                (376, 32760, 1000, 1): "0x192w 0x192w 0x192w", (1552, 7672, 1352, 1): "0x224w 0x224w 0x224w",
                (8184, 2040, 328, 3): "0x256w 0x256w 1x128w", (8184, 6136, 520, 1): "0x256w 0x256w 0x256w",
                (7000, 4600, 1000, 1): "0x256w 0x256w 0x256w", (1024, 25003, 768, 1): "0x256w 0x256w 0x256w", (8192, 2048, 512, 2): "0x256w 0x256w 0x256w"},

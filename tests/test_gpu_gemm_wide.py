@@ -13,8 +13,8 @@ pytestmark = pytest.mark.gpu
 # (M, N, K, steps), which the planner gives to 256-column tiles in NN and NT and, mostly, in TN: heights 160, 192, 224 and 256 with
 # ragged edges, K of a part of a stage behind whole ones, three steps (rotated starts in NT), three tiles a block, a last row and column
 # of tiles with few elements, an odd last column; three stages to a tile, each of them a part of one (as short as the kernel
-# takes: every stage is the last of its step, every third of its tile); slices of three stages (NT and TN)
-SHAPES = [(300, 50257, 40, 3), (4100, 4090, 328, 1), (300, 32768, 1016, 1), (376, 32760, 1000, 1), (1552, 7672, 1352, 1), (8184, 2040, 328, 3), (8184, 6136, 520, 1),
+# takes: every stage is the last of its step, every third of its tile); slices of three and four stages (NT and TN)
+SHAPES = [(300, 50257, 40, 3), (4100, 4090, 392, 1), (300, 32768, 1016, 1), (376, 32760, 1000, 1), (1552, 7672, 1352, 1), (8184, 2040, 328, 3), (8184, 6136, 520, 1),
           (7000, 4600, 1000, 1), (1024, 25003, 768, 1), (8192, 2048, 512, 2)]
 
 # shapes that the planner gives to 128 x 128 tiles of two groups, in one orientation at least: ragged last tiles of either direction, K
