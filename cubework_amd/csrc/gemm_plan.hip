@@ -311,6 +311,10 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         // 6080 53.4 / 43.5; from some 11000 of k on both are alike. Not so with k-contiguous A: 660 x 4096 x 12288 NT 71 / 78.
         if (layout == CW_TN && cfg == 0 && full == 0 && slices > 3) reduce_us += 3.0 - 0.48 * slices + 0.37 * q.partial_bytes / 6.6e6 * q.rows / 256;
         if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor * pitch_factor(trips / slices)) + reduce_us;
+        // At most one 128 x 256 tile a unit and a short k: nothing hides a block's first loads and its stores, where 128 x 128 ones share the
+        // unit (us, M x N x K, 128 x 256 / 128 x 128): 2820 x 1632 x 166 TN 11.3 / 8.9, 6243 x 832 x 256 NT 12.8 / 10.8; above 576 of k
+        // the costs hold as they are.
+        if (cfg == 1 && full == tiles && tiles <= 256 && trips < 18) us += 1.5;
         // Weight gradients of so few tokens that a 256 x 256 tile has fewer than 7 stages: its stores do not drain under the next one's products,
         // and where the last round is a quarter full or less the smaller tiles' finer rounds are the faster ones (us, M x N x K, TN, 256 x
         // 256 / 128 x 256): 50257 x 1024 x 166 44.4 / 38.1, 50272 x 2048 x 188 76 / 67; fuller last rounds: 50257 x 2560 x 250 98 / 104.

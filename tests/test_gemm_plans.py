@@ -66,6 +66,12 @@ def test_vocabulary_gradients_of_few_tokens(plans, M, N, K, cfg):
     assert plans([("TN", M, N, K, 1)])[0][0] == cfg
 
 
+@pytest.mark.parametrize("layout,M,N,K", [("TN", 2820, 1632, 166), ("TN", 3520, 1664, 407), ("NT", 6243, 832, 256), ("NN", 6620, 544, 288)])
+def test_short_products_of_half_a_round_take_128_x_128_tiles(plans, layout, M, N, K):
+    """160 to 200 tiles of 128 x 256 would leave each of its blocks alone on its unit (15 to 25 % slower)."""
+    assert plans([(layout, M, N, K, 1)])[0][:2] == (2, 128)
+
+
 # What the lists of the GPU tests are there for: configuration, tile height, and w (whole tiles), s (every tile cut along k) or m (the
 # last round's cut), in NN, NT and TN. A plan that moves takes a kernel's coverage with it: find the list another shape then.
 WIDE_PLANS = {
@@ -77,7 +83,7 @@ WIDE_PLANS = {
                (4001, 1000, 1032, 3): "5x128w 5x128w 5x128w", (2040, 2040, 1416, 1): "2x128w 5x128w 2x128w",
                (4001, 1000, 4200, 1): "5x128w 5x128w 5x128w", (2040, 2047, 4200, 1): "5x128w 5x128w 5x128w",
                (1016, 768, 5000, 1): "5x128s 5x128s 4x64w", (300, 2048, 8192, 1): "5x128s 5x128s 5x128s", (4096, 1024, 4096, 1): "5x128w 5x128w 5x128w"},
-    "NARROW": {(300, 16384, 40, 5): "6x160w 6x160w 1x128w", (4100, 2047, 1000, 3): "6x192w 6x192m 5x128m", (496, 2560, 520, 5): "3x64w 7x128s 3x64w",
+    "NARROW": {(300, 16384, 40, 5): "6x160w 6x160w 2x128w", (4100, 2047, 1000, 3): "6x192w 6x192m 5x128m", (496, 2560, 520, 5): "3x64w 7x128s 3x64w",
                (300, 16376, 2056, 1): "6x160w 6x160w 0x160s", (1554, 2559, 1000, 3): "6x192w 6x192w 3x64w",
                (496, 8184, 2056, 1): "7x128w 5x128w 5x128w", (300, 4090, 12296, 1): "6x160s 6x160s 0x160s", (1554, 2560, 2560, 1): "6x192w 6x192w 3x64w"},
     "RAGGED_K": {(300, 50257, 37, 3): "0x160w 0x160w", (300, 16384, 37, 5): "6x160w 6x160w", (8184, 2040, 331, 3): "0x256w 0x256w",
