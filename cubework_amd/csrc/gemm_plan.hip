@@ -319,6 +319,10 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         // and where the last round is a quarter full or less the smaller tiles' finer rounds are the faster ones (us, M x N x K, TN, 256 x
         // 256 / 128 x 256): 50257 x 1024 x 166 44.4 / 38.1, 50272 x 2048 x 188 76 / 67; fuller last rounds: 50257 x 2560 x 250 98 / 104.
         if (layout == CW_TN && cfg == 0 && trips < 7 && tiles % 256 > 0 && tiles % 256 <= 64) us += (double)((full + 255) / 256);
+        // 128-column tiles of NN products over a long k in more than two and a half rounds: their first rounds are no slower than the costs say,
+        // the later ones, under the power cap, are (us, M x N x K, such tiles / 128 x 256 or 256 x 256): 7948 x 2560 x 2560 126 / 109, 2465 x 7680
+        // x 2560 121 / 106, 14502 x 2560 x 2560 188 / 169, 5280 x 4096 x 4096 177 / 171.
+        if (layout == CW_NN && cfg >= kNarrowConfig && full == tiles && tiles > 640 && K * n_steps >= 2496) us *= 1.07;
         // behind whole tiles: the slices start under the last tile's stores, and nothing hides theirs (146 launches: 3 us too high in the median)
         if (cfg == 0 && rest > 0 && full > 0) us += 1.2 * q.partial_bytes / 6.6e6 - 8.0;
         us = us > memory_us ? us + 0.1 * memory_us : memory_us + 0.1 * us;

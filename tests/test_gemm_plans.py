@@ -72,6 +72,12 @@ def test_short_products_of_half_a_round_take_128_x_128_tiles(plans, layout, M, N
     assert plans([(layout, M, N, K, 1)])[0][:2] == (2, 128)
 
 
+@pytest.mark.parametrize("M,N,K,cfg", [(7948, 2560, 2560, 1), (2465, 7680, 2560, 1), (2028, 10240, 2560, 1), (14502, 2560, 2560, 0), (1554, 10240, 2560, 6)])
+def test_forward_products_of_many_rounds_take_256_columns(plans, M, N, K, cfg):
+    """More than two and a half rounds of 128-column tiles are slower than the larger ones' (7 to 15 %)."""
+    assert plans([("NN", M, N, K, 1)])[0][0] == cfg
+
+
 # What the lists of the GPU tests are there for: configuration, tile height, and w (whole tiles), s (every tile cut along k) or m (the
 # last round's cut), in NN, NT and TN. A plan that moves takes a kernel's coverage with it: find the list another shape then.
 WIDE_PLANS = {
