@@ -1,5 +1,5 @@
 // bf16 / fp16 block GEMM: choice of kernel and launch (the same for both element types).
-//   - the tile kernels (gemm_tile.h) take every shape whose operand rows are 16-byte aligned, and the others after a copy to
+//   - the tile kernels (gemm_wide.h, gemm_tile.h) take every shape whose operand rows are 16-byte aligned, and the others after a copy to
 //     aligned rows, which the caller's scratch holds. tile_plan (gemm_plan.hip) chooses the tile size and which tiles are
 //     cut along k, by a cost model of the launch;
 //   - a call with less scratch than that (or none) is planned by gemm_half_plan;

@@ -44,16 +44,17 @@ struct GemmPlan {
 GemmPlan gemm_half_plan(const GemmArgs& args, int layout, bool dma_enabled, bool strip_enabled);
 
 // ---- tile kernels (gemm_wide.h: configurations 0 and 5 to 7; gemm_tile.h: the others) ---------------------------------------
-// Their configurations: block tile 64 tm x 64 tn, k extent of a trip in units of 32, ring stages, resident
-// blocks per compute unit, and what a trip costs (us; one block on the unit / two) and a block besides its trips. The
-// costs were a fit to 2000 launches over 110 shapes (products of 64 .. 8192 tokens with the model widths 768 .. 4096, in the
-// forward and weight-gradient orientations; rms error 11 %). Configurations 0 and 5 to 7, what cutting along k costs them, and where the
-// choice against them lies (1 and 2, the factors of TN) were fitted to some 250 later launches of 30 of these shapes; 3 and 4 to 14000
-// launches of every configuration over 1000 shapes (also layers of any width and vocabularies), the others held. Over those launches the
-// error is 14 % rms (3 and 4: 20 to 24), and choosing by the costs costs 1.6 % over the best launch of a shape on average. 3 and 4
-// at 0.440, 0.800, 2.60 and 0.289, 0.460, 2.06 (2.1 %) gave short products 64 x 64 tiles in two rounds (us, M x N x K): 2394 x 576 x
-// 1536 NT 15.8 / 12.9 on 64 x 128, 1894 x 1024 x 1024 NT 11.2 / 9.5, 1280 x 1024 x 1024 NT 10.5 / 9.1, 473 x 3072 x 768 NN 9.7 /
-// 8.8. (The launches' times are not kept in this tree: a change of the kernels' speed means measuring and fitting again.)
+// Their configurations: block tile 64 tm x 64 tn, k extent of a trip in units of 32, ring stages, resident blocks per compute unit,
+// and what a trip costs (us; one block on the unit / two) and a block besides its trips. The costs were a fit to 2000 launches over
+// 110 shapes (products of 64 .. 8192 tokens with the model widths 768 .. 4096, in the forward and weight-gradient orientations; rms
+// error 11 %). Configurations 0 and 5 to 7, what cutting along k costs them, and where the choice against them lies (1 and 2, the
+// factors of TN) were fitted to some 250 later launches of 30 of these shapes; 3 and 4 to 14000 launches of every configuration over
+// 1000 shapes (also layers of any width and vocabularies), the others held; the same launches gave the four corrections in tile_plan
+// that name their shapes. Over them the error is 14 % rms (3 and 4: 20 to 24), and choosing by the costs costs 1.4 % over the best
+// launch of a shape on average. 3 and 4 at 0.440, 0.800, 2.60 and 0.289, 0.460, 2.06 (2.1 %) gave short products 64 x 64 tiles in
+// two rounds (us, M x N x K): 2394 x 576 x 1536 NT 15.8 / 12.9 on 64 x 128, 1894 x 1024 x 1024 NT 11.2 / 9.5, 1280 x 1024 x 1024 NT
+// 10.5 / 9.1, 473 x 3072 x 768 NN 9.7 / 8.8. (The launches' times are not kept in this tree: a change of the kernels' speed means
+// measuring and fitting again.)
 struct TileConfig {
     int tm, tn, kb, stages, resident;
     float trip1, trip2, fixed;
