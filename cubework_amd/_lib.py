@@ -63,6 +63,14 @@ SIGNATURES = {
     "cw_colsum_static_max_bytes": (_i64, []),
     "cw_colsum_static": (_int, [_i64, _i64, _ptr, _i64, _ptr, _int, _int, _ptr]),
     "cw_act_bwd_colsum": (_int, [_int, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _int, _ptr, _i64, _int, _ptr]),
+    "cw_colsum_peers": (_int, [_i64, _i64, _ptr, _i64, _ptr, _int, _ptr, _i64, _pp, _int, _i64, _i64, _ptr, _int, _int, _ptr]),
+    "cw_act_bwd_colsum_peers": (_int, [_int, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _i64, _ptr, _int, _ptr, _i64, _pp, _int, _i64,
+                                       _i64, _ptr, _int, _int, _ptr]),
+    "cw_ln_partial_stats_gather": (_int, [_i64, _i64, _ptr, _i64, _ptr, _pp, _pp, _int, _ptr, _ptr, _int, _ptr]),
+    "cw_ln_normalize_peers": (_int, [_i64, _i64, _ptr, _i64, _ptr, _pp, _int, _int, _i64, _f32, _ptr, _ptr, _ptr, _i64, _ptr, _int,
+                                     _ptr]),
+    "cw_ln_bwd_dx_close_peers": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _pp, _int, _i64, _ptr, _i64, _ptr, _i64,
+                                        _ptr, _ptr, _int, _pp, _pp, _int, _i64, _i64, _ptr, _ptr, _int, _int, _ptr]),
     "cw_ln_partial_stats": (_int, [_i64, _i64, _ptr, _i64, _int, _ptr, _ptr, _int, _ptr]),
     "cw_ln_normalize": (_int, [_i64, _i64, _ptr, _i64, _ptr, _int, _i64, _f32, _ptr, _ptr, _ptr, _i64, _ptr, _int,
                                _ptr]),
@@ -111,8 +119,9 @@ def load():
 
 #: entry points that the native operator calls (csrc/host_ops.cpp) use
 HOST_ENTRIES = ("cw_gemm_scratch_bytes", "cw_gemm_ksteps_ws", "cw_colsum_workspace_bytes", "cw_colsum", "cw_act_bwd_colsum",
-                "cw_ln_partial_stats", "cw_ln_normalize", "cw_ln_forward_fused", "cw_ln_backward_fused",
-                "cw_ln_bwd_partials_open", "cw_ln_bwd_dx_close")
+                "cw_colsum_peers", "cw_act_bwd_colsum_peers", "cw_ln_partial_stats", "cw_ln_partial_stats_gather",
+                "cw_ln_normalize_peers", "cw_ln_forward_fused", "cw_ln_backward_fused", "cw_ln_bwd_partials_open",
+                "cw_ln_bwd_dx_close_peers")
 
 
 def host():

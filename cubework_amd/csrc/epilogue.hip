@@ -102,7 +102,8 @@ constexpr int kFinGroups = 16;
 __global__ __launch_bounds__(kFinGroups * 64) void finalize_cols_kernel(const float* __restrict__ ws, int64_t nparts,
                                                                         int64_t part_stride, int64_t C,
                                                                         void* __restrict__ out0,
-                                                                        void* __restrict__ out1, int out_dtype) {
+                                                                        void* __restrict__ out1, int out_dtype,
+                                                                        const PeerCols peers) {
     __shared__ float red[kFinGroups][64];
     const int lane = threadIdx.x & 63;
     const int grp = threadIdx.x >> 6;
@@ -132,13 +133,14 @@ __global__ __launch_bounds__(kFinGroups * 64) void finalize_cols_kernel(const fl
         for (int g = 1; g < kFinGroups; ++g) total += red[g][lane];
         void* out = (k == 0) ? out0 : out1;
         if (out != nullptr) store_col_total(out, c, total, out_dtype);
+        add_peer_cols(peers, k, c, total);
     }
 }
 
 template <typename T, int MODE>
 int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void* pre, int64_t ld_pre, void* dPre,
                 int64_t ld_dpre, int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes,
-                hipStream_t s) {
+                const PeerCols* peers, hipStream_t s) {
     constexpr int V = elem<T>::kVec;
     const int want_sum = out != nullptr ? 1 : 0;
     bool vec = aligned16(dY) && (ld_dy % V) == 0 && (N % V) == 0;
@@ -170,16 +172,39 @@ int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void*
     }
     int rc = check_launch("colsum kernel");
     if (rc != CW_OK || !want_sum) return rc;
-    return finalize_col_partials((const float*)workspace, slabs, N, 1, N, out, nullptr, out_dtype, s);
+    return finalize_col_partials((const float*)workspace, slabs, N, 1, N, out, nullptr, out_dtype, s, peers);
 }
 
 }  // namespace
 
 int finalize_col_partials(const float* ws, int64_t nparts, int64_t part_stride, int nsets, int64_t C, void* out0,
-                          void* out1, int out_dtype, hipStream_t s) {
+                          void* out1, int out_dtype, hipStream_t s, const PeerCols* peers) {
     hipLaunchKernelGGL(finalize_cols_kernel, dim3((unsigned)((C + 63) / 64), (unsigned)nsets), dim3(kFinGroups * 64), 0, s, ws,
-                       nparts, part_stride, C, out0, out1, out_dtype);
+                       nparts, part_stride, C, out0, out1, out_dtype, peers != nullptr ? *peers : PeerCols{});
     return check_launch("finalize_cols_kernel");
+}
+
+int peer_cols(const char* fn, int sets, const float* const* peers0, const float* const* peers1, int n_peers, int64_t C, int64_t c0,
+              int64_t count, void* out0, void* out1, int out_dtype, PeerCols* p) {
+    *p = PeerCols{};
+    if (n_peers == 0) return CW_OK;
+    if (n_peers < 0 || n_peers > CW_MAX_ADDENDS) return fail(CW_ERR_INVALID, "%s: n_peers=%d outside 0..%d", fn, n_peers, CW_MAX_ADDENDS);
+    if (c0 < 0 || count < 0 || c0 > C - count) return fail(CW_ERR_INVALID, "%s: columns %lld + %lld of %lld", fn, (long long)c0, (long long)count, (long long)C);
+    if (!col_out_dtype_ok(out_dtype)) return fail(CW_ERR_INVALID, "%s: bad type %d of the reduced sums", fn, out_dtype);
+    if (peers0 == nullptr || out0 == nullptr || (sets > 1 && (peers1 == nullptr || out1 == nullptr)))
+        return fail(CW_ERR_INVALID, "%s: the peers' tables and the reduced sums are both needed", fn);
+    for (int set = 0; set < sets; ++set)
+        for (int k = 0; k < n_peers; ++k) {
+            p->peer[set][k] = (set == 0 ? peers0 : peers1)[k];
+            if (p->peer[set][k] == nullptr) return fail(CW_ERR_INVALID, "%s: peer %d is NULL", fn, k);
+        }
+    p->c0 = c0;
+    p->count = count;
+    p->out[0] = out0;
+    p->out[1] = out1;
+    p->n_peers = n_peers;
+    p->out_dtype = out_dtype;
+    return CW_OK;
 }
 
 // ---- library-owned scratch for the entry point that allocates nothing ------------------------------
@@ -257,21 +282,30 @@ extern "C" int64_t cw_colsum_workspace_bytes(int64_t M, int64_t N) {
 
 extern "C" int cw_colsum(int64_t M, int64_t N, const void* dY, int64_t ld, void* out, int out_dtype, void* workspace,
                          int64_t workspace_bytes, int io_dtype, void* stream) {
+    return cw_colsum_peers(M, N, dY, ld, out, out_dtype, workspace, workspace_bytes, nullptr, 0, 0, 0, nullptr, CW_F32, io_dtype, stream);
+}
+
+extern "C" int cw_colsum_peers(int64_t M, int64_t N, const void* dY, int64_t ld, void* out, int out_dtype, void* workspace,
+                               int64_t workspace_bytes, const float* const* peers, int n_peers, int64_t c0, int64_t count,
+                               void* reduced, int reduced_dtype, int io_dtype, void* stream) {
     if (M < 0 || N <= 0) return fail(CW_ERR_INVALID, "cw_colsum: bad shape M=%lld N=%lld", (long long)M, (long long)N);
     if (io_dtype != CW_BF16 && io_dtype != CW_F32 && io_dtype != CW_F16)
         return fail(CW_ERR_INVALID, "cw_colsum: bad io_dtype %d", io_dtype);
     if (out == nullptr) return fail(CW_ERR_INVALID, "cw_colsum: out is NULL");
     if (!col_out_dtype_ok(out_dtype)) return fail(CW_ERR_INVALID, "cw_colsum: bad out_dtype %d", out_dtype);
+    PeerCols pc;
+    if (const int prc = peer_cols("cw_colsum_peers", 1, peers, nullptr, n_peers, N, c0, count, reduced, nullptr, reduced_dtype, &pc); prc != CW_OK)
+        return prc;
     if (const int drc = require_gfx950("cw_colsum"); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
-    if (M == 0) return finalize_col_partials(nullptr, 0, N, 1, N, out, nullptr, out_dtype, s);  // zero fill
+    if (M == 0) return finalize_col_partials(nullptr, 0, N, 1, N, out, nullptr, out_dtype, s, &pc);  // zero fill
     if (dY == nullptr || workspace == nullptr || ld < N)
         return fail(CW_ERR_INVALID, "cw_colsum: null pointer or ld < N");
     if (io_dtype == CW_F16)
-        return colsum_impl<f16_t, 0>(M, N, dY, ld, nullptr, 0, nullptr, 0, 0, out, out_dtype, workspace, workspace_bytes, s);
+        return colsum_impl<f16_t, 0>(M, N, dY, ld, nullptr, 0, nullptr, 0, 0, out, out_dtype, workspace, workspace_bytes, &pc, s);
     return io_dtype == CW_BF16
-               ? colsum_impl<bf16_t, 0>(M, N, dY, ld, nullptr, 0, nullptr, 0, 0, out, out_dtype, workspace, workspace_bytes, s)
-               : colsum_impl<float, 0>(M, N, dY, ld, nullptr, 0, nullptr, 0, 0, out, out_dtype, workspace, workspace_bytes, s);
+               ? colsum_impl<bf16_t, 0>(M, N, dY, ld, nullptr, 0, nullptr, 0, 0, out, out_dtype, workspace, workspace_bytes, &pc, s)
+               : colsum_impl<float, 0>(M, N, dY, ld, nullptr, 0, nullptr, 0, 0, out, out_dtype, workspace, workspace_bytes, &pc, s);
 }
 
 extern "C" int64_t cw_colsum_static_max_bytes(void) { return kStaticScratchBytes; }
@@ -308,6 +342,14 @@ extern "C" int cw_act_bwd_colsum(int activation, int64_t M, int64_t N, const voi
                                  const void* preact, int64_t ld_pre, void* dPre, int64_t ld_dpre, void* dbias,
                                  int dbias_dtype, void* workspace, int64_t workspace_bytes, int io_dtype,
                                  void* stream) {
+    return cw_act_bwd_colsum_peers(activation, M, N, dY, ld_dy, preact, ld_pre, dPre, ld_dpre, dbias, dbias_dtype, workspace,
+                                   workspace_bytes, nullptr, 0, 0, 0, nullptr, CW_F32, io_dtype, stream);
+}
+
+extern "C" int cw_act_bwd_colsum_peers(int activation, int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void* preact,
+                                       int64_t ld_pre, void* dPre, int64_t ld_dpre, void* dbias, int dbias_dtype, void* workspace,
+                                       int64_t workspace_bytes, const float* const* peers, int n_peers, int64_t c0, int64_t count,
+                                       void* reduced, int reduced_dtype, int io_dtype, void* stream) {
     if (M < 0 || N <= 0)
         return fail(CW_ERR_INVALID, "cw_act_bwd_colsum: bad shape M=%lld N=%lld", (long long)M, (long long)N);
     if (io_dtype != CW_BF16 && io_dtype != CW_F32 && io_dtype != CW_F16)
@@ -317,11 +359,16 @@ extern "C" int cw_act_bwd_colsum(int activation, int64_t M, int64_t N, const voi
         return fail(CW_ERR_INVALID, "cw_act_bwd_colsum: bad activation %d", activation);
     if (dbias != nullptr && !col_out_dtype_ok(dbias_dtype))
         return fail(CW_ERR_INVALID, "cw_act_bwd_colsum: bad dbias_dtype %d", dbias_dtype);
+    if (dbias == nullptr && n_peers != 0) return fail(CW_ERR_INVALID, "cw_act_bwd_colsum_peers: peers' sums without dbias");
+    PeerCols pc;
+    if (const int prc = peer_cols("cw_act_bwd_colsum_peers", 1, peers, nullptr, n_peers, N, c0, count, reduced, nullptr, reduced_dtype, &pc);
+        prc != CW_OK)
+        return prc;
     if (const int drc = require_gfx950("cw_act_bwd_colsum"); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
     if (M == 0) {
         if (dbias == nullptr) return CW_OK;
-        return finalize_col_partials(nullptr, 0, N, 1, N, dbias, nullptr, dbias_dtype, s);  // zero fill
+        return finalize_col_partials(nullptr, 0, N, 1, N, dbias, nullptr, dbias_dtype, s, &pc);  // zero fill
     }
     if (dY == nullptr || preact == nullptr || dPre == nullptr || ld_dy < N || ld_pre < N || ld_dpre < N)
         return fail(CW_ERR_INVALID, "cw_act_bwd_colsum: null pointer or leading dimension < N");
@@ -329,9 +376,9 @@ extern "C" int cw_act_bwd_colsum(int activation, int64_t M, int64_t N, const voi
         return fail(CW_ERR_INVALID, "cw_act_bwd_colsum: workspace is NULL");
     if (io_dtype == CW_F16)
         return colsum_impl<f16_t, 1>(M, N, dY, ld_dy, preact, ld_pre, dPre, ld_dpre, activation, dbias, dbias_dtype,
-                                     workspace, workspace_bytes, s);
+                                     workspace, workspace_bytes, &pc, s);
     return io_dtype == CW_BF16 ? colsum_impl<bf16_t, 1>(M, N, dY, ld_dy, preact, ld_pre, dPre, ld_dpre, activation, dbias,
-                                                        dbias_dtype, workspace, workspace_bytes, s)
+                                                        dbias_dtype, workspace, workspace_bytes, &pc, s)
                                : colsum_impl<float, 1>(M, N, dY, ld_dy, preact, ld_pre, dPre, ld_dpre, activation, dbias,
-                                                       dbias_dtype, workspace, workspace_bytes, s);
+                                                       dbias_dtype, workspace, workspace_bytes, &pc, s);
 }

@@ -18,8 +18,9 @@ using OptTensor = std::optional<Tensor>;
 
 #define CW_HOST_ENTRIES(X)                                                                                             \
     X(cw_gemm_scratch_bytes) X(cw_gemm_ksteps_ws) X(cw_colsum_workspace_bytes) X(cw_colsum) X(cw_act_bwd_colsum)       \
-    X(cw_ln_partial_stats) X(cw_ln_normalize) X(cw_ln_forward_fused) X(cw_ln_backward_fused) X(cw_ln_bwd_partials_open) \
-    X(cw_ln_bwd_dx_close)
+    X(cw_colsum_peers) X(cw_act_bwd_colsum_peers) X(cw_ln_partial_stats) X(cw_ln_partial_stats_gather)                 \
+    X(cw_ln_normalize_peers) X(cw_ln_forward_fused) X(cw_ln_backward_fused) X(cw_ln_bwd_partials_open)                 \
+    X(cw_ln_bwd_dx_close_peers)
 struct Entries {
 #define X(name) decltype(&::name) name = nullptr;
     CW_HOST_ENTRIES(X)
@@ -79,6 +80,37 @@ OptTensor vec(const OptTensor& t, at::ScalarType type) {
     return t->to(type).contiguous();
 }
 Tensor colsum_workspace(int64_t M, int64_t N, const Tensor& like) { return bytes(std::max<int64_t>(lib.cw_colsum_workspace_bytes(M, N), 16), like); }
+
+// The other ranks' summands of a vector or of rows' pairs. The kernels read them where they arrived if they are what a rank of this
+// kind sends (fp32, contiguous, as many elements); anything else that torch can add is added here, in the same order.
+using Peers = std::vector<Tensor>;
+bool direct(const Peers& peers, const Tensor& own) {
+    if (peers.size() > CW_MAX_ADDENDS || own.scalar_type() != at::kFloat) return false;
+    for (const auto& t : peers)
+        if (t.scalar_type() != at::kFloat || t.sizes() != own.sizes() || !t.is_contiguous() || t.device() != own.device()) return false;
+    return true;
+}
+std::vector<const float*> pointers(const Peers& peers) {
+    std::vector<const float*> p;
+    for (const auto& t : peers) p.push_back((const float*)ptr(t));
+    return p;
+}
+Tensor add_peers(Tensor own, const Peers& peers) {
+    for (const auto& t : peers) own = own + t;
+    return own;
+}
+// This rank's share of column sums that are reduce-scattered over `world` ranks, stored as `type`.
+struct Scatter {
+    Peers peers;
+    int64_t world = 1, rank = 0;
+    at::ScalarType type = at::kFloat;
+    bool fused(const Tensor& own) const {
+        return !peers.empty() && own.dim() == 1 && own.size(0) % world == 0 && (type == at::kFloat || type == at::kBFloat16 || type == at::kHalf) &&
+               direct(peers, own);
+    }
+    int64_t count(const Tensor& own) const { return own.size(0) / world; }
+    Tensor general(const Tensor& own) const { return add_peers(own, peers).chunk(world, -1).at(rank).contiguous().to(type); }
+};
 
 // -> (C, preact or None). See ops.gemm_ksteps.
 std::tuple<Tensor, OptTensor> gemm_ksteps(int layout, std::vector<Tensor> A, std::vector<Tensor> B, const OptTensor& bias_in, int epilogue,
@@ -178,6 +210,61 @@ std::tuple<Tensor, OptTensor> act_bwd_colsum(int activation, const Tensor& dy_in
     return {dpre, dbias};
 }
 
+// Column sums (of dPre = dy * act'(pre) if there is an activation) reduce-scattered over the ranks: -> (dPre or None, this rank's share).
+std::tuple<OptTensor, Tensor> colsum_scattered(const Tensor& dy_in, int activation, const OptTensor& pre_in, Peers peers, int64_t world,
+                                               int64_t rank, at::ScalarType type) {
+    const Tensor dy = rows(dy_in);
+    on_device(dy);
+    const int64_t M = dy.size(0), N = dy.size(1);
+    const Scatter sc{std::move(peers), world, rank, type};
+    Tensor own = empty({N}, dy, at::kFloat), ws = colsum_workspace(M, N, dy);
+    const bool fused = sc.fused(own);
+    const int64_t count = fused ? sc.count(own) : 0;
+    OptTensor reduced, pre, dpre;
+    if (fused) reduced = empty({count}, dy, sum_type(type));
+    const auto table = pointers(fused ? sc.peers : Peers{});
+    if (pre_in) {
+        pre = rows(*pre_in);
+        on_device(pre);
+        TORCH_CHECK_VALUE(dy.sizes() == pre->sizes() && dy.scalar_type() == pre->scalar_type(), "dy and preact must agree in shape and dtype");
+        dpre = empty({M, N}, dy);
+        check(lib.cw_act_bwd_colsum_peers(activation, M, N, ptr(dy), ld(dy), ptr(pre), ld(pre), ptr(dpre), ld(dpre), ptr(own), CW_F32, ptr(ws),
+                                          ws.numel(), table.data(), (int)table.size(), rank * count, count, ptr(reduced),
+                                          fused ? dtype_code(type) : CW_F32, dtype_code(dy.scalar_type()), stream()),
+              "cw_act_bwd_colsum_peers");
+    } else {
+        check(lib.cw_colsum_peers(M, N, ptr(dy), ld(dy), ptr(own), CW_F32, ptr(ws), ws.numel(), table.data(), (int)table.size(), rank * count,
+                                  count, ptr(reduced), fused ? dtype_code(type) : CW_F32, dtype_code(dy.scalar_type()), stream()),
+              "cw_colsum_peers");
+    }
+    return {dpre, fused ? *reduced : sc.general(own)};
+}
+
+// Statistics of x and, by the same launch, the affine parameters gathered from their ranks' parts: -> (stats, gamma, beta).
+std::tuple<Tensor, Tensor, Tensor> ln_partial_stats_gather(const Tensor& x_in, std::vector<Tensor> gammas, std::vector<Tensor> betas) {
+    const Tensor x = rows(x_in);
+    on_device(x);
+    const int64_t R = x.size(0), C = x.size(1), n = (int64_t)gammas.size();
+    bool fused = R > 0 && n >= 1 && n <= CW_MAX_ADDENDS && betas.size() == gammas.size() && C % n == 0;
+    for (const auto* set : {&gammas, &betas})
+        for (const auto& t : *set)
+            fused = fused && t.dim() == 1 && t.numel() * n == C && t.scalar_type() == x.scalar_type() && t.is_contiguous() && t.device() == x.device();
+    Tensor stats = empty({R, 2}, x, at::kFloat);
+    if (!fused) {
+        check(lib.cw_ln_partial_stats(R, C, ptr(x), ld(x), CW_LN_ONE_PASS, nullptr, (float*)ptr(stats), dtype_code(x.scalar_type()), stream()),
+              "cw_ln_partial_stats");
+        return {stats, at::cat(gammas, -1), at::cat(betas, -1)};
+    }
+    Tensor gamma = empty({C}, x), beta = empty({C}, x);
+    std::vector<const void*> pg, pb;
+    for (const auto& t : gammas) pg.push_back(ptr(t));
+    for (const auto& t : betas) pb.push_back(ptr(t));
+    check(lib.cw_ln_partial_stats_gather(R, C, ptr(x), ld(x), (float*)ptr(stats), pg.data(), pb.data(), (int)n, ptr(gamma), ptr(beta),
+                                         dtype_code(x.scalar_type()), stream()),
+          "cw_ln_partial_stats_gather");
+    return {stats, gamma, beta};
+}
+
 Tensor ln_partial_stats(const Tensor& x_in, int mode, const OptTensor& mean_in) {
     const Tensor x = rows(x_in);
     on_device(x);
@@ -194,9 +281,9 @@ Tensor ln_partial_stats(const Tensor& x_in, int mode, const OptTensor& mean_in) 
     return stats;
 }
 
-// stats given: ln_normalize; else ln_forward_fused.
-std::tuple<Tensor, OptTensor> ln_forward(const Tensor& x_in, const OptTensor& stats_in, int64_t hidden, double eps, const OptTensor& gamma_in,
-                                         const OptTensor& beta_in, int mode, bool save_mean_rstd) {
+// stats given: ln_normalize of their sum with the peers'; else ln_forward_fused.
+std::tuple<Tensor, OptTensor> ln_forward(const Tensor& x_in, const OptTensor& stats_in, Peers peers, int64_t hidden, double eps,
+                                         const OptTensor& gamma_in, const OptTensor& beta_in, int mode, bool save_mean_rstd) {
     const Tensor x = rows(x_in);
     on_device(x);
     on_device(stats_in);
@@ -204,7 +291,11 @@ std::tuple<Tensor, OptTensor> ln_forward(const Tensor& x_in, const OptTensor& st
     on_device(beta_in);
     const int64_t R = x.size(0), C = x.size(1);
     OptTensor stats;
-    if (stats_in) stats = stats_in->reshape({R, 2}).to(at::kFloat).contiguous();
+    if (stats_in) {
+        if (!direct(peers, *stats_in)) stats = add_peers(*stats_in, std::exchange(peers, {}));
+        stats = stats.value_or(*stats_in).reshape({R, 2}).to(at::kFloat).contiguous();
+    }
+    const auto table = pointers(peers);
     const OptTensor gamma = vec(gamma_in, x.scalar_type()), beta = vec(beta_in, x.scalar_type());
     if (stats)
         for (const auto* v : {&gamma, &beta}) TORCH_CHECK_VALUE(!*v || (*v)->numel() == C, "gamma/beta must have C elements");
@@ -213,9 +304,9 @@ std::tuple<Tensor, OptTensor> ln_forward(const Tensor& x_in, const OptTensor& st
     if (save_mean_rstd) mr = empty({R, 2}, x, at::kFloat);
     const int dt = dtype_code(x.scalar_type());
     if (stats)
-        check(lib.cw_ln_normalize(R, C, ptr(x), ld(x), (const float*)ptr(stats), mode, hidden, (float)eps, ptr(gamma), ptr(beta), ptr(y), ld(y),
-                                  (float*)ptr(mr), dt, stream()),
-              "cw_ln_normalize");
+        check(lib.cw_ln_normalize_peers(R, C, ptr(x), ld(x), (const float*)ptr(stats), table.data(), (int)table.size(), mode, hidden, (float)eps,
+                                        ptr(gamma), ptr(beta), ptr(y), ld(y), (float*)ptr(mr), dt, stream()),
+              "cw_ln_normalize_peers");
     else
         check(lib.cw_ln_forward_fused(R, C, ptr(x), ld(x), mode, (float)eps, ptr(gamma), ptr(beta), ptr(y), ld(y), (float*)ptr(mr), dt, stream()),
               "cw_ln_forward_fused");
@@ -286,17 +377,37 @@ std::tuple<Tensor, Tensor, int64_t> ln_bwd_partials_open(const Tensor& dy_in, co
     return {row_sums, ws, parts};
 }
 
+// sums: this rank's; the row peers' are added. With column peers dgamma and dbeta come back reduce-scattered, as the given types.
 std::tuple<Tensor, Tensor, Tensor> ln_bwd_dx_close(const Tensor& dy_in, const Tensor& x_in, const Tensor& mean_rstd, const Tensor& sums_in,
-                                                   int64_t hidden, const Tensor& ws, int64_t parts, const OptTensor& gamma,
-                                                   std::optional<at::ScalarType> param_type) {
+                                                   Peers row_peers, int64_t hidden, const Tensor& ws, int64_t parts, const OptTensor& gamma,
+                                                   std::optional<at::ScalarType> param_type, Peers dgamma_peers, Peers dbeta_peers, int64_t world,
+                                                   int64_t rank, at::ScalarType gamma_type, at::ScalarType beta_type) {
     const LnBackward b = ln_backward_inputs(dy_in, x_in, mean_rstd, sums_in, gamma);
-    const Tensor sums = sums_in.reshape({b.R, 2}).to(at::kFloat).contiguous();
+    const bool rows_direct = direct(row_peers, sums_in);
+    const Tensor sums = (rows_direct ? sums_in : add_peers(sums_in, row_peers)).reshape({b.R, 2}).to(at::kFloat).contiguous();
     const at::ScalarType pt = sum_type(param_type);
     Tensor dx = empty({b.R, b.C}, b.x), dgamma = empty({b.C}, b.x, pt), dbeta = empty({b.C}, b.x, pt);
-    check(lib.cw_ln_bwd_dx_close(b.R, b.C, ptr(b.dy), ld(b.dy), ptr(b.x), ld(b.x), (const float*)ptr(mean_rstd), ptr(b.gamma),
-                                 (const float*)ptr(sums), hidden, ptr(dx), ld(dx), ptr(ws), parts, ptr(dgamma), ptr(dbeta), dtype_code(pt), b.dt,
-                                 stream()),
-          "cw_ln_bwd_dx_close");
+    const Scatter sg{std::move(dgamma_peers), world, rank, gamma_type}, sb{std::move(dbeta_peers), world, rank, beta_type};
+    const bool fused = sg.fused(dgamma) && sb.fused(dbeta) && sg.peers.size() == sb.peers.size() && gamma_type == beta_type;
+    const int64_t count = fused ? sg.count(dgamma) : 0;
+    OptTensor rg, rb;
+    if (fused) {
+        rg = empty({count}, b.x, sum_type(gamma_type));
+        rb = empty({count}, b.x, gamma_type);
+    }
+    const auto tr = pointers(rows_direct ? row_peers : Peers{}), tg = pointers(fused ? sg.peers : Peers{}), tb = pointers(fused ? sb.peers : Peers{});
+    check(lib.cw_ln_bwd_dx_close_peers(b.R, b.C, ptr(b.dy), ld(b.dy), ptr(b.x), ld(b.x), (const float*)ptr(mean_rstd), ptr(b.gamma),
+                                       (const float*)ptr(sums), tr.data(), (int)tr.size(), hidden, ptr(dx), ld(dx), ptr(ws), parts, ptr(dgamma),
+                                       ptr(dbeta), dtype_code(pt), tg.data(), tb.data(), (int)tg.size(), rank * count, count, ptr(rg), ptr(rb),
+                                       fused ? dtype_code(gamma_type) : CW_F32, b.dt, stream()),
+          "cw_ln_bwd_dx_close_peers");
+    if (fused) {
+        dgamma = *rg;
+        dbeta = *rb;
+    } else if (world > 1) {
+        dgamma = sg.general(dgamma);
+        dbeta = sb.general(dbeta);
+    }
     return {dx.sizes() == x_in.sizes() ? dx : dx.reshape(x_in.sizes()), dgamma, dbeta};
 }
 
@@ -308,7 +419,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     CW_HOST_DEF(gemm_ksteps);
     CW_HOST_DEF(colsum);
     CW_HOST_DEF(act_bwd_colsum);
+    CW_HOST_DEF(colsum_scattered);
     CW_HOST_DEF(ln_partial_stats);
+    CW_HOST_DEF(ln_partial_stats_gather);
     CW_HOST_DEF(ln_forward);
     CW_HOST_DEF(ln_backward_fused);
     CW_HOST_DEF(ln_bwd_partials_open);

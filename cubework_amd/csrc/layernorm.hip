@@ -31,6 +31,43 @@ constexpr int kRowsAt2Chunks = 1;
 constexpr int kRowsAt4Chunks = 1;
 constexpr int kTileBlocksPerCu = 8;
 
+// The other ranks' pairs of the same rows ([R, 2] fp32 each), added in rank order to this rank's where they are used: an all-reduce
+// of the pairs without a launch of its own (n = 0: nothing to add).
+struct RowPeers {
+    const float* p[CW_MAX_ADDENDS];
+    int n;
+};
+__device__ __forceinline__ void row_pair(const float* __restrict__ own, const RowPeers& peers, int64_t row, float& a, float& b) {
+    a = own[2 * row];
+    b = own[2 * row + 1];
+    if (peers.n == 0) return;
+#pragma unroll
+    for (int k = 0; k < CW_MAX_ADDENDS; ++k)
+        if (k < peers.n) {
+            a += peers.p[k][2 * row];
+            b += peers.p[k][2 * row + 1];
+        }
+}
+
+// Two vectors of parameters gathered from their ranks' parts by the leading `blocks` workgroups of the statistics launch, which does
+// not read them (their concatenations were two launches of 5 us): part k, `part` elements, goes to [k * part, (k + 1) * part) of
+// out0 and out1.
+struct GatherParams {
+    const uint16_t *p0[CW_MAX_ADDENDS], *p1[CW_MAX_ADDENDS];  // as 16-bit units, `part` of them (two to an fp32 element)
+    uint16_t *out0, *out1;
+    int64_t part;
+    int blocks;
+};
+__device__ __forceinline__ void gather_params(const GatherParams& g) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, k = i / g.part;
+#pragma unroll
+    for (int n = 0; n < CW_MAX_ADDENDS; ++n)
+        if (n == k && g.p0[n] != nullptr) {
+            g.out0[i] = g.p0[n][i - k * g.part];
+            g.out1[i] = g.p1[n][i - k * g.part];
+        }
+}
+
 // Sum of (x-mu) and (x-mu)^2 over one row; every lane returns the full sums.
 template <typename T>
 __device__ __forceinline__ void row_moments(const T* __restrict__ xr, int64_t C, float mu, bool vec_ok,
@@ -68,10 +105,11 @@ __device__ __forceinline__ void row_moments(const T* __restrict__ xr, int64_t C,
 template <typename T>
 __global__ __launch_bounds__(kLnBlock) void ln_stats_kernel(int64_t R, int64_t C, const T* __restrict__ x,
                                                             int64_t ld, int mode, const float* __restrict__ mean,
-                                                            float* __restrict__ stats, int vec_ok) {
+                                                            float* __restrict__ stats, int vec_ok, const GatherParams gather) {
+    if ((int)blockIdx.x < gather.blocks) return gather_params(gather);
     const int lane = threadIdx.x & 63;
-    const int64_t wave = (int64_t)blockIdx.x * (kLnBlock / 64) + (threadIdx.x >> 6);
-    const int64_t nwaves = (int64_t)gridDim.x * (kLnBlock / 64);
+    const int64_t wave = (int64_t)((int)blockIdx.x - gather.blocks) * (kLnBlock / 64) + (threadIdx.x >> 6);
+    const int64_t nwaves = (int64_t)((int)gridDim.x - gather.blocks) * (kLnBlock / 64);
     for (int64_t row = wave; row < R; row += nwaves) {
         const float mu = (mode == CW_LN_TWO_PASS && mean != nullptr) ? mean[row] : 0.0f;
         float s1, s2;
@@ -104,7 +142,7 @@ __global__ __launch_bounds__(kLnBlock) void ln_normalize_kernel(int64_t R, int64
                                                                 const T* __restrict__ gamma,
                                                                 const T* __restrict__ beta, T* __restrict__ y,
                                                                 int64_t ldy, float* __restrict__ mean_rstd,
-                                                                int vec_ok) {
+                                                                int vec_ok, const RowPeers peers) {
     constexpr int V = elem<T>::kVec;
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)blockIdx.x * (kLnBlock / 64) + (threadIdx.x >> 6);
@@ -125,7 +163,9 @@ __global__ __launch_bounds__(kLnBlock) void ln_normalize_kernel(int64_t R, int64
                 finish_stats(mode, s1, s2, inv_h, eps, mean, rstd);
             }
         } else {
-            finish_stats(mode, stats[2 * row], stats[2 * row + 1], inv_h, eps, mean, rstd);
+            float s1, s2;
+            row_pair(stats, peers, row, s1, s2);
+            finish_stats(mode, s1, s2, inv_h, eps, mean, rstd);
         }
         if (mean_rstd != nullptr && lane == 0) {
             mean_rstd[2 * row] = mean;
@@ -266,10 +306,11 @@ template <typename T, int NCH, int NR, bool EXACT>
 __global__ __launch_bounds__(kTileWaves * 64) void ln_stats_tile_kernel(int64_t R, int64_t C,
                                                                         const T* __restrict__ x, int64_t ld, int mode,
                                                                         const float* __restrict__ mean,
-                                                                        float* __restrict__ stats) {
+                                                                        float* __restrict__ stats, const GatherParams gather) {
+    if ((int)blockIdx.x < gather.blocks) return gather_params(gather);
     const int lane = threadIdx.x & 63;
-    const int64_t wave = (int64_t)blockIdx.x * kTileWaves + (threadIdx.x >> 6);
-    const int64_t step = (int64_t)gridDim.x * kTileWaves * NR;
+    const int64_t wave = (int64_t)((int)blockIdx.x - gather.blocks) * kTileWaves + (threadIdx.x >> 6);
+    const int64_t step = (int64_t)((int)gridDim.x - gather.blocks) * kTileWaves * NR;
     const bool centred = mode == CW_LN_TWO_PASS && mean != nullptr;
     if constexpr (EXACT) {
         // plain sums (the one-pass statistics and the first exchange of the two-pass flavour): no mean to fetch
@@ -339,7 +380,7 @@ template <typename T, int NCH, int NR, bool FUSED, bool EXACT>
 __global__ __launch_bounds__(kTileWaves * 64) void ln_normalize_tile_kernel(
     int64_t R, int64_t C, const T* __restrict__ x, int64_t ld, const float* __restrict__ stats, int mode, float inv_h,
     float eps, const T* __restrict__ gamma, const T* __restrict__ beta, T* __restrict__ y, int64_t ldy,
-    float* __restrict__ mean_rstd) {
+    float* __restrict__ mean_rstd, const RowPeers peers) {
     constexpr int V = elem<T>::kVec;
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)blockIdx.x * kTileWaves + (threadIdx.x >> 6);
@@ -379,7 +420,9 @@ __global__ __launch_bounds__(kTileWaves * 64) void ln_normalize_tile_kernel(
                     finish_stats(mode, s1, s2, inv_h, eps, mean, rstd);
                 }
             } else {
-                finish_stats(mode, stats[2 * row_c], stats[2 * row_c + 1], inv_h, eps, mean, rstd);
+                float s1, s2;
+                row_pair(stats, peers, row_c, s1, s2);
+                finish_stats(mode, s1, s2, inv_h, eps, mean, rstd);
             }
             if (mean_rstd != nullptr && lane == 0 && row < R) {
                 mean_rstd[2 * row] = mean;
@@ -420,7 +463,9 @@ template <typename T, int NCH, int MAXW>
 __global__ __launch_bounds__(MAXW * 64) void ln_stats_split_kernel(int64_t R, int64_t C, const T* __restrict__ x,
                                                                    int64_t ld, int mode,
                                                                    const float* __restrict__ mean,
-                                                                   float* __restrict__ stats, int wpr) {
+                                                                   float* __restrict__ stats, int wpr,
+                                                                   const GatherParams gather) {
+    if ((int)blockIdx.x < gather.blocks) return gather_params(gather);
     constexpr int V = elem<T>::kVec;
     __shared__ float lds_sums[2][MAXW][2];  // [trip parity][wavefront][moment]
     const int lane = threadIdx.x & 63;
@@ -431,8 +476,8 @@ __global__ __launch_bounds__(MAXW * 64) void ln_stats_split_kernel(int64_t R, in
     const int64_t Cs = C - col0;
     x += col0;
     const bool centred = mode == CW_LN_TWO_PASS && mean != nullptr;
-    const int64_t step = (int64_t)gridDim.x * nrg;
-    int64_t base = (int64_t)blockIdx.x * nrg;
+    const int64_t step = (int64_t)((int)gridDim.x - gather.blocks) * nrg;
+    int64_t base = (int64_t)((int)blockIdx.x - gather.blocks) * nrg;
     RowTile<T, NCH, 1> t;
     if (base < R) t.load(x, ld, base + rg, R, Cs, lane);
     for (int trip = 0; base < R; base += step, ++trip) {
@@ -553,7 +598,7 @@ template <typename T, int NCH, int NR, bool EXACT>
 __global__ __launch_bounds__(kTileWaves * 64) void ln_bwd_dx_tile_kernel(
     int64_t R, int64_t C, const T* __restrict__ dY, int64_t ld_dy, const T* __restrict__ x, int64_t ld_x,
     const float* __restrict__ mean_rstd, const T* __restrict__ gamma, const float* __restrict__ row_sums, float inv_h,
-    T* __restrict__ dx, int64_t ld_dx, const FinishCols fin) {
+    T* __restrict__ dx, int64_t ld_dx, const FinishCols fin, const RowPeers peers) {
     constexpr int V = elem<T>::kVec;
     if (fin.blocks > 0 && (int)blockIdx.x < fin.blocks) {  // the leading workgroups finish the column sums
         __shared__ float fin_red[kTileWaves * 64];
@@ -576,7 +621,10 @@ __global__ __launch_bounds__(kTileWaves * 64) void ln_bwd_dx_tile_kernel(
             const int64_t row = row0 + r;
             const int64_t row_c = row < R ? row : R - 1;
             const float mean = mean_rstd[2 * row_c], rstd = mean_rstd[2 * row_c + 1];
-            const float c1 = row_sums[2 * row_c] * inv_h, c2 = row_sums[2 * row_c + 1] * inv_h;
+            float c1, c2;
+            row_pair(row_sums, peers, row_c, c1, c2);
+            c1 *= inv_h;
+            c2 *= inv_h;
 #pragma unroll
             for (int j = 0; j < NCH; ++j) {
                 float dy[V], xv[V], g[V];
@@ -954,7 +1002,7 @@ __global__ __launch_bounds__(kLnBlock) void ln_bwd_dx_kernel(int64_t R, int64_t 
                                                              const T* __restrict__ gamma,
                                                              const float* __restrict__ row_sums, float inv_h,
                                                              T* __restrict__ dx, int64_t ld_dx, int vec_ok,
-                                                             const FinishCols fin) {
+                                                             const FinishCols fin, const RowPeers peers) {
     constexpr int V = elem<T>::kVec;
     if (fin.blocks > 0 && (int)blockIdx.x < fin.blocks) {  // the leading workgroups finish the column sums
         __shared__ float fin_red[kLnBlock];
@@ -967,8 +1015,10 @@ __global__ __launch_bounds__(kLnBlock) void ln_bwd_dx_kernel(int64_t R, int64_t 
     for (int64_t row = wave; row < R; row += nwaves) {
         const float mean = mean_rstd[2 * row];
         const float rstd = mean_rstd[2 * row + 1];
-        const float c1 = row_sums[2 * row] * inv_h;
-        const float c2 = row_sums[2 * row + 1] * inv_h;
+        float c1, c2;
+        row_pair(row_sums, peers, row, c1, c2);
+        c1 *= inv_h;
+        c2 *= inv_h;
         const T* dyr = dY + row * ld_dy;
         const T* xr = x + row * ld_x;
         T* dxr = dx + row * ld_dx;
@@ -1041,45 +1091,54 @@ FwdSplitShape fwd_split_shape(int64_t R, int64_t nch) {
 
 template <typename T>
 int stats_impl(int64_t R, int64_t C, const void* x, int64_t ld, int mode, const float* mean, float* stats,
-               hipStream_t s) {
+               hipStream_t s, const GatherParams* params = nullptr) {
+    GatherParams gather = params != nullptr ? *params : GatherParams{};
+    // leading workgroups of `threads` threads that a launch carries for the gathering
+    auto extra = [&](int threads) {
+        if (params != nullptr) gather.blocks = (int)((C * (int64_t)(sizeof(T) / 2) + threads - 1) / threads);
+        return (unsigned)gather.blocks;
+    };
     const int vec_ok = rows_vec_ok<T>(x, ld);
     const int64_t nch = row_chunks<T>(C);
     if (vec_ok && exact_chunks<T>(C, nch) && R <= (int64_t)1 << 30) {
         return dispatch_exact<8>(nch, [&](auto nch_c, auto nr_c) {
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
-            hipLaunchKernelGGL((ln_stats_tile_kernel<T, NCH, NR, true>), dim3(exact_grid(R, NR)), dim3(kTileWaves * 64),
-                               0, s, R, C, (const T*)x, ld, mode, mean, stats);
+            const unsigned fb = extra(kTileWaves * 64);
+            hipLaunchKernelGGL((ln_stats_tile_kernel<T, NCH, NR, true>), dim3(exact_grid(R, NR) + fb), dim3(kTileWaves * 64),
+                               0, s, R, C, (const T*)x, ld, mode, mean, stats, gather);
             return check_launch("ln_stats_tile_kernel");
         });
     }
     if (vec_ok && (C % elem<T>::kVec) == 0 && nch <= 8) {
         return dispatch_tile(nch, [&](auto nch_c, auto nr_c) {
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
-            hipLaunchKernelGGL((ln_stats_tile_kernel<T, NCH, NR, false>), dim3(tile_grid(R, NR)), dim3(kTileWaves * 64),
-                               0, s, R, C, (const T*)x, ld, mode, mean, stats);
+            const unsigned fb = extra(kTileWaves * 64);
+            hipLaunchKernelGGL((ln_stats_tile_kernel<T, NCH, NR, false>), dim3(tile_grid(R, NR) + fb), dim3(kTileWaves * 64),
+                               0, s, R, C, (const T*)x, ld, mode, mean, stats, gather);
             return check_launch("ln_stats_tile_kernel");
         });
     }
     const FwdSplitShape sh = fwd_split_shape(R, nch);
     if (vec_ok && (C % elem<T>::kVec) == 0 && sh.takes) {
-        const dim3 grid((unsigned)sh.blocks), block(sh.wpr * sh.nrg * 64);
+        const dim3 grid((unsigned)sh.blocks + extra(sh.wpr * sh.nrg * 64)), block(sh.wpr * sh.nrg * 64);
         if (sh.wide)
             hipLaunchKernelGGL((ln_stats_split_kernel<T, kFwdSplitChunks, 16>), grid, block, 0, s, R, C, (const T*)x,
-                               ld, mode, mean, stats, sh.wpr);
+                               ld, mode, mean, stats, sh.wpr, gather);
         else
             hipLaunchKernelGGL((ln_stats_split_kernel<T, kFwdSplitChunks, kFwdSplitBlockWaves>), grid, block, 0, s,
-                               R, C, (const T*)x, ld, mode, mean, stats, sh.wpr);
+                               R, C, (const T*)x, ld, mode, mean, stats, sh.wpr, gather);
         return check_launch("ln_stats_split_kernel");
     }
-    hipLaunchKernelGGL(ln_stats_kernel<T>, dim3(ln_grid(R)), dim3(kLnBlock), 0, s, R, C, (const T*)x, ld, mode,
-                       mean, stats, vec_ok);
+    const unsigned fb = extra(kLnBlock);
+    hipLaunchKernelGGL(ln_stats_kernel<T>, dim3(ln_grid(R) + fb), dim3(kLnBlock), 0, s, R, C, (const T*)x, ld, mode,
+                       mean, stats, vec_ok, gather);
     return check_launch("ln_stats_kernel");
 }
 
 template <typename T, bool FUSED>
 int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float* stats, int mode, int64_t H,
                    float eps, const void* gamma, const void* beta, void* y, int64_t ldy, float* mean_rstd,
-                   hipStream_t s) {
+                   hipStream_t s, const RowPeers& peers = RowPeers{}) {
     const int vec_ok = rows_vec_ok<T>(x, ld) && rows_vec_ok<T>(y, ldy) && (gamma == nullptr || aligned16(gamma)) &&
                        (beta == nullptr || aligned16(beta));
     const int64_t nch = row_chunks<T>(C);
@@ -1093,7 +1152,7 @@ int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float*
             constexpr int NR = NCH == 2 ? 2 : decltype(nr_c)::value;
             hipLaunchKernelGGL((ln_normalize_tile_kernel<T, NCH, NR, FUSED, true>), dim3(exact_grid(R, NR)),
                                dim3(kTileWaves * 64), 0, s, R, C, (const T*)x, ld, stats, mode, 1.0f / (float)H, eps,
-                               (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd);
+                               (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd, peers);
             return check_launch("ln_normalize_tile_kernel");
         });
     }
@@ -1102,7 +1161,7 @@ int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float*
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
             hipLaunchKernelGGL((ln_normalize_tile_kernel<T, NCH, NR, FUSED, false>), dim3(tile_grid(R, NR)),
                                dim3(kTileWaves * 64), 0, s, R, C, (const T*)x, ld, stats, mode, 1.0f / (float)H, eps,
-                               (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd);
+                               (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd, peers);
             return check_launch("ln_normalize_tile_kernel");
         });
     }
@@ -1123,7 +1182,7 @@ int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float*
     }
     hipLaunchKernelGGL((ln_normalize_kernel<T, FUSED>), dim3(ln_grid(R)), dim3(kLnBlock), 0, s, R, C, (const T*)x,
                        ld, stats, mode, 1.0f / (float)H, eps, (const T*)gamma, (const T*)beta, (T*)y, ldy,
-                       mean_rstd, vec_ok);
+                       mean_rstd, vec_ok, peers);
     return check_launch("ln_normalize_kernel");
 }
 
@@ -1319,7 +1378,7 @@ int bwd_partials_impl(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const
 template <typename T>
 int bwd_dx_impl(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void* x, int64_t ld_x,
                 const float* mean_rstd, const void* gamma, const float* row_sums, int64_t H, void* dx, int64_t ld_dx,
-                hipStream_t s, const FinishCols* finish = nullptr) {
+                hipStream_t s, const FinishCols* finish = nullptr, const RowPeers& peers = RowPeers{}) {
     const int vec_ok = rows_vec_ok<T>(dY, ld_dy) && rows_vec_ok<T>(x, ld_x) && rows_vec_ok<T>(dx, ld_dx) &&
                        (gamma == nullptr || aligned16(gamma));
     const FinishCols fin = finish != nullptr ? *finish : FinishCols{};
@@ -1331,7 +1390,7 @@ int bwd_dx_impl(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void*
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
             hipLaunchKernelGGL((ln_bwd_dx_tile_kernel<T, NCH, NR, true>), dim3(exact_grid(R, NR) + fb), dim3(kTileWaves * 64),
                                0, s, R, C, (const T*)dY, ld_dy, (const T*)x, ld_x, mean_rstd, (const T*)gamma, row_sums,
-                               1.0f / (float)H, (T*)dx, ld_dx, fin);
+                               1.0f / (float)H, (T*)dx, ld_dx, fin, peers);
             return check_launch("ln_bwd_dx_tile_kernel");
         });
     }
@@ -1340,14 +1399,27 @@ int bwd_dx_impl(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void*
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
             hipLaunchKernelGGL((ln_bwd_dx_tile_kernel<T, NCH, NR, false>), dim3(tile_grid(R, NR) + fb), dim3(kTileWaves * 64),
                                0, s, R, C, (const T*)dY, ld_dy, (const T*)x, ld_x, mean_rstd, (const T*)gamma, row_sums,
-                               1.0f / (float)H, (T*)dx, ld_dx, fin);
+                               1.0f / (float)H, (T*)dx, ld_dx, fin, peers);
             return check_launch("ln_bwd_dx_tile_kernel");
         });
     }
     hipLaunchKernelGGL(ln_bwd_dx_kernel<T>, dim3(ln_grid(R) + fb), dim3(kLnBlock), 0, s, R, C, (const T*)dY, ld_dy,
                        (const T*)x, ld_x, mean_rstd, (const T*)gamma, row_sums, 1.0f / (float)H, (T*)dx, ld_dx,
-                       vec_ok, fin);
+                       vec_ok, fin, peers);
     return check_launch("ln_bwd_dx_kernel");
+}
+
+int row_peers(const char* fn, const float* const* peers, int n_peers, RowPeers* p) {
+    *p = RowPeers{};
+    if (n_peers == 0) return CW_OK;
+    if (n_peers < 0 || n_peers > CW_MAX_ADDENDS || peers == nullptr)
+        return fail(CW_ERR_INVALID, "%s: n_peers=%d outside 0..%d, or no table", fn, n_peers, CW_MAX_ADDENDS);
+    for (int k = 0; k < n_peers; ++k) {
+        p->p[k] = peers[k];
+        if (peers[k] == nullptr) return fail(CW_ERR_INVALID, "%s: peer %d is NULL", fn, k);
+    }
+    p->n = n_peers;
+    return CW_OK;
 }
 
 int check_rc(const char* fn, int64_t R, int64_t C, int io_dtype) {
@@ -1384,13 +1456,48 @@ extern "C" int cw_ln_partial_stats(int64_t R, int64_t C, const void* x, int64_t 
     });
 }
 
+extern "C" int cw_ln_partial_stats_gather(int64_t R, int64_t C, const void* x, int64_t ld, float* stats, const void* const* gamma_parts,
+                                          const void* const* beta_parts, int n_parts, void* gamma, void* beta, int io_dtype,
+                                          void* stream) {
+    int rc = check_rc("cw_ln_partial_stats_gather", R, C, io_dtype);
+    if (rc != CW_OK) return rc;
+    if (n_parts < 1 || n_parts > CW_MAX_ADDENDS || C % n_parts != 0 || C > ((int64_t)1 << 30))
+        return fail(CW_ERR_INVALID, "cw_ln_partial_stats_gather: %d parts of %lld columns", n_parts, (long long)C);
+    if (gamma_parts == nullptr || beta_parts == nullptr || gamma == nullptr || beta == nullptr)
+        return fail(CW_ERR_INVALID, "cw_ln_partial_stats_gather: null pointer");
+    GatherParams g = {};
+    for (int k = 0; k < n_parts; ++k) {
+        g.p0[k] = (const uint16_t*)gamma_parts[k];
+        g.p1[k] = (const uint16_t*)beta_parts[k];
+        if (g.p0[k] == nullptr || g.p1[k] == nullptr) return fail(CW_ERR_INVALID, "cw_ln_partial_stats_gather: part %d is NULL", k);
+    }
+    g.out0 = (uint16_t*)gamma;
+    g.out1 = (uint16_t*)beta;
+    g.part = C / n_parts * (io_dtype == CW_F32 ? 2 : 1);
+    if (R == 0) return fail(CW_ERR_UNSUPPORTED, "cw_ln_partial_stats_gather: no rows");
+    if (x == nullptr || stats == nullptr || ld < C) return fail(CW_ERR_INVALID, "cw_ln_partial_stats_gather: null pointer or ld < C");
+    if (const int drc = require_gfx950("cw_ln_partial_stats_gather"); drc != CW_OK) return drc;
+    hipStream_t s = (hipStream_t)stream;
+    return with_elem_type(io_dtype, [&](auto* tag) {
+        return stats_impl<std::remove_pointer_t<decltype(tag)>>(R, C, x, ld, CW_LN_ONE_PASS, nullptr, stats, s, &g);
+    });
+}
+
 extern "C" int cw_ln_normalize(int64_t R, int64_t C, const void* x, int64_t ld, const float* stats, int mode,
                                int64_t H, float eps, const void* gamma, const void* beta, void* y, int64_t ldy,
                                float* mean_rstd, int io_dtype, void* stream) {
+    return cw_ln_normalize_peers(R, C, x, ld, stats, nullptr, 0, mode, H, eps, gamma, beta, y, ldy, mean_rstd, io_dtype, stream);
+}
+
+extern "C" int cw_ln_normalize_peers(int64_t R, int64_t C, const void* x, int64_t ld, const float* stats, const float* const* peers,
+                                     int n_peers, int mode, int64_t H, float eps, const void* gamma, const void* beta, void* y,
+                                     int64_t ldy, float* mean_rstd, int io_dtype, void* stream) {
     int rc = check_rc("cw_ln_normalize", R, C, io_dtype);
     if (rc != CW_OK) return rc;
     if (mode != CW_LN_ONE_PASS && mode != CW_LN_TWO_PASS) return fail(CW_ERR_INVALID, "cw_ln_normalize: bad mode %d", mode);
     if (H < C) return fail(CW_ERR_INVALID, "cw_ln_normalize: hidden size H=%lld smaller than local C=%lld", (long long)H, (long long)C);
+    RowPeers rp;
+    if (const int prc = row_peers("cw_ln_normalize_peers", peers, n_peers, &rp); prc != CW_OK) return prc;
     if (R == 0) return CW_OK;
     if (x == nullptr || y == nullptr || stats == nullptr || ld < C || ldy < C)
         return fail(CW_ERR_INVALID, "cw_ln_normalize: null pointer or leading dimension < C");
@@ -1398,7 +1505,7 @@ extern "C" int cw_ln_normalize(int64_t R, int64_t C, const void* x, int64_t ld, 
     hipStream_t s = (hipStream_t)stream;
     return with_elem_type(io_dtype, [&](auto* tag) {
         return normalize_impl<std::remove_pointer_t<decltype(tag)>, false>(R, C, x, ld, stats, mode, H, eps, gamma, beta,
-                                                                           y, ldy, mean_rstd, s);
+                                                                           y, ldy, mean_rstd, s, rp);
     });
 }
 
@@ -1544,18 +1651,35 @@ extern "C" int cw_ln_bwd_dx_close(int64_t R, int64_t C, const void* dY, int64_t 
                                   const float* mean_rstd, const void* gamma, const float* row_sums, int64_t H, void* dx,
                                   int64_t ld_dx, const void* workspace, int64_t n_parts, void* dgamma, void* dbeta,
                                   int param_dtype, int io_dtype, void* stream) {
+    return cw_ln_bwd_dx_close_peers(R, C, dY, ld_dy, x, ld_x, mean_rstd, gamma, row_sums, nullptr, 0, H, dx, ld_dx, workspace, n_parts,
+                                    dgamma, dbeta, param_dtype, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, CW_F32, io_dtype, stream);
+}
+
+extern "C" int cw_ln_bwd_dx_close_peers(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void* x, int64_t ld_x,
+                                        const float* mean_rstd, const void* gamma, const float* row_sums, const float* const* row_peers_in,
+                                        int n_row_peers, int64_t H, void* dx, int64_t ld_dx, const void* workspace, int64_t n_parts,
+                                        void* dgamma, void* dbeta, int param_dtype, const float* const* dgamma_peers,
+                                        const float* const* dbeta_peers, int n_col_peers, int64_t c0, int64_t count, void* dgamma_reduced,
+                                        void* dbeta_reduced, int reduced_dtype, int io_dtype, void* stream) {
     int rc = check_rc("cw_ln_bwd_dx_close", R, C, io_dtype);
     if (rc != CW_OK) return rc;
     if (!col_out_dtype_ok(param_dtype)) return fail(CW_ERR_INVALID, "cw_ln_bwd_dx_close: bad param_dtype %d", param_dtype);
     if (H < C) return fail(CW_ERR_INVALID, "cw_ln_bwd_dx_close: hidden size H=%lld smaller than local C=%lld", (long long)H, (long long)C);
     if (dgamma == nullptr || dbeta == nullptr) return fail(CW_ERR_INVALID, "cw_ln_bwd_dx_close: dgamma and dbeta are both needed");
+    RowPeers rp;
+    if (const int prc = row_peers("cw_ln_bwd_dx_close_peers", row_peers_in, n_row_peers, &rp); prc != CW_OK) return prc;
+    PeerCols pc;
+    if (const int prc = peer_cols("cw_ln_bwd_dx_close_peers", 2, dgamma_peers, dbeta_peers, n_col_peers, C, c0, count, dgamma_reduced,
+                                  dbeta_reduced, reduced_dtype, &pc);
+        prc != CW_OK)
+        return prc;
     if (n_parts < 0 || n_parts > (1 << 20) || (n_parts > 0 && workspace == nullptr) || C > ((int64_t)1 << 30))
         return fail(CW_ERR_INVALID, "cw_ln_bwd_dx_close: bad partial count %lld, NULL workspace or C too large", (long long)n_parts);
     if (const int drc = require_gfx950("cw_ln_bwd_dx_close"); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
     if (R == 0 || n_parts == 0) {
         // no rows: the column sums are zero (the finalize kernel over zero partial rows writes them)
-        rc = finalize_col_partials(nullptr, 0, 2 * C, 2, C, dgamma, dbeta, param_dtype, s);
+        rc = finalize_col_partials(nullptr, 0, 2 * C, 2, C, dgamma, dbeta, param_dtype, s, &pc);
         if (rc != CW_OK || R == 0) return rc;
     }
     if (dY == nullptr || x == nullptr || mean_rstd == nullptr || row_sums == nullptr || dx == nullptr || ld_dy < C ||
@@ -1570,8 +1694,9 @@ extern "C" int cw_ln_bwd_dx_close(int64_t R, int64_t C, const void* dY, int64_t 
     fin.out1 = dbeta;
     fin.out_dtype = param_dtype;
     fin.blocks = n_parts > 0 ? 2 * (int)((C + 63) / 64) : 0;
+    fin.peers = pc;
     return with_elem_type(io_dtype, [&](auto* tag) {
         return bwd_dx_impl<std::remove_pointer_t<decltype(tag)>>(R, C, dY, ld_dy, x, ld_x, mean_rstd, gamma, row_sums, H, dx,
-                                                                 ld_dx, s, &fin);
+                                                                 ld_dx, s, &fin, rp);
     });
 }

@@ -52,6 +52,33 @@ __device__ __forceinline__ void block_flat_reduce(const float (&acc)[NREG], floa
     }
 }
 
+// What follows the column sums where other ranks own the rest of the reduction: their sums of the same columns, as they arrived
+// (fp32, [C] of each rank and set), are added in rank order to this rank's, and columns [c0, c0 + count) of the totals are stored in
+// the parameter's type: a reduce-scatter's addition, slicing and cast (three launches of some 4 us a vector) in the launch
+// that finishes the sums. n_peers = 0: nothing.
+struct PeerCols {
+    const float* peer[2][CW_MAX_ADDENDS];
+    int64_t c0, count;
+    void* out[2];
+    int n_peers, out_dtype;
+};
+
+// One finished column total into an output vector of the given element type.
+__device__ __forceinline__ void store_col_total(void* out, int64_t c, float total, int out_dtype) {
+    if (out_dtype == CW_F32) reinterpret_cast<float*>(out)[c] = total;
+    else if (out_dtype == CW_BF16) store_elem(reinterpret_cast<bf16_t*>(out) + c, total);
+    else store_elem(reinterpret_cast<f16_t*>(out) + c, total);
+}
+
+// Column c of set `set` (0 or 1), whose sum over this rank's rows is `total`.
+__device__ __forceinline__ void add_peer_cols(const PeerCols& p, int set, int64_t c, float total) {
+    if (p.n_peers == 0 || c < p.c0 || c >= p.c0 + p.count) return;
+#pragma unroll
+    for (int k = 0; k < CW_MAX_ADDENDS; ++k)  // constant indices: a table read with a variable one would be copied to scratch
+        if (k < p.n_peers) total += (set == 0 ? p.peer[0][k] : p.peer[1][k])[c];
+    store_col_total(set == 0 ? p.out[0] : p.out[1], c - p.c0, total, p.out_dtype);
+}
+
 // The column finalize as the leading workgroups of another launch: the first `blocks` workgroups of a kernel that
 // was handed a FinishCols add the partial rows (out_k[c] = sum_p ws[p*part_stride + k*C + c], k < 2) and return, the
 // others do the kernel's own work with their index shifted. blocks = 2 * ceil(C / 64); 0 = nothing to finish.
@@ -62,14 +89,8 @@ struct FinishCols {
     void* out1;
     int blocks;
     int out_dtype;  // CW_F32 / CW_BF16 / CW_F16: the type the totals are stored in (rounded once, to nearest even)
+    PeerCols peers;
 };
-
-// One finished column total into an output vector of the given element type.
-__device__ __forceinline__ void store_col_total(void* out, int64_t c, float total, int out_dtype) {
-    if (out_dtype == CW_F32) reinterpret_cast<float*>(out)[c] = total;
-    else if (out_dtype == CW_BF16) store_elem(reinterpret_cast<bf16_t*>(out) + c, total);
-    else store_elem(reinterpret_cast<f16_t*>(out) + c, total);
-}
 
 // Workgroup `block` (< f.blocks) of THREADS threads: 64 columns of one of the two sets. The THREADS / 64 groups
 // of 64 threads split the partial rows, 16 independent loads in flight each, and are combined in index order.
@@ -103,13 +124,19 @@ __device__ __forceinline__ void finish_cols_block(const FinishCols& f, int block
         for (int g = 1; g < G; ++g) total += red[g * 64 + lane];
         void* out = (k == 0) ? f.out0 : f.out1;
         if (out != nullptr) store_col_total(out, c, total, f.out_dtype);
+        add_peer_cols(f.peers, k, c, total);
     }
 }
 
 // out_k[c] = sum_p ws[p*part_stride + k*C + c], k < nsets (nsets is 1 or 2;
 // out1 is ignored when nsets == 1), stored as out_dtype. Enqueued on `s`.
 int finalize_col_partials(const float* ws, int64_t nparts, int64_t part_stride, int nsets, int64_t C, void* out0,
-                          void* out1, int out_dtype, hipStream_t s);
+                          void* out1, int out_dtype, hipStream_t s, const PeerCols* peers = nullptr);
+
+// Checks and collects an entry point's arguments: `sets` sets of n_peers vectors of C sums; columns [c0, c0 + count) of the totals
+// go to out0 (and out1).
+int peer_cols(const char* fn, int sets, const float* const* peers0, const float* const* peers1, int n_peers, int64_t C, int64_t c0,
+              int64_t count, void* out0, void* out1, int out_dtype, PeerCols* p);
 
 inline bool col_out_dtype_ok(int dt) { return dt == CW_F32 || dt == CW_BF16 || dt == CW_F16; }
 

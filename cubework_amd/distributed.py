@@ -145,13 +145,17 @@ def initialize(tensor_parallel: Optional[str] = None, tensor_parallel_size: int 
 # collectives: identity at world size 1, mailbox otherwise
 # (signatures of cubework/distributed/collective.py:6-97)
 # --------------------------------------------------------------------------
-def all_gather(tensor, dim, parallel_mode, async_op=False):
+def gather_parts(tensor, parallel_mode):
+    """What an all-gather delivers, every rank's tensor in rank order, for a kernel that reads the parts."""
     if parallel_mode.world_size == 1:
-        out = tensor
-    else:
-        peers = list(parallel_mode.take("all_gather"))  # world_size entries, own slot ignored
-        peers[parallel_mode.local_rank] = tensor
-        out = torch.cat(peers, dim=dim)
+        return [tensor]
+    parts = list(parallel_mode.take("all_gather"))  # world_size entries, own slot ignored
+    parts[parallel_mode.local_rank] = tensor
+    return parts
+
+
+def all_gather(tensor, dim, parallel_mode, async_op=False):
+    out = tensor if parallel_mode.world_size == 1 else torch.cat(gather_parts(tensor, parallel_mode), dim=dim)
     return (out, None) if async_op else out
 
 

@@ -18,7 +18,7 @@ import torch
 from torch import Tensor
 
 from ... import ops
-from ...distributed import ParallelMode, all_gather, all_reduce, broadcast, reduce_scatter
+from ...distributed import ParallelMode, all_gather, all_reduce, broadcast, gather_parts, reduce_scatter
 from .._amp import bwd, fp32_fwd, gemm_fwd
 from ..._lib import CW_LN_ONE_PASS
 
@@ -65,12 +65,15 @@ class _SUMMA_AB(torch.autograd.Function):
         # across ranks the fp32 sums are reduced first and rounded once afterwards
         sum_dtype = bias_dtype if has_bias and col_mode.world_size == 1 else None
         with torch.no_grad():
-            if activation is not None:
-                g, dbias = ops.act_bwd_colsum(activation, g, pre, want_dbias=has_bias, out_dtype=sum_dtype)
+            if has_bias and col_mode.world_size > 1:
+                # the launch that finishes the column sums adds the peers' and stores this rank's share
+                dpre, bias_grad = ops.colsum_scattered(g, col_mode.take("reduce_scatter"), col_mode.world_size, col_mode.local_rank,
+                                                       bias_dtype, activation, pre)
+                g = g if dpre is None else dpre
+            elif activation is not None:
+                g, bias_grad = ops.act_bwd_colsum(activation, g, pre, want_dbias=has_bias, out_dtype=sum_dtype)
             elif has_bias:
-                dbias = ops.colsum(g, out_dtype=sum_dtype)
-            if has_bias:
-                bias_grad = reduce_scatter(dbias, -1, col_mode).to(bias_dtype)
+                bias_grad = ops.colsum(g, out_dtype=sum_dtype)
             g = g.reshape(output_grad.shape)
             # operands of one type need none of the operators' casting: the products alone, without a node (12 us) each
             abt, atb = (_abt, _atb) if A.dtype == B.dtype == g.dtype else (summa_ABT, summa_ATB)
@@ -197,8 +200,12 @@ class _SUMMAbias(torch.autograd.Function):
         col_mode, skipped, bias_dtype = ctx.meta
         if skipped:
             return None, reduce_scatter(output_grad, -1, col_mode), None, None, None
-        dbias = ops.colsum(_flat(output_grad), out_dtype=bias_dtype if col_mode.world_size == 1 else None)
-        return output_grad, reduce_scatter(dbias, -1, col_mode).to(bias_dtype), None, None, None
+        if col_mode.world_size == 1:
+            dbias = ops.colsum(_flat(output_grad), out_dtype=bias_dtype)
+        else:
+            _, dbias = ops.colsum_scattered(_flat(output_grad), col_mode.take("reduce_scatter"), col_mode.world_size,
+                                            col_mode.local_rank, bias_dtype)
+        return output_grad, dbias, None, None, None
 
 
 def add_bias_2d(input_: Optional[Tensor], bias: Tensor, row_parallel_mode: ParallelMode,
@@ -216,13 +223,16 @@ class _Layernorm2D(torch.autograd.Function):
     @staticmethod
     @fp32_fwd()
     def forward(ctx, input_, weight, bias, hidden_size, eps, row_parallel_mode, col_parallel_mode, fork_residual=False):
-        gamma = all_gather(weight, -1, col_parallel_mode)
-        beta = all_gather(bias, -1, col_parallel_mode)
         if row_parallel_mode.world_size == 1:
+            gamma = all_gather(weight, -1, col_parallel_mode)
+            beta = all_gather(bias, -1, col_parallel_mode)
             out, mean_rstd = ops.ln_forward_fused(input_, eps, gamma, beta, mode=CW_LN_ONE_PASS)
         else:
-            stats = all_reduce(ops.ln_partial_stats(input_, CW_LN_ONE_PASS), row_parallel_mode)
-            out, mean_rstd = ops.ln_normalize(input_, stats, hidden_size, eps, gamma, beta, mode=CW_LN_ONE_PASS)
+            # what the exchanges deliver enters the two launches: the parameters' parts the statistics', the peers' sums the other
+            stats, gamma, beta = ops.ln_partial_stats_gather(input_, gather_parts(weight, col_parallel_mode),
+                                                             gather_parts(bias, col_parallel_mode))
+            out, mean_rstd = ops.ln_normalize(input_, stats, hidden_size, eps, gamma, beta, mode=CW_LN_ONE_PASS,
+                                              peers=row_parallel_mode.take("all_reduce"))
         ctx.save_for_backward(input_, gamma, mean_rstd)
         ctx.meta = (hidden_size, row_parallel_mode, col_parallel_mode, weight.dtype, bias.dtype)
         if fork_residual:
@@ -245,11 +255,17 @@ class _Layernorm2D(torch.autograd.Function):
                                                                   dx_addend=residual_grad)
                 residual_grad = None
             else:
-                # the dx launch also finishes the column sums that the first launch leaves as partial rows
+                # the dx launch also finishes the column sums that the first launch leaves as partial rows, and adds the peers'
                 row_sums, pending = ops.ln_bwd_partials_open(output_grad, x, mean_rstd, gamma)
-                row_sums = all_reduce(row_sums, row_mode)
-                input_grad, dgamma, dbeta = ops.ln_bwd_dx_close(output_grad, x, mean_rstd, row_sums, hidden_size, pending,
-                                                                gamma, param_dtype=pd)
+                scatter = None
+                row_peers = row_mode.take("all_reduce")
+                if col_mode.world_size > 1:
+                    scatter = (col_mode.take("reduce_scatter"), col_mode.take("reduce_scatter"), col_mode.world_size,
+                               col_mode.local_rank, w_dtype, b_dtype)
+                input_grad, dgamma, dbeta = ops.ln_bwd_dx_close(output_grad, x, mean_rstd, row_sums, hidden_size, pending, gamma,
+                                                                param_dtype=pd, row_peers=row_peers, scatter=scatter)
+                if scatter is not None:
+                    return input_grad if residual_grad is None else input_grad + residual_grad, dgamma, dbeta, None, None, None, None, None
             if residual_grad is not None:
                 input_grad = input_grad + residual_grad
             weight_grad = reduce_scatter(dgamma, -1, col_mode).to(w_dtype)

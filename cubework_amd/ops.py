@@ -154,6 +154,24 @@ def act_bwd_colsum(activation: Optional[str], dy: torch.Tensor, preact: torch.Te
     return _lib.host().act_bwd_colsum(ACTIVATIONS[activation], dy, preact, want_dbias, out_dtype)
 
 
+def _summands(own, peers):
+    """(own, peers) with the peers as tensors; staged plain numbers are added to own at once."""
+    peers = list(peers)
+    if not all(isinstance(t, torch.Tensor) for t in peers):
+        for t in peers:
+            own = own + t
+        peers = []
+    return own, peers
+
+
+def colsum_scattered(dy: torch.Tensor, peers: Sequence[torch.Tensor], world: int, rank: int, out_dtype: torch.dtype,
+                     activation: Optional[str] = None, preact: Optional[torch.Tensor] = None):
+    """Column sums of a [M,N] tensor (of dPre = dy * act'(preact) with an activation) reduce-scattered over `world` ranks, whose
+    other members' [N] sums are `peers`: (dPre or None, this rank's N / world columns of the totals as out_dtype).
+    See cw_colsum_peers."""
+    return _lib.host().colsum_scattered(dy, ACTIVATIONS[activation], preact, list(peers), world, rank, out_dtype)
+
+
 # --------------------------------------------------------------------------
 # LayerNorm
 # --------------------------------------------------------------------------
@@ -162,17 +180,24 @@ def ln_partial_stats(x: torch.Tensor, mode: int = CW_LN_ONE_PASS, mean: Optional
     return _lib.host().ln_partial_stats(x, mode, mean)
 
 
+def ln_partial_stats_gather(x: torch.Tensor, gammas: Sequence[torch.Tensor], betas: Sequence[torch.Tensor]):
+    """(one-pass statistics of x, gamma [C], beta [C]): the parameters are gathered from their ranks' parts by the launch that
+    forms the statistics. See cw_ln_partial_stats_gather."""
+    return _lib.host().ln_partial_stats_gather(x, list(gammas), list(betas))
+
+
 def ln_normalize(x: torch.Tensor, stats: torch.Tensor, hidden: int, eps: float,
                  gamma: Optional[torch.Tensor] = None, beta: Optional[torch.Tensor] = None,
-                 mode: int = CW_LN_ONE_PASS, save_mean_rstd: bool = True):
-    """y = gamma*(x-mean)*rstd+beta from whole-hidden-size stats; returns (y, mean_rstd)."""
-    return _lib.host().ln_forward(x, stats, hidden, eps, gamma, beta, mode, save_mean_rstd)
+                 mode: int = CW_LN_ONE_PASS, save_mean_rstd: bool = True, peers: Sequence[torch.Tensor] = ()):
+    """y = gamma*(x-mean)*rstd+beta from whole-hidden-size stats (stats + the peers', in order); returns (y, mean_rstd)."""
+    stats, peers = _summands(stats, peers)
+    return _lib.host().ln_forward(x, stats, peers, hidden, eps, gamma, beta, mode, save_mean_rstd)
 
 
 def ln_forward_fused(x: torch.Tensor, eps: float, gamma: Optional[torch.Tensor] = None,
                      beta: Optional[torch.Tensor] = None, mode: int = CW_LN_ONE_PASS, save_mean_rstd: bool = True):
     """LayerNorm over the last dimension when this rank holds the whole hidden size."""
-    return _lib.host().ln_forward(x, None, 0, eps, gamma, beta, mode, save_mean_rstd)
+    return _lib.host().ln_forward(x, None, [], 0, eps, gamma, beta, mode, save_mean_rstd)
 
 
 def ln_bwd_partials(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor,
@@ -226,11 +251,17 @@ def ln_bwd_partials_open(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Ten
 
 
 def ln_bwd_dx_close(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor, row_sums: torch.Tensor, hidden: int,
-                    pending, gamma: Optional[torch.Tensor] = None, param_dtype: Optional[torch.dtype] = None):
-    """(dx, dgamma [C], dbeta [C]): ln_bwd_dx whose launch also finishes the column sums that
-    ln_bwd_partials_open left pending (stored as param_dtype, default float32). See cw_ln_bwd_dx_close."""
+                    pending, gamma: Optional[torch.Tensor] = None, param_dtype: Optional[torch.dtype] = None,
+                    row_peers: Sequence[torch.Tensor] = (), scatter=None):
+    """(dx, dgamma [C], dbeta [C]): ln_bwd_dx of row_sums + the row peers' whose launch also finishes the column sums that
+    ln_bwd_partials_open left pending (stored as param_dtype, default float32). See cw_ln_bwd_dx_close.
+    scatter = (the peers' dgamma, the peers' dbeta, ranks, rank, gamma's dtype, beta's dtype): dgamma and dbeta are
+    reduce-scattered, C / ranks columns of the totals each. See cw_ln_bwd_dx_close_peers."""
     ws, n_parts = pending
-    return _lib.host().ln_bwd_dx_close(dy, x, mean_rstd, row_sums, hidden, ws, n_parts, gamma, param_dtype)
+    row_sums, row_peers = _summands(row_sums, row_peers)
+    dgammas, dbetas, *rest = scatter or ((), (), 1, 0, torch.float32, torch.float32)
+    return _lib.host().ln_bwd_dx_close(dy, x, mean_rstd, row_sums, row_peers, hidden, ws, n_parts, gamma, param_dtype,
+                                       list(dgammas), list(dbetas), *rest)
 
 
 def ln_backward_fused(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor,

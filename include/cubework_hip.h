@@ -201,6 +201,20 @@ int cw_act_bwd_colsum(int activation, int64_t M, int64_t N,
                       void* dPre, int64_t ld_dpre, void* dbias, int dbias_dtype,
                       void* workspace, int64_t workspace_bytes, int io_dtype, void* stream);
 
+/*
+ * cw_colsum and cw_act_bwd_colsum for a rank whose column sums are reduce-scattered (parallel_2d/_operation.py:287 behind :286):
+ * besides out / dbias, this rank's own sums of all N columns, the launch that finishes them adds the n_peers (<= CW_MAX_ADDENDS)
+ * other ranks' sums (fp32, [N] each, in the order given) and stores columns [c0, c0 + count) of the totals as reduced_dtype in
+ * reduced[count]: the same bits as out + peers[0] + ..., sliced and cast. n_peers == 0: as the plain entry points.
+ */
+int cw_colsum_peers(int64_t M, int64_t N, const void* dY, int64_t ld, void* out, int out_dtype, void* workspace,
+                    int64_t workspace_bytes, const float* const* peers, int n_peers, int64_t c0, int64_t count,
+                    void* reduced, int reduced_dtype, int io_dtype, void* stream);
+int cw_act_bwd_colsum_peers(int activation, int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void* preact,
+                            int64_t ld_pre, void* dPre, int64_t ld_dpre, void* dbias, int dbias_dtype, void* workspace,
+                            int64_t workspace_bytes, const float* const* peers, int n_peers, int64_t c0, int64_t count,
+                            void* reduced, int reduced_dtype, int io_dtype, void* stream);
+
 /* ---- LayerNorm ---------------------------------------------------------- */
 /*
  * Local partial statistics of x[R,C] (this rank's C of the H hidden columns).
@@ -227,6 +241,20 @@ int cw_ln_partial_stats(int64_t R, int64_t C, const void* x, int64_t ld, int mod
 int cw_ln_normalize(int64_t R, int64_t C, const void* x, int64_t ld, const float* stats,
                     int mode, int64_t H, float eps, const void* gamma, const void* beta,
                     void* y, int64_t ldy, float* mean_rstd, int io_dtype, void* stream);
+
+/*
+ * What a rank of a larger grid does around the exchanges, in the launches it has anyway:
+ *   cw_ln_partial_stats_gather: cw_ln_partial_stats (one-pass) whose launch also gathers the affine parameters from the n_parts
+ *     (<= CW_MAX_ADDENDS) ranks that hold C / n_parts of them each, into gamma[C] and beta[C] (the all-gathers of
+ *     parallel_2d/module.py:155-169). R == 0 is refused with CW_ERR_UNSUPPORTED.
+ *   cw_ln_normalize_peers: cw_ln_normalize of stats + peers[0] + ... (fp32 [R,2] each, added in that order: the bits of the
+ *     all-reduced statistics, parallel_2d/module.py:145,149). n_peers == 0: cw_ln_normalize.
+ */
+int cw_ln_partial_stats_gather(int64_t R, int64_t C, const void* x, int64_t ld, float* stats, const void* const* gamma_parts,
+                               const void* const* beta_parts, int n_parts, void* gamma, void* beta, int io_dtype, void* stream);
+int cw_ln_normalize_peers(int64_t R, int64_t C, const void* x, int64_t ld, const float* stats, const float* const* peers,
+                          int n_peers, int mode, int64_t H, float eps, const void* gamma, const void* beta, void* y,
+                          int64_t ldy, float* mean_rstd, int io_dtype, void* stream);
 
 /*
  * Statistics and normalise in one launch for the case with no peers (H == C):
@@ -276,6 +304,17 @@ int cw_ln_bwd_dx_close(int64_t R, int64_t C, const void* dY, int64_t ld_dy, cons
                        const float* mean_rstd, const void* gamma, const float* row_sums, int64_t H, void* dx,
                        int64_t ld_dx, const void* workspace, int64_t n_parts, void* dgamma, void* dbeta,
                        int param_dtype, int io_dtype, void* stream);
+/*
+ * cw_ln_bwd_dx_close of row_sums + row_peers[0] + ... (as cw_ln_normalize_peers adds), which also reduces the column sums over
+ * the ranks: besides dgamma and dbeta, this rank's own sums, columns [c0, c0 + count) of own + peers go to dgamma_reduced and
+ * dbeta_reduced as reduced_dtype (as in cw_colsum_peers).
+ */
+int cw_ln_bwd_dx_close_peers(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void* x, int64_t ld_x,
+                             const float* mean_rstd, const void* gamma, const float* row_sums, const float* const* row_peers,
+                             int n_row_peers, int64_t H, void* dx, int64_t ld_dx, const void* workspace, int64_t n_parts,
+                             void* dgamma, void* dbeta, int param_dtype, const float* const* dgamma_peers,
+                             const float* const* dbeta_peers, int n_col_peers, int64_t c0, int64_t count,
+                             void* dgamma_reduced, void* dbeta_reduced, int reduced_dtype, int io_dtype, void* stream);
 
 /*
  * cw_ln_bwd_partials + cw_ln_bwd_dx with H = C in one pass over dY and x, for rows that are complete on
