@@ -86,6 +86,10 @@ SIGNATURES = {
     "cw_vpce_fwd_local": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _int, _ptr]),
     "cw_vpce_finalize": (_int, [_i64, _int, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "cw_vpce_finalize_peers": (_int, [_i64, _int, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "cw_vpce_fwd_local_mean": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _int, _ptr]),
+    "cw_vpce_mean_workspace_bytes": (_i64, [_i64]),
+    "cw_vpce_finalize_mean": (_int, [_i64, _int, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr]),
+    "cw_vpce_bwd_mean": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _int, _int, _ptr]),
     "cw_vpce_bwd": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _f32, _ptr, _i64, _int, _int, _ptr]),
 }
 
@@ -121,7 +125,8 @@ def load():
 HOST_ENTRIES = ("cw_gemm_scratch_bytes", "cw_gemm_ksteps_ws", "cw_colsum_workspace_bytes", "cw_colsum", "cw_act_bwd_colsum",
                 "cw_colsum_peers", "cw_act_bwd_colsum_peers", "cw_ln_partial_stats", "cw_ln_partial_stats_gather",
                 "cw_ln_normalize_peers", "cw_ln_forward_fused", "cw_ln_backward_fused", "cw_ln_bwd_partials_open",
-                "cw_ln_bwd_dx_close_peers")
+                "cw_ln_bwd_dx_close_peers", "cw_vpce_fwd_local_mean", "cw_vpce_mean_workspace_bytes", "cw_vpce_finalize_mean",
+                "cw_vpce_bwd_mean")
 
 
 def host():

@@ -20,7 +20,8 @@ using OptTensor = std::optional<Tensor>;
     X(cw_gemm_scratch_bytes) X(cw_gemm_ksteps_ws) X(cw_colsum_workspace_bytes) X(cw_colsum) X(cw_act_bwd_colsum)       \
     X(cw_colsum_peers) X(cw_act_bwd_colsum_peers) X(cw_ln_partial_stats) X(cw_ln_partial_stats_gather)                 \
     X(cw_ln_normalize_peers) X(cw_ln_forward_fused) X(cw_ln_backward_fused) X(cw_ln_bwd_partials_open)                 \
-    X(cw_ln_bwd_dx_close_peers)
+    X(cw_ln_bwd_dx_close_peers) X(cw_vpce_fwd_local_mean) X(cw_vpce_mean_workspace_bytes) X(cw_vpce_finalize_mean)     \
+    X(cw_vpce_bwd_mean)
 struct Entries {
 #define X(name) decltype(&::name) name = nullptr;
     CW_HOST_ENTRIES(X)
@@ -411,6 +412,51 @@ std::tuple<Tensor, Tensor, Tensor> ln_bwd_dx_close(const Tensor& dy_in, const Te
     return {dx.sizes() == x_in.sizes() ? dx : dx.reshape(x_in.sizes()), dgamma, dbeta};
 }
 
+// Mean vocabulary-parallel loss of [T, V] logits, T >= 1: -> (loss, [2, T] global maxima and sums). peers: as ops.vpce_finalize_peers.
+std::tuple<Tensor, Tensor> vpce_mean(const Tensor& logits_in, const Tensor& targets_in, int64_t vocab_start, std::vector<Tensor> peers) {
+    const Tensor logits = rows(logits_in);
+    on_device(logits);
+    on_device(targets_in);
+    const int64_t T = logits.size(0), V = logits.size(1);
+    const Tensor targets = targets_in.reshape({-1}).to(at::kLong).contiguous();
+    TORCH_CHECK_VALUE(targets.numel() == T, "one target per logits row is required");
+    Tensor own = empty({3, T}, logits, at::kFloat), mask = bytes(T, logits), total = empty({2, T}, logits, at::kFloat);
+    Tensor loss = empty({}, logits, at::kFloat), ws = bytes(lib.cw_vpce_mean_workspace_bytes(T), logits);
+    float *f = (float*)ptr(own), *g = (float*)ptr(total);
+    uint8_t* m = (uint8_t*)ptr(mask);
+    int64_t n = 0;
+    TORCH_CHECK_VALUE(peers.empty() || peers.size() == 4, "the peers' max, sumexp, pred and mask must come from the same ranks");
+    for (size_t i = 0; i < peers.size(); ++i) {
+        on_device(peers[i]);
+        peers[i] = peers[i].to(i < 3 ? at::kFloat : at::kByte).reshape({-1, T}).contiguous();
+        n = peers[0].size(0);
+        TORCH_CHECK_VALUE(peers[i].size(0) == n, "the peers' max, sumexp, pred and mask must come from the same ranks");
+    }
+    auto peer = [&](size_t i) { return peers.empty() ? nullptr : ptr(peers[i]); };
+    check(lib.cw_vpce_fwd_local_mean(T, V, ptr(logits), ld(logits), (const int64_t*)ptr(targets), vocab_start, f, f + T, f + 2 * T, m, (int*)ptr(ws),
+                                     dtype_code(logits.scalar_type()), stream()),
+          "cw_vpce_fwd_local_mean");
+    check(lib.cw_vpce_finalize_mean(T, (int)n, f, f + T, f + 2 * T, m, (const float*)peer(0), (const float*)peer(1), (const float*)peer(2),
+                                    (const uint8_t*)peer(3), (float*)ptr(loss), g, g + T, ptr(ws), ws.numel(), stream()),
+          "cw_vpce_finalize_mean");
+    return {loss, total};
+}
+
+// Gradient of the logits, contiguous and of their type, for the gradient `dloss` of vpce_mean's loss.
+Tensor vpce_mean_bwd(const Tensor& logits_in, const Tensor& targets_in, int64_t vocab_start, const Tensor& total, const Tensor& dloss_in) {
+    const Tensor logits = rows(logits_in), targets = targets_in.reshape({-1}).to(at::kLong).contiguous(), dloss = dloss_in.to(at::kFloat);
+    on_device(logits);
+    on_device(dloss);
+    const int64_t T = logits.size(0), V = logits.size(1);
+    Tensor grad = empty({T, V}, logits);
+    const float* g = (const float*)ptr(total);
+    const int dt = dtype_code(logits.scalar_type());
+    check(lib.cw_vpce_bwd_mean(T, V, ptr(logits), ld(logits), (const int64_t*)ptr(targets), vocab_start, g, g + T, (const float*)ptr(dloss), ptr(grad),
+                               ld(grad), dt, dt, stream()),
+          "cw_vpce_bwd_mean");
+    return grad;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -426,4 +472,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     CW_HOST_DEF(ln_backward_fused);
     CW_HOST_DEF(ln_bwd_partials_open);
     CW_HOST_DEF(ln_bwd_dx_close);
+    CW_HOST_DEF(vpce_mean);
+    CW_HOST_DEF(vpce_mean_bwd);
 }

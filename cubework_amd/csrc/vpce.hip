@@ -93,7 +93,9 @@ __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int6
                                                             const T* __restrict__ logits, int64_t ld,
                                                             const int64_t* __restrict__ targets, int64_t vocab_start,
                                                             float* __restrict__ out_max, float* __restrict__ out_sumexp,
-                                                            float* __restrict__ out_pred, uint8_t* __restrict__ out_mask) {
+                                                            float* __restrict__ out_pred, uint8_t* __restrict__ out_mask,
+                                                            int* __restrict__ arrived) {
+    if (arrived != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *arrived = 0;  // for the launch behind this one (MeanOut)
     constexpr int V = elem<T>::kVec;
     __shared__ float red_m[kCeBlock / 64];
     __shared__ float red_s[kCeBlock / 64];
@@ -158,28 +160,61 @@ struct CeStats {
     const float* pred;
     const uint8_t* mask;
 };
+// The mean over the rows, finished by the launch that forms the losses: every block leaves its sum, and the one that arrives last
+// (`arrived`, zeroed by the launch of the statistics) adds the blocks' sums in block order. Behind a launch of per-row losses the
+// mean was one more (4.8 us at 8192 rows, where this takes the launch from 4.0 to 5.5 us), and its backward two autograd nodes and
+// a launch that writes dloss / T for every row (2.9 us), which the gradient kernel now reads as one scalar.
+struct MeanOut {
+    float* mean;      // nullptr: the losses of the rows are wanted
+    float* partials;  // one a block
+    int* arrived;
+};
+constexpr int kMeanBlocks = 128;  // blocks at most; each release of a partial sum costs its XCD's L2 a write-back
+
 // This rank's statistics and the peers' as they arrived, combined in that order: stacking them first took four launches
 // (14 us of the GPU at 8192 rows of 4 ranks, and as much of the host) in front of this one (5 us): the loss, forward and
 // backward, 173 -> 144 us.
 __global__ __launch_bounds__(256) void vpce_finalize_kernel(int64_t T_rows, int n_peers, const CeStats own, const CeStats peers,
                                                             float* __restrict__ loss, float* __restrict__ gmax,
-                                                            float* __restrict__ gsum) {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= T_rows) return;
-    float m = own.max[t];
-    for (int r = 0; r < n_peers; ++r) m = fmaxf(m, peers.max[(int64_t)r * T_rows + t]);
-    float s = 0.0f, p = 0.0f;
-    auto add = [&](const CeStats& st, int64_t i) {
-        const float mr = st.max[i];
-        const float f = (mr == kNegInf) ? 0.0f : expf(mr - m);
-        s += st.sumexp[i] * f;
-        if (st.mask[i] == 0) p += st.pred[i] - m;
-    };
-    add(own, t);
-    for (int r = 0; r < n_peers; ++r) add(peers, (int64_t)r * T_rows + t);
-    loss[t] = logf(s) - p;
-    if (gmax != nullptr) gmax[t] = m;
-    if (gsum != nullptr) gsum[t] = s;
+                                                            float* __restrict__ gsum, const MeanOut mean) {
+    __shared__ float red[256 / 64];
+    __shared__ int last;
+    float total = 0.0f;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < T_rows; t += (int64_t)gridDim.x * 256) {
+        float m = own.max[t];
+        for (int r = 0; r < n_peers; ++r) m = fmaxf(m, peers.max[(int64_t)r * T_rows + t]);
+        float s = 0.0f, p = 0.0f;
+        auto add = [&](const CeStats& st, int64_t i) {
+            const float mr = st.max[i];
+            const float f = (mr == kNegInf) ? 0.0f : expf(mr - m);
+            s += st.sumexp[i] * f;
+            if (st.mask[i] == 0) p += st.pred[i] - m;
+        };
+        add(own, t);
+        for (int r = 0; r < n_peers; ++r) add(peers, (int64_t)r * T_rows + t);
+        const float l = logf(s) - p;
+        total += l;
+        if (loss != nullptr) loss[t] = l;
+        if (gmax != nullptr) gmax[t] = m;
+        if (gsum != nullptr) gsum[t] = s;
+    }
+    if (mean.mean == nullptr) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    total = wave_sum(total);
+    if (lane == 0) red[wave] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float block = red[0];
+        for (int w = 1; w < 256 / 64; ++w) block += red[w];
+        __hip_atomic_store(mean.partials + blockIdx.x, block, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = __hip_atomic_fetch_add(mean.arrived, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last || wave != 0) return;
+    float sum = 0.0f;
+    for (int b = lane; b < (int)gridDim.x; b += 64) sum += __hip_atomic_load(mean.partials + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sum = wave_sum(sum);
+    if (lane == 0) *mean.mean = sum / (float)T_rows;
 }
 
 // The gradient is written once and not read again by this kernel: streaming stores.
@@ -239,6 +274,13 @@ __device__ __forceinline__ void grad_quad(raw8_t raw, int64_t i, int64_t tcol, f
     store_raw_stream_any(gr + i * 4, pack_raw(v, (const float*)nullptr));
 }
 
+// The loss's gradient: one value a row, or one for all (stride 0), times scale; no pointer: scale alone.
+struct DLoss {
+    const float* p;
+    int stride;
+    float scale;
+};
+
 // Per-row scalars of the backward: fetched after the row's first loads have been issued.
 struct CeRowScalars {
     float m2, dl, scale;
@@ -246,11 +288,10 @@ struct CeRowScalars {
 };
 __device__ __forceinline__ CeRowScalars ce_row_scalars(int64_t row, int64_t V_cols, const int64_t* __restrict__ targets,
                                                        int64_t vocab_start, const float* __restrict__ gmax,
-                                                       const float* __restrict__ gsum,
-                                                       const float* __restrict__ dloss_rows, float dloss_scale) {
+                                                       const float* __restrict__ gsum, const DLoss& dloss) {
     CeRowScalars r;
     r.m2 = gmax[row] * kLog2e;
-    r.dl = (dloss_rows != nullptr ? dloss_rows[row] : 1.0f) * dloss_scale;
+    r.dl = (dloss.p != nullptr ? dloss.p[row * dloss.stride] : 1.0f) * dloss.scale;
     r.scale = r.dl / gsum[row];
     const int64_t t = targets[row];
     const bool masked = (t < vocab_start) || (t >= vocab_start + V_cols);
@@ -264,8 +305,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                                                                const int64_t* __restrict__ targets, int64_t vocab_start,
                                                                const float* __restrict__ gmax,
                                                                const float* __restrict__ gsum,
-                                                               const float* __restrict__ dloss_rows, float dloss_scale,
-                                                               G* __restrict__ grad, int64_t ld_grad) {
+                                                               const DLoss dloss, G* __restrict__ grad, int64_t ld_grad) {
     constexpr int V = elem<T>::kVec;
     constexpr int B = kCeBwdBlock;
     const int tid = threadIdx.x;
@@ -288,7 +328,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                     const int64_t i = base + (int64_t)u * B;
                     raw[u] = __builtin_nontemporal_load(reinterpret_cast<const raw8_any_t*>(xb + (i < nq ? i : nq - 1) * 4));
                 }
-                if (base == tid) rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
+                if (base == tid) rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss);
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const int64_t i = base + (int64_t)u * B;
@@ -296,7 +336,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                 }
             }
             if (nq * 4 < V_cols) {
-                rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
+                rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss);
                 for (int64_t c = nq * 4 + tid; c < V_cols; c += B) {
                     float y = __builtin_amdgcn_exp2f(__builtin_fmaf(load_elem(xr + c), kLog2e, -rs.m2)) * rs.scale;
                     if (c == rs.tcol) y -= rs.dl;
@@ -309,7 +349,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
             if constexpr (sizeof(T) == 2) {
                 // 16-bit in, 16-bit out: one vector per thread and trip. Sixteen wavefronts per row and two rows
                 // per compute unit keep enough loads in flight; batching loads per thread measured slower here.
-                rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
+                rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss);
                 for (int64_t i = tid; i < nvec; i += B)
                     grad_vector<T, G, V>(load_raw_stream_any(xr + i * V), i, rs.tcol, rs.m2, rs.scale, rs.dl, gr);
             } else {
@@ -321,7 +361,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                         const int64_t i = base + (int64_t)u * B;
                         raw[u] = load_raw_stream_any(xr + (i < nvec ? i : nvec - 1) * V);
                     }
-                    if (base == tid) rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
+                    if (base == tid) rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss);
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
                         const int64_t i = base + (int64_t)u * B;
@@ -330,7 +370,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                 }
             }
             if (nvec * V < V_cols) {
-                rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale);
+                rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss);
                 for (int64_t c = nvec * V + tid; c < V_cols; c += B) {
                     float y = __builtin_amdgcn_exp2f(__builtin_fmaf(load_elem(xr + c), kLog2e, -rs.m2)) * rs.scale;
                     if (c == rs.tcol) y -= rs.dl;
@@ -348,11 +388,10 @@ int ce_grid(int64_t T_rows) {
 
 template <typename T, typename G>
 int bwd_impl(int64_t T_rows, int64_t V_cols, const void* logits, int64_t ld, const int64_t* targets,
-             int64_t vocab_start, const float* gmax, const float* gsum, const float* dloss_rows, float dloss_scale,
-             void* grad, int64_t ld_grad, hipStream_t s) {
+             int64_t vocab_start, const float* gmax, const float* gsum, const DLoss& dloss, void* grad, int64_t ld_grad,
+             hipStream_t s) {
     hipLaunchKernelGGL((vpce_bwd_kernel<T, G>), dim3(ce_grid(T_rows)), dim3(kCeBwdBlock), 0, s, T_rows, V_cols,
-                       (const T*)logits, ld, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale, (G*)grad,
-                       ld_grad);
+                       (const T*)logits, ld, targets, vocab_start, gmax, gsum, dloss, (G*)grad, ld_grad);
     return check_launch("vpce_bwd_kernel");
 }
 
@@ -364,6 +403,12 @@ using namespace cw;
 extern "C" int cw_vpce_fwd_local(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets,
                                  int64_t vocab_start, float* out_max, float* out_sumexp, float* out_pred,
                                  uint8_t* out_mask, int io_dtype, void* stream) {
+    return cw_vpce_fwd_local_mean(T, V, logits, ld, targets, vocab_start, out_max, out_sumexp, out_pred, out_mask, nullptr, io_dtype, stream);
+}
+
+extern "C" int cw_vpce_fwd_local_mean(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets, int64_t vocab_start,
+                                      float* out_max, float* out_sumexp, float* out_pred, uint8_t* out_mask, int* arrived, int io_dtype,
+                                      void* stream) {
     if (T < 0 || V <= 0) return fail(CW_ERR_INVALID, "cw_vpce_fwd_local: bad shape T=%lld V=%lld", (long long)T, (long long)V);
     if (io_dtype != CW_BF16 && io_dtype != CW_F32 && io_dtype != CW_F16)
         return fail(CW_ERR_INVALID, "cw_vpce_fwd_local: bad io_dtype %d", io_dtype);
@@ -377,7 +422,7 @@ extern "C" int cw_vpce_fwd_local(int64_t T, int64_t V, const void* logits, int64
     return with_elem_type(io_dtype, [&](auto* tag) {
         using E = std::remove_pointer_t<decltype(tag)>;
         hipLaunchKernelGGL(vpce_fwd_kernel<E>, dim3(ce_grid(T)), dim3(kCeBlock), 0, s, T, V, (const E*)logits, ld, targets,
-                           vocab_start, out_max, out_sumexp, out_pred, out_mask);
+                           vocab_start, out_max, out_sumexp, out_pred, out_mask, arrived);
         return check_launch("vpce_fwd_kernel");
     });
 }
@@ -404,14 +449,56 @@ extern "C" int cw_vpce_finalize_peers(int64_t T, int n_peers, const float* max, 
         return fail(CW_ERR_INVALID, "cw_vpce_finalize_peers: null pointer");
     if (const int drc = require_gfx950("cw_vpce_finalize_peers"); drc != CW_OK) return drc;
     hipLaunchKernelGGL(vpce_finalize_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, (hipStream_t)stream, T, n_peers,
-                       (CeStats{max, sumexp, pred, mask}), (CeStats{max_peers, sumexp_peers, pred_peers, mask_peers}), loss, gmax, gsum);
+                       (CeStats{max, sumexp, pred, mask}), (CeStats{max_peers, sumexp_peers, pred_peers, mask_peers}), loss, gmax, gsum, MeanOut{});
     return check_launch("vpce_finalize_kernel");
 }
+
+extern "C" int64_t cw_vpce_mean_workspace_bytes(int64_t T) {
+    const int64_t blocks = (T + 255) / 256;
+    return T <= 0 ? 0 : (1 + (blocks < kMeanBlocks ? blocks : kMeanBlocks)) * (int64_t)sizeof(float);
+}
+
+extern "C" int cw_vpce_finalize_mean(int64_t T, int n_peers, const float* max, const float* sumexp, const float* pred, const uint8_t* mask,
+                                     const float* max_peers, const float* sumexp_peers, const float* pred_peers,
+                                     const uint8_t* mask_peers, float* loss_mean, float* gmax, float* gsum, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+    if (T <= 0 || n_peers < 0) return fail(CW_ERR_INVALID, "cw_vpce_finalize_mean: bad T=%lld or n_peers=%d", (long long)T, n_peers);
+    if (max == nullptr || sumexp == nullptr || pred == nullptr || mask == nullptr || loss_mean == nullptr || workspace == nullptr ||
+        (n_peers > 0 && (max_peers == nullptr || sumexp_peers == nullptr || pred_peers == nullptr || mask_peers == nullptr)))
+        return fail(CW_ERR_INVALID, "cw_vpce_finalize_mean: null pointer");
+    const int64_t need = cw_vpce_mean_workspace_bytes(T);
+    if (workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 3u) != 0)
+        return fail(CW_ERR_INVALID, "cw_vpce_finalize_mean: workspace too small (%lld bytes) or not 4-byte aligned", (long long)workspace_bytes);
+    if (const int drc = require_gfx950("cw_vpce_finalize_mean"); drc != CW_OK) return drc;
+    hipLaunchKernelGGL(vpce_finalize_kernel, dim3((unsigned)(need / (int64_t)sizeof(float) - 1)), dim3(256), 0, (hipStream_t)stream, T, n_peers,
+                       (CeStats{max, sumexp, pred, mask}), (CeStats{max_peers, sumexp_peers, pred_peers, mask_peers}), nullptr, gmax, gsum,
+                       (MeanOut{loss_mean, (float*)workspace + 1, (int*)workspace}));
+    return check_launch("vpce_finalize_kernel (mean)");
+}
+
+static int vpce_bwd(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets, int64_t vocab_start,
+                    const float* gmax, const float* gsum, const DLoss& dloss, void* grad, int64_t ld_grad, int io_dtype,
+                    int grad_dtype, void* stream);
 
 extern "C" int cw_vpce_bwd(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets,
                            int64_t vocab_start, const float* gmax, const float* gsum, const float* dloss_rows,
                            float dloss_scale, void* grad, int64_t ld_grad, int io_dtype, int grad_dtype,
                            void* stream) {
+    return vpce_bwd(T, V, logits, ld, targets, vocab_start, gmax, gsum, DLoss{dloss_rows, 1, dloss_scale}, grad, ld_grad, io_dtype,
+                    grad_dtype, stream);
+}
+
+extern "C" int cw_vpce_bwd_mean(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets, int64_t vocab_start,
+                                const float* gmax, const float* gsum, const float* dloss, void* grad, int64_t ld_grad, int io_dtype,
+                                int grad_dtype, void* stream) {
+    if (dloss == nullptr) return fail(CW_ERR_INVALID, "cw_vpce_bwd_mean: null pointer");
+    return vpce_bwd(T, V, logits, ld, targets, vocab_start, gmax, gsum, DLoss{dloss, 0, 1.0f / (float)T}, grad, ld_grad, io_dtype,
+                    grad_dtype, stream);
+}
+
+static int vpce_bwd(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets, int64_t vocab_start,
+                    const float* gmax, const float* gsum, const DLoss& dloss, void* grad, int64_t ld_grad, int io_dtype,
+                    int grad_dtype, void* stream) {
     if (T < 0 || V <= 0) return fail(CW_ERR_INVALID, "cw_vpce_bwd: bad shape T=%lld V=%lld", (long long)T, (long long)V);
     if (io_dtype != CW_BF16 && io_dtype != CW_F32 && io_dtype != CW_F16)
         return fail(CW_ERR_INVALID, "cw_vpce_bwd: bad io_dtype %d", io_dtype);
@@ -426,12 +513,12 @@ extern "C" int cw_vpce_bwd(int64_t T, int64_t V, const void* logits, int64_t ld,
     if (const int drc = require_gfx950("cw_vpce_bwd"); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
     if (io_dtype == CW_F16 && grad_dtype == CW_F16)
-        return bwd_impl<f16_t, f16_t>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale, grad, ld_grad, s);
+        return bwd_impl<f16_t, f16_t>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss, grad, ld_grad, s);
     if (io_dtype == CW_F16)
-        return bwd_impl<f16_t, float>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale, grad, ld_grad, s);
+        return bwd_impl<f16_t, float>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss, grad, ld_grad, s);
     if (io_dtype == CW_BF16 && grad_dtype == CW_BF16)
-        return bwd_impl<bf16_t, bf16_t>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale, grad, ld_grad, s);
+        return bwd_impl<bf16_t, bf16_t>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss, grad, ld_grad, s);
     if (io_dtype == CW_BF16)
-        return bwd_impl<bf16_t, float>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale, grad, ld_grad, s);
-    return bwd_impl<float, float>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss_rows, dloss_scale, grad, ld_grad, s);
+        return bwd_impl<bf16_t, float>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss, grad, ld_grad, s);
+    return bwd_impl<float, float>(T, V, logits, ld, targets, vocab_start, gmax, gsum, dloss, grad, ld_grad, s);
 }

@@ -43,6 +43,37 @@ class _VocabParallelCrossEntropy(torch.autograd.Function):
         return grad.reshape(shape), None, None
 
 
+class _VocabParallelCrossEntropyMean(torch.autograd.Function):
+    """The loss averaged over the tokens (loss_1d.py:90-91): the launch that forms the losses finishes their mean, and the gradient
+    kernel reads the mean's gradient."""
+
+    @staticmethod
+    @loss_fwd()
+    def forward(ctx, logits, targets, parallel_mode):
+        vocab = logits.size(-1)
+        vocab_start = parallel_mode.local_rank * vocab
+        logits_2d, targets = logits.reshape(-1, vocab), targets.reshape(-1)
+        peers = () if parallel_mode.world_size == 1 else parallel_mode.take("vpce_stats")
+        loss, stats = ops.vpce_mean(logits_2d, targets, vocab_start, peers)
+        ctx.save_for_backward(logits_2d, targets, stats)
+        ctx.meta = (vocab_start, logits.shape)
+        return loss
+
+    @staticmethod
+    @bwd()
+    def backward(ctx, output_grad):
+        logits_2d, targets, stats = ctx.saved_tensors
+        vocab_start, shape = ctx.meta
+        return ops.vpce_mean_bwd(logits_2d, targets, vocab_start, stats, output_grad).reshape(shape), None, None
+
+
 def vocab_parallel_cross_entropy(logits, targets, parallel_mode):
     """Per-token loss [targets.shape] for this rank's vocabulary slice."""
     return _VocabParallelCrossEntropy.apply(logits, targets, parallel_mode)
+
+
+def vocab_parallel_cross_entropy_mean(logits, targets, parallel_mode):
+    """Mean loss over the tokens for this rank's vocabulary slice."""
+    if targets.numel() == 0:  # a mean of nothing: NaN, as torch gives it
+        return _VocabParallelCrossEntropy.apply(logits, targets, parallel_mode).mean()
+    return _VocabParallelCrossEntropyMean.apply(logits, targets, parallel_mode)

@@ -10,7 +10,7 @@ from ..parallel_2d._utils import assert_summa_initialization, reduce_by_batch_2d
 from ..parallel_3d._utils import (get_input_parallel_mode, get_output_parallel_mode, get_weight_parallel_mode,
                                   reduce_by_batch_3d, split_batch_3d)
 from ..utils import get_tensor_parallel_mode
-from ._operation import vocab_parallel_cross_entropy
+from ._operation import vocab_parallel_cross_entropy, vocab_parallel_cross_entropy_mean
 
 
 class VocabParallelCrossEntropyLoss1D(nn.Module):
@@ -19,8 +19,8 @@ class VocabParallelCrossEntropyLoss1D(nn.Module):
         self.reduction_mean = reduction
 
     def forward(self, logits, targets):
-        loss = vocab_parallel_cross_entropy(logits, targets, pm.PARALLEL_1D)
-        return loss.mean() if self.reduction_mean else loss
+        loss_of = vocab_parallel_cross_entropy_mean if self.reduction_mean else vocab_parallel_cross_entropy
+        return loss_of(logits, targets, pm.PARALLEL_1D)
 
 
 class VocabParallelCrossEntropyLoss2D(nn.Module):
@@ -33,10 +33,9 @@ class VocabParallelCrossEntropyLoss2D(nn.Module):
 
     def forward(self, logits, targets):
         targets = split_batch_2d(targets)
-        loss = vocab_parallel_cross_entropy(logits, targets, pm.PARALLEL_2D_ROW)
-        if self.reduction_mean:
-            loss = reduce_by_batch_2d(loss.mean(), True)
-        return loss
+        if not self.reduction_mean:
+            return vocab_parallel_cross_entropy(logits, targets, pm.PARALLEL_2D_ROW)
+        return reduce_by_batch_2d(vocab_parallel_cross_entropy_mean(logits, targets, pm.PARALLEL_2D_ROW), True)
 
 
 class VocabParallelCrossEntropyLoss3D(nn.Module):
@@ -50,10 +49,10 @@ class VocabParallelCrossEntropyLoss3D(nn.Module):
     def forward(self, logits, targets):
         targets = split_batch_3d(targets, input_parallel_mode=self.input_parallel_mode,
                                  weight_parallel_mode=self.weight_parallel_mode)
-        loss = vocab_parallel_cross_entropy(logits, targets, self.output_parallel_mode)
-        if self.reduction_mean:
-            loss = reduce_by_batch_3d(loss.mean(), self.input_parallel_mode, self.weight_parallel_mode, True)
-        return loss
+        if not self.reduction_mean:
+            return vocab_parallel_cross_entropy(logits, targets, self.output_parallel_mode)
+        loss = vocab_parallel_cross_entropy_mean(logits, targets, self.output_parallel_mode)
+        return reduce_by_batch_3d(loss, self.input_parallel_mode, self.weight_parallel_mode, True)
 
 
 class CrossEntropyLoss2D(nn.Module):

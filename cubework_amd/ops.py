@@ -330,6 +330,17 @@ def vpce_finalize_peers(local: Sequence[torch.Tensor], peers: Sequence[torch.Ten
     return loss, gmax, gsum
 
 
+def vpce_mean(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, peers: Sequence[torch.Tensor] = ()):
+    """(mean loss, statistics for vpce_mean_bwd) of at least one row: vpce_fwd_local, vpce_finalize(_peers) and the mean over the
+    rows. See cw_vpce_finalize_mean."""
+    return _lib.host().vpce_mean(logits, targets, vocab_start, list(peers))
+
+
+def vpce_mean_bwd(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, stats: torch.Tensor, dloss: torch.Tensor):
+    """Gradient of the logits slice for the gradient `dloss` (one value) of vpce_mean's loss."""
+    return _lib.host().vpce_mean_bwd(logits, targets, vocab_start, stats, dloss)
+
+
 def vpce_bwd(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, gmax: torch.Tensor, gsum: torch.Tensor,
              dloss_rows: Optional[torch.Tensor] = None, dloss_scale: float = 1.0,
              grad_dtype: Optional[torch.dtype] = None, aligned_rows: bool = False) -> torch.Tensor:

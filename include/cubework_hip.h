@@ -376,6 +376,25 @@ int cw_vpce_bwd(int64_t T, int64_t V, const void* logits, int64_t ld,
                 const float* gmax, const float* gsum,
                 const float* dloss_rows, float dloss_scale,
                 void* grad, int64_t ld_grad, int io_dtype, int grad_dtype, void* stream);
+/*
+ * The same for a loss that is averaged over the T rows (`loss.mean()`, cubework/module/loss/loss_1d.py:90-91), T >= 1:
+ *   cw_vpce_fwd_local_mean: cw_vpce_fwd_local that also zeroes *arrived (may be NULL): the first 4 bytes of the workspace that
+ *     cw_vpce_finalize_mean is given next on the same stream;
+ *   cw_vpce_finalize_mean: cw_vpce_finalize_peers with the rows' mean (fp32, added in a fixed order) in place of their losses, in
+ *     one launch; workspace of cw_vpce_mean_workspace_bytes(T) bytes, 4-byte aligned;
+ *   cw_vpce_bwd_mean: cw_vpce_bwd with the gradient of the mean, one fp32 on the device; every row's is dloss[0] / T.
+ */
+int cw_vpce_fwd_local_mean(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets, int64_t vocab_start,
+                           float* out_max, float* out_sumexp, float* out_pred, uint8_t* out_mask, int* arrived, int io_dtype,
+                           void* stream);
+int64_t cw_vpce_mean_workspace_bytes(int64_t T);
+int cw_vpce_finalize_mean(int64_t T, int n_peers, const float* max, const float* sumexp, const float* pred, const uint8_t* mask,
+                          const float* max_peers, const float* sumexp_peers, const float* pred_peers, const uint8_t* mask_peers,
+                          float* loss_mean, float* gmax, float* gsum, void* workspace, int64_t workspace_bytes, void* stream);
+int cw_vpce_bwd_mean(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets, int64_t vocab_start,
+                     const float* gmax, const float* gsum, const float* dloss, void* grad, int64_t ld_grad, int io_dtype,
+                     int grad_dtype, void* stream);
+
 
 /* ---- vocab-parallel embedding -------------------------------------------- */
 /*
