@@ -74,6 +74,66 @@ __global__ __launch_bounds__(kColWaves * 64) void colsum_vec_kernel(
     }
 }
 
+// Few rows: one launch that finishes the sums. A block of 16 wavefronts owns 16 vectors of columns (256 bytes of a row, whole
+// lines) and walks over all rows, 64 at a time: a wavefront's four groups of 16 lanes read four of them.
+constexpr int kShortWaves = 16, kShortLanes = 16;
+template <typename T, int MODE, int ACT>
+__global__ __launch_bounds__(kShortWaves * 64) void colsum_short_kernel(int M, int64_t N, const T* __restrict__ dY, int64_t ld_dy,
+                                                                        const T* __restrict__ pre, int64_t ld_pre, T* __restrict__ dPre,
+                                                                        int64_t ld_dpre, void* __restrict__ out, int out_dtype,
+                                                                        const PeerCols peers) {
+    constexpr int V = elem<T>::kVec, U = MODE == 0 ? 4 : 2, kRows = kShortWaves * 64 / kShortLanes, kCols = kShortLanes * V;
+    __shared__ float red[kShortWaves][kCols];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lc = lane % kShortLanes, lr = lane / kShortLanes;
+    const int64_t c0 = (int64_t)blockIdx.x * kCols + lc * V;
+    const bool valid = c0 < N;
+    const int64_t c = valid ? c0 : 0;  // no load under a branch: what is outside is read elsewhere and dropped
+    float acc[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] = 0.0f;
+    for (int base = wave * (64 / kShortLanes); base < M; base += kRows * U) {
+        raw16_t d_raw[U], p_raw[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int rr = base + lr + u * kRows;
+            const int64_t rc = rr < M ? rr : M - 1;
+            d_raw[u] = load_raw_stream(dY + rc * ld_dy + c);
+            if constexpr (MODE == 1) p_raw[u] = load_raw_stream(pre + rc * ld_pre + c);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int rr = base + lr + u * kRows;
+            const bool live = rr < M && valid;
+            float dy[V];
+            unpack_raw(d_raw[u], dy, (const T*)nullptr);
+            if constexpr (MODE == 1) {
+                float p[V];
+                unpack_raw(p_raw[u], p, (const T*)nullptr);
+#pragma unroll
+                for (int e = 0; e < V; ++e) dy[e] *= act_grad_of<ACT>(p[e]);
+                if (live) store_raw_stream(dPre + rr * ld_dpre + c, pack_raw(dy, (const T*)nullptr));
+            }
+#pragma unroll
+            for (int e = 0; e < V; ++e) acc[e] += live ? dy[e] : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+#pragma unroll
+        for (int off = kShortLanes; off < 64; off <<= 1) acc[e] += __shfl_xor(acc[e], off, 64);
+        if (lr == 0) red[wave][lc * V + e] = acc[e];
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    const int64_t col = (int64_t)blockIdx.x * kCols + t;
+    if (t >= kCols || col >= N) return;
+    float total = red[0][t];
+#pragma unroll
+    for (int w = 1; w < kShortWaves; ++w) total += red[w][t];
+    store_col_total(out, col, total, out_dtype);
+    add_peer_cols(peers, 0, col, total);
+}
+
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) void colsum_generic_kernel(int64_t M, int64_t N, const T* __restrict__ dY,
                                                              int64_t ld_dy, const T* __restrict__ pre,
@@ -137,6 +197,12 @@ __global__ __launch_bounds__(kFinGroups * 64) void finalize_cols_kernel(const fl
     }
 }
 
+// Up to here one launch of few blocks takes less time than one that fills the chip and the finalize behind it (us, one launch / two,
+// in a graph, bf16): sums of 128 x 2304 3.3 / 5.3, 256 x 4096 4.0 / 6.2, 512 x 768 4.7 / 5.8, 512 x 12288 6.1 / 8.1, from 777 rows on
+// the two are the faster ones at small widths (777 x 768 6.3 / 6.0); with an activation's derivative, which reads and writes three
+// times as much, 128 x 768 3.7 / 5.7, 256 x 768 6.8 / 6.8, 256 x 12288 8.7 / 9.7, 512 x 2304 12.3 / 7.5.
+constexpr int64_t kShortRows = 512, kShortRowsAct = 256;
+
 template <typename T, int MODE>
 int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void* pre, int64_t ld_pre, void* dPre,
                 int64_t ld_dpre, int act, void* out, int out_dtype, void* workspace, int64_t workspace_bytes,
@@ -146,6 +212,20 @@ int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void*
     bool vec = aligned16(dY) && (ld_dy % V) == 0 && (N % V) == 0;
     if (MODE == 1) vec = vec && aligned16(pre) && (ld_pre % V) == 0 && aligned16(dPre) && (ld_dpre % V) == 0;
     int64_t slabs, rows_per_slab;
+    const auto with_act = [&](auto&& launch) {
+        if (MODE == 0 || act == CW_ACT_NONE) launch(std::integral_constant<int, CW_ACT_NONE>{});
+        else if (act == CW_ACT_GELU_TANH) launch(std::integral_constant<int, CW_ACT_GELU_TANH>{});
+        else if (act == CW_ACT_GELU_ERF) launch(std::integral_constant<int, CW_ACT_GELU_ERF>{});
+        else launch(std::integral_constant<int, CW_ACT_RELU>{});
+    };
+    if (vec && want_sum && M <= (MODE == 0 ? kShortRows : kShortRowsAct)) {
+        with_act([&](auto act_c) {
+            hipLaunchKernelGGL((colsum_short_kernel<T, MODE, decltype(act_c)::value>), dim3((unsigned)((N + kShortLanes * V - 1) / (kShortLanes * V))),
+                               dim3(kShortWaves * 64), 0, s, (int)M, N, (const T*)dY, ld_dy, (const T*)pre, ld_pre, (T*)dPre, ld_dpre, out, out_dtype,
+                               peers != nullptr ? *peers : PeerCols{});
+        });
+        return check_launch("colsum_short_kernel");
+    }
     if (vec) {
         const int64_t coltiles = (N + 64 * V - 1) / (64 * V);
         colsum_plan(M, N, V, true, slabs, rows_per_slab);
@@ -153,15 +233,11 @@ int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void*
             return fail(CW_ERR_INVALID, "column sum: workspace too small (%lld bytes)", (long long)workspace_bytes);
         const size_t lds = tree_reduce_lds_bytes(V, kColWaves);
         const dim3 grid((unsigned)coltiles, (unsigned)slabs), block(kColWaves * 64);
-        auto launch = [&](auto act_c) {
+        with_act([&](auto act_c) {
             constexpr int ACT = decltype(act_c)::value;
             hipLaunchKernelGGL((colsum_vec_kernel<T, MODE, ACT>), grid, block, lds, s, M, N, (const T*)dY, ld_dy,
                                (const T*)pre, ld_pre, (T*)dPre, ld_dpre, (float*)workspace, rows_per_slab, want_sum);
-        };
-        if (MODE == 0 || act == CW_ACT_NONE) launch(std::integral_constant<int, CW_ACT_NONE>{});
-        else if (act == CW_ACT_GELU_TANH) launch(std::integral_constant<int, CW_ACT_GELU_TANH>{});
-        else if (act == CW_ACT_GELU_ERF) launch(std::integral_constant<int, CW_ACT_GELU_ERF>{});
-        else launch(std::integral_constant<int, CW_ACT_RELU>{});
+        });
     } else {
         colsum_plan(M, N, V, false, slabs, rows_per_slab);
         if (want_sum && workspace_bytes < slabs * N * (int64_t)sizeof(float))
