@@ -126,11 +126,13 @@ HOST_ENTRIES = ("cw_gemm_scratch_bytes", "cw_gemm_ksteps_ws", "cw_colsum_workspa
                 "cw_colsum_peers", "cw_act_bwd_colsum_peers", "cw_ln_partial_stats", "cw_ln_partial_stats_gather",
                 "cw_ln_normalize_peers", "cw_ln_forward_fused", "cw_ln_backward_fused", "cw_ln_bwd_partials_open",
                 "cw_ln_bwd_dx_close_peers", "cw_vpce_fwd_local_mean", "cw_vpce_mean_workspace_bytes", "cw_vpce_finalize_mean",
-                "cw_vpce_bwd_mean")
+                "cw_vpce_bwd_mean", "cw_attn_fwd", "cw_attn_narrow_fwd", "cw_attn_bwd", "cw_attn_narrow_bwd",
+                "cw_attn_bwd_workspace_bytes", "cw_embed_fwd", "cw_embed_bwd_ids_supported", "cw_embed_bwd_ids",
+                "cw_embed_sort_workspace_bytes", "cw_embed_sort_ids", "cw_embed_bwd")
 
 
 def host():
-    """The native operator calls, bound to the loaded library (once)."""
+    """The native operator calls and autograd nodes, bound to the loaded library (once)."""
     global _host
     if _host is None:
         lib = load()

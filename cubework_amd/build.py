@@ -28,7 +28,7 @@ DIAG_SOURCES = ["diag_gemm.hip", "diag.hip"]
 DIAG_LIB_PATH = os.path.join(HERE, "libcubework_diag.so")
 
 # the operators' native host side: a Python extension on torch's C++ API
-HOST_SOURCE = "host_ops.cpp"
+HOST_SOURCES = ["host_ops.cpp", "host_nodes.cpp"]
 HOST_PATH = os.path.join(HERE, "_host.so")
 
 # Packed-fp32 VALU forms are kept off: plain float code only.
@@ -70,14 +70,20 @@ def build_host(verbose=True):
     include = [os.path.join(os.path.dirname(HERE), "include"), os.path.join(root, "include"),
                os.path.join(root, "include", "torch", "csrc", "api", "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
     tmp = HOST_PATH + ".tmp"
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
-           "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H", "-DTORCH_EXTENSION_NAME=_host",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, *["-I" + d for d in include],
-           os.path.join(CSRC, HOST_SOURCE), "-o", tmp, "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
-           "-ltorch_python"]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError("host extension failed:\n%s\n%s" % (proc.stdout, proc.stderr))
+    cxx = [os.environ.get("CXX", "g++")]
+    flags = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+             "-DTORCH_EXTENSION_NAME=_host", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, *["-I" + d for d in include]]
+    objs = [os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".host.o") for src in HOST_SOURCES]
+
+    def run(cmd):
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError("host extension failed:\n%s\n%s" % (proc.stdout, proc.stderr))
+
+    os.makedirs(OBJ_DIR, exist_ok=True)
+    with ThreadPoolExecutor(len(HOST_SOURCES)) as pool:
+        list(pool.map(lambda pair: run([*cxx, *flags, "-c", os.path.join(CSRC, pair[0]), "-o", pair[1]]), zip(HOST_SOURCES, objs)))
+    run([*cxx, "-shared", *objs, "-o", tmp, "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python"])
     os.replace(tmp, HOST_PATH)
     if verbose:
         print("built", HOST_PATH, os.path.getsize(HOST_PATH), "bytes")

@@ -5,28 +5,13 @@
 // The entry points' addresses come from the library that cubework_amd._lib loaded (bind), so a measurement build selected
 // there is the one that runs. Calls run without the interpreter lock. Errors: ValueError, TypeError and RuntimeError as
 // the Python wrappers document, CubeworkHipError (raised by cubework_amd._lib.check) for a status of the library.
-#include <torch/extension.h>
+#include "host_ops.h"
 
 #include <c10/hip/HIPStream.h>
 
-#include "cubework_hip.h"
+namespace cw_host {
 
-namespace {
-
-using at::Tensor;
-using OptTensor = std::optional<Tensor>;
-
-#define CW_HOST_ENTRIES(X)                                                                                             \
-    X(cw_gemm_scratch_bytes) X(cw_gemm_ksteps_ws) X(cw_colsum_workspace_bytes) X(cw_colsum) X(cw_act_bwd_colsum)       \
-    X(cw_colsum_peers) X(cw_act_bwd_colsum_peers) X(cw_ln_partial_stats) X(cw_ln_partial_stats_gather)                 \
-    X(cw_ln_normalize_peers) X(cw_ln_forward_fused) X(cw_ln_backward_fused) X(cw_ln_bwd_partials_open)                 \
-    X(cw_ln_bwd_dx_close_peers) X(cw_vpce_fwd_local_mean) X(cw_vpce_mean_workspace_bytes) X(cw_vpce_finalize_mean)     \
-    X(cw_vpce_bwd_mean)
-struct Entries {
-#define X(name) decltype(&::name) name = nullptr;
-    CW_HOST_ENTRIES(X)
-#undef X
-} lib;
+Entries lib;
 
 void bind(const std::map<std::string, uintptr_t>& addresses) {
 #define X(name) lib.name = reinterpret_cast<decltype(lib.name)>(addresses.at(#name));
@@ -61,7 +46,6 @@ void on_device(const OptTensor& t) {
     if (t) on_device(*t);
 }
 
-// View as [rows, cols] with unit column stride (copy only if unavoidable).
 Tensor rows(const Tensor& t) {
     Tensor r = t.dim() == 2 ? t : t.reshape({-1, t.size(-1)});
     if (r.stride(1) != 1 || (r.size(0) > 1 && r.stride(0) < r.size(1))) r = r.contiguous();
@@ -69,13 +53,8 @@ Tensor rows(const Tensor& t) {
 }
 int64_t ld(const Tensor& t) { return t.size(0) > 1 ? t.stride(0) : std::max<int64_t>(t.size(1), 1); }
 int64_t ld(const OptTensor& t) { return t ? ld(*t) : 0; }
-void* ptr(const Tensor& t) { return t.data_ptr(); }
 void* ptr(const OptTensor& t) { return t ? t->data_ptr() : nullptr; }
-bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
-Tensor empty(at::IntArrayRef shape, const Tensor& like, at::ScalarType t) { return at::empty(shape, like.options().dtype(t)); }
-Tensor empty(at::IntArrayRef shape, const Tensor& like) { return at::empty(shape, like.options()); }
-Tensor bytes(int64_t n, const Tensor& like) { return empty({n}, like, at::kByte); }
 OptTensor vec(const OptTensor& t, at::ScalarType type) {
     if (!t) return t;
     return t->to(type).contiguous();
@@ -457,7 +436,9 @@ Tensor vpce_mean_bwd(const Tensor& logits_in, const Tensor& targets_in, int64_t 
     return grad;
 }
 
-}  // namespace
+}  // namespace cw_host
+
+using namespace cw_host;
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("bind", &bind);
@@ -474,4 +455,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     CW_HOST_DEF(ln_bwd_dx_close);
     CW_HOST_DEF(vpce_mean);
     CW_HOST_DEF(vpce_mean_bwd);
+    def_nodes(m);
 }

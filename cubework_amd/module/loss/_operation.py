@@ -49,11 +49,8 @@ class _VocabParallelCrossEntropyMean(torch.autograd.Function):
 
     @staticmethod
     @loss_fwd()
-    def forward(ctx, logits, targets, parallel_mode):
-        vocab = logits.size(-1)
-        vocab_start = parallel_mode.local_rank * vocab
-        logits_2d, targets = logits.reshape(-1, vocab), targets.reshape(-1)
-        peers = () if parallel_mode.world_size == 1 else parallel_mode.take("vpce_stats")
+    def forward(ctx, logits, targets, vocab_start, peers):
+        logits_2d, targets = logits.reshape(-1, logits.size(-1)), targets.reshape(-1)
         loss, stats = ops.vpce_mean(logits_2d, targets, vocab_start, peers)
         ctx.save_for_backward(logits_2d, targets, stats)
         ctx.meta = (vocab_start, logits.shape)
@@ -64,7 +61,7 @@ class _VocabParallelCrossEntropyMean(torch.autograd.Function):
     def backward(ctx, output_grad):
         logits_2d, targets, stats = ctx.saved_tensors
         vocab_start, shape = ctx.meta
-        return ops.vpce_mean_bwd(logits_2d, targets, vocab_start, stats, output_grad).reshape(shape), None, None
+        return ops.vpce_mean_bwd(logits_2d, targets, vocab_start, stats, output_grad).reshape(shape), None, None, None
 
 
 def vocab_parallel_cross_entropy(logits, targets, parallel_mode):
@@ -76,4 +73,7 @@ def vocab_parallel_cross_entropy_mean(logits, targets, parallel_mode):
     """Mean loss over the tokens for this rank's vocabulary slice."""
     if targets.numel() == 0:  # a mean of nothing: NaN, as torch gives it
         return _VocabParallelCrossEntropy.apply(logits, targets, parallel_mode).mean()
-    return _VocabParallelCrossEntropyMean.apply(logits, targets, parallel_mode)
+    vocab_start = parallel_mode.local_rank * logits.size(-1)
+    peers = () if parallel_mode.world_size == 1 else parallel_mode.take("vpce_stats")
+    loss = ops.mean_loss(logits, targets, vocab_start, peers)
+    return _VocabParallelCrossEntropyMean.apply(logits, targets, vocab_start, peers) if loss is None else loss

@@ -62,7 +62,8 @@ class _LinearNT(torch.autograd.Function):
 def linear_nt(input_: Tensor, weight: Tensor, bias: Optional[Tensor] = None,
               activation: Optional[str] = None) -> Tensor:
     """F.linear(input_, weight, bias) (+ fused activation) on the HIP path."""
-    return _LinearNT.apply(input_, weight, bias, activation)
+    out = ops.linear("NT", input_, weight, bias, activation)
+    return _LinearNT.apply(input_, weight, bias, activation) if out is None else out
 
 
 class _ReduceGrad(torch.autograd.Function):
@@ -110,6 +111,8 @@ class _GatherForwardSplitBackward(torch.autograd.Function):
 
 
 def reduce_grad(input_, parallel_mode):
+    if parallel_mode.world_size == 1:
+        return input_
     return _ReduceGrad.apply(input_, parallel_mode)
 
 

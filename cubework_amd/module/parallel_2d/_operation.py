@@ -86,13 +86,17 @@ class _SUMMA_AB(torch.autograd.Function):
 def summa_AB(A: Tensor, B: Tensor, summa_dim: int, out_shape: Tuple[int, ...], row_parallel_mode: ParallelMode,
              col_parallel_mode: ParallelMode) -> Tensor:
     """Reference signature (_operation.py:83-91)."""
-    return _SUMMA_AB.apply(A, B, None, summa_dim, out_shape, row_parallel_mode, col_parallel_mode, None, None)
+    return summa_AB_bias_act(A, B, None, summa_dim, out_shape, row_parallel_mode, col_parallel_mode)
 
 
 def summa_AB_bias_act(A: Tensor, B: Tensor, bias: Optional[Tensor], summa_dim: int, out_shape: Tuple[int, ...],
                       row_parallel_mode: ParallelMode, col_parallel_mode: ParallelMode,
                       activation: Optional[str] = None, residual: Optional[Tensor] = None) -> Tensor:
     """summa_AB + add_bias_2d (+ activation, or + a residual of the output's shape) in one kernel."""
+    if summa_dim == row_parallel_mode.world_size == col_parallel_mode.world_size == 1 and out_shape == A.shape[:-1] + (B.shape[-1],):
+        out = ops.linear("NN", A, B, bias, activation, residual)
+        if out is not None:
+            return out
     return _SUMMA_AB.apply(A, B, bias, summa_dim, out_shape, row_parallel_mode, col_parallel_mode, activation, residual)
 
 
@@ -276,6 +280,10 @@ class _Layernorm2D(torch.autograd.Function):
 def layernorm_2d(input_: Tensor, weight: Tensor, bias: Tensor, hidden_size: int, eps: float,
                  row_parallel_mode: ParallelMode, col_parallel_mode: ParallelMode, fork_residual: bool = False):
     """fork_residual (additive option, default off): returns (normalised, input) - see _Layernorm2D.forward."""
+    if row_parallel_mode.world_size == col_parallel_mode.world_size == 1:
+        out = ops.layernorm(input_, weight, bias, eps, fork_residual)
+        if out is not None:
+            return out
     return _Layernorm2D.apply(input_, weight, bias, hidden_size, eps, row_parallel_mode, col_parallel_mode, fork_residual)
 
 

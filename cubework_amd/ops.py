@@ -90,6 +90,13 @@ def _ptr_table(tensors: Sequence[torch.Tensor]):
 # --------------------------------------------------------------------------
 # block GEMM
 # --------------------------------------------------------------------------
+def linear(layout: str, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+           activation: Optional[str] = None, residual: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """act(x W + bias) + residual as a native autograd node, W [in, out] ("NN") or [out, in] ("NT"); None for a call that is not
+    an ordinary one (csrc/host_nodes.cpp says which), which the caller's own node takes."""
+    return _lib.host().linear(x, weight, bias, residual, LAYOUTS[layout], ACTIVATIONS[activation])
+
+
 def gemm_ksteps(layout: str, A_steps: Sequence[torch.Tensor], B_steps: Sequence[torch.Tensor],
                 bias: Optional[torch.Tensor] = None, activation: Optional[str] = None,
                 addends: Sequence[torch.Tensor] = (), want_preact: bool = False,
@@ -178,6 +185,12 @@ def colsum_scattered(dy: torch.Tensor, peers: Sequence[torch.Tensor], world: int
 def ln_partial_stats(x: torch.Tensor, mode: int = CW_LN_ONE_PASS, mean: Optional[torch.Tensor] = None) -> torch.Tensor:
     """[R,2] fp32 partial statistics of the local columns of x [R,C]."""
     return _lib.host().ln_partial_stats(x, mode, mean)
+
+
+def layernorm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: float, fork_residual: bool = False):
+    """One-pass LayerNorm over whole rows as a native autograd node (with fork_residual: and x again, for a residual branch); None
+    as linear."""
+    return _lib.host().layernorm(x, weight, bias, eps, fork_residual)
 
 
 def ln_partial_stats_gather(x: torch.Tensor, gammas: Sequence[torch.Tensor], betas: Sequence[torch.Tensor]):
@@ -328,6 +341,11 @@ def vpce_finalize_peers(local: Sequence[torch.Tensor], peers: Sequence[torch.Ten
     rc = lib.cw_vpce_finalize_peers(T, n, *map(_p, local), *map(_p, peers), _p(loss), _p(gmax), _p(gsum), _stream())
     _lib.check(rc, "cw_vpce_finalize_peers")
     return loss, gmax, gsum
+
+
+def mean_loss(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, peers: Sequence[torch.Tensor] = ()):
+    """vpce_mean's loss as a native autograd node; None as linear."""
+    return _lib.host().mean_loss(logits, targets, vocab_start, list(peers))
 
 
 def vpce_mean(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, peers: Sequence[torch.Tensor] = ()):
@@ -498,7 +516,8 @@ class _AttentionCore(torch.autograd.Function):
 
 def attention_core(qkv: torch.Tensor, heads: int, scale: Optional[float] = None, causal: bool = True) -> torch.Tensor:
     """Differentiable fused attention core on the qkv projection's output."""
-    return _AttentionCore.apply(qkv, heads, scale, causal)
+    out = _lib.host().attention(qkv, heads, scale, causal)
+    return _AttentionCore.apply(qkv, heads, scale, causal) if out is None else out
 
 
 # --------------------------------------------------------------------------
@@ -591,5 +610,6 @@ def vocab_embedding(ids: torch.Tensor, weight: torch.Tensor, vocab_start: int = 
                     padding_idx: Optional[int] = None) -> torch.Tensor:
     """Differentiable masked embedding lookup of one vocabulary slice. padding_idx is the row of `weight`
     that receives no gradient (what F.embedding's padding_idx means for the tensor it is handed)."""
-    skip = -1 if padding_idx is None else int(padding_idx)
-    return _VocabEmbedding.apply(ids, weight, int(vocab_start), skip)
+    skip, vocab_start = -1 if padding_idx is None else int(padding_idx), int(vocab_start)
+    out = _lib.host().embedding(ids, weight, vocab_start, skip)
+    return _VocabEmbedding.apply(ids, weight, vocab_start, skip) if out is None else out
