@@ -13,8 +13,11 @@
 //     (partial sums through scratch in accumulator order, finished by tile_reduce_kernel): the last, partly empty
 //     round of tiles, or a problem with few tiles and a long reduction, is spread over the whole chip.
 //
-// LDS images per stage: k-contiguous operand [BM rows][32 k], chunk c of row r at c ^ ((r >> 2) & 3);
-// k-slow operand [32 k][BM rows], chunk c of k row k at c ^ ((k & 3) << 2). Both read conflict free.
+// LDS images per stage: k-contiguous operand [BM rows][32 k], chunk c of row r at c ^ ((r >> 2) & 3), or, where a trip is 64 k,
+// [BM rows][64 k], chunk c of row r at c ^ ((r >> 1) & 7); k-slow operand [32 k][BM rows], chunk c of k row k at c ^ ((k & 3) << 2),
+// one image per 32 k. All read conflict free.
+// Rows of 64 k are whole 128-byte lines: a load instruction of 8 of them takes the load unit 17 cycles, one of 16 pieces of 64 bytes
+// (two images of 32 k a trip, as before) 35, and that bounded the small tiles: 16 such instructions a trip of a 64 x 64 NT tile.
 #pragma once
 #include <cstddef>
 
@@ -71,17 +74,26 @@ __device__ __forceinline__ int kslow_swizzle(int k) {
     return W == 1 ? (k >> 1) & 1 : k & 3;
 }
 
-// Loader of one operand: W MFMA tiles per wavefront, 64 W rows per block, W load instructions per wavefront and k tile.
-template <bool TRANS, int W>
+// Loader of one operand: W MFMA tiles per wavefront, 64 W rows per block, W load instructions per wavefront and 32 k of a trip of KB.
+template <bool TRANS, int W, int KB>
 struct Loader {
     static constexpr int kRows = 64 * W;
-    static constexpr int kBytes = kRows * kBK * 2;
+    static constexpr int kImage = kRows * kBK * 2, kBytes = KB * kImage;  // of 32 k, of a trip
     static constexpr int kKPer = 1024 / (kRows * 2);  // TRANS: k rows per instruction
-    uint32_t voff[W];
-    int klane;  // !TRANS: first k of the lane's chunk; TRANS: the lane's k row in instruction 0
+    static constexpr bool kLines = !TRANS && KB == 2;  // rows of 64 k
+    static constexpr int kOffsets = kLines ? 2 * W : W;
+    static_assert(KB == 1 || KB == 2, "");
+    uint32_t voff[kOffsets];
+    int klane;  // !TRANS: first k of the lane's chunk (of instruction 0); TRANS: the lane's k row in instruction 0
     // row0: first operand row of the block; rmax: rows of the operand
     __device__ __forceinline__ void init(int lane, int wave, int64_t ld, int row0, int rmax) {
-        if constexpr (!TRANS) {
+        if constexpr (kLines) {
+            const int r = wave * 16 * W + (lane >> 3), c = (lane & 7) ^ (lane >> 4);
+            klane = c * 8;
+#pragma unroll
+            for (int i = 0; i < kOffsets; ++i)
+                voff[i] = row0 + r + 8 * i < rmax ? (uint32_t)(((int64_t)(r + 8 * i) * ld + (c ^ (i & 1) * 4) * 8) * 2) : kRange;
+        } else if constexpr (!TRANS) {
             const int r = wave * 16 * W + (lane >> 2), c = (lane & 3) ^ (lane >> 4);
             klane = c * 8;
 #pragma unroll
@@ -98,11 +110,16 @@ struct Loader {
             }
         }
     }
-    // base: the block's first row at the tile's first k; k_rem: k values left from there (<= 0: nothing is fetched)
+    // base: the block's first row at the trip's first k, adv: bytes from there to the next 32 k; k_rem: k values left from base on
+    // (<= 0: nothing is fetched)
     template <int I>
-    __device__ __forceinline__ void issue(const char* base, int k_rem, uint32_t lds_oper, int wave) const {
-        if constexpr (!TRANS) dma16_buffer(base, klane < k_rem ? voff[I] : kRange, lds_oper + (wave * 16 * W + I * 16) * 64);
-        else dma16_buffer(base, klane + I * kKPer < k_rem ? voff[I] : kRange, lds_oper + (wave * 8 + I * kKPer) * (kRows * 2));
+    __device__ __forceinline__ void issue(const char* base, int64_t adv, int k_rem, uint32_t lds_oper, int wave) const {
+        constexpr int H = I / W, O = I % W;  // the 32 k of the trip and the instruction there, of images of 32 k
+        if constexpr (kLines) dma16_buffer(base, (klane ^ (I & 1) * 32) < k_rem ? voff[I] : kRange, lds_oper + (wave * 2 * W + I) * 1024);
+        else if constexpr (!TRANS) dma16_buffer(base, klane < k_rem ? voff[I] : kRange, lds_oper + (wave * 16 * W + I * 16) * 64);
+        else
+            dma16_buffer(base + H * adv, klane + O * kKPer < k_rem - H * kBK ? voff[O] : kRange,
+                         lds_oper + H * kImage + (wave * 8 + O * kKPer) * (kRows * 2));
     }
     // !TRANS: zero what lies past k_rem in the chunks that straddle it, in the rows this wavefront loaded (W * 16)
     __device__ __forceinline__ void fix_tail(lds_char* oper, int k_rem, int lane, int wave) const {
@@ -110,22 +127,23 @@ struct Loader {
             const int c = k_rem >> 3;
             if (lane < 16 * W) {
                 const int r = wave * 16 * W + lane;
-                lds_u16* p = (lds_u16*)(oper + r * 64 + ((c ^ ((r >> 2) & 3)) << 4));
+                lds_u16* p = (lds_u16*)(oper + (kLines ? r * 128 + ((c ^ ((r >> 1) & 7)) << 4) : r * 64 + ((c ^ ((r >> 2) & 3)) << 4)));
                 for (int e = k_rem & 7; e < 8; ++e) p[e] = 0;
             }
         }
     }
 };
 
-template <bool TRANS, int W>
+template <bool TRANS, int W, int KB>
 struct Frags {
     static constexpr int kRows = 64 * W;
-    uint32_t off[TRANS ? W : 2];
+    static constexpr bool kLines = Loader<TRANS, W, KB>::kLines;
+    uint32_t off[TRANS ? W : 2 * KB];
     __device__ __forceinline__ void init(int lane, int wrow) {
         if constexpr (!TRANS) {
-            const int r = lane & 31, g = lane >> 5, swz = (r >> 2) & 3;
+            const int r = lane & 31, g = lane >> 5, swz = kLines ? (r >> 1) & 7 : (r >> 2) & 3;
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) off[ks] = (uint32_t)((wrow + r) * 64 + (((2 * ks + g) ^ swz) << 4));
+            for (int ks = 0; ks < 2 * KB; ++ks) off[ks] = (uint32_t)((wrow + r) * (kLines ? 128 : 64) + (((2 * ks + g) ^ swz) << 4));
         } else {
             const int i = lane & 15, grp = lane >> 4, g = grp >> 1, kk = (i >> 2) & 3;
             const int lane_const = (8 * g + (i >> 2)) * (kRows * 2) + ((2 * (grp & 1) + ((i & 3) >> 1)) << 4) + 8 * (i & 1);
@@ -136,9 +154,9 @@ struct Frags {
     template <int T, int KS>
     __device__ __forceinline__ bf16x8_t read(lds_char* oper) const {
         if constexpr (!TRANS) {
-            return *(__attribute__((address_space(3))) const bf16x8_t*)(oper + off[KS] + T * 32 * 64);
+            return *(__attribute__((address_space(3))) const bf16x8_t*)(oper + off[KS] + T * 32 * (kLines ? 128 : 64));
         } else {
-            lds_char* p = oper + off[T] + KS * 16 * (kRows * 2);
+            lds_char* p = oper + off[T] + KS * 16 * (kRows * 2);  // the next 32 k's image follows: 32 rows further
             const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)p);
             const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + 4 * (kRows * 2)));
             const s16x8_t v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -321,10 +339,9 @@ constexpr int kBlocksPerCU = kLdsBytes<TM, TN, KB, NS> <= 80 * 1024 ? 2 : 1;
 template <bool TRANS_A, bool TRANS_B, int TM, int TN, int KB, int NS, int EPI, typename E>
 __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm_tile_kernel(const TileArgs args) {
     constexpr int BM = 64 * TM, BN = 64 * TN, BK = KB * kBK;
-    using LA = Loader<TRANS_A, TM>;
-    using LB = Loader<TRANS_B, TN>;
-    constexpr int kBlock = LA::kBytes + LB::kBytes;  // one k block: A image, B image
-    constexpr int kStage = KB * kBlock;
+    using LA = Loader<TRANS_A, TM, KB>;
+    using LB = Loader<TRANS_B, TN, KB>;
+    constexpr int kStage = LA::kBytes + LB::kBytes;  // of a trip: A, B
     constexpr int kPer = KB * (TM + TN);             // load instructions per wavefront and trip
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     lds_char* lds_base = (lds_char*)lds;
@@ -366,8 +383,8 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
     LB lb;
     la.init(lane, wave, args.lda, m0, M);
     lb.init(lane, wave, args.ldb, n0, N);
-    Frags<TRANS_A, TM> fa;
-    Frags<TRANS_B, TN> fb;
+    Frags<TRANS_A, TM, KB> fa;
+    Frags<TRANS_B, TN, KB> fb;
     fa.init(lane, wm * 32 * TM);
     fb.init(lane, wn * 32 * TN);
     // byte distance of the block's origin and of one k block
@@ -394,10 +411,9 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
     const char* is_b = step_ptr(kTabB, is_step) + b_org + (is_k / kBK) * b_adv;
     int is_rem = is_left > 0 ? K - is_k : 0;
     auto issue_one = [&](auto op) {  // instruction `op` of the trip's kPer
-        constexpr int H = op.value / (TM + TN), O = op.value % (TM + TN);
-        const uint32_t st = lds_addr0 + is_stage * kStage + H * kBlock;
-        if constexpr (O < TM) la.template issue<O>(is_a + H * a_adv, is_rem - H * kBK, st, wave);
-        else lb.template issue<O - TM>(is_b + H * b_adv, is_rem - H * kBK, st + LA::kBytes, wave);
+        const uint32_t st = lds_addr0 + is_stage * kStage;
+        if constexpr (op.value < KB * TM) la.template issue<op.value>(is_a, a_adv, is_rem, st, wave);
+        else lb.template issue<op.value - KB * TM>(is_b, b_adv, is_rem, st + LA::kBytes, wave);
     };
     auto issue_advance = [&]() {
         is_stage = (is_stage + 1 == NS) ? 0 : is_stage + 1;
@@ -421,9 +437,9 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
     const bool odd_tail = (!TRANS_A || !TRANS_B) && (K & 7) != 0;
     auto publish = [&]() {
         if (odd_tail && pub_rem < BK) {
-            lds_char* st = lds_base + pub_stage * kStage + (pub_rem / kBK) * kBlock;
-            la.fix_tail(st, pub_rem % kBK, lane, wave);
-            lb.fix_tail(st + LA::kBytes, pub_rem % kBK, lane, wave);
+            lds_char* st = lds_base + pub_stage * kStage;
+            la.fix_tail(st, pub_rem, lane, wave);
+            lb.fix_tail(st + LA::kBytes, pub_rem, lane, wave);
         }
         pub_rem -= BK;
         if (pub_rem <= 0) pub_rem = K;
@@ -443,9 +459,8 @@ __global__ __launch_bounds__(kThreads, (kBlocksPerCU<TM, TN, KB, NS>)) void gemm
     bf16x8_t af[2][2 * KB][TM], bfr[2][2 * KB][TN];
     auto read_one = [&](auto set, auto op) {  // fragment `op` of a trip: [k step][A fragments, B fragments]
         constexpr int KS = op.value / (TM + TN), O = op.value % (TM + TN);
-        lds_char* blk = rd + (KS / 2) * kBlock;
-        if constexpr (O < TM) af[set.value][KS][O] = fa.template read<O, KS % 2>(blk);
-        else bfr[set.value][KS][O - TM] = fb.template read<O - TM, KS % 2>(blk + LA::kBytes);
+        if constexpr (O < TM) af[set.value][KS][O] = fa.template read<O, KS>(rd);
+        else bfr[set.value][KS][O - TM] = fb.template read<O - TM, KS>(rd + LA::kBytes);
     };
     // prologue: trips 0 .. NS-1 requested, trip 0 published and its fragments on the way
     for (int p = 0; p < NS; ++p) {
