@@ -27,8 +27,8 @@ constexpr int TM = 4, TN = 4, NS = 4;  // MFMA tiles of a wavefront, LDS stages 
 template <int ABL>
 __global__ __launch_bounds__(kThreads, 1) void ring_kernel(const TileArgs args) {
     constexpr int BM = 64 * TM, BN = 64 * TN;
-    using LA = Loader<false, TM>;
-    using LB = Loader<true, TN>;
+    using LA = Loader<false, TM, 1>;
+    using LB = Loader<true, TN, 1>;
     constexpr int kStage = LA::kBytes + LB::kBytes, kPer = TM + TN;  // bytes of a stage, load instructions per wavefront and k tile
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     lds_char* lds_base = (lds_char*)lds;
@@ -49,8 +49,8 @@ __global__ __launch_bounds__(kThreads, 1) void ring_kernel(const TileArgs args) 
     LB lb;
     la.init(lane, wave, args.lda, m0, args.M);
     lb.init(lane, wave, args.ldb, n0, args.N);
-    Frags<false, TM> fa;
-    Frags<true, TN> fb;
+    Frags<false, TM, 1> fa;
+    Frags<true, TN, 1> fb;
     fa.init(lane, wm * 32 * TM);
     fb.init(lane, wn * 32 * TN);
     const int64_t a_org = (int64_t)m0 * args.lda * 2, a_adv = 2 * kBK, b_org = (int64_t)n0 * 2, b_adv = args.ldb * (2 * kBK);
@@ -71,8 +71,8 @@ __global__ __launch_bounds__(kThreads, 1) void ring_kernel(const TileArgs args) 
     int is_rem = K - is_k;
     auto issue_one = [&](auto op) {
         const uint32_t st = lds_addr0 + is_stage * kStage;
-        if constexpr (op.value < TM) la.template issue<op.value>(is_a, is_rem, st, wave);
-        else lb.template issue<op.value - TM>(is_b, is_rem, st + LA::kBytes, wave);
+        if constexpr (op.value < TM) la.template issue<op.value>(is_a, 0, is_rem, st, wave);
+        else lb.template issue<op.value - TM>(is_b, 0, is_rem, st + LA::kBytes, wave);
     };
     auto issue_advance = [&]() {
         is_stage = (is_stage + 1 == NS) ? 0 : is_stage + 1;
