@@ -5,7 +5,7 @@
 // softmax from the logits and the global (max, sum) and writes the gradient;
 // the logits are never modified.
 // Both are bound by memory. 16-byte accesses serve rows of any alignment (an odd vocabulary puts every row at another
-// offset): 1023 x 50257 bf16, forward 27 us where single elements took 75, backward 41 us for 44; aligned rows
+// offset): 1023 x 50257 bf16, forward 19 us where single elements took 75, backward 41 us for 44; aligned rows
 // (8192 x 12568 bf16, 33 and 69 us, 6 TB/s) run as they did with loads that assumed their alignment.
 #include <type_traits>
 
@@ -88,6 +88,14 @@ __device__ __forceinline__ void lse_merge(float& m_a, float& s_a, float m_b, flo
     m_a = m;
 }
 
+// 1 for a row of 16-bit elements that begins off a multiple of 4 bytes: its vectors are taken from the second element on. 16-byte
+// loads at odd elements take the load unit longer, at even ones they run as aligned ones do (1023 x 50257 bf16, where every other row
+// is odd, forward 24.5 -> 18.9 us, as at 50258 columns; 8192 x 12567 forward 42.4 -> 34.7, backward 81 -> 72, at 12568 33 and 68).
+template <typename T>
+__device__ __forceinline__ int odd_row(const T* row) {
+    return sizeof(T) == 2 ? (int)(reinterpret_cast<uintptr_t>(row) >> 1) & 1 : 0;
+}
+
 template <typename T>
 __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int64_t V_cols,
                                                             const T* __restrict__ logits, int64_t ld,
@@ -103,9 +111,13 @@ __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int6
     const int lane = tid & 63;
     const int wave = tid >> 6;
     for (int64_t row = blockIdx.x; row < T_rows; row += gridDim.x) {
-        const T* xr = logits + row * ld;
+        const T* row_begin = logits + row * ld;
+        const int odd = odd_row(row_begin);
+        const T* xr = row_begin + odd;
+        const int64_t cols = V_cols - odd;
         OnlineLse st{kNegInf, 0.0f, 0.0f};
-        const int64_t nvec = V_cols / V;
+        if (odd != 0 && tid == kCeBlock - 1) lse_add_one(st, load_elem(row_begin));
+        const int64_t nvec = cols / V;
         int64_t i = tid;
         // kCeUnroll independent 16-byte streaming loads in flight per trip
         for (; i + (kCeUnroll - 1) * kCeBlock < nvec; i += kCeUnroll * kCeBlock) {
@@ -122,7 +134,7 @@ __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int6
             unpack_raw(load_raw_stream_any(xr + i * V), v0, (const T*)nullptr);
             lse_add_chunk<V>(st, v0);
         }
-        for (int64_t c = nvec * V + tid; c < V_cols; c += kCeBlock) lse_add_one(st, load_elem(xr + c));
+        for (int64_t c = nvec * V + tid; c < cols; c += kCeBlock) lse_add_one(st, load_elem(xr + c));
         // wavefront, then block
         float m = st.m, s = st.s;
 #pragma unroll
@@ -147,7 +159,7 @@ __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int6
             const bool masked = (t < vocab_start) || (t >= vocab_start + V_cols);
             const int64_t idx = masked ? 0 : (t - vocab_start);
             out_mask[row] = masked ? 1 : 0;
-            out_pred[row] = masked ? 0.0f : load_elem(xr + idx);
+            out_pred[row] = masked ? 0.0f : load_elem(row_begin + idx);
         }
         __syncthreads();
     }
@@ -344,14 +356,16 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                 }
             }
         } else {
-            const int64_t nvec = V_cols / V;
+            // where logits and gradient are odd rows both, the vectors of both begin at the second element
+            const int odd = odd_row(xr) & odd_row(gr);
+            const int64_t nvec = (V_cols - odd) / V;
             CeRowScalars rs;
             if constexpr (sizeof(T) == 2) {
                 // 16-bit in, 16-bit out: one vector per thread and trip. Sixteen wavefronts per row and two rows
                 // per compute unit keep enough loads in flight; batching loads per thread measured slower here.
                 rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss);
                 for (int64_t i = tid; i < nvec; i += B)
-                    grad_vector<T, G, V>(load_raw_stream_any(xr + i * V), i, rs.tcol, rs.m2, rs.scale, rs.dl, gr);
+                    grad_vector<T, G, V>(load_raw_stream_any(xr + odd + i * V), i, rs.tcol - odd, rs.m2, rs.scale, rs.dl, gr + odd);
             } else {
                 constexpr int U = 4;  // 16-byte vectors per thread and batch
                 for (int64_t base = tid; base < nvec; base += (int64_t)U * B) {
@@ -369,12 +383,14 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
                     }
                 }
             }
-            if (nvec * V < V_cols) {
+            if (odd + nvec * V < V_cols || odd != 0) {
                 rs = ce_row_scalars(row, V_cols, targets, vocab_start, gmax, gsum, dloss);
-                for (int64_t c = nvec * V + tid; c < V_cols; c += B) {
-                    float y = __builtin_amdgcn_exp2f(__builtin_fmaf(load_elem(xr + c), kLog2e, -rs.m2)) * rs.scale;
-                    if (c == rs.tcol) y -= rs.dl;
-                    store_elem(gr + c, y);
+                // the columns behind the vectors, and the first one of an odd row
+                for (int64_t c = odd + nvec * V + tid; c < V_cols + odd; c += B) {
+                    const int64_t col = c < V_cols ? c : 0;
+                    float y = __builtin_amdgcn_exp2f(__builtin_fmaf(load_elem(xr + col), kLog2e, -rs.m2)) * rs.scale;
+                    if (col == rs.tcol) y -= rs.dl;
+                    store_elem(gr + col, y);
                 }
             }
         }

@@ -115,3 +115,30 @@ def test_logits_gradient_is_contiguous(V):
     logits.retain_grad()
     VocabParallelCrossEntropyLoss1D()(logits, torch.zeros((2, 61), dtype=torch.int64, device=DEV)).backward()
     assert seen == [2 * 61 * V] and logits.grad.is_contiguous() and logits.grad.untyped_storage().nbytes() == 2 * 61 * V * 2
+
+
+@pytest.mark.parametrize("V", [1, 2, 7, 9, 767, 769, 6143, 6145, 8191])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_cross_entropy_of_odd_rows(V, dtype):
+    """Rows at every alignment of their elements, in both kernels: vectors from the first or the second element on."""
+    from cubework_amd import ops
+
+    T = 5
+    for first in (0, 1):
+        buf = randn((T * V + 1,), dtype, V, std=3.0, device=DEV)
+        x = buf[first:first + T * V].view(T, V)
+        t = torch.tensor([0, V - 1, min(1, V - 1), V // 2, V + 3], device=DEV)  # the last one: another slice's
+        m, s, p, k = ops.vpce_fwd_local(x, t, 0)
+        ref = x.double()
+        top = ref.max(1).values
+        assert torch.equal(m.double(), top) and k.tolist() == [0, 0, 0, 0, 1]
+        # exponentials to 2^-22 or so, V terms at most 2^-24 each in chains of V / 2048 + 32
+        want = (ref - top[:, None]).exp().sum(1)
+        assert ((s.double() - want).abs() <= (V / 2048 + 40) * 2.0 ** -23 * want).all()
+        assert torch.equal(p[:4], x[torch.arange(4), t[:4]].float()) and p[4] == 0
+        soft = (ref - top[:, None]).exp() / want[:, None]
+        soft[torch.arange(4), t[:4]] -= 1.0
+        for aligned in (False, True):
+            g = ops.vpce_bwd(x, t, 0, m, s, aligned_rows=aligned)
+            rel = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+            assert ((g.double() - soft).abs() <= rel * soft.abs() + 2.0 ** -20 * (1 if dtype == torch.bfloat16 else 2.0 ** -4)).all()
