@@ -421,13 +421,16 @@ std::tuple<Tensor, Tensor> vpce_mean(const Tensor& logits_in, const Tensor& targ
     return {loss, total};
 }
 
-// Gradient of the logits, contiguous and of their type, for the gradient `dloss` of vpce_mean's loss.
-Tensor vpce_mean_bwd(const Tensor& logits_in, const Tensor& targets_in, int64_t vocab_start, const Tensor& total, const Tensor& dloss_in) {
+// Gradient of the logits, of their type, for the gradient `dloss` of vpce_mean's loss: contiguous, or with rows that begin at multiples
+// of 16 bytes.
+Tensor vpce_mean_bwd(const Tensor& logits_in, const Tensor& targets_in, int64_t vocab_start, const Tensor& total, const Tensor& dloss_in,
+                     bool aligned) {
     const Tensor logits = rows(logits_in), targets = targets_in.reshape({-1}).to(at::kLong).contiguous(), dloss = dloss_in.to(at::kFloat);
     on_device(logits);
     on_device(dloss);
     const int64_t T = logits.size(0), V = logits.size(1);
-    Tensor grad = empty({T, V}, logits);
+    const int64_t unit = aligned ? 16 / logits.element_size() : 1;
+    Tensor grad = empty({T, (V + unit - 1) / unit * unit}, logits).narrow(1, 0, V);
     const float* g = (const float*)ptr(total);
     const int dt = dtype_code(logits.scalar_type());
     check(lib.cw_vpce_bwd_mean(T, V, ptr(logits), ld(logits), (const int64_t*)ptr(targets), vocab_start, g, g + T, (const float*)ptr(dloss), ptr(grad),

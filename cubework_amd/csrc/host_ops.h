@@ -49,7 +49,8 @@ std::tuple<Tensor, OptTensor, OptTensor> ln_backward_fused(const Tensor& dy_in, 
                                                            const OptTensor& gamma, bool want_param_grads,
                                                            std::optional<at::ScalarType> param_type, const OptTensor& addend);
 std::tuple<Tensor, Tensor> vpce_mean(const Tensor& logits_in, const Tensor& targets_in, int64_t vocab_start, std::vector<Tensor> peers);
-Tensor vpce_mean_bwd(const Tensor& logits_in, const Tensor& targets_in, int64_t vocab_start, const Tensor& total, const Tensor& dloss_in);
+Tensor vpce_mean_bwd(const Tensor& logits_in, const Tensor& targets_in, int64_t vocab_start, const Tensor& total, const Tensor& dloss_in,
+                     bool aligned);
 
 void def_nodes(py::module_& m);
 

@@ -356,7 +356,7 @@ def vpce_mean(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, pee
 
 def vpce_mean_bwd(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, stats: torch.Tensor, dloss: torch.Tensor):
     """Gradient of the logits slice for the gradient `dloss` (one value) of vpce_mean's loss."""
-    return _lib.host().vpce_mean_bwd(logits, targets, vocab_start, stats, dloss)
+    return _lib.host().vpce_mean_bwd(logits, targets, vocab_start, stats, dloss, False)
 
 
 def vpce_bwd(logits: torch.Tensor, targets: torch.Tensor, vocab_start: int, gmax: torch.Tensor, gsum: torch.Tensor,

@@ -276,3 +276,52 @@ def test_threads_and_streams():
         t.join()
     for a, b in zip(alone, together):
         assert len(a) == len(b) > 0 and all(torch.equal(p, q) for p, q in zip(a, b))
+
+
+@pytest.mark.parametrize("rows,vocab,bias", [(33, 1001, False), (257, 516, True), (64, 1000, False), (1, 7, True)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_head_and_loss_of_any_vocabulary(rows, vocab, bias, dtype):
+    """The head's gradients are the ones of a dense gradient of the logits, and whoever sees that gradient sees a dense one."""
+    from cubework_amd import ops
+    from cubework_amd.module.loss._operation import _VocabParallelCrossEntropyMean
+    from cubework_amd.module.parallel_1d._operation import _LinearNT
+
+    leaves = [randn((rows, 64), dtype, 1, device=DEV).requires_grad_(True), randn((vocab, 64), dtype, 2, std=0.1, device=DEV).requires_grad_(True),
+              randn((vocab,), dtype, 3, device=DEV).requires_grad_(True) if bias else None]
+    t = torch.randint(0, vocab, (rows,), generator=torch.Generator().manual_seed(4)).to(DEV)
+    scale = lambda o, k: torch.full_like(o, 64.0)  # noqa: E731
+    want = _compare(lambda x, w, b: ops.mean_loss(ops.linear("NT", x, w, b), t, 0),
+                    lambda x, w, b: _VocabParallelCrossEntropyMean.apply(_LinearNT.apply(x, w, b, None), t, 0, ()), leaves, scale)
+    x, w, b = leaves
+    seen = []
+    forward = lambda: ops.linear("NT", x, w, b)  # noqa: E731
+    for watch in ("hook", "retain", "post", "asked", "inputs", "view"):
+        for leaf in leaves:
+            if leaf is not None:
+                leaf.grad = None
+        logits = forward()
+        loss = ops.mean_loss(logits.view(rows, 1, vocab) if watch == "view" else logits, t, 0)
+        dy = torch.full_like(loss, 64.0)
+        if watch == "hook":
+            logits.register_hook(seen.append)
+        elif watch == "retain":
+            logits.retain_grad()
+        elif watch == "post":
+            loss.grad_fn.register_hook(lambda outputs, _: seen.append(outputs[0]))
+        if watch == "asked":
+            seen.append(torch.autograd.grad(loss, logits, dy)[0])
+            continue
+        loss.backward(dy, inputs=[logits, x] if watch == "inputs" else None)
+        if watch in ("retain", "inputs"):
+            seen.append(logits.grad)
+        assert torch.equal(x.grad, want[1])
+        if watch != "inputs":
+            assert torch.equal(w.grad, want[2])
+    assert len(seen) == 5
+    assert all(g.shape == (rows, vocab) and g.is_contiguous() and torch.equal(g, seen[0]) for g in seen)
+    # the logits read a second time: their gradients are added before the product sees them
+    logits = forward()
+    (twice,) = torch.autograd.grad(ops.mean_loss(logits, t, 0) + logits.float().sum() / 16, x)
+    ref = torch.autograd.grad(ops.mean_loss(forward(), t, 0), x)[0].double() + (w.double().sum(0) / 16)
+    # 16-bit rounding of the added gradient and of the results
+    assert (twice.double() - ref).abs().max() <= 2.0 ** (-7 if dtype == torch.bfloat16 else -10) * ref.abs().max()
