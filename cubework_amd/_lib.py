@@ -17,7 +17,7 @@ CW_NN, CW_NT, CW_TN = 0, 1, 2
 CW_EPI_NONE, CW_EPI_BIAS, CW_EPI_BIAS_GELU_TANH, CW_EPI_BIAS_GELU_ERF, CW_EPI_BIAS_RELU = 0, 1, 2, 3, 4
 CW_ACT_NONE, CW_ACT_GELU_TANH, CW_ACT_GELU_ERF, CW_ACT_RELU = 0, 2, 3, 4
 CW_LN_ONE_PASS, CW_LN_TWO_PASS = 0, 1
-CW_MAX_KSTEPS, CW_MAX_ADDENDS = 16, 8
+CW_MAX_KSTEPS, CW_MAX_ADDENDS, CW_MAX_CASTS = 16, 8, 4
 CW_ERR_INVALID, CW_ERR_ALIGNMENT, CW_ERR_UNSUPPORTED, CW_ERR_LAUNCH, CW_ERR_DEVICE = -1, -2, -3, -4, -5
 
 _i64 = ctypes.c_int64
@@ -90,6 +90,7 @@ SIGNATURES = {
     "cw_vpce_mean_workspace_bytes": (_i64, [_i64]),
     "cw_vpce_finalize_mean": (_int, [_i64, _int, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr]),
     "cw_vpce_bwd_mean": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _int, _int, _ptr]),
+    "cw_cast_many": (_int, [_int, _pp, _pp, _ptr, _int, _int, _ptr]),
     "cw_vpce_bwd": (_int, [_i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _f32, _ptr, _i64, _int, _int, _ptr]),
 }
 
@@ -128,7 +129,7 @@ HOST_ENTRIES = ("cw_gemm_scratch_bytes", "cw_gemm_ksteps_ws", "cw_colsum_workspa
                 "cw_ln_bwd_dx_close_peers", "cw_vpce_fwd_local_mean", "cw_vpce_mean_workspace_bytes", "cw_vpce_finalize_mean",
                 "cw_vpce_bwd_mean", "cw_attn_fwd", "cw_attn_narrow_fwd", "cw_attn_bwd", "cw_attn_narrow_bwd",
                 "cw_attn_bwd_workspace_bytes", "cw_embed_fwd", "cw_embed_bwd_ids_supported", "cw_embed_bwd_ids",
-                "cw_embed_sort_workspace_bytes", "cw_embed_sort_ids", "cw_embed_bwd")
+                "cw_embed_sort_workspace_bytes", "cw_embed_sort_ids", "cw_embed_bwd", "cw_cast_many")
 
 
 def host():

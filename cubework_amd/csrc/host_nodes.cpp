@@ -40,9 +40,13 @@ bool half_type(at::ScalarType t) { return t == at::kBFloat16 || t == at::kHalf; 
 OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); }
 Tensor def(const OptTensor& t) { return t ? *t : Tensor(); }
 
-// What custom_fwd does to an input in an autocast region (nothing outside one), and the state in which the bodies run.
-Tensor cast_to(const Tensor& t, at::ScalarType type) {
-    return t.defined() && t.is_floating_point() && t.is_cuda() && t.scalar_type() != at::kDouble ? t.to(type) : t;
+// What custom_fwd does to inputs in an autocast region (nothing outside one), and the state in which the bodies run.
+void cast_inputs(std::initializer_list<Tensor*> ts, at::ScalarType type) {
+    Tensor none, *cast[CW_MAX_CASTS] = {&none, &none, &none, &none};
+    int n = 0;
+    for (Tensor* t : ts)
+        if (t->defined() && t->is_floating_point() && t->scalar_type() != at::kDouble) cast[n++] = t;
+    cast_together({cast[0], cast[1], cast[2], cast[3]}, type);
 }
 bool autocast() { return at::autocast::is_autocast_enabled(at::kCUDA); }
 struct Body {
@@ -61,17 +65,26 @@ Tensor aligned_rows(const Tensor& t_in) {
     return out.copy_(t);
 }
 
+// Which of the tensors are fp32, as bits.
+int64_t fp32_inputs(std::initializer_list<const Tensor*> ts) {
+    int64_t bits = 0, bit = 1;
+    for (const Tensor* t : ts) {
+        if (t->defined() && t->scalar_type() == at::kFloat) bits |= bit;
+        bit *= 2;
+    }
+    return bits;
+}
+
 // act(x W + bias) + residual, W [in, out] (CW_NN) or [out, in] (CW_NT): parallel_2d._operation._SUMMA_AB, parallel_1d._operation._LinearNT.
 struct Linear : Function<Linear> {
     static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& w_in, const OptTensor& bias_in, const OptTensor& residual_in,
                           int64_t layout, int64_t act) {
         Tensor x = x_in, w = w_in, bias = def(bias_in), residual = def(residual_in);
-        if (autocast()) {
-            const auto asked = at::autocast::get_autocast_dtype(at::kCUDA);
-            const auto type = half_type(asked) ? asked : at::kHalf;
-            for (Tensor* t : {&x, &w, &bias, &residual}) *t = cast_to(*t, type);
-        }
+        const bool cast = autocast();
+        const auto asked = cast ? at::autocast::get_autocast_dtype(at::kCUDA) : at::kHalf;
+        const int64_t given = fp32_inputs({&x, &w, &bias});
         Body body;
+        if (cast) cast_inputs({&x, &w, &bias, &residual}, half_type(asked) ? asked : at::kHalf);
         const int64_t N = w.size(layout == CW_NN ? 1 : 0);
         std::vector<Tensor> addends;
         if (residual.defined()) addends.push_back(residual.reshape({-1, N}));
@@ -80,7 +93,7 @@ struct Linear : Function<Linear> {
                                       act != CW_ACT_NONE ? (int)act : bias.defined() ? CW_EPI_BIAS : CW_EPI_NONE, addends,
                                       act != CW_ACT_NONE && act != CW_ACT_RELU, {});
         ctx->save_for_backward({x, w, act == CW_ACT_RELU ? out : def(pre)});
-        keep(ctx, {layout, act, bias.defined() ? (int64_t)bias.scalar_type() : -1, residual.defined()});
+        keep(ctx, {layout, act, bias.defined() ? (int64_t)bias.scalar_type() : -1, residual.defined(), given & ~fp32_inputs({&x, &w, &bias})});
         auto shape = x.sizes().vec();
         shape.back() = N;
         return out.reshape(shape);
@@ -107,6 +120,11 @@ struct Linear : Function<Linear> {
         if (need_w)
             dw = std::get<0>(layout == CW_NN ? gemm_ksteps(CW_TN, {x2}, {g}, {}, CW_EPI_NONE, {}, false, {})
                                              : gemm_ksteps(CW_TN, {g}, {x2}, {}, CW_EPI_NONE, {}, false, {}));
+        // gradients of inputs that were cast, which autograd would cast one by one
+        if (const int64_t was_fp32 = meta[4]; was_fp32 != 0) {
+            Tensor none;
+            cast_together({was_fp32 & 1 ? &dx : &none, was_fp32 & 2 ? &dw : &none, was_fp32 & 4 ? &dbias : &none}, at::kFloat);
+        }
         // absent operands are no inputs of the node, and have no index there
         const bool need_residual = meta[3] != 0 && ctx->needs_input_grad(has_bias ? 3 : 2);
         return {dx, dw, dbias, need_residual ? grads[0] : Tensor(), Tensor(), Tensor()};
@@ -134,9 +152,9 @@ py::object linear(py::handle x_in, py::handle w_in, py::handle bias_in, py::hand
 struct LayerNorm : Function<LayerNorm> {
     static variable_list forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& w_in, const Tensor& b_in, double eps, bool fork) {
         Tensor x = x_in, w = w_in, b = b_in;
-        if (autocast())
-            for (Tensor* t : {&x, &w, &b}) *t = cast_to(*t, at::kFloat);
+        const bool cast = autocast();
         Body body;
+        if (cast) cast_inputs({&x, &w, &b}, at::kFloat);
         auto [out, mean_rstd] = ln_forward(x, {}, {}, 0, eps, w, b, CW_LN_ONE_PASS, true);
         ctx->save_for_backward({x, w, *mean_rstd});
         keep(ctx, {(int64_t)w.scalar_type(), (int64_t)b.scalar_type()});

@@ -160,6 +160,35 @@ std::tuple<Tensor, OptTensor> gemm_ksteps(int layout, std::vector<Tensor> A, std
     return {out, pre};
 }
 
+void cast_together(std::initializer_list<Tensor*> ts, at::ScalarType type) {
+    auto half = [](at::ScalarType t) { return t == at::kBFloat16 || t == at::kHalf; };
+    const void* src[CW_MAX_CASTS];
+    void* dst[CW_MAX_CASTS];
+    int64_t n[CW_MAX_CASTS];
+    Tensor to[CW_MAX_CASTS], *of[CW_MAX_CASTS];
+    int count = 0;
+    at::ScalarType from = at::kFloat;
+    for (Tensor* t : ts) {
+        if (!t->defined() || t->scalar_type() == type) continue;
+        const at::ScalarType own = t->scalar_type();
+        const bool ours = (own == at::kFloat ? half(type) : half(own) && type == at::kFloat) && (count == 0 || own == from) && count < CW_MAX_CASTS &&
+                          t->is_contiguous() && aligned16(*t) && t->numel() > 0 && t->numel() < ((int64_t)1 << 33);
+        if (!ours) {
+            *t = t->to(type);
+            continue;
+        }
+        from = own;
+        to[count] = empty(t->sizes(), *t, type);
+        src[count] = ptr(*t);
+        dst[count] = ptr(to[count]);
+        n[count] = t->numel();
+        of[count++] = t;
+    }
+    if (count == 0) return;
+    check(lib.cw_cast_many(count, src, dst, n, dtype_code(from), dtype_code(type), stream()), "cw_cast_many");
+    for (int i = 0; i < count; ++i) *of[i] = to[i];
+}
+
 Tensor colsum(const Tensor& dy_in, std::optional<at::ScalarType> out_type) {
     const Tensor dy = rows(dy_in);
     on_device(dy);

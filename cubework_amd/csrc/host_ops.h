@@ -16,7 +16,7 @@ using OptTensor = std::optional<Tensor>;
     X(cw_ln_bwd_dx_close_peers) X(cw_vpce_fwd_local_mean) X(cw_vpce_mean_workspace_bytes) X(cw_vpce_finalize_mean)     \
     X(cw_vpce_bwd_mean) X(cw_attn_fwd) X(cw_attn_narrow_fwd) X(cw_attn_bwd) X(cw_attn_narrow_bwd)                      \
     X(cw_attn_bwd_workspace_bytes) X(cw_embed_fwd) X(cw_embed_bwd_ids_supported) X(cw_embed_bwd_ids)                   \
-    X(cw_embed_sort_workspace_bytes) X(cw_embed_sort_ids) X(cw_embed_bwd)
+    X(cw_embed_sort_workspace_bytes) X(cw_embed_sort_ids) X(cw_embed_bwd) X(cw_cast_many)
 struct Entries {
 #define X(name) decltype(&::name) name = nullptr;
     CW_HOST_ENTRIES(X)
@@ -40,6 +40,8 @@ inline Tensor bytes(int64_t n, const Tensor& like) { return empty({n}, like, at:
 
 std::tuple<Tensor, OptTensor> gemm_ksteps(int layout, std::vector<Tensor> A, std::vector<Tensor> B, const OptTensor& bias_in, int epilogue,
                                           std::vector<Tensor> addends, bool want_preact, const OptTensor& out_in);
+// Each of the tensors (undefined ones stay so) as `type`: those that are contiguous between fp32 and a 16-bit type in one launch.
+void cast_together(std::initializer_list<Tensor*> ts, at::ScalarType type);
 Tensor colsum(const Tensor& dy_in, std::optional<at::ScalarType> out_type);
 std::tuple<Tensor, OptTensor> act_bwd_colsum(int activation, const Tensor& dy_in, const Tensor& pre_in, bool want_dbias,
                                              std::optional<at::ScalarType> out_type);

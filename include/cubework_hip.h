@@ -74,6 +74,7 @@ typedef enum { CW_LN_ONE_PASS = 0, CW_LN_TWO_PASS = 1 } cw_ln_mode;
 
 #define CW_MAX_KSTEPS 16
 #define CW_MAX_ADDENDS 8
+#define CW_MAX_CASTS 4
 
 /* ---- sanity ------------------------------------------------------------ */
 const char* cw_version(void);
@@ -394,6 +395,13 @@ int cw_vpce_finalize_mean(int64_t T, int n_peers, const float* max, const float*
 int cw_vpce_bwd_mean(int64_t T, int64_t V, const void* logits, int64_t ld, const int64_t* targets, int64_t vocab_start,
                      const float* gmax, const float* gsum, const float* dloss, void* grad, int64_t ld_grad, int io_dtype,
                      int grad_dtype, void* stream);
+
+/*
+ * Casts of up to CW_MAX_CASTS dense tensors (numels[i] elements at src[i] to dst[i], all 16-byte aligned) between fp32 and one 16-bit
+ * type in one launch, rounding to nearest even: what custom_fwd(cast_inputs=...) does to a linear layer's input, weight and bias
+ * (cubework/module/parallel_2d/_operation.py:17), and autograd to their gradients.
+ */
+int cw_cast_many(int count, const void* const* src, void* const* dst, const int64_t* numels, int src_dtype, int dst_dtype, void* stream);
 
 
 /* ---- vocab-parallel embedding -------------------------------------------- */
