@@ -63,7 +63,9 @@ class OPTBlock(nn.Module):
         """(layer(x), x for the residual branch): through LayerNorm2D's `fork_residual` option where the layer is
         one, so that the two branches' gradients are added inside its backward kernel."""
         inner = getattr(layer, "norm", layer)
-        if isinstance(inner, LayerNorm2D) and x.dtype == inner.weight.dtype and not torch.is_autocast_enabled("cuda"):
+        # under autocast the layer works on an fp32 copy of a 16-bit input: the residual branch keeps the input itself
+        if (isinstance(inner, LayerNorm2D) and x.dtype == inner.weight.dtype
+                and (x.dtype == torch.float32 or not torch.is_autocast_enabled("cuda"))):
             return layer(x, fork_residual=True)
         return layer(x), x
 

@@ -1,4 +1,4 @@
-"""Casts of several tensors in one launch against torch's, bit for bit."""
+"""Casts of several tensors in one launch against torch's, bit for bit, and what a block under autocast does with them."""
 import ctypes
 
 import pytest
@@ -40,3 +40,41 @@ def test_refusals():
     assert _cast([x[1:]], torch.float16)[0] == -2  # not 16-byte aligned
     assert _cast([x.half()], torch.bfloat16)[0] == -3
     assert _cast([x] * 5, torch.float16)[0] == -1
+
+
+@pytest.mark.parametrize("amp", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_block_under_autocast_keeps_its_types(amp, dtype):
+    """A block's parameters and stream in either type: the residual branch carries the input's own type, gradients the parameters'."""
+    from cubework_amd.distributed import initialize
+    from cubework_amd.opt_block import OPTBlock
+    initialize("2d", 1)
+    blk = OPTBlock(hidden=128, heads=2, ffn=512, dtype=dtype).to(DEV)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    with torch.no_grad():
+        for name, p in blk.named_parameters():
+            p.copy_(torch.randn(p.shape, generator=g, device=DEV) * 0.05 + (1.0 if "norm" in name and name.endswith("weight") else 0.0))
+
+    def run(plain):
+        x = randn((2, 33, 128), dtype, 5, device=DEV).requires_grad_(True)
+        keep = OPTBlock._norm_fork
+        if plain:  # the two branches' gradients added by autograd
+            OPTBlock._norm_fork = staticmethod(lambda layer, t: (layer(t), t))
+        try:
+            for p in blk.parameters():
+                p.grad = None
+            with torch.autocast("cuda", dtype=amp):
+                y = blk(x)
+            y.backward(torch.ones_like(y))
+        finally:
+            OPTBlock._norm_fork = staticmethod(keep)
+        assert x.grad.dtype == dtype and all(p.grad.dtype == dtype for p in blk.parameters())
+        return y, [x.grad] + [p.grad for p in blk.parameters()]
+
+    y, grads = run(False)
+    want, want_grads = run(True)
+    assert y.dtype == want.dtype and torch.equal(y, want)
+    # one fp32 addition in another place: what it changes is rounded to 16 bits on the way back
+    bar = 2.0 ** (-9 if amp == torch.float16 else -6)
+    for a, b in zip(grads, want_grads):
+        assert (a.double() - b.double()).norm() <= bar * b.double().norm()
