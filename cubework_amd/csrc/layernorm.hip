@@ -945,6 +945,125 @@ __global__ __launch_bounds__(MAXW * 64, 4) void ln_bwd_split_kernel(
             }
 }
 
+// Backward over whole rows (FUSE_DX as above), few of them: one launch that finishes everything. The leading workgroups own 8 vectors
+// of columns each (whole lines) and walk over all rows, 64 at a time, for dgamma and dbeta, which need the rows' mean and rstd but not their
+// sums; the others take a row per wavefront for the row sums and dx. dY and x are read twice, the second time from cache; what
+// that saves is the launch that adds the partial rows and the partial rows themselves. Bound by latency: a wavefront's loads, its
+// sums, its stores (512 x 4096 bf16 9 us, 15.7 before), and by the columns' walk as the rows get more (short_bwd_rows).
+constexpr int kShortWaves = 8, kShortLanes = 8;
+template <typename T, int NCH, int FUSE_DX>
+__global__ __launch_bounds__(kShortWaves * 64) void ln_bwd_short_kernel(
+    int R, int64_t C, const T* __restrict__ dY, int64_t ld_dy, const T* __restrict__ x, int64_t ld_x,
+    const float* __restrict__ mean_rstd, const T* __restrict__ gamma, float* __restrict__ row_sums, T* __restrict__ dx, int64_t ld_dx,
+    float inv_h, const T* __restrict__ dx_add, int64_t ld_add, int col_blocks, void* __restrict__ dgamma, void* __restrict__ dbeta,
+    int param_dtype) {
+    constexpr int V = elem<T>::kVec;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if ((int)blockIdx.x < col_blocks) {
+        constexpr int U = 4, kRows = kShortWaves * 64 / kShortLanes, kCols = kShortLanes * V;
+        __shared__ float red[2][kShortWaves][kCols];
+        const int lc = lane % kShortLanes, lr = lane / kShortLanes;
+        const int64_t c0 = (int64_t)blockIdx.x * kCols + lc * V, c = c0 < C ? c0 : 0;  // columns outside are read elsewhere and dropped
+        float acc[2][V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[0][e] = acc[1][e] = 0.0f;
+        for (int base = wave * (64 / kShortLanes) + lr; base < R; base += kRows * U) {
+            raw16_t d_raw[U], x_raw[U];
+            float mean[U], rstd[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int r = base + u * kRows, rc = r < R ? r : R - 1;
+                d_raw[u] = load_raw(dY + rc * ld_dy + c);
+                x_raw[u] = load_raw(x + rc * ld_x + c);
+                mean[u] = mean_rstd[2 * rc];
+                rstd[u] = mean_rstd[2 * rc + 1];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const bool live = base + u * kRows < R;
+                float d[V], xv[V];
+                unpack_raw(d_raw[u], d, (const T*)nullptr);
+                unpack_raw(x_raw[u], xv, (const T*)nullptr);
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    acc[0][e] += live ? d[e] * ((xv[e] - mean[u]) * rstd[u]) : 0.0f;
+                    acc[1][e] += live ? d[e] : 0.0f;
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+#pragma unroll
+                for (int off = kShortLanes; off < 64; off <<= 1) acc[k][e] += __shfl_xor(acc[k][e], off, 64);
+                if (lr == 0) red[k][wave][lc * V + e] = acc[k][e];
+            }
+        __syncthreads();
+        const int k = (int)threadIdx.x / kCols, t = (int)threadIdx.x % kCols;
+        const int64_t col = (int64_t)blockIdx.x * kCols + t;
+        if (k > 1 || col >= C) return;
+        float total = red[k][0][t];
+#pragma unroll
+        for (int w = 1; w < kShortWaves; ++w) total += red[k][w][t];
+        store_col_total(k == 0 ? dgamma : dbeta, col, total, param_dtype);
+        return;
+    }
+    const int64_t row = (int64_t)((int)blockIdx.x - col_blocks) * kShortWaves + wave;
+    if (row >= R) return;
+    RowTile<T, NCH, 1> tdy, tx, tadd;
+    tdy.load(dY, ld_dy, row, R, C, lane);
+    tx.load(x, ld_x, row, R, C, lane);
+    if constexpr (FUSE_DX == 2) tadd.load(dx_add, ld_add, row, R, C, lane);
+    raw16_t g_raw[NCH];
+    load_param_chunks<T, NCH>(gamma, C, lane, g_raw);
+    const float mean = mean_rstd[2 * row], rstd = mean_rstd[2 * row + 1];
+    float s1 = 0.0f, s2 = 0.0f;
+    auto vectors = [&](int j, float (&gd)[V], float (&xh)[V]) {
+        float d[V], xv[V], g[V];
+        unpack_raw(tdy.raw[0][j], d, (const T*)nullptr);
+        unpack_raw(tx.raw[0][j], xv, (const T*)nullptr);
+        unpack_raw(g_raw[j], g, (const T*)nullptr);
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            xh[e] = (xv[e] - mean) * rstd;
+            gd[e] = gamma != nullptr ? d[e] * g[e] : d[e];
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+        float gd[V], xh[V];
+        vectors(j, gd, xh);
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            s1 += gd[e];
+            s2 += gd[e] * xh[e];
+        }
+    }
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    if (lane == 0) {
+        row_sums[2 * row] = s1;
+        row_sums[2 * row + 1] = s2;
+    }
+    if constexpr (FUSE_DX == 0) return;
+    const float c1 = s1 * inv_h, c2 = s2 * inv_h;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+        float gd[V], xh[V];
+        vectors(j, gd, xh);
+#pragma unroll
+        for (int e = 0; e < V; ++e) gd[e] = (gd[e] - xh[e] * c2 - c1) * rstd;
+        if constexpr (FUSE_DX == 2) {
+            float av[V];
+            unpack_raw(tadd.raw[0][j], av, (const T*)nullptr);
+#pragma unroll
+            for (int e = 0; e < V; ++e) gd[e] += av[e];
+        }
+        if (chunk_valid<T>(j, lane, C)) store_raw_stream(dx + row * ld_dx + ((int64_t)j * 64 + lane) * V, pack_raw(gd, (const T*)nullptr));
+    }
+}
+
 // Backward partials for shapes the vector kernel does not take (ragged C,
 // unaligned rows, very wide rows). Row sums only; the column sums of this
 // path come from ln_bwd_cols_generic_kernel.
@@ -1302,6 +1421,49 @@ int bwd_split_launch(const SplitShape& sh, int64_t R, int64_t C, const void* dY,
 #undef CW_SPLIT
 }
 
+// Where the two passes over the rows cost more than the second launch: us with a residual gradient, operands from the Infinity Cache and
+// memory, before / here: up to four chunks a row (bf16, rows x 2048) 128 11.1 / 5.4, 512 11.9 / 8.3, 777 12.6 / 11.2, 1024 13.1 / 13.2;
+// (x 768) 512 10.3 / 7.5, 777 10.5 / 9.5, fp32 9.2 / 9.8; more of them (bf16, x 2560) 512 12.7 / 8.8, 1024 19.3 / 14.0, 1554 23.5 / 21.1,
+// 2048 25.3 / 27.3, (x 4096) 1024 23.9 / 15.7, 2048 31.5 / 28.3; fp32 (x 2048) 1024 17.1 / 14.4, 1554 21.7 / 21.2. Blocks of 4 wavefronts, 4
+// or 16 vectors of columns, 8 rows in flight: slower.
+template <typename T>
+int64_t short_bwd_rows(int64_t nch) {
+    return nch <= kSplitMinChunks ? 640 : sizeof(T) == 2 ? 1792 : 1536;
+}
+
+template <typename T>
+bool bwd_short_takes(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void* x, int64_t ld_x, const void* gamma, const void* dx,
+                     int64_t ld_dx, const void* dgamma, int64_t workspace_bytes, const DxAdd& add) {
+    // dx is written while other workgroups read dY and x: a caller that works in place takes the kernels that read each row once
+    auto apart = [&](const void* p, int64_t ld) {
+        const char *a = (const char*)p, *b = (const char*)dx;
+        return b == nullptr || a + ((R - 1) * ld + C) * (int64_t)sizeof(T) <= b || b + ((R - 1) * ld_dx + C) * (int64_t)sizeof(T) <= a;
+    };
+    // the scratch that the entry point asks for, though this launch needs none: with less the others decide
+    return dgamma != nullptr && workspace_bytes >= ln_bwd_workspace_bytes(R, C) && C % elem<T>::kVec == 0 && row_chunks<T>(C) <= 8 &&
+           R <= short_bwd_rows<T>(row_chunks<T>(C)) && rows_vec_ok<T>(dY, ld_dy) && rows_vec_ok<T>(x, ld_x) &&
+           (dx == nullptr || rows_vec_ok<T>(dx, ld_dx)) && (gamma == nullptr || aligned16(gamma)) && apart(dY, ld_dy) && apart(x, ld_x) &&
+           (add.p == nullptr || rows_vec_ok<T>(add.p, add.ld));
+}
+
+template <typename T>
+int bwd_short_launch(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void* x, int64_t ld_x, const float* mean_rstd,
+                     const void* gamma, float* row_sums, void* dx, int64_t ld_dx, void* dgamma, void* dbeta, int param_dtype,
+                     hipStream_t s, const DxAdd& add) {
+    const int cols = kShortLanes * elem<T>::kVec, col_blocks = (int)((C + cols - 1) / cols);
+    const dim3 grid((unsigned)(col_blocks + (R + kShortWaves - 1) / kShortWaves));
+    auto launch = [&](auto nch_c, auto fuse_c) {
+        hipLaunchKernelGGL((ln_bwd_short_kernel<T, decltype(nch_c)::value, decltype(fuse_c)::value>), grid, dim3(kShortWaves * 64), 0, s, (int)R, C,
+                           (const T*)dY, ld_dy, (const T*)x, ld_x, mean_rstd, (const T*)gamma, row_sums, (T*)dx, ld_dx, 1.0f / (float)C,
+                           (const T*)add.p, add.ld, col_blocks, dgamma, dbeta, param_dtype);
+        return check_launch("ln_bwd_short_kernel");
+    };
+    return dispatch_tile(row_chunks<T>(C), [&](auto nch_c, auto) {
+        if (dx == nullptr) return launch(nch_c, std::integral_constant<int, 0>{});
+        return add.p != nullptr ? launch(nch_c, std::integral_constant<int, 2>{}) : launch(nch_c, std::integral_constant<int, 1>{});
+    });
+}
+
 constexpr int64_t kGenericSlabRows = 64;
 
 // dx != nullptr asks for the fused backward (C is the whole hidden size); *dx_done tells whether the
@@ -1318,6 +1480,10 @@ int bwd_partials_impl(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const
     const int want_cols = (dgamma != nullptr || dbeta != nullptr || open_parts != nullptr) ? 1 : 0;
     const bool vec = rows_vec_ok<T>(dY, ld_dy) && rows_vec_ok<T>(x, ld_x) && (gamma == nullptr || aligned16(gamma)) &&
                      (C % V) == 0 && (add.p == nullptr || rows_vec_ok<T>(add.p, add.ld));
+    if (open_parts == nullptr && bwd_short_takes<T>(R, C, dY, ld_dy, x, ld_x, gamma, dx, ld_dx, dgamma, workspace_bytes, add)) {
+        if (dx_done != nullptr) *dx_done = dx != nullptr;
+        return bwd_short_launch<T>(R, C, dY, ld_dy, x, ld_x, mean_rstd, gamma, row_sums, dx, ld_dx, dgamma, dbeta, param_dtype, s, add);
+    }
     const int64_t nch = (C + 64 * V - 1) / (64 * V);
     int64_t nparts = 0;
     int rc;

@@ -1,0 +1,91 @@
+"""LayerNorm of few rows: the forward with a wavefront a chunk and the backward that finishes everything in one launch, at the edges of
+their rules and of their tiles, against float64."""
+import ctypes
+
+import pytest
+import torch
+
+from tests.util import randn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+CODE = {torch.bfloat16: 0, torch.float32: 1, torch.float16: 2}
+# one rounding of the result, and fp32 sums of up to 4096 terms in chains of 64 and trees
+REL = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -18}
+
+
+def _reference(x, dy, g, b, add, eps):
+    x, dy, g, b, add = (t.double() for t in (x, dy, g, b, add))
+    mean = x.mean(1, keepdim=True)
+    rstd = (x.var(1, unbiased=False, keepdim=True) + eps).rsqrt()
+    xh = (x - mean) * rstd
+    gd = dy * g
+    dx = (gd - gd.mean(1, keepdim=True) - xh * (gd * xh).mean(1, keepdim=True)) * rstd
+    return xh * g + b, dx + add, (dy * xh).sum(0), dy.sum(0)
+
+
+def _close(got, want, rel, scale=None):
+    scale = want.abs() + want.abs().mean() if scale is None else scale
+    assert ((got.double() - want).abs() <= rel * scale).all()
+
+
+SHAPES = [(1, 8), (2, 520), (7, 768), (8, 1032), (9, 1536), (63, 2056), (64, 4096), (65, 1024), (257, 2048), (512, 4096), (513, 4096), (640, 768),
+          (641, 768), (819, 2560), (820, 2560), (1024, 2048), (1025, 2048), (1365, 776), (1366, 776), (1536, 2048), (1537, 2048), (1792, 2560),
+          (1793, 2560)]
+
+
+@pytest.mark.parametrize("R,C", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("pitched", [False, True])
+def test_few_rows_forward_and_backward(R, C, dtype, pitched):
+    from cubework_amd import ops
+
+    def rows(seed):
+        t = randn((R, C + (64 if pitched else 0)), dtype, seed, device=DEV)
+        return t[:, :C]
+    x, dy, add = rows(1), rows(2), rows(3)
+    g, b = (randn((C,), torch.float32, 4) * 0.2 + 1).to(dtype).to(DEV), randn((C,), dtype, 5, device=DEV)
+    y, dx, dg, db = _reference(x, dy, g, b, add, 1e-5)
+    got, mean_rstd = ops.ln_forward_fused(x, 1e-5, g, b)
+    _close(got, y, REL[dtype])
+    got_dx, got_dg, got_db = ops.ln_backward_fused(dy, x, mean_rstd, g, param_dtype=torch.float32, dx_addend=add)
+    _close(got_dx, dx, REL[dtype] * 2)
+    # x_hat is off by some 2^-22 of (|x - mean| + the row's largest |x|, which rounds the mean) times rstd, its sums over R rows by 2^-20 of
+    # their magnitudes: 2^-19 of both
+    xd = x.double()
+    centred = (xd - xd.mean(1, keepdim=True)).abs() + xd.abs().amax(1, keepdim=True)
+    bound = (dy.double().abs() * centred * (xd.var(1, unbiased=False, keepdim=True) + 1e-5).rsqrt()).sum(0)
+    _close(got_dg, dg, 2.0 ** -19, bound)
+    _close(got_db, db, 2.0 ** -20, dy.double().abs().sum(0))
+    plain = ops.ln_backward_fused(dy, x, mean_rstd, g, param_dtype=dtype)
+    _close(plain[0], dx - add.double(), REL[dtype] * 2)
+    assert plain[1].dtype == dtype and torch.equal(plain[2], got_db.to(dtype))
+
+
+def _backward(dy, x, mean_rstd, g, dx, ws_bytes):
+    from cubework_amd import _lib
+    R, C = x.shape
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    row_sums, out = torch.empty((R, 2), device=DEV), [torch.full((C,), float("nan"), device=DEV) for _ in range(2)]
+    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=DEV)
+    rc = _lib.load().cw_ln_backward_fused(R, C, p(dy), C, p(x), C, p(mean_rstd), p(g), p(row_sums), p(dx), C, None, 0, p(out[0]), p(out[1]), 1, p(ws),
+                                          ws_bytes, CODE[x.dtype], ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    return rc, row_sums, out
+
+
+def test_in_place_and_scratch():
+    """dx in the place of dY: the kernels that read every row once. Less scratch than the entry point asks for: refused as before."""
+    from cubework_amd import _lib, ops
+    R, C = 96, 1024
+    x, dy, g = randn((R, C), torch.float32, 1, device=DEV), randn((R, C), torch.float32, 2, device=DEV), randn((C,), torch.float32, 3, device=DEV)
+    _, mean_rstd = ops.ln_forward_fused(x, 1e-5, g, g)
+    need = _lib.load().cw_colsum_workspace_bytes(R, C)
+    dx = torch.empty_like(x)
+    rc, sums, cols = _backward(dy, x, mean_rstd, g, dx, need)
+    assert rc == 0
+    own = dy.clone()
+    rc, own_sums, own_cols = _backward(own, x, mean_rstd, g, own, need)
+    assert rc == 0
+    for a, b in zip([dx, sums] + cols, [own, own_sums] + own_cols):
+        _close(a, b.double(), 2.0 ** -18, b.double().abs() + b.double().abs().mean())
+    assert _backward(dy, x, mean_rstd, g, dx, 16)[0] == -1
