@@ -1261,6 +1261,17 @@ int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float*
     const int vec_ok = rows_vec_ok<T>(x, ld) && rows_vec_ok<T>(y, ldy) && (gamma == nullptr || aligned16(gamma)) &&
                        (beta == nullptr || aligned16(beta));
     const int64_t nch = row_chunks<T>(C);
+    if constexpr (FUSED) {
+        // As many wavefronts a row as it has chunks, one load each, where all of them fit the chip at once (16 per compute unit): with a row a
+        // wavefront the launch is that wavefront's chain (us, bf16 from memory: 300 x 4096 5.6 -> 3.9, 1024 x 2048 5.8 -> 4.3, 777 x 2560 5.5 -> 4.4; beyond,
+        // from cache, 1554 x 2560 5.6 -> 6.2; rows of two chunks, 128 x 768 2.7 -> 2.8).
+        if (vec_ok && (C % elem<T>::kVec) == 0 && nch >= 3 && nch <= kFwdSplitBlockWaves && R * nch <= 16 * 256) {
+            const int nrg = kFwdSplitBlockWaves / (int)nch;
+            hipLaunchKernelGGL((ln_forward_split_kernel<T, 1, kFwdSplitBlockWaves>), dim3((unsigned)((R + nrg - 1) / nrg)), dim3((unsigned)(nch * nrg * 64)),
+                               0, s, R, C, (const T*)x, ld, mode, 1.0f / (float)H, eps, (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd, (int)nch);
+            return check_launch("ln_forward_split_kernel");
+        }
+    }
     if (vec_ok && exact_chunks<T>(C, nch) && R <= (int64_t)1 << 30) {
         // rows per wavefront, by measurement (one tile per wavefront, 16-bit rows): four rows of one chunk (12.8 us
         // on 32768 x 512 against 14.8 with two and 14.5 with eight), two rows of two chunks (16384 x 1024: 11.9
