@@ -15,10 +15,10 @@
 // as the A operand uses the same permutation, which the transposing LDS
 // read of V provides).
 //
-// Block = 8 wavefronts x 32 query rows; K/V tiles of 64 rows are staged in
+// Block = 2, 4 or 8 wavefronts x 32 query rows (fwd_waves); K/V tiles of 64 rows are staged in
 // LDS (two stages, the next tile loaded straight into LDS while this one is
 // used), K as [kv][d] read with ds_read_b128, V as [kv][d] read with
-// ds_read_b64_tr_b16. At head size 64 two blocks are resident per compute
+// ds_read_b64_tr_b16. At head size 64 four blocks of 4 are resident per compute
 // unit (four wavefronts per SIMD); the softmax arithmetic (one v_exp_f32 per
 // score) weighs about as much as the matrix products there.
 #include "attention_common.h"
@@ -30,12 +30,9 @@ namespace {
 using namespace attn;
 
 constexpr int kQT = 1;                    // 32-row query tiles per wavefront
-constexpr int kWaves = 8;                 // wavefronts per block
-constexpr int kThreads = kWaves * 64;
 constexpr int kQPerWave = 32 * kQT;
 constexpr float kLazy = 8.0f;             // log2 of the largest probability taken against a stale reference
 constexpr float kNoKey = -1.0e30f;        // reference of a row that has met no live key yet (finite on purpose)
-constexpr int kQPerBlock = kWaves * kQPerWave;
 
 struct AttnArgs {
     const uint16_t* q;
@@ -54,10 +51,11 @@ struct AttnArgs {
 // HS: the head's shape (HeadShape). A tile of NP x 64 columns is NP images side by side ("panels"); everything that
 // runs over the head dimension runs over KB 16-wide k blocks (scores) or DT 32-wide output blocks (O^T). Heads up to
 // 80 columns keep two blocks per compute unit, 128 has the registers of one.
-template <typename HS, typename E>
-__global__ __launch_bounds__(kThreads, HS::NP == 1 ? 2 : 1) void attn_fwd_kernel(const AttnArgs a) {
+template <typename HS, int W, typename E>
+__global__ __launch_bounds__(64 * W, HS::NP == 1 ? 2 : 1) void attn_fwd_kernel(const AttnArgs a) {
     constexpr int NP = HS::NP, KB = HS::KB, DT = HS::DT;
     constexpr bool MASK = HS::MASK;
+    constexpr int kQPerBlock = W * kQPerWave;
     constexpr int kStage = 2 * NP * kImage;  // K panels (row images), then V panels (transpose images)
     __shared__ __attribute__((aligned(16))) char lds_raw[2 * kStage];
     lds_char* lds = (lds_char*)lds_raw;
@@ -77,7 +75,7 @@ __global__ __launch_bounds__(kThreads, HS::NP == 1 ? 2 : 1) void attn_fwd_kernel
     // Under the causal mask a wavefront's work grows with its query position, and wavefront w always runs on
     // SIMD w % 4: half of the blocks deal the query tiles in reverse so that no SIMD collects the long ones
     // (blocks 256 apart, which share a compute unit when the launch starts, differ in bit 8).
-    const int wq = (a.causal && (((blockIdx.x >> 8) ^ blockIdx.x) & 1)) ? kWaves - 1 - wave : wave;
+    const int wq = (a.causal && (((blockIdx.x >> 8) ^ blockIdx.x) & 1)) ? W - 1 - wave : wave;
     const int qw0 = q0 + wq * kQPerWave;
 
     const uint16_t* qp = a.q + b * a.sb + h * a.sh;
@@ -118,7 +116,7 @@ __global__ __launch_bounds__(kThreads, HS::NP == 1 ? 2 : 1) void attn_fwd_kernel
     const int kv_end = a.causal ? q_hi : S;
     const int n_tiles = (kv_end + kTile - 1) / kTile;
 
-    TileDma<kThreads> dma;
+    TileDma<64 * W> dma;
     dma.init(tid);
     const uint32_t lds_addr = (uint32_t)(uintptr_t)lds;
     ReadOffsets ro;
@@ -271,12 +269,24 @@ using namespace cw;
 
 namespace {
 
+// Wavefronts of a block. Few of them where they all fit the chip at once: a block's wavefronts wait for each other at every tile, and under
+// the causal mask for the longest of them. us, bf16, 8 / 4 / 2 wavefronts (batch x tokens x heads x columns): 1 x 300 x 32 x 128 15.1 / 12.8 /
+// 12.5, 1 x 1024 x 16 x 64 23.9 / 18.6 / 17.8, 2 x 777 x 32 x 64 20.7 / 16.9 / 16.9, 2 x 777 x 32 x 80 26.0 / 25.0 / 27.0. With more blocks than
+// units they read K and V more often: 4 x 2048 x 32 x 64 91.6 / 89.0 / 108, 4 x 2048 x 16 x 64 56 / 50 / 59, x 128 columns 88 / 98 / 126.
+template <typename HS>
+int fwd_waves(int64_t BH, int64_t S) {
+    const bool all64 = BH * ((S + 63) / 64) <= kUnits, all256 = BH * ((S + 255) / 256) <= kUnits;
+    if (HS::NP == 1) return all64 ? 2 : 4;
+    if (all64 && (HS::DT == 4 || S <= 128)) return 2;  // 1 x 777 x 16 x 80: 22.1 with 4, 23.4 with 2
+    return all256 ? 4 : 8;
+}
+
 int attn_fwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
              int64_t stride_b, int64_t stride_s, int64_t stride_h, float scale, int causal, void* out, int64_t out_stride_b,
              int64_t out_stride_s, int64_t out_stride_h, float* lse, int io_dtype, void* stream) {
     if (B == 0 || H == 0 || S == 0) return CW_OK;
     if (q == nullptr || k == nullptr || v == nullptr || out == nullptr) return fail(CW_ERR_INVALID, "%s: null pointer", who);
-    if (S > INT32_MAX / 2 || B * H > (1 << 20) || ((S + kQPerBlock - 1) / kQPerBlock) * B * H > INT32_MAX)
+    if (S > INT32_MAX / 2 || B * H > (1 << 20) || ((S + 255) / 256) * B * H > INT32_MAX)
         return fail(CW_ERR_INVALID, "%s: S or B*H too large", who);
     const bool aligned = aligned16(q) && aligned16(k) && aligned16(v) && (reinterpret_cast<uintptr_t>(out) & 7u) == 0 &&
                          stride_b % 8 == 0 && stride_s % 8 == 0 && stride_h % 8 == 0 && out_stride_b % 4 == 0 &&
@@ -295,15 +305,24 @@ int attn_fwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const 
     a.S = (int)S; a.H = (int)H; a.BH = (int)(B * H); a.D = (int)D;
     a.scale_log2e = scale * kLog2e;
     a.causal = causal ? 1 : 0;
-    a.n_qblocks = (int)((S + kQPerBlock - 1) / kQPerBlock);
-    const dim3 grid((unsigned)(a.n_qblocks * B * H));
     if (const int drc = require_gfx950(who); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
     return with_head_shape(D, [&](auto hs) {
         using HS = decltype(hs);
-        if (io_dtype == CW_F16) hipLaunchKernelGGL((attn_fwd_kernel<HS, f16_t>), grid, dim3(kThreads), 0, s, a);
-        else hipLaunchKernelGGL((attn_fwd_kernel<HS, bf16_t>), grid, dim3(kThreads), 0, s, a);
-        return check_launch("attn_fwd_kernel");
+        const int waves = fwd_waves<HS>(B * H, S);
+        auto launch = [&](auto w) {
+            constexpr int W = decltype(w)::value;
+            a.n_qblocks = (int)((S + W * kQPerWave - 1) / (W * kQPerWave));
+            const dim3 grid((unsigned)(a.n_qblocks * B * H));
+            if (io_dtype == CW_F16) hipLaunchKernelGGL((attn_fwd_kernel<HS, W, f16_t>), grid, dim3(64 * W), 0, s, a);
+            else hipLaunchKernelGGL((attn_fwd_kernel<HS, W, bf16_t>), grid, dim3(64 * W), 0, s, a);
+            return check_launch("attn_fwd_kernel");
+        };
+        if (waves == 2) return launch(std::integral_constant<int, 2>{});
+        if constexpr (HS::NP == 2) {
+            if (waves == 8) return launch(std::integral_constant<int, 8>{});
+        }
+        return launch(std::integral_constant<int, 4>{});
     });
 }
 

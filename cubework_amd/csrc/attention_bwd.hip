@@ -9,13 +9,13 @@
 // reference (scaled bmm, mask, softmax, bmm).
 //
 // Two kernels, no atomics (results are bit-reproducible):
-//   attn_dq_kernel    : a block owns 256 query rows (32 per wavefront, Q and dO
+//   attn_dq_kernel    : a block owns 64, 128 or 256 query rows (32 per wavefront, Q and dO
 //                       fragments in registers; D_i from them and the same rows
 //                       of O, also left in scratch for the second kernel) and
 //                       walks the K/V tiles; all
 //                       products are formed transposed (lane = query row), so
 //                       L_i and D_i are per-lane scalars.
-//   attn_dkdv_kernel  : a block owns 256 key rows (32 per wavefront, K and V
+//   attn_dkdv_kernel  : a block owns 64, 128 or 256 key rows (32 per wavefront, K and V
 //                       fragments in registers) and walks the Q/dO tiles;
 //                       products are formed with lane = key row.
 // In both, the fp32 probabilities / score gradients of a lane, rounded to
@@ -31,11 +31,8 @@ namespace {
 
 using namespace attn;
 
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * 64;
 constexpr int kRowsPerWave = 32;
-constexpr int kRowsPerBlock = kWaves * kRowsPerWave;
-// dK/dV kernel: 4 wavefronts (128 keys) per workgroup. At head size 64 a wavefront needs 218 registers and two
+// dK/dV kernel: 4 wavefronts (128 keys) per workgroup (bwd_waves: fewer of few blocks). At head size 64 a wavefront needs 218 registers and two
 // workgroups share a compute unit (two wavefronts per SIMD, 2 x 65 KB of LDS): they run out of step, so that one's
 // MFMA groups overlap the other's vector work, where the 8 wavefronts of one workgroup met at a barrier per tile
 // and ran the same phase at the same time (302 -> 291 us for the whole backward at batch 4 x 32 heads x 2048
@@ -43,9 +40,8 @@ constexpr int kRowsPerBlock = kWaves * kRowsPerWave;
 // of 32 keys per wavefront (every LDS operand read feeding two MFMAs, 510 registers) ran 278 us against 190 us.
 // Heads of 65 to 80 columns also leave room for one workgroup only (130 KB of LDS), but need no more than 256 registers:
 // 8 wavefronts then share the workgroup's tiles, two per SIMD. Whole backward at 32 heads of 80, 4 against 8
-// wavefronts: 4 x 1500 tokens 344 -> 290 us, 8 x 200 tokens 48 -> 42 us, 2 x 777 tokens 80 and 81 us. At head size 128
+// wavefronts: 4 x 1500 tokens 344 -> 290 us, 2 x 777 tokens 80 and 81 us. At head size 128
 // the same would spill (4 x 512 tokens 81 -> 100 us).
-constexpr int kDkdvWaves = 4;
 
 struct BwdArgs {
     const uint16_t* q;
@@ -69,11 +65,11 @@ struct BwdArgs {
 
 // ---- dQ ---------------------------------------------------------------------
 // LDS per stage: K row images, K transpose images, V row images (NP panels of 64 columns of each).
-template <typename HS, typename E>
-__global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
+template <typename HS, int W, typename E>
+__global__ __launch_bounds__(64 * W, 1) void attn_dq_kernel(const BwdArgs a) {
     constexpr int NP = HS::NP, KB = HS::KB, DT = HS::DT;
     constexpr bool MASK = HS::MASK;
-    constexpr int kStage = 3 * NP * kImage;
+    constexpr int kStage = 3 * NP * kImage, kRowsPerBlock = W * kRowsPerWave;
     __shared__ __attribute__((aligned(16))) char lds_raw[2 * kStage];
     lds_char* lds = (lds_char*)lds_raw;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, l32 = lane & 31;
@@ -126,7 +122,7 @@ __global__ __launch_bounds__(kThreads, 1) void attn_dq_kernel(const BwdArgs a) {
 
     ReadOffsets ro;
     ro.init(lane);
-    TileDma<kThreads> dma;
+    TileDma<64 * W> dma;
     dma.init(tid);
     const uint32_t lds_addr = (uint32_t)(uintptr_t)lds;
     // stage = K row images, K transpose images, V row images, filled by the load unit
@@ -438,21 +434,57 @@ __global__ __launch_bounds__(NW * 64, HS::NP == 1 ? 2 : 1) void attn_dkdv_kernel
     }
 }
 
+// Wavefronts of a dQ and of a dK/dV block: fewer of them where the blocks all fit the chip at once (of 32 rows each: 64, or 256 together), as
+// in the forward. us of both launches, bf16, causal, before (dQ 8, dK/dV 4, at 65 to 80 columns 8) / here (batch x tokens x heads x
+// columns): 1 x 300 x 32 x 64 25.5 / 20.7, 1 x 512 x 32 x 128 58.1 / 48.9, 1 x 512 x 32 x 80 52.3 / 40.5, 2 x 777 x 16 x 80 71.5 / 61.8, 4 x 512 x 16 x
+// 64 36.3 / 32.7, 1 x 2048 x 32 x 64 101 / 98.9. Beyond, dQ of 4: 4 x 1024 x 32 x 64 95.1 / 95.1, 4 x 2048 x 32 x 64 272 / 284; at 80 columns and 256
+// blocks of 256 rows 2 x 777 x 32 75.9 / 79.5 (dK/dV of 4 73.7, but 4 x 512 x 32 60.6 / 65.4).
+struct BwdWaves {
+    int dq, dkdv;
+};
+template <typename HS>
+BwdWaves bwd_waves(int64_t BH, int64_t S) {
+    const bool all64 = BH * ((S + 63) / 64) <= kUnits;
+    const int64_t blocks = BH * ((S + 255) / 256);
+    if (HS::KB == 5) return all64 ? BwdWaves{2, 2} : blocks <= kUnits / 2 ? BwdWaves{4, 4} : BwdWaves{8, 8};
+    return BwdWaves{all64 && HS::NP == 1 ? 2 : blocks <= kUnits ? 4 : 8, all64 ? 2 : 4};
+}
+
 // The two launches of the backward for element type E.
 template <typename E>
-int launch_bwd(const BwdArgs& a, int64_t B, int64_t H, int64_t S, int64_t D, int64_t nblk, hipStream_t s) {
+int launch_bwd(BwdArgs a, int64_t B, int64_t H, int64_t S, int64_t D, hipStream_t s) {
     return with_head_shape(D, [&](auto hs) {
         using HS = decltype(hs);
-        hipLaunchKernelGGL((attn_dq_kernel<HS, E>), dim3((unsigned)(nblk * B * H)), dim3(kThreads), 0, s, a);
-        if (const int rc = check_launch("attn_dq_kernel"); rc != CW_OK) return rc;
-        constexpr int NW = HS::KB == 5 ? 2 * kDkdvWaves : kDkdvWaves;
-        const int64_t nkv = (S + NW * kRowsPerWave - 1) / (NW * kRowsPerWave);
-        if (nkv * B * H > INT32_MAX) return fail(CW_ERR_INVALID, "cw_attn_bwd: S or B*H too large");
-        constexpr int lds_bytes = 2 * dkdv_stage_bytes<HS::NP>();
-        auto kern = attn_dkdv_kernel<HS, NW, 1, E>;
-        if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)(lds_bytes), "attn_dkdv_kernel"); lrc != CW_OK) return lrc;
-        hipLaunchKernelGGL(kern, dim3((unsigned)(nkv * B * H)), dim3(NW * 64), lds_bytes, s, a);
-        return check_launch("attn_dkdv_kernel");
+        const BwdWaves waves = bwd_waves<HS>(B * H, S);
+        auto dq = [&](auto w) {
+            constexpr int W = decltype(w)::value;
+            a.n_blocks = (int)((S + W * kRowsPerWave - 1) / (W * kRowsPerWave));
+            hipLaunchKernelGGL((attn_dq_kernel<HS, W, E>), dim3((unsigned)(a.n_blocks * B * H)), dim3(64 * W), 0, s, a);
+            return check_launch("attn_dq_kernel");
+        };
+        constexpr std::integral_constant<int, 2> two{};
+        constexpr std::integral_constant<int, 4> four{};
+        constexpr std::integral_constant<int, 8> eight{};
+        int rc = CW_OK;
+        if (waves.dq == 8) rc = dq(eight);
+        else if (waves.dq == 4) rc = dq(four);
+        else if constexpr (HS::KB <= 5) rc = dq(two);
+        if (rc != CW_OK) return rc;
+        auto dkdv = [&](auto w) {
+            constexpr int NW = decltype(w)::value;
+            const int64_t nkv = (S + NW * kRowsPerWave - 1) / (NW * kRowsPerWave);
+            if (nkv * B * H > INT32_MAX) return fail(CW_ERR_INVALID, "cw_attn_bwd: S or B*H too large");
+            constexpr int lds_bytes = 2 * dkdv_stage_bytes<HS::NP>();
+            auto kern = attn_dkdv_kernel<HS, NW, 1, E>;
+            if (const int lrc = ensure_dynamic_lds((const void*)kern, (int)(lds_bytes), "attn_dkdv_kernel"); lrc != CW_OK) return lrc;
+            hipLaunchKernelGGL(kern, dim3((unsigned)(nkv * B * H)), dim3(NW * 64), lds_bytes, s, a);
+            return check_launch("attn_dkdv_kernel");
+        };
+        if (waves.dkdv == 2) return dkdv(two);
+        if constexpr (HS::KB == 5) {
+            if (waves.dkdv == 8) return dkdv(eight);
+        }
+        return dkdv(four);
     });
 }
 
@@ -480,8 +512,7 @@ int attn_bwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const 
         return fail(CW_ERR_INVALID, "%s: null pointer", who);
     if (workspace_bytes < cw_attn_bwd_workspace_bytes(B, H, S))
         return fail(CW_ERR_INVALID, "%s: workspace too small (%lld bytes)", who, (long long)workspace_bytes);
-    const int64_t nblk = (S + kRowsPerBlock - 1) / kRowsPerBlock;
-    if (S > INT32_MAX / 2 || B * H > (1 << 20) || nblk * B * H > INT32_MAX)
+    if (S > INT32_MAX / 2 || B * H > (1 << 20) || ((S + 255) / 256) * B * H > INT32_MAX)
         return fail(CW_ERR_INVALID, "%s: S or B*H too large", who);
     const bool aligned = aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out) && aligned16(d_out) &&
                          stride_b % 8 == 0 && stride_s % 8 == 0 && stride_h % 8 == 0 && out_stride_b % 8 == 0 &&
@@ -501,13 +532,13 @@ int attn_bwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const 
     a.sb = stride_b; a.ss = stride_s; a.sh = stride_h;
     a.ob = out_stride_b; a.os = out_stride_s; a.oh = out_stride_h;
     a.gb = grad_stride_b; a.gs = grad_stride_s; a.gh = grad_stride_h;
-    a.S = (int)S; a.H = (int)H; a.BH = (int)(B * H); a.n_blocks = (int)nblk;
+    a.S = (int)S; a.H = (int)H; a.BH = (int)(B * H); 
     a.scale = scale; a.scale_log2e = scale * kLog2e;
     a.causal = causal ? 1 : 0;
     a.D = (int)D;
     if (const int drc = require_gfx950(who); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
-    return io_dtype == CW_F16 ? launch_bwd<f16_t>(a, B, H, S, D, nblk, s) : launch_bwd<bf16_t>(a, B, H, S, D, nblk, s);
+    return io_dtype == CW_F16 ? launch_bwd<f16_t>(a, B, H, S, D, s) : launch_bwd<bf16_t>(a, B, H, S, D, s);
 }
 
 }  // namespace

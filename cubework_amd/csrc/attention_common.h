@@ -20,6 +20,7 @@ typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x8_t __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) char lds_char;
 
+constexpr int kUnits = 256;                // compute units
 constexpr int kHead = 64;                  // columns of one LDS image (a head of 128 is two images side by side)
 constexpr int kTile = 64;                  // rows of a streamed tile
 constexpr int kImage = kTile * kHead * 2;  // 8 KB: one LDS image of a tile

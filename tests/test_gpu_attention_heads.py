@@ -60,3 +60,15 @@ def test_unaligned_rows(d, form):
     for a, e in zip(got, want):
         # the padded copy adds products with zeros only; its 64 or 128 columns are the same sums
         assert_parity(a, e.float(), torch.bfloat16, "unaligned %s, head size %d" % (form, d))
+
+
+@pytest.mark.parametrize("D", [48, 56, 64, 80, 96, 128])
+@pytest.mark.parametrize("B,H,S,causal", [(9, 16, 130, True), (5, 16, 257, True), (5, 32, 300, False), (18, 16, 130, True), (17, 16, 260, True)])
+def test_blocks_of_any_number_of_wavefronts_give_the_same_bits(B, H, S, D, causal):
+    """A batch on each side of the rules that choose a block's wavefronts, against its sequences one by one: whole batches run on blocks of 4
+    or 8, single sequences on blocks of 2 or 4."""
+    qkv, d_out = randn((B, S, H * 3 * D), torch.bfloat16, D + S, device=DEV), randn((B, S, H * D), torch.bfloat16, D, device=DEV)
+    whole = _run(qkv, H, d_out, causal)
+    for b in (0, B - 1):
+        for one, all_of in zip(_run(qkv[b:b + 1].contiguous(), H, d_out[b:b + 1].contiguous(), causal), whole):
+            assert torch.equal(one, all_of[b:b + 1])
