@@ -551,14 +551,24 @@ __global__ __launch_bounds__(kThreads) void tile_reduce_kernel(const TileArgs ar
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[j][e] = 0.0f;
     const float* part = args.partial + (int64_t)r * (BM * BN) + (int64_t)slab * (TN * 4 * kThreads * 4) + tid * 4;
-    for (int z = 0; z < args.slices; ++z, part += (int64_t)rest * (BM * BN)) {
+    // several slices' pieces requested together: a launch of a few tiles waits for memory alone
+    constexpr int kAhead = TN == 4 ? 2 : 4;
+    const int64_t slice = (int64_t)rest * (BM * BN);
+    for (int z = 0; z < args.slices; z += kAhead, part += kAhead * slice) {
+        raw16_t u[kAhead][TN * 4];
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int a = 0; a < kAhead; ++a) {
+            const float* p = part + (z + a < args.slices ? a * slice : 0);
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const raw16_t u = load_raw_stream(part + (j * 4 + g) * (kThreads * 4));
+            for (int i = 0; i < TN * 4; ++i) u[a][i] = load_raw_stream(p + i * (kThreads * 4));
+        }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[j][4 * g + e] += __uint_as_float(u[e]);
+        for (int a = 0; a < kAhead; ++a)
+            if (z + a < args.slices) {
+#pragma unroll
+                for (int i = 0; i < TN * 4; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i / 4][4 * (i % 4) + e] += __uint_as_float(u[a][i][e]);
             }
     }
     int buf = 0;
