@@ -291,7 +291,10 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         if (max_scratch >= 0 && q.scratch() > max_scratch) return;
         // TN on the kernels of gemm_tile.h: k-contiguous operands move as pieces of 64 bytes, k-slow ones as whole lines. On the
         // paired one: the two groups' transposing reads take more LDS cycles than their products.
-        const double layout_factor = cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9;
+        // 64 x 128 tiles of an NT product, at most one a unit: both operands move as whole lines, where the costs were fitted to pieces of 64 bytes
+        // (us, M x N x K, as chosen before / such tiles: 1554 x 768 x 2304 20.3 / 16.0, 489 x 2560 x 2560 22.5 / 17.4, 2561 x 768 x 3072 25.8 / 21.5).
+        const double lines_factor = cfg == 3 && layout == CW_NT && full == tiles && tiles <= 256 ? 0.86 : 1.0;
+        const double layout_factor = lines_factor * (cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9);
         // Rows that are not whole 128-byte lines cost the paired kernel's loads more the longer a block walks along them (us, M x N x K):
         // whole tiles, paired / 256 x 256 in slices: 4096 x 1024 x 4104 NT 41 / 44, 4000 x 1000 x 8200 NT 70 / 81, 4096 x 1024 x 12568 NN
         // 131 / 104; the blocks of a sliced product are short, paired / 128 x 128 of one group: 1023 x 768 x 50257 NN in 5 slices 99 / 111,
@@ -303,9 +306,13 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         if (rows != 64 * c.tm) trips *= 0.2 + 0.8 * rows / (64 * c.tm);
         // The kernels of gemm_wide.h: 4 us a tile, whose stores drain under the next one's products, and 3 us for the last one's. Their
         // reduction waits about 0.9 us a slice whatever its size, and its bytes come from the cache.
+        // The small tiles' waits less for a slice, but priced as if it did not, outputs of few rows were cut into up to 16 of them (us, M x N x K,
+        // NT, before / now: 58 x 876 x 3712 13.1 / 10.7, 49 x 896 x 2752 12.1 / 10.1, 185 x 768 x 2304 11.4 / 10.1). Of 2415 shapes of the layers in
+        // every configuration this and lines_factor make 109 more than 3 % faster and none slower, all 0.5 % on average. (TN, whose k-slow
+        // operands always moved as lines: as fitted.)
         const bool walks = cfg == 0 || cfg >= kPairedConfig;
         double us = tile_rounds(c, (double)full, trips, layout_factor * pitch_factor(trips)) + (walks && full > 0 ? 3.0 : 0.0);
-        double reduce_us = (walks ? 2.0 + 0.9 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
+        double reduce_us = (walks ? 2.0 + 0.9 * slices : layout != CW_TN ? 3.0 + 0.3 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
         // Weight gradients cut in many slices of 256 x 256 tiles: all blocks write their partial sums at once and have walked little besides
         // (us, M x N x K, TN, on such slices / as chosen now): 768 x 3072 x 4416 42.7 / 35.2, 3072 x 768 x 5295 46.4 / 38.4, 1024 x 3072 x
         // 6080 53.4 / 43.5; from some 11000 of k on both are alike. Not so with k-contiguous A: 660 x 4096 x 12288 NT 71 / 78.

@@ -46,6 +46,19 @@ def test_long_rows_in_long_blocks_leave_the_paired_kernel(plans):
     assert cfg != PAIRED
 
 
+@pytest.mark.parametrize("M,N,K", [(1554, 768, 2304), (489, 2560, 2560), (2561, 768, 3072)])
+def test_input_gradients_of_one_round_take_64_x_128_tiles(plans, M, N, K):
+    """At most 256 tiles of 64 x 128, whose operands move as whole lines: 17 to 23 % faster than slices of the paired kernel's."""
+    assert plans([("NT", M, N, K, 1)]) == [(3, 64, -(-M // 64) * -(-N // 128), 1, 0)]
+
+
+@pytest.mark.parametrize("M,N,K", [(58, 876, 3712), (49, 896, 2752), (185, 768, 2304)])
+def test_few_rows_are_not_cut_into_more_slices_than_pay(plans, M, N, K):
+    """Every slice is a wait of the reduction: 4 to 6 are 11 to 18 % faster than the 7 to 15 that fill the chip."""
+    (cfg, _, full, slices, _), = plans([("NT", M, N, K, 1)])
+    assert (cfg, full) == (4, 0) and 3 <= slices <= 6
+
+
 @pytest.mark.parametrize("layout,M,N,K", [("NT", 2394, 576, 1536), ("NT", 1894, 1024, 1024), ("NT", 1280, 1024, 1024), ("NN", 1777, 768, 768),
                                           ("NN", 473, 3072, 768), ("NN", 351, 3072, 1024)])
 def test_short_products_of_one_round_take_64_x_128_tiles(plans, layout, M, N, K):
