@@ -56,8 +56,12 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
     return static_cast<uint32_t>(__builtin_bit_cast(uint16_t, b));
 }
 
+// Two in one v_cvt_pk_bf16_f32; converted one by one they are two of them, a shift and an or. The epilogues and the softmax of
+// attention issue one per pair of results.
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo, hi}), bf16x2_t));
 }
 
 // fp16 <-> fp32: v_cvt_f32_f16 is exact, v_cvt_f16_f32 rounds to nearest even (the mode the kernels run in),
@@ -70,8 +74,7 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float f) {
 }
 __device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {
     typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-    const half2_t h = {static_cast<_Float16>(lo), static_cast<_Float16>(hi)};
-    return __builtin_bit_cast(uint32_t, h);
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t{lo, hi}), half2_t));  // v_cvt_pk_f16_f32
 }
 
 // The two 16-bit element types share every kernel; what differs is the conversion.

@@ -50,6 +50,7 @@ namespace gemm_wide {
 using gemm_bf16::bf16x8_t;
 using gemm_bf16::static_for;
 using gemm_bf16::u32x4_t;
+using gemm_tile::u32x2_t;
 using gemm_tile::kRange;
 using gemm_tile::kTabA;
 using gemm_tile::kTabAddend;
@@ -161,41 +162,40 @@ struct Frags {
     }
 };
 
-// What follows the sums: a wavefront's accumulators go through LDS of its own, one row of TN MFMA tiles (16 x 16 TN fp32)
-// at a time, and come back as 8 columns of a row per lane: bias, addends and results move as 16 bytes per lane, 128-byte
+// What follows the sums: a wavefront's accumulators go through LDS of its own, one row of TN MFMA tiles (16 x 16 TN)
+// at a time, and come back as 8 columns of a row per lane: addends and results move as 16 bytes per lane, 128-byte
 // lines per 8 lanes (TN = 2: 64 bytes per 4), edges are a matter of one lane, and no accumulator is copied to another register.
-// Chunk c (4 columns) of row r stands at c ^ r.
+// With addends, and for TN = 2, the sums go through as fp32: chunk c (4 columns) of row r stands at c ^ r. Without addends TN = 4
+// applies bias and activation first and sends rounded results, half of the bytes, chunk c (8 columns) of row r at c ^ (r / 2). No load
+// runs beside any of this, so its instructions count: rounded results, a pair of them converted at a time and addresses of whole tiles
+// as a scalar took 4096 x 3072 x 768 from 27.2 / 26.7 / 28.0 us (NN / NT / TN) to 25.6 / 24.9 / 26.5, 8192 x 10240 x 2560 from 324 / 325 /
+// 335 to 322 / 317 / 325, GELU of 4096 x 3072 x 768 from 30.6 to 29.5. TN = 2 gains nothing by it (1554 x 10240 x 2560 NN 97.6 -> 98.6).
 template <int TN, int EPI, typename E>
 struct Out {
     static constexpr int kPitch = 64 * TN, kPatch = 16 * kPitch;  // bytes of a row, of the wavefront's patch
     static constexpr int LPR = 2 * TN, kHalves = TN / 2, kHalfRows = 64 / LPR;  // lanes of a row, passes, rows of a pass
     static_assert(TN == 2 || TN == 4, "");
-    lds_char *wr, *rd;  // the lane's addresses in the wavefront's patch
+    static constexpr int kPitch16 = 128, kPatch16 = 16 * kPitch16;  // the same of rounded results (TN = 4): two patches of a half
+    lds_char *wr, *rd;      // the lane's addresses in the wavefront's patch
+    lds_char *wr16, *rd16;  // the same of rounded results
+    int col4;               // the lane's first column of the accumulators
+    int row0, col0;         // of the wavefront
     int row, col, M, N;  // of the lane's piece in half 0 of row 0 of the tiles
+    static constexpr int64_t kFastPitch = 1 << 26;  // 16 rows' offset in 32 bits
     bool whole;
-    u32x4_t bias;
-    __device__ __forceinline__ Out(const TileArgs& a, lds_char* patch, int row0, int col0, bool whole_tile, int lane) {
+    __device__ __forceinline__ Out(const TileArgs& a, lds_char* patch, int row0, int col0, bool whole_tile, int lane) : row0(row0), col0(col0) {
         asm volatile("" : "+v"(lane));  // opaque: nothing of this is kept in registers between tiles
         const int r = lane & 15, q = lane >> 4, rr = lane / LPR, c = lane % LPR, m = 4 * TN - 1;
         wr = patch + r * kPitch + ((q ^ (r & m)) << 4);
         rd = patch + rr * kPitch + (((2 * c) ^ (rr & m)) << 4);
+        wr16 = patch + r * kPitch16 + (((q >> 1) ^ (r >> 1)) << 4) + 8 * (q & 1);
+        rd16 = patch + rr * kPitch16 + ((c ^ (rr >> 1)) << 4);
+        col4 = col0 + 4 * q;
         row = row0 + rr;
         col = col0 + 8 * c;
         M = a.M;
         N = a.N;
         whole = whole_tile;
-        bias = u32x4_t{0u, 0u, 0u, 0u};
-        if (a.bias != nullptr) {
-            const uint16_t* b = reinterpret_cast<const uint16_t*>(a.bias) + col;
-            if (whole && ((uintptr_t)a.bias & 15) == 0) {
-                bias = *reinterpret_cast<const u32x4_t*>(b);
-            } else {
-                uint32_t w[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) w[e] = col + e < N ? b[e] : 0u;
-                bias = u32x4_t{w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16};
-            }
-        }
     }
     static __device__ __forceinline__ lds_char* flip(lds_char* p, uint32_t bits) { return (lds_char*)(uintptr_t)((uint32_t)(uintptr_t)p ^ bits); }
     __device__ __forceinline__ void put(const f32x4_t (&acc)[TN]) const {
@@ -231,6 +231,9 @@ struct Out {
         u32x4_t o;
 #pragma unroll
         for (int d = 0; d < 4; ++d) o[d] = half_conv<E>::pack2(v[2 * d], v[2 * d + 1]);
+        store_piece(o, dst, ld, r);
+    }
+    __device__ __forceinline__ void store_piece(u32x4_t o, void* dst, int64_t ld, int r) const {
         uint16_t* out = reinterpret_cast<uint16_t*>(dst) + (int64_t)r * ld + col;
         if (whole) {
             *reinterpret_cast<u32x4_t*>(out) = o;
@@ -251,10 +254,107 @@ struct Out {
         for (int e = 0; e < 8; ++e) v[e] = gemm_tile::tile_act<EPI>(v[e]);
         store(v, a.C, a.ldc, r);
     }
+    // of the lane's piece
+    __device__ __forceinline__ u32x4_t bias8(const TileArgs& a) const {
+        if (a.bias == nullptr) return u32x4_t{0u, 0u, 0u, 0u};
+        const uint16_t* b = reinterpret_cast<const uint16_t*>(a.bias) + col;
+        if (whole && ((uintptr_t)a.bias & 15) == 0) return *reinterpret_cast<const u32x4_t*>(b);
+        uint32_t w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = col + e < N ? b[e] : 0u;
+        return u32x4_t{w[0] | w[1] << 16, w[2] | w[3] << 16, w[4] | w[5] << 16, w[6] | w[7] << 16};
+    }
+    // bias and activation where the sums are: a lane has 4 columns of a row in each MFMA tile
+    template <bool ACT, bool BIAS>
+    __device__ __forceinline__ void put_rounded(const f32x4_t (&acc)[TN], const u32x2_t (&bias4)[TN], int buf) const {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            f32x4_t v = acc[j];
+            if constexpr (BIAS) {
+                v[0] += half_conv<E>::lo(bias4[j].x);
+                v[1] += half_conv<E>::hi(bias4[j].x);
+                v[2] += half_conv<E>::lo(bias4[j].y);
+                v[3] += half_conv<E>::hi(bias4[j].y);
+            }
+            if constexpr (ACT) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = gemm_tile::tile_act<EPI>(v[e]);
+            }
+            *(__attribute__((address_space(3))) u32x2_t*)(flip(wr16, 32 * j) + buf * kPatch16) =
+                u32x2_t{half_conv<E>::pack2(v[0], v[1]), half_conv<E>::pack2(v[2], v[3])};
+        }
+    }
+    // row I of the tiles; FAST: of a whole tile, whose addresses are a scalar and one offset of the lane
+    template <int I, bool FAST>
+    __device__ __forceinline__ void store_rounded(int buf, void* dst, int64_t ld, int r) const {
+        u32x4_t o[kHalves];
+#pragma unroll
+        for (int h = 0; h < kHalves; ++h) o[h] = *(__attribute__((address_space(3))) const u32x4_t*)(flip(rd16, 64 * h) + h * 1024 + buf * kPatch16);
+#pragma unroll
+        for (int h = 0; h < kHalves; ++h) {
+            if constexpr (FAST) {
+                char* base = reinterpret_cast<char*>(dst) + 2 * ((int64_t)(row0 + 16 * I + kHalfRows * h) * ld + col0);
+                *reinterpret_cast<u32x4_t*>(base + 2u * ((uint32_t)(row - row0) * (uint32_t)ld + (uint32_t)(col - col0))) = o[h];
+            } else {
+                store_piece(o[h], dst, ld, r + kHalfRows * h);
+            }
+        }
+    }
+    template <bool FAST, bool BIAS, bool PREACT, int TM>
+    __device__ __forceinline__ void walk_rounded(const f32x4_t (&acc)[TM][TN], const u32x2_t (&bias4)[TN], const TileArgs& a) const {
+        if constexpr (!PREACT) put_rounded<true, BIAS>(acc[0], bias4, 0);
+        static_for<TM>([&](auto i) {
+            constexpr int I = i.value;
+            int r = row + 16 * I;
+            asm volatile("" : "+v"(r));  // opaque: the addresses of a row are formed here and not for all rows at once
+            if constexpr (PREACT) {
+                put_rounded<false, BIAS>(acc[I], bias4, 0);
+                put_rounded<true, BIAS>(acc[I], bias4, 1);
+                store_rounded<I, FAST>(0, a.preact, a.ldp, r);
+                store_rounded<I, FAST>(1, a.C, a.ldc, r);
+            } else {
+                if constexpr (I + 1 < TM) put_rounded<true, BIAS>(acc[I + 1], bias4, (I + 1) & 1);
+                store_rounded<I, FAST>(I & 1, a.C, a.ldc, r);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    }
+    template <int TM>
+    __device__ __forceinline__ void rows_rounded(const f32x4_t (&acc)[TM][TN], const TileArgs& a) const {
+        u32x2_t bias4[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int c = col4 + 16 * j;
+            const uint16_t* b = reinterpret_cast<const uint16_t*>(a.bias) + c;
+            bias4[j] = u32x2_t{0x80008000u, 0x80008000u};  // no bias: -0, which changes no sum, not even one of -0
+            if (a.bias != nullptr) {
+                if (whole && ((uintptr_t)a.bias & 7) == 0) {
+                    bias4[j] = *reinterpret_cast<const u32x2_t*>(b);
+                } else {
+                    uint32_t w[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) w[e] = c + e < N ? b[e] : 0u;
+                    bias4[j] = u32x2_t{w[0] | w[1] << 16, w[2] | w[3] << 16};
+                }
+            }
+        }
+        const bool fast = whole && a.ldc < kFastPitch && (a.preact == nullptr || a.ldp < kFastPitch);
+        // whole tiles have walks of their own, edges share one: a -0 as the bias of none costs 1 us a tile where all take it
+        if (fast && a.preact == nullptr && a.bias == nullptr) return walk_rounded<true, false, false>(acc, bias4, a);
+        if (fast && a.preact == nullptr) return walk_rounded<true, true, false>(acc, bias4, a);
+        if constexpr (EPI != CW_EPI_BIAS)
+            if (fast) return walk_rounded<true, true, true>(acc, bias4, a);
+        if (a.preact == nullptr) walk_rounded<false, true, false>(acc, bias4, a);
+        else walk_rounded<false, true, true>(acc, bias4, a);
+    }
     template <int TM>
     __device__ __forceinline__ void rows(const f32x4_t (&acc)[TM][TN], const TileArgs& a) const {
+        if constexpr (TN == 4) {
+            if (a.n_addends == 0) return rows_rounded(acc, a);
+        }
+        const u32x4_t bias = bias8(a);
         put(acc[0]);
-        if (a.n_addends == 0) {
+        if (TN == 2 && a.n_addends == 0) {
             static_for<TM>([&](auto i) {
                 float v[kHalves][8];
                 static_for<kHalves>([&](auto h) { get<h.value>(v[h.value]); });

@@ -113,3 +113,30 @@ def test_rows_that_end_inside_16_bytes(layout, shape):
     want = sum(a[rows].double() @ (b.double().t().contiguous() if layout == "NT" else b.double()) for a, b in zip(A, B))
     assert_parity(got[rows], want, torch.bfloat16, "%s %s" % (layout, shape))
     assert bool(torch.isfinite(got).all())
+
+
+# without addends rounded results go through LDS: tiles that lie whole in C and ones that don't (M, N, odd N), every height, sliced tiles;
+# the bias absent, 16-byte aligned, 8-byte aligned, and neither; with and without the sums before the activation. Whole numbers: the sums
+# are exact in fp32 (at most 9 K + 64 < 2^24), so every result is the exact one rounded once.
+@pytest.mark.parametrize("shape", [(8192, 2048, 512), (8184, 2040, 328), (1552, 7672, 1352), (300, 32767, 1016), (7000, 4600, 1000), (4352, 4096, 1024)], ids=str)
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_results_of_no_addends(layout, shape, dtype):
+    from cubework_amd import ops
+
+    M, N, K = shape
+    gen = torch.Generator().manual_seed(M + N)
+    whole = lambda *s: torch.randint(-3, 4, s, generator=gen).to(dtype).cuda()  # noqa: E731
+    A = whole(*((K, M) if layout == "TN" else (M, K)))
+    B = whole(N, K) if layout == "NT" else whole(K, N + -N % 8)[:, :N]
+    sums = (A.t() if layout == "TN" else A).float() @ (B.t() if layout == "NT" else B).float()
+    many = torch.randint(-64, 65, (N + 8,), generator=gen).to(dtype).cuda()
+    for skip, act, preact in ((None, None, False), (0, None, False), (4, "relu", True), (1, "relu", False), (None, "relu", True), (0, "relu", True)):
+        if layout == "TN" and act is not None:
+            continue
+        bias = None if skip is None else many[skip:skip + N]
+        want = sums if bias is None else sums + bias.float()
+        got = ops.gemm_ksteps(layout, [A], [B], bias, act, [], want_preact=preact)
+        out, pre = got if preact else (got, None)
+        assert torch.equal(out, (want if act is None else want.relu()).to(dtype)), (skip, act, preact)
+        assert pre is None or torch.equal(pre, want.to(dtype)), (skip, act, preact)
