@@ -312,12 +312,28 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         // operands always moved as lines: as fitted.)
         const bool walks = cfg == 0 || cfg >= kPairedConfig;
         double us = tile_rounds(c, (double)full, trips, layout_factor * pitch_factor(trips)) + (walks && full > 0 ? 3.0 : 0.0);
-        double reduce_us = (walks ? 2.0 + 0.9 * slices : layout != CW_TN ? 3.0 + 0.3 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
+        // All tiles of an output of more than 128 rows and columns sliced: behind the eighth slice the reduction, which requests four together,
+        // waits a tenth of that, and up to 32 slices are tried (us, M x N x K, NN, up to 16 / as chosen now): 1023 x 768 x 50257 121 / 90
+        // (TN 102 / 86, NT 143 / 103), 1280 x 408 x 50304 94 / 75, 178 x 1536 x 51072 66 / 48, 391 x 2048 x 32000 81 / 66. Of 330 products of
+        // a long k and of the 2415 shapes of the layers this and the slower walks below make 33 more than 3 % faster and none slower. Fewer
+        // rows or columns are left to the small tiles: 34 x 3072 x 56535 TN 72 / 87.
+        const bool deep = full == 0 && M > 128 && N > 128;
+        const double waits = deep && slices > 8 ? 7.2 + 0.1 * (slices - 8) : 0.9 * slices;
+        double reduce_us = (walks ? 2.0 + waits : layout != CW_TN ? 3.0 + 0.3 * slices : 5.0) + (walks ? 1.2 : 2.0) * q.partial_bytes / 6.6e6 * q.rows / (64 * c.tm);
+        // Slices of the paired kernel slow down from some 50 trips on (NN at any pitch; NT, from 60, off the 128-byte lines; measured / priced without:
+        // 1.19 in the median of 40 to 59 trips of NN, 1.28 of 60 to 79; 2048 x 512 x 30001 NT in 4 of 59 trips 94, of 256 x 256 tiles 100).
+        auto slice_factor = [&](double block_trips) {
+            const double pitch = pitch_factor(block_trips), longer = (block_trips - (layout == CW_NN ? 48.0 : 56.0)) / 15.0;
+            const bool slows = layout == CW_NN || (layout == CW_NT && (p.lda % 64 != 0 || p.ldb % 64 != 0));
+            if (!deep || cfg != kPairedConfig || !slows || longer <= 0.0) return pitch;
+            const double slow = 1.0 + 0.25 * (longer < 1.0 ? longer : 1.0);
+            return pitch > slow ? pitch : slow;
+        };
         // Weight gradients cut in many slices of 256 x 256 tiles: all blocks write their partial sums at once and have walked little besides
         // (us, M x N x K, TN, on such slices / as chosen now): 768 x 3072 x 4416 42.7 / 35.2, 3072 x 768 x 5295 46.4 / 38.4, 1024 x 3072 x
         // 6080 53.4 / 43.5; from some 11000 of k on both are alike. Not so with k-contiguous A: 660 x 4096 x 12288 NT 71 / 78.
-        if (layout == CW_TN && cfg == 0 && full == 0 && slices > 3) reduce_us += 3.0 - 0.48 * slices + 0.37 * q.partial_bytes / 6.6e6 * q.rows / 256;
-        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor * pitch_factor(trips / slices)) + reduce_us;
+        if (layout == CW_TN && cfg == 0 && full == 0 && slices > 3) reduce_us += 3.0 - 0.48 * (slices < 16 ? slices : 16) + 0.37 * q.partial_bytes / 6.6e6 * q.rows / 256;
+        if (rest > 0) us += tile_rounds(c, (double)(rest * slices), trips / slices, layout_factor * slice_factor(trips / slices)) + reduce_us;
         // At most one 128 x 256 tile a unit and a short k: nothing hides a block's first loads and its stores, where 128 x 128 ones share the
         // unit (us, M x N x K, 128 x 256 / 128 x 128): 2820 x 1632 x 166 TN 11.3 / 8.9, 6243 x 832 x 256 NT 12.8 / 10.8; above 576 of k
         // the costs hold as they are.
@@ -350,7 +366,9 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         // all tiles sliced, to fill the chip about once; or only those of the partial last round
         if (ordered) return;
         const int64_t last = tiles % cap;
-        for (int slices = 2; slices <= 16; ++slices) {
+        // more of 256-column tiles and of 128-column ones of 160 or 192 rows, where so many slices of all tiles are one round (consider)
+        const int most = (cfg == 0 || cfg == kNarrowConfig) && M > 128 && N > 128 && tiles * 17 <= cap ? 32 : 16;
+        for (int slices = 2; slices <= most; ++slices) {
             if (trips / slices < least) break;
             if (tiles * slices <= cap) consider(cfg, rows, tiles, 0, slices);
             else if (tiles > cap && last > 0 && last * slices <= cap) consider(cfg, rows, tiles, tiles - last, slices);

@@ -66,6 +66,19 @@ def test_short_products_of_one_round_take_64_x_128_tiles(plans, layout, M, N, K)
     assert plans([(layout, M, N, K, 1)]) == [(3, 64, -(-M // 64) * -(-N // 128), 1, 0)]
 
 
+@pytest.mark.parametrize("layout,M,N,K", [("NN", 1023, 768, 50257), ("TN", 1023, 768, 50257), ("NT", 1023, 768, 50257), ("NN", 403, 1280, 50304)])
+def test_few_large_tiles_of_a_long_k_fill_the_chip(plans, layout, M, N, K):
+    """Sixteen slices of 10 or 12 tiles of 256 x 256 would leave a third of the units idle, and the paired kernel was chosen (up to 40 % slower)."""
+    (cfg, _, full, slices, rest), = plans([(layout, M, N, K, 1)])
+    assert (cfg, full) == (0, 0) and slices > 16 and slices * rest <= 256
+
+
+@pytest.mark.parametrize("M,N,K", [(34, 3072, 56535), (68, 2048, 50304), (128, 2048, 50257)])
+def test_few_rows_are_left_to_the_small_tiles(plans, M, N, K):
+    (cfg, _, _, slices, _), = plans([("TN", M, N, K, 1)])
+    assert cfg != 0 and slices <= 16
+
+
 @pytest.mark.parametrize("M,N,K", [(768, 3072, 4416), (3072, 768, 5295), (3072, 768, 6528), (1024, 3072, 6080)])
 def test_weight_gradients_are_not_cut_into_many_slices_of_large_tiles(plans, M, N, K):
     """Six or seven slices of 36 tiles of 256 x 256 took 20 % longer than three of 128 x 256 or whole 128 x 128 tiles."""

@@ -140,3 +140,19 @@ def test_results_of_no_addends(layout, shape, dtype):
         out, pre = got if preact else (got, None)
         assert torch.equal(out, (want if act is None else want.relu()).to(dtype)), (skip, act, preact)
         assert pre is None or torch.equal(pre, want.to(dtype)), (skip, act, preact)
+
+
+# more than 16 slices: 256-column tiles of 256 and 224 rows, 128-column ones of 192, slices of unequal lengths, a ragged last k. Products of
+# -1, 0 and 1, whose sums (at most K < 2^24) are exact in fp32 in any order.
+@pytest.mark.parametrize("layout,M,N,K", [("NN", 1023, 768, 50257), ("TN", 1023, 768, 50257), ("NT", 1023, 768, 50257), ("NN", 403, 1280, 50304),
+                                          ("NN", 178, 1536, 51072)])
+def test_many_slices(layout, M, N, K):
+    from cubework_amd import ops
+
+    gen = torch.Generator().manual_seed(K)
+    sign = lambda *s: torch.randint(-1, 2, s, generator=gen).bfloat16().cuda()  # noqa: E731
+    rows8 = lambda r, c: sign(r, c + -c % 8)[:, :c]  # noqa: E731
+    A = rows8(K, M) if layout == "TN" else rows8(M, K)
+    B = rows8(N, K) if layout == "NT" else rows8(K, N)
+    want = (A.t() if layout == "TN" else A).float() @ (B.t() if layout == "NT" else B).float()
+    assert torch.equal(ops.gemm_ksteps(layout, [A], [B]), want.bfloat16())
