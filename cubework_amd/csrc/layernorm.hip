@@ -594,6 +594,59 @@ __global__ __launch_bounds__(MAXW * 64) void ln_forward_split_kernel(
     }
 }
 
+// Fused forward of few rows: a wavefront for every one of a row's NCH chunks, one load a lane. The wavefronts leave their chunks in LDS and
+// each forms the row's sums from there itself, in the order of the kernel that has a wavefront for the whole row (tile_moments): the number of
+// rows decides which of the two runs, and a row has the same bits in any batch, as the products behind the layer promise (a
+// ReLU behind them sees the same signs). Bound by latency: a load, the barrier, the sums' chain. Registers for 6 wavefronts a SIMD, so that
+// the line below fits at once (6 chunks, 682 x 3072: 5.3 -> 4.3 us); 7 and 8 chunks would spill (512 x 4096: 4.4 -> 6.8).
+constexpr int kFwdShortWaves = 8;
+template <typename T, int NCH>
+__global__ __launch_bounds__(kFwdShortWaves * 64, NCH <= 6 ? 6 : 4) void ln_forward_short_kernel(int64_t R, int64_t C, const T* __restrict__ x, int64_t ld, int mode,
+                                                                              float inv_h, float eps, const T* __restrict__ gamma,
+                                                                              const T* __restrict__ beta, T* __restrict__ y, int64_t ldy,
+                                                                              float* __restrict__ mean_rstd) {
+    constexpr int V = elem<T>::kVec;
+    __shared__ raw16_t chunks[kFwdShortWaves][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, first = wave / NCH * NCH;  // wavefront of the row's first chunk
+    const int64_t row = (int64_t)blockIdx.x * (kFwdShortWaves / NCH) + wave / NCH;
+    const bool live = row < R, ok = chunk_valid<T>(wave - first, lane, C);
+    const int64_t c0 = ok ? ((int64_t)(wave - first) * 64 + lane) * V : 0;
+    const raw16_t zero = {0u, 0u, 0u, 0u};
+    const raw16_t own = load_raw_stream(x + (live ? row : R - 1) * ld + c0);
+    const raw16_t g_raw = gamma != nullptr ? load_raw(gamma + c0) : zero, b_raw = beta != nullptr ? load_raw(beta + c0) : zero;
+    chunks[wave][lane] = ok ? own : zero;
+    __syncthreads();
+    RowTile<T, NCH, 1> t;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) t.raw[0][j] = chunks[first + j][lane];
+    float s1, s2, mean, rstd;
+    tile_moments(t, 0, C, 0.0f, lane, s1, s2);
+    if (mode == CW_LN_TWO_PASS) {
+        const float mu = s1 * inv_h;
+        float d1, d2;
+        tile_moments(t, 0, C, mu, lane, d1, d2);
+        finish_stats(mode, mu, d2, inv_h, eps, mean, rstd);
+    } else {
+        finish_stats(mode, s1, s2, inv_h, eps, mean, rstd);
+    }
+    if (mean_rstd != nullptr && wave == first && lane == 0 && live) {
+        mean_rstd[2 * row] = mean;
+        mean_rstd[2 * row + 1] = rstd;
+    }
+    float v[V], g[V], b[V];
+    unpack_raw(own, v, (const T*)nullptr);
+    unpack_raw(g_raw, g, (const T*)nullptr);
+    unpack_raw(b_raw, b, (const T*)nullptr);
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        float xh = (v[e] - mean) * rstd;
+        if (gamma != nullptr) xh *= g[e];
+        if (beta != nullptr) xh += b[e];
+        v[e] = xh;
+    }
+    if (live && ok) store_raw_stream(y + row * ldy + c0, pack_raw(v, (const T*)nullptr));
+}
+
 template <typename T, int NCH, int NR, bool EXACT>
 __global__ __launch_bounds__(kTileWaves * 64) void ln_bwd_dx_tile_kernel(
     int64_t R, int64_t C, const T* __restrict__ dY, int64_t ld_dy, const T* __restrict__ x, int64_t ld_x,
@@ -1262,14 +1315,22 @@ int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float*
                        (beta == nullptr || aligned16(beta));
     const int64_t nch = row_chunks<T>(C);
     if constexpr (FUSED) {
-        // As many wavefronts a row as it has chunks, one load each, where all of them fit the chip at once (16 per compute unit): with a row a
-        // wavefront the launch is that wavefront's chain (us, bf16 from memory: 300 x 4096 5.6 -> 3.9, 1024 x 2048 5.8 -> 4.3, 777 x 2560 5.5 -> 4.4; beyond,
-        // from cache, 1554 x 2560 5.6 -> 6.2; rows of two chunks, 128 x 768 2.7 -> 2.8).
-        if (vec_ok && (C % elem<T>::kVec) == 0 && nch >= 3 && nch <= kFwdSplitBlockWaves && R * nch <= 16 * 256) {
-            const int nrg = kFwdSplitBlockWaves / (int)nch;
-            hipLaunchKernelGGL((ln_forward_split_kernel<T, 1, kFwdSplitBlockWaves>), dim3((unsigned)((R + nrg - 1) / nrg)), dim3((unsigned)(nch * nrg * 64)),
-                               0, s, R, C, (const T*)x, ld, mode, 1.0f / (float)H, eps, (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd, (int)nch);
-            return check_launch("ln_forward_split_kernel");
+        // Where all of the rows' chunks fit the chip at once, 16 wavefronts per compute unit (us, bf16 from memory, a wavefront a row / a chunk: 300 x
+        // 4096 5.5 / 4.0, 512 x 4096 5.6 / 4.4, 1024 x 2048 5.6 / 3.9, 777 x 2560 5.4 / 4.0, fp32 1365 x 768 4.2 / 3.4, 512 x 2048 4.8 / 3.6; beyond, 625 x 4096
+        // 5.7 / 5.8, 1024 x 4096 6.2 / 7.4, 2730 x 1536 5.1 / 6.2). Rows of two chunks, 128 x 768, with the sums through LDS: 2.7 / 2.8.
+        if (vec_ok && (C % elem<T>::kVec) == 0 && nch >= 3 && nch <= kFwdShortWaves && R * nch <= 16 * 256) {
+            auto launch = [&](auto nch_c) {
+                constexpr int NCH = decltype(nch_c)::value, NRG = kFwdShortWaves / NCH;
+                hipLaunchKernelGGL((ln_forward_short_kernel<T, NCH>), dim3((unsigned)((R + NRG - 1) / NRG)), dim3(NCH * NRG * 64), 0, s, R, C, (const T*)x, ld,
+                                   mode, 1.0f / (float)H, eps, (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd);
+                return check_launch("ln_forward_short_kernel");
+            };
+            if (nch == 3) return launch(std::integral_constant<int, 3>{});
+            if (nch == 4) return launch(std::integral_constant<int, 4>{});
+            if (nch == 5) return launch(std::integral_constant<int, 5>{});
+            if (nch == 6) return launch(std::integral_constant<int, 6>{});
+            if (nch == 7) return launch(std::integral_constant<int, 7>{});
+            return launch(std::integral_constant<int, 8>{});
         }
     }
     if (vec_ok && exact_chunks<T>(C, nch) && R <= (int64_t)1 << 30) {

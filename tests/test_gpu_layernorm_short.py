@@ -89,3 +89,20 @@ def test_in_place_and_scratch():
     for a, b in zip([dx, sums] + cols, [own, own_sums] + own_cols):
         _close(a, b.double(), 2.0 ** -18, b.double().abs() + b.double().abs().mean())
     assert _backward(dy, x, mean_rstd, g, dx, 16)[0] == -1
+
+
+@pytest.mark.parametrize("C", [512, 776, 1536, 2048, 2056, 2560, 3072, 3584, 4096])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("mode", ["one_pass", "two_pass"])
+def test_a_row_has_the_same_bits_in_any_batch(C, dtype, mode):
+    """On both sides of the number of rows from which a row is one wavefront's, and on the block's edges: what the ordered products
+    behind the layer keep (test_forward_rows_do_not_depend_on_the_batch) begins here."""
+    from cubework_amd import _lib, ops
+    mode = _lib.CW_LN_ONE_PASS if mode == "one_pass" else _lib.CW_LN_TWO_PASS
+    chunks = -(-C * torch.empty((), dtype=dtype).element_size() // 1024)
+    edge = 4096 // chunks
+    x, g, b = randn((edge + 9, C), dtype, 1, device=DEV) + 0.5, randn((C,), dtype, 2, device=DEV), randn((C,), dtype, 3, device=DEV)
+    want = ops.ln_forward_fused(x, 1e-5, g, b, mode)
+    for R in (1, 2, 7, 128, edge, edge + 1):
+        for got, whole in zip(ops.ln_forward_fused(x[:R], 1e-5, g, b, mode), want):
+            assert torch.equal(got, whole[:R])
