@@ -55,7 +55,7 @@ struct Body {
 };
 
 void keep(AutogradContext* ctx, std::vector<int64_t> meta) { ctx->saved_data["meta"] = std::move(meta); }
-std::vector<int64_t> kept(AutogradContext* ctx) { return ctx->saved_data["meta"].toIntVector(); }
+std::vector<int64_t> kept(const AutogradContext* ctx) { return ctx->saved_data.at("meta").toIntVector(); }
 
 // A 16-bit operand of two products with rows that begin at multiples of 16 bytes (ops.aligned_rows).
 Tensor aligned_rows(const Tensor& t_in) {
@@ -126,9 +126,10 @@ struct Linear : Function<Linear> {
             cast_together({was_fp32 & 1 ? &dx : &none, was_fp32 & 2 ? &dw : &none, was_fp32 & 4 ? &dbias : &none}, at::kFloat);
         }
         // absent operands are no inputs of the node, and have no index there
-        const bool need_residual = meta[3] != 0 && ctx->needs_input_grad(has_bias ? 3 : 2);
+        const bool need_residual = has_residual(*ctx) && ctx->needs_input_grad(has_bias ? 3 : 2);
         return {dx, dw, dbias, need_residual ? grads[0] : Tensor(), Tensor(), Tensor()};
     }
+    static bool has_residual(const AutogradContext& ctx) { return kept(&ctx)[3] != 0; }
 };
 
 py::object linear(py::handle x_in, py::handle w_in, py::handle bias_in, py::handle residual_in, int layout, int act) {
@@ -295,16 +296,18 @@ py::object embedding(py::handle ids_in, py::handle weight_in, int64_t start, int
     return py::cast(out);
 }
 
-// Whether the gradient that the running node hands to its first input's node is read by that node alone, which is a layer's product:
-// no hook sees it and nobody asked for it. It may then have rows that begin at multiples of 16 bytes whatever their length, as both
-// gradient products read them. (autograd's other readers, a logits tensor with a second use among them, take any strides.)
+// Whether the gradient that the running node hands to its first input's node is read by that node's own kernels alone, those of a
+// layer without a residual (which would hand the gradient on as it is): no hook before, at or behind that node sees it and nobody asked
+// for it. It may then have rows that begin at multiples of 16 bytes whatever their length, as both gradient products read them.
+// (autograd's other readers, a logits tensor with a second use among them, take any strides.)
 bool for_a_product_only() {
     const auto node = torch::autograd::get_current_node();
     const auto* asked = torch::autograd::get_current_graph_task_exec_info();  // empty for backward() without inputs
     if (!node || !node->post_hooks().empty() || asked == nullptr || !asked->empty() || node->num_outputs() == 0) return false;
     const auto& next = node->next_edge(0).function;
-    return next && dynamic_cast<torch::autograd::CppNode<Linear>*>(next.get()) != nullptr && next->pre_hooks().empty() &&
-           next->tensor_pre_hooks().empty() && next->retains_grad_hooks().empty();
+    const auto* linear = dynamic_cast<torch::autograd::CppNode<Linear>*>(next.get());
+    return linear != nullptr && !Linear::has_residual(linear->ctx_) && next->pre_hooks().empty() && next->tensor_pre_hooks().empty() &&
+           next->retains_grad_hooks().empty() && next->post_hooks().empty();
 }
 
 // loss._operation._VocabParallelCrossEntropyMean.

@@ -295,7 +295,7 @@ def test_head_and_loss_of_any_vocabulary(rows, vocab, bias, dtype):
     x, w, b = leaves
     seen = []
     forward = lambda: ops.linear("NT", x, w, b)  # noqa: E731
-    for watch in ("hook", "retain", "post", "asked", "inputs", "view"):
+    for watch in ("hook", "retain", "post", "behind", "asked", "inputs", "view"):
         for leaf in leaves:
             if leaf is not None:
                 leaf.grad = None
@@ -308,6 +308,8 @@ def test_head_and_loss_of_any_vocabulary(rows, vocab, bias, dtype):
             logits.retain_grad()
         elif watch == "post":
             loss.grad_fn.register_hook(lambda outputs, _: seen.append(outputs[0]))
+        elif watch == "behind":  # the layer's own node: its hooks are handed what it was given
+            logits.grad_fn.register_hook(lambda _, given: seen.append(given[0]))
         if watch == "asked":
             seen.append(torch.autograd.grad(loss, logits, dy)[0])
             continue
@@ -317,7 +319,7 @@ def test_head_and_loss_of_any_vocabulary(rows, vocab, bias, dtype):
         assert torch.equal(x.grad, want[1])
         if watch != "inputs":
             assert torch.equal(w.grad, want[2])
-    assert len(seen) == 5
+    assert len(seen) == 6
     assert all(g.shape == (rows, vocab) and g.is_contiguous() and torch.equal(g, seen[0]) for g in seen)
     # the logits read a second time: their gradients are added before the product sees them
     logits = forward()
@@ -325,3 +327,26 @@ def test_head_and_loss_of_any_vocabulary(rows, vocab, bias, dtype):
     ref = torch.autograd.grad(ops.mean_loss(forward(), t, 0), x)[0].double() + (w.double().sum(0) / 16)
     # 16-bit rounding of the added gradient and of the results
     assert (twice.double() - ref).abs().max() <= 2.0 ** (-7 if dtype == torch.bfloat16 else -10) * ref.abs().max()
+
+
+@pytest.mark.parametrize("watch", ["hook", "retain", "asked"])
+def test_residual_of_a_head_of_an_odd_vocabulary(watch):
+    """A layer hands its residual the gradient it was given: a dense one, which a hook may view as it likes."""
+    from cubework_amd import ops
+
+    x, w = randn((33, 64), torch.bfloat16, 1, device=DEV).requires_grad_(True), randn((64, 1001), torch.bfloat16, 2, std=0.1, device=DEV).requires_grad_(True)
+    leaf = randn((33, 1001), torch.bfloat16, 3, device=DEV).requires_grad_(True)
+    t = torch.randint(0, 1001, (33,), generator=torch.Generator().manual_seed(4)).to(DEV)
+    residual = leaf * 1.0
+    loss = ops.mean_loss(ops.linear("NN", x, w, residual=residual), t, 0)
+    seen = []
+    if watch == "hook":
+        residual.register_hook(lambda g: seen.append(g.view(-1)))
+    elif watch == "retain":
+        residual.retain_grad()
+    if watch == "asked":
+        seen.append(torch.autograd.grad(loss, residual)[0])
+    else:
+        loss.backward()
+        seen.append(leaf.grad if watch == "hook" else residual.grad)
+    assert len(seen) == (2 if watch == "hook" else 1) and all(g.is_contiguous() and g.numel() == 33 * 1001 for g in seen)
