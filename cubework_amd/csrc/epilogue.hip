@@ -212,6 +212,10 @@ int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void*
     bool vec = aligned16(dY) && (ld_dy % V) == 0 && (N % V) == 0;
     if (MODE == 1) vec = vec && aligned16(pre) && (ld_pre % V) == 0 && aligned16(dPre) && (ld_dpre % V) == 0;
     int64_t slabs, rows_per_slab;
+    colsum_plan(M, N, V, vec, slabs, rows_per_slab);
+    // also of a call whose launch needs none: the sizes that a caller passes are wrong or right whatever the number of rows
+    if (want_sum && workspace_bytes < slabs * N * (int64_t)sizeof(float))
+        return fail(CW_ERR_INVALID, "column sum: workspace too small (%lld bytes)", (long long)workspace_bytes);
     const auto with_act = [&](auto&& launch) {
         if (MODE == 0 || act == CW_ACT_NONE) launch(std::integral_constant<int, CW_ACT_NONE>{});
         else if (act == CW_ACT_GELU_TANH) launch(std::integral_constant<int, CW_ACT_GELU_TANH>{});
@@ -228,9 +232,6 @@ int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void*
     }
     if (vec) {
         const int64_t coltiles = (N + 64 * V - 1) / (64 * V);
-        colsum_plan(M, N, V, true, slabs, rows_per_slab);
-        if (want_sum && workspace_bytes < slabs * N * (int64_t)sizeof(float))
-            return fail(CW_ERR_INVALID, "column sum: workspace too small (%lld bytes)", (long long)workspace_bytes);
         const size_t lds = tree_reduce_lds_bytes(V, kColWaves);
         const dim3 grid((unsigned)coltiles, (unsigned)slabs), block(kColWaves * 64);
         with_act([&](auto act_c) {
@@ -239,9 +240,6 @@ int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void*
                                (const T*)pre, ld_pre, (T*)dPre, ld_dpre, (float*)workspace, rows_per_slab, want_sum);
         });
     } else {
-        colsum_plan(M, N, V, false, slabs, rows_per_slab);
-        if (want_sum && workspace_bytes < slabs * N * (int64_t)sizeof(float))
-            return fail(CW_ERR_INVALID, "column sum: workspace too small (%lld bytes)", (long long)workspace_bytes);
         hipLaunchKernelGGL((colsum_generic_kernel<T, MODE>), dim3((unsigned)((N + 255) / 256), (unsigned)slabs),
                            dim3(256), 0, s, M, N, (const T*)dY, ld_dy, (const T*)pre, ld_pre, (T*)dPre, ld_dpre, act,
                            (float*)workspace, rows_per_slab, want_sum);

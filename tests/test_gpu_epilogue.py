@@ -153,3 +153,23 @@ def test_column_sums_of_few_rows(M, N, dtype):
     # the sums are of the unrounded products: 16-bit rounding of each on top where dPre is 16 bits
     per = 2.0 ** -24 * M + (0 if dtype == torch.float32 else torch.finfo(dtype).eps / 2)
     assert (db.double() - dpre.double().sum(0)).abs().le(dpre.double().abs().sum(0) * per * 1.01 + 1e-6).all()
+
+
+@pytest.mark.parametrize("M", [1, 256, 257, 512, 513])
+def test_column_sums_refuse_scratch_that_is_too_small_at_every_size(M):
+    """Less than one row of partial sums, also where the launch needs none: refused before anything is written."""
+    import ctypes
+
+    from cubework_amd import _lib
+
+    N, lib = 64, _lib.load()
+    dy, pre = (randn((M, N), torch.bfloat16, k, device=DEV) for k in range(2))
+    dpre, out = torch.zeros_like(dy), torch.zeros(N, device=DEV)
+    need = lib.cw_colsum_workspace_bytes(M, N)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for size, rc in ((N * 4 - 1, _lib.CW_ERR_INVALID), (need, 0)):
+        assert lib.cw_colsum(M, N, p(dy), N, p(out), 1, p(ws), size, 0, stream) == rc
+        assert lib.cw_act_bwd_colsum(2, M, N, p(dy), N, p(pre), N, p(dpre), N, p(out), 1, p(ws), size, 0, stream) == rc
+        assert out.any().item() == dpre.any().item() == (rc == 0)
