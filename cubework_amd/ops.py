@@ -161,14 +161,9 @@ def act_bwd_colsum(activation: Optional[str], dy: torch.Tensor, preact: torch.Te
     return _lib.host().act_bwd_colsum(ACTIVATIONS[activation], dy, preact, want_dbias, out_dtype)
 
 
-def _summands(own, peers):
-    """(own, peers) with the peers as tensors; staged plain numbers are added to own at once."""
-    peers = list(peers)
-    if not all(isinstance(t, torch.Tensor) for t in peers):
-        for t in peers:
-            own = own + t
-        peers = []
-    return own, peers
+def _tensors(peers):
+    """The peers as tensors: staged plain numbers, which torch adds as well, among them."""
+    return [t if isinstance(t, torch.Tensor) else torch.as_tensor(t) for t in peers]
 
 
 def colsum_scattered(dy: torch.Tensor, peers: Sequence[torch.Tensor], world: int, rank: int, out_dtype: torch.dtype,
@@ -176,7 +171,7 @@ def colsum_scattered(dy: torch.Tensor, peers: Sequence[torch.Tensor], world: int
     """Column sums of a [M,N] tensor (of dPre = dy * act'(preact) with an activation) reduce-scattered over `world` ranks, whose
     other members' [N] sums are `peers`: (dPre or None, this rank's N / world columns of the totals as out_dtype).
     See cw_colsum_peers."""
-    return _lib.host().colsum_scattered(dy, ACTIVATIONS[activation], preact, list(peers), world, rank, out_dtype)
+    return _lib.host().colsum_scattered(dy, ACTIVATIONS[activation], preact, _tensors(peers), world, rank, out_dtype)
 
 
 # --------------------------------------------------------------------------
@@ -203,8 +198,7 @@ def ln_normalize(x: torch.Tensor, stats: torch.Tensor, hidden: int, eps: float,
                  gamma: Optional[torch.Tensor] = None, beta: Optional[torch.Tensor] = None,
                  mode: int = CW_LN_ONE_PASS, save_mean_rstd: bool = True, peers: Sequence[torch.Tensor] = ()):
     """y = gamma*(x-mean)*rstd+beta from whole-hidden-size stats (stats + the peers', in order); returns (y, mean_rstd)."""
-    stats, peers = _summands(stats, peers)
-    return _lib.host().ln_forward(x, stats, peers, hidden, eps, gamma, beta, mode, save_mean_rstd)
+    return _lib.host().ln_forward(x, stats, _tensors(peers), hidden, eps, gamma, beta, mode, save_mean_rstd)
 
 
 def ln_forward_fused(x: torch.Tensor, eps: float, gamma: Optional[torch.Tensor] = None,
@@ -271,10 +265,9 @@ def ln_bwd_dx_close(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor, 
     scatter = (the peers' dgamma, the peers' dbeta, ranks, rank, gamma's dtype, beta's dtype): dgamma and dbeta are
     reduce-scattered, C / ranks columns of the totals each. See cw_ln_bwd_dx_close_peers."""
     ws, n_parts = pending
-    row_sums, row_peers = _summands(row_sums, row_peers)
     dgammas, dbetas, *rest = scatter or ((), (), 1, 0, torch.float32, torch.float32)
-    return _lib.host().ln_bwd_dx_close(dy, x, mean_rstd, row_sums, row_peers, hidden, ws, n_parts, gamma, param_dtype,
-                                       list(dgammas), list(dbetas), *rest)
+    return _lib.host().ln_bwd_dx_close(dy, x, mean_rstd, row_sums, _tensors(row_peers), hidden, ws, n_parts, gamma, param_dtype,
+                                       _tensors(dgammas), _tensors(dbetas), *rest)
 
 
 def ln_backward_fused(dy: torch.Tensor, x: torch.Tensor, mean_rstd: torch.Tensor,

@@ -84,6 +84,18 @@ def test_peers_that_torch_adds():
     own = ops.colsum(x)
     assert torch.equal(ops.colsum_scattered(x, [own, own, own], 4, 3, torch.float16)[1], _scattered(own, [own] * 3, 4, 3, torch.float16))
     assert torch.equal(ops.colsum_scattered(x, [own], 2, 1, torch.float64)[1], _scattered(own, [own], 2, 1, torch.float64))
+    dy = randn((40, 30), torch.bfloat16, 2, device=DEV)
+    mr = ops.ln_normalize(x, stats, 90, 1e-5)[1]
+    sums, pending = ops.ln_bwd_partials_open(dy, x, mr)
+    dx, dg, db = ops.ln_bwd_dx_close(dy, x, mr, sums, 90, pending)
+    for numbers in ([3.0], [own, 2], [0.25, own.bfloat16()]):
+        world = len(numbers) + 1
+        assert torch.equal(ops.colsum_scattered(x, numbers, world, 0, torch.bfloat16)[1], _scattered(own, numbers, world, 0, torch.bfloat16))
+        got = ops.ln_bwd_dx_close(dy, x, mr, sums, 90, pending, scatter=(numbers, [own] * len(numbers), world, 0, torch.bfloat16, torch.float32))
+        assert torch.equal(got[0], dx) and torch.equal(got[1], _scattered(dg, numbers, world, 0, torch.bfloat16))
+        assert torch.equal(got[2], _scattered(db, [own] * len(numbers), world, 0, torch.float32))
+        shifted = ops.ln_bwd_dx_close(dy, x, mr, sums, 90, pending, row_peers=[2.0])
+        assert torch.equal(shifted[0], ops.ln_bwd_dx_close(dy, x, mr, sums + 2.0, 90, pending)[0])
     none = ops.colsum_scattered(x[:0], [own], 2, 0, torch.float32)[1]
     assert torch.equal(none, own[:15])
     w = [randn((15,), torch.bfloat16, 5, device=DEV), randn((15,), torch.float32, 6, device=DEV)]
