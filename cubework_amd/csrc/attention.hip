@@ -269,16 +269,24 @@ using namespace cw;
 
 namespace {
 
-// Wavefronts of a block. Few of them where they all fit the chip at once: a block's wavefronts wait for each other at every tile, and under
-// the causal mask for the longest of them. us, bf16, 8 / 4 / 2 wavefronts (batch x tokens x heads x columns): 1 x 300 x 32 x 128 15.1 / 12.8 /
-// 12.5, 1 x 1024 x 16 x 64 23.9 / 18.6 / 17.8, 2 x 777 x 32 x 64 20.7 / 16.9 / 16.9, 2 x 777 x 32 x 80 26.0 / 25.0 / 27.0. With more blocks than
-// units they read K and V more often: 4 x 2048 x 32 x 64 91.6 / 89.0 / 108, 4 x 2048 x 16 x 64 56 / 50 / 59, x 128 columns 88 / 98 / 126.
+// Wavefronts of a block. Few of them where their blocks all fit the chip at once: a block's wavefronts wait for each other at every tile, and
+// under the causal mask for the longest of them. us, bf16, 8 / 4 / 2 wavefronts (batch x tokens x heads x columns), causal: 1 x 300 x 32 x 128
+// 15.1 / 12.8 / 12.5, 1 x 1024 x 16 x 64 23.9 / 18.6 / 17.8, 2 x 777 x 32 x 64 20.7 / 16.9 / 16.9, 2 x 777 x 32 x 80 26.0 / 25.0 / 27.0. With more
+// blocks than units they read K and V more often: 4 x 2048 x 32 x 64 91.6 / 89.0 / 108, 4 x 2048 x 16 x 64 56 / 50 / 59, x 128 columns 88 / 98 / 126.
+// Without the mask all of a block's wavefronts walk alike: blocks of 4 that do not fit cost a second round (1 x 1456 x 32 x 128 47.1 / 58.3,
+// causal 45.1 / 44.5; 1 x 1040 x 32 x 80 31.4 / 37.8, of 16 heads of 1314 34.5 / 33.8).
+// Heads of up to 64 columns leave room for four blocks of 4 a unit; those of more heads than units and many tokens each read their K and V from
+// beyond the L2, blocks of 4 twice as often: 8 x 1497 x 32 x 48 169 / 216, causal 100 / 117 (4 x 1497 x 16 93 / 91, causal 54 / 52), 8 x 2048 x
+// 32 x 64 315 / 342, causal 182 / 188 (4 x 1800 x 32 147 / 141). Left to 4: 2 x 1612 x 32 x 48 59.4 / 62.6, 2 x 1255 x 40 x 64 50.3 / 52.4.
 template <typename HS>
-int fwd_waves(int64_t BH, int64_t S) {
-    const bool all64 = BH * ((S + 63) / 64) <= kUnits, all256 = BH * ((S + 255) / 256) <= kUnits;
-    if (HS::NP == 1) return all64 ? 2 : 4;
+int fwd_waves(int64_t BH, int64_t S, bool causal) {
+    const bool all64 = BH * ((S + 63) / 64) <= kUnits;
+    if (HS::NP == 1) {
+        const bool far = causal ? HS::MASK && BH >= kUnits && S >= 1400 : BH * S >= 1024 * kUnits && S >= (HS::MASK ? 1024 : 1400);
+        return all64 ? 2 : far ? 8 : 4;
+    }
     if (all64 && (HS::DT == 4 || S <= 128)) return 2;  // 1 x 777 x 16 x 80: 22.1 with 4, 23.4 with 2
-    return all256 ? 4 : 8;
+    return S <= 128 || BH * ((S + 127) / 128) <= (causal ? kUnits * 3 / 2 : kUnits) ? 4 : 8;
 }
 
 int attn_fwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const void* q, const void* k, const void* v,
@@ -309,7 +317,7 @@ int attn_fwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const 
     hipStream_t s = (hipStream_t)stream;
     return with_head_shape(D, [&](auto hs) {
         using HS = decltype(hs);
-        const int waves = fwd_waves<HS>(B * H, S);
+        const int waves = fwd_waves<HS>(B * H, S, causal != 0);
         auto launch = [&](auto w) {
             constexpr int W = decltype(w)::value;
             a.n_qblocks = (int)((S + W * kQPerWave - 1) / (W * kQPerWave));
@@ -319,9 +327,7 @@ int attn_fwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const 
             return check_launch("attn_fwd_kernel");
         };
         if (waves == 2) return launch(std::integral_constant<int, 2>{});
-        if constexpr (HS::NP == 2) {
-            if (waves == 8) return launch(std::integral_constant<int, 8>{});
-        }
+        if (waves == 8) return launch(std::integral_constant<int, 8>{});
         return launch(std::integral_constant<int, 4>{});
     });
 }

@@ -434,20 +434,24 @@ __global__ __launch_bounds__(NW * 64, HS::NP == 1 ? 2 : 1) void attn_dkdv_kernel
     }
 }
 
-// Wavefronts of a dQ and of a dK/dV block: fewer of them where the blocks all fit the chip at once (of 32 rows each: 64, or 256 together), as
+// Wavefronts of a dQ and of a dK/dV block: fewer of them where their blocks all fit the chip at once, as
 // in the forward. us of both launches, bf16, causal, before (dQ 8, dK/dV 4, at 65 to 80 columns 8) / here (batch x tokens x heads x
 // columns): 1 x 300 x 32 x 64 25.5 / 20.7, 1 x 512 x 32 x 128 58.1 / 48.9, 1 x 512 x 32 x 80 52.3 / 40.5, 2 x 777 x 16 x 80 71.5 / 61.8, 4 x 512 x 16 x
 // 64 36.3 / 32.7, 1 x 2048 x 32 x 64 101 / 98.9. Beyond, dQ of 4: 4 x 1024 x 32 x 64 95.1 / 95.1, 4 x 2048 x 32 x 64 272 / 284; at 80 columns and 256
 // blocks of 256 rows 2 x 777 x 32 75.9 / 79.5 (dK/dV of 4 73.7, but 4 x 512 x 32 60.6 / 65.4).
+// Under the mask blocks of 4 may be somewhat more than that, the short ones fill the gaps: dQ of 8 / 4 at 1 x 1456 x 32 x 128 123 / 112, 4 x 706 x 16
+// 81.6 / 79.5, not with few tiles a block (8 x 161 x 32 44.7 / 49.4, 4 x 303 x 32 49.8 / 52.2). Without it they are a second round: 1 x 1456 x
+// 32 x 128 189 / 219, 1 x 1624 x 24 x 64 91.7 / 102, 3 x 635 x 16 x 64, which fit, 40.2 / 37.0. Up to 128 tokens blocks of 8 are half empty.
 struct BwdWaves {
     int dq, dkdv;
 };
 template <typename HS>
-BwdWaves bwd_waves(int64_t BH, int64_t S) {
+BwdWaves bwd_waves(int64_t BH, int64_t S, bool causal) {
     const bool all64 = BH * ((S + 63) / 64) <= kUnits;
-    const int64_t blocks = BH * ((S + 255) / 256);
+    const int64_t blocks128 = BH * ((S + 127) / 128), blocks = BH * ((S + 255) / 256);
     if (HS::KB == 5) return all64 ? BwdWaves{2, 2} : blocks <= kUnits / 2 ? BwdWaves{4, 4} : BwdWaves{8, 8};
-    return BwdWaves{all64 && HS::NP == 1 ? 2 : blocks <= kUnits ? 4 : 8, all64 ? 2 : 4};
+    const bool more = causal && (HS::NP == 1 ? blocks <= kUnits : blocks128 <= kUnits * 3 / 2 && S > 640);
+    return BwdWaves{all64 && HS::NP == 1 ? 2 : S <= 128 || blocks128 <= kUnits || more ? 4 : 8, all64 ? 2 : 4};
 }
 
 // The two launches of the backward for element type E.
@@ -455,7 +459,7 @@ template <typename E>
 int launch_bwd(BwdArgs a, int64_t B, int64_t H, int64_t S, int64_t D, hipStream_t s) {
     return with_head_shape(D, [&](auto hs) {
         using HS = decltype(hs);
-        const BwdWaves waves = bwd_waves<HS>(B * H, S);
+        const BwdWaves waves = bwd_waves<HS>(B * H, S, a.causal != 0);
         auto dq = [&](auto w) {
             constexpr int W = decltype(w)::value;
             a.n_blocks = (int)((S + W * kRowsPerWave - 1) / (W * kRowsPerWave));
@@ -532,7 +536,7 @@ int attn_bwd(const char* who, int64_t B, int64_t H, int64_t S, int64_t D, const 
     a.sb = stride_b; a.ss = stride_s; a.sh = stride_h;
     a.ob = out_stride_b; a.os = out_stride_s; a.oh = out_stride_h;
     a.gb = grad_stride_b; a.gs = grad_stride_s; a.gh = grad_stride_h;
-    a.S = (int)S; a.H = (int)H; a.BH = (int)(B * H); 
+    a.S = (int)S; a.H = (int)H; a.BH = (int)(B * H);
     a.scale = scale; a.scale_log2e = scale * kLog2e;
     a.causal = causal ? 1 : 0;
     a.D = (int)D;

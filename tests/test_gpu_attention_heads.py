@@ -63,7 +63,8 @@ def test_unaligned_rows(d, form):
 
 
 @pytest.mark.parametrize("D", [48, 56, 64, 80, 96, 128])
-@pytest.mark.parametrize("B,H,S,causal", [(9, 16, 130, True), (5, 16, 257, True), (5, 32, 300, False), (18, 16, 130, True), (17, 16, 260, True)])
+@pytest.mark.parametrize("B,H,S,causal", [(9, 16, 130, True), (5, 16, 257, True), (5, 32, 300, False), (18, 16, 130, True), (17, 16, 260, True),
+                                           (5, 32, 500, False), (16, 16, 1024, False), (16, 16, 1400, True)])
 def test_blocks_of_any_number_of_wavefronts_give_the_same_bits(B, H, S, D, causal):
     """A batch on each side of the rules that choose a block's wavefronts, against its sequences one by one: whole batches run on blocks of 4
     or 8, single sequences on blocks of 2 or 4."""
