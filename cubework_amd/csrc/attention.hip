@@ -72,11 +72,7 @@ __global__ __launch_bounds__(64 * W, HS::NP == 1 ? 2 : 1) void attn_fwd_kernel(c
     const int b = bh / a.H, h = bh - b * a.H;
     const int qblk = a.n_qblocks - 1 - (int)(blockIdx.x / (unsigned)a.BH);
     const int q0 = qblk * kQPerBlock;
-    // Under the causal mask a wavefront's work grows with its query position, and wavefront w always runs on
-    // SIMD w % 4: half of the blocks deal the query tiles in reverse so that no SIMD collects the long ones
-    // (blocks 256 apart, which share a compute unit when the launch starts, differ in bit 8).
-    const int wq = (a.causal && (((blockIdx.x >> 8) ^ blockIdx.x) & 1)) ? W - 1 - wave : wave;
-    const int qw0 = q0 + wq * kQPerWave;
+    const int qw0 = q0 + wave * kQPerWave;
 
     const uint16_t* qp = a.q + b * a.sb + h * a.sh;
     const uint16_t* kp = a.k + b * a.sb + h * a.sh;
