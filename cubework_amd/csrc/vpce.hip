@@ -88,22 +88,31 @@ __device__ __forceinline__ void lse_merge(float& m_a, float& s_a, float m_b, flo
     m_a = m;
 }
 
-// 1 for a row of 16-bit elements that begins off a multiple of 4 bytes: its vectors are taken from the second element on. 16-byte
+// 1 for a row of 16-bit elements that begins off a multiple of 4 bytes: where ODD, its vectors are taken from the second element on. 16-byte
 // loads at odd elements take the load unit longer, at even ones they run as aligned ones do (1023 x 50257 bf16, where every other row
 // is odd, forward 24.5 -> 18.9 us, as at 50258 columns; 8192 x 12567 forward 42.4 -> 34.7, backward 81 -> 72, at 12568 33 and 68).
-template <typename T>
+// Long rows only, for it costs every wavefront some 20 instructions, of which a block of short rows does little else (us, without / with it:
+// forward 8192 x 4097 20.1 / 19.5, 1853 x 4097 6.2 / 6.3, 1853 x 3073 5.9 / 6.0; backward 8192 x 8193 56.2 / 51.9, 437 x 8193 4.8 / 5.0, 8192 x
+// 6145 43.9 / 43.9, 8192 x 1097 25.9 / 31.0).
+template <bool ODD, typename T>
 __device__ __forceinline__ int odd_row(const T* row) {
-    return sizeof(T) == 2 ? (int)(reinterpret_cast<uintptr_t>(row) >> 1) & 1 : 0;
+    return ODD ? (int)(reinterpret_cast<uintptr_t>(row) >> 1) & 1 : 0;
+}
+constexpr int64_t kOddForward = 4096, kOddBackward = 8192;  // columns
+template <typename T>
+bool odd_rows(const void* p, int64_t ld, int64_t rows) {
+    return sizeof(T) == 2 && ((reinterpret_cast<uintptr_t>(p) >> 1 & 1) != 0 || (rows > 1 && ld % 2 != 0));
 }
 
-template <typename T>
+// MEAN: for the launch of the mean behind this one (MeanOut); a test of every block for it took 8192 rows of 301 from 11.1 to 11.6 us.
+template <typename T, bool ODD, bool MEAN>
 __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int64_t V_cols,
                                                             const T* __restrict__ logits, int64_t ld,
                                                             const int64_t* __restrict__ targets, int64_t vocab_start,
                                                             float* __restrict__ out_max, float* __restrict__ out_sumexp,
                                                             float* __restrict__ out_pred, uint8_t* __restrict__ out_mask,
                                                             int* __restrict__ arrived) {
-    if (arrived != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *arrived = 0;  // for the launch behind this one (MeanOut)
+    if (MEAN && blockIdx.x == 0 && threadIdx.x == 0) *arrived = 0;
     constexpr int V = elem<T>::kVec;
     __shared__ float red_m[kCeBlock / 64];
     __shared__ float red_s[kCeBlock / 64];
@@ -112,7 +121,7 @@ __global__ __launch_bounds__(kCeBlock) void vpce_fwd_kernel(int64_t T_rows, int6
     const int wave = tid >> 6;
     for (int64_t row = blockIdx.x; row < T_rows; row += gridDim.x) {
         const T* row_begin = logits + row * ld;
-        const int odd = odd_row(row_begin);
+        const int odd = odd_row<ODD>(row_begin);
         const T* xr = row_begin + odd;
         const int64_t cols = V_cols - odd;
         OnlineLse st{kNegInf, 0.0f, 0.0f};
@@ -311,7 +320,7 @@ __device__ __forceinline__ CeRowScalars ce_row_scalars(int64_t row, int64_t V_co
     return r;
 }
 
-template <typename T, typename G>
+template <typename T, typename G, bool ODD>
 __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, int64_t V_cols,
                                                                const T* __restrict__ logits, int64_t ld,
                                                                const int64_t* __restrict__ targets, int64_t vocab_start,
@@ -357,7 +366,7 @@ __global__ __launch_bounds__(kCeBwdBlock) void vpce_bwd_kernel(int64_t T_rows, i
             }
         } else {
             // where logits and gradient are odd rows both, the vectors of both begin at the second element
-            const int odd = odd_row(xr) & odd_row(gr);
+            const int odd = odd_row<ODD>(xr) & odd_row<ODD>(gr);
             const int64_t nvec = (V_cols - odd) / V;
             CeRowScalars rs;
             if constexpr (sizeof(T) == 2) {
@@ -406,9 +415,14 @@ template <typename T, typename G>
 int bwd_impl(int64_t T_rows, int64_t V_cols, const void* logits, int64_t ld, const int64_t* targets,
              int64_t vocab_start, const float* gmax, const float* gsum, const DLoss& dloss, void* grad, int64_t ld_grad,
              hipStream_t s) {
-    hipLaunchKernelGGL((vpce_bwd_kernel<T, G>), dim3(ce_grid(T_rows)), dim3(kCeBwdBlock), 0, s, T_rows, V_cols,
-                       (const T*)logits, ld, targets, vocab_start, gmax, gsum, dloss, (G*)grad, ld_grad);
-    return check_launch("vpce_bwd_kernel");
+    auto launch = [&](auto odd) {
+        hipLaunchKernelGGL((vpce_bwd_kernel<T, G, decltype(odd)::value>), dim3(ce_grid(T_rows)), dim3(kCeBwdBlock), 0, s, T_rows, V_cols,
+                           (const T*)logits, ld, targets, vocab_start, gmax, gsum, dloss, (G*)grad, ld_grad);
+        return check_launch("vpce_bwd_kernel");
+    };
+    if constexpr (sizeof(G) == 2)
+        if (V_cols >= kOddBackward && odd_rows<T>(logits, ld, T_rows) && odd_rows<G>(grad, ld_grad, T_rows)) return launch(std::true_type{});
+    return launch(std::false_type{});
 }
 
 }  // namespace
@@ -437,9 +451,15 @@ extern "C" int cw_vpce_fwd_local_mean(int64_t T, int64_t V, const void* logits, 
     hipStream_t s = (hipStream_t)stream;
     return with_elem_type(io_dtype, [&](auto* tag) {
         using E = std::remove_pointer_t<decltype(tag)>;
-        hipLaunchKernelGGL(vpce_fwd_kernel<E>, dim3(ce_grid(T)), dim3(kCeBlock), 0, s, T, V, (const E*)logits, ld, targets,
-                           vocab_start, out_max, out_sumexp, out_pred, out_mask, arrived);
-        return check_launch("vpce_fwd_kernel");
+        auto launch = [&](auto odd, auto mean) {
+            hipLaunchKernelGGL((vpce_fwd_kernel<E, decltype(odd)::value, decltype(mean)::value>), dim3(ce_grid(T)), dim3(kCeBlock), 0, s, T, V,
+                               (const E*)logits, ld, targets, vocab_start, out_max, out_sumexp, out_pred, out_mask, arrived);
+            return check_launch("vpce_fwd_kernel");
+        };
+        auto any = [&](auto odd) { return arrived != nullptr ? launch(odd, std::true_type{}) : launch(odd, std::false_type{}); };
+        if constexpr (sizeof(E) == 2)
+            if (V >= kOddForward && odd_rows<E>(logits, ld, T)) return any(std::true_type{});
+        return any(std::false_type{});
     });
 }
 

@@ -117,7 +117,7 @@ def test_logits_gradient_is_contiguous(V):
     assert seen == [2 * 61 * V] and logits.grad.is_contiguous() and logits.grad.untyped_storage().nbytes() == 2 * 61 * V * 2
 
 
-@pytest.mark.parametrize("V", [1, 2, 7, 9, 767, 769, 6143, 6145, 8191])
+@pytest.mark.parametrize("V", [1, 2, 7, 9, 767, 769, 4095, 4097, 6143, 6145, 8191, 8193, 16384])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_cross_entropy_of_odd_rows(V, dtype):
     """Rows at every alignment of their elements, in both kernels: vectors from the first or the second element on."""
