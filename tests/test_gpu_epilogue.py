@@ -128,11 +128,11 @@ def test_gemm_part_diagnostic_takes_k_of_128(steps):
     torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("M", [1, 3, 63, 64, 65, 255, 256, 257, 511, 512, 513])  # the last rows of the one-launch kernels among them
+@pytest.mark.parametrize("M", [1, 3, 63, 64, 65, 160, 161, 224, 225, 255, 256, 257, 511, 512, 513])  # the last rows of the one-launch kernels among them
 @pytest.mark.parametrize("N", [8, 120, 136, 1000])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_column_sums_of_few_rows(M, N, dtype):
-    """One launch up to 512 rows (256 with an activation), NaN outside the operands' columns; fp32 sums of M values in any order lie
+    """One launch up to 512 rows (256 with an activation, 160 or 224 of the GELUs in 16 bits), NaN outside the operands' columns; fp32 sums of M values in any order lie
     within M 2^-24 of the sum of magnitudes. dPre does not depend on the kernel."""
     from cubework_amd import ops
 
@@ -147,12 +147,13 @@ def test_column_sums_of_few_rows(M, N, dtype):
         want, room = dy.double().sum(0), dy.double().abs().sum(0) * M * 2.0 ** -24
         room = room + want.abs() * (0 if out == torch.float32 else torch.finfo(out).eps / 2) * 1.001
         assert got.dtype == out and (got.double() - want).abs().le(room).all()
-    dpre, db = ops.act_bwd_colsum("gelu_tanh", dy, pre)
-    alone, none = ops.act_bwd_colsum("gelu_tanh", dy, pre, want_dbias=False)
-    assert none is None and torch.equal(dpre, alone)
-    # the sums are of the unrounded products: 16-bit rounding of each on top where dPre is 16 bits
-    per = 2.0 ** -24 * M + (0 if dtype == torch.float32 else torch.finfo(dtype).eps / 2)
-    assert (db.double() - dpre.double().sum(0)).abs().le(dpre.double().abs().sum(0) * per * 1.01 + 1e-6).all()
+    for act in ("gelu_tanh", "gelu_erf", "relu"):
+        dpre, db = ops.act_bwd_colsum(act, dy, pre)
+        alone, none = ops.act_bwd_colsum(act, dy, pre, want_dbias=False)
+        assert none is None and torch.equal(dpre, alone)
+        # the sums are of the unrounded products: 16-bit rounding of each on top where dPre is 16 bits
+        per = 2.0 ** -24 * M + (0 if dtype == torch.float32 else torch.finfo(dtype).eps / 2)
+        assert (db.double() - dpre.double().sum(0)).abs().le(dpre.double().abs().sum(0) * per * 1.01 + 1e-6).all()
 
 
 @pytest.mark.parametrize("M", [1, 256, 257, 512, 513])
