@@ -77,11 +77,11 @@ __global__ __launch_bounds__(kColWaves * 64) void colsum_vec_kernel(
 // Few rows: one launch that finishes the sums. A block of 16 wavefronts owns 16 vectors of columns (256 bytes of a row, whole
 // lines) and walks over all rows, 64 at a time: a wavefront's four groups of 16 lanes read four of them.
 constexpr int kShortWaves = 16, kShortLanes = 16;
-template <typename T, int MODE, int ACT>
+template <typename T, int MODE, int ACT, typename P>
 __global__ __launch_bounds__(kShortWaves * 64) void colsum_short_kernel(int M, int64_t N, const T* __restrict__ dY, int64_t ld_dy,
                                                                         const T* __restrict__ pre, int64_t ld_pre, T* __restrict__ dPre,
                                                                         int64_t ld_dpre, void* __restrict__ out, int out_dtype,
-                                                                        const PeerCols peers) {
+                                                                        const P peers) {
     constexpr int V = elem<T>::kVec, U = MODE == 0 ? 4 : 2, kRows = kShortWaves * 64 / kShortLanes, kCols = kShortLanes * V;
     __shared__ float red[kShortWaves][kCols];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lc = lane % kShortLanes, lr = lane / kShortLanes;
@@ -159,11 +159,12 @@ __global__ __launch_bounds__(256) void colsum_generic_kernel(int64_t M, int64_t 
 // grid (ceil(C/64), nsets); 16 groups of 64 threads split the partials, each
 // with 16 independent loads in flight, and are combined in a fixed order.
 constexpr int kFinGroups = 16;
+template <typename P>
 __global__ __launch_bounds__(kFinGroups * 64) void finalize_cols_kernel(const float* __restrict__ ws, int64_t nparts,
                                                                         int64_t part_stride, int64_t C,
                                                                         void* __restrict__ out0,
                                                                         void* __restrict__ out1, int out_dtype,
-                                                                        const PeerCols peers) {
+                                                                        const P peers) {
     __shared__ float red[kFinGroups][64];
     const int lane = threadIdx.x & 63;
     const int grp = threadIdx.x >> 6;
@@ -195,6 +196,13 @@ __global__ __launch_bounds__(kFinGroups * 64) void finalize_cols_kernel(const fl
         if (out != nullptr) store_col_total(out, c, total, out_dtype);
         add_peer_cols(peers, k, c, total);
     }
+}
+
+// Calls f with the peers, or with nothing where there are none.
+template <typename F>
+void with_peers(const PeerCols* peers, F&& f) {
+    if (peers != nullptr && peers->n_peers > 0) f(*peers);
+    else f(NoPeerCols{});
 }
 
 // Up to here one launch of few blocks takes less time than one that fills the chip and the finalize behind it (us, one launch / two,
@@ -230,10 +238,12 @@ int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void*
         else launch(std::integral_constant<int, CW_ACT_RELU>{});
     };
     if (vec && want_sum && M <= short_rows<T, MODE>(act)) {
-        with_act([&](auto act_c) {
-            hipLaunchKernelGGL((colsum_short_kernel<T, MODE, decltype(act_c)::value>), dim3((unsigned)((N + kShortLanes * V - 1) / (kShortLanes * V))),
-                               dim3(kShortWaves * 64), 0, s, (int)M, N, (const T*)dY, ld_dy, (const T*)pre, ld_pre, (T*)dPre, ld_dpre, out, out_dtype,
-                               peers != nullptr ? *peers : PeerCols{});
+        with_peers(peers, [&](const auto& p) {
+            with_act([&](auto act_c) {
+                hipLaunchKernelGGL((colsum_short_kernel<T, MODE, decltype(act_c)::value, std::decay_t<decltype(p)>>),
+                                   dim3((unsigned)((N + kShortLanes * V - 1) / (kShortLanes * V))), dim3(kShortWaves * 64), 0, s, (int)M, N, (const T*)dY, ld_dy,
+                                   (const T*)pre, ld_pre, (T*)dPre, ld_dpre, out, out_dtype, p);
+            });
         });
         return check_launch("colsum_short_kernel");
     }
@@ -260,8 +270,10 @@ int colsum_impl(int64_t M, int64_t N, const void* dY, int64_t ld_dy, const void*
 
 int finalize_col_partials(const float* ws, int64_t nparts, int64_t part_stride, int nsets, int64_t C, void* out0,
                           void* out1, int out_dtype, hipStream_t s, const PeerCols* peers) {
-    hipLaunchKernelGGL(finalize_cols_kernel, dim3((unsigned)((C + 63) / 64), (unsigned)nsets), dim3(kFinGroups * 64), 0, s, ws,
-                       nparts, part_stride, C, out0, out1, out_dtype, peers != nullptr ? *peers : PeerCols{});
+    with_peers(peers, [&](const auto& p) {
+        hipLaunchKernelGGL((finalize_cols_kernel<std::decay_t<decltype(p)>>), dim3((unsigned)((C + 63) / 64), (unsigned)nsets), dim3(kFinGroups * 64), 0, s, ws,
+                           nparts, part_stride, C, out0, out1, out_dtype, p);
+    });
     return check_launch("finalize_cols_kernel");
 }
 

@@ -32,7 +32,7 @@ constexpr int kRowsAt4Chunks = 1;
 constexpr int kTileBlocksPerCu = 8;
 
 // The other ranks' pairs of the same rows ([R, 2] fp32 each), added in rank order to this rank's where they are used: an all-reduce
-// of the pairs without a launch of its own (n = 0: nothing to add).
+// of the pairs without a launch of its own.
 struct RowPeers {
     const float* p[CW_MAX_ADDENDS];
     int n;
@@ -40,13 +40,19 @@ struct RowPeers {
 __device__ __forceinline__ void row_pair(const float* __restrict__ own, const RowPeers& peers, int64_t row, float& a, float& b) {
     a = own[2 * row];
     b = own[2 * row + 1];
-    if (peers.n == 0) return;
 #pragma unroll
     for (int k = 0; k < CW_MAX_ADDENDS; ++k)
         if (k < peers.n) {
             a += peers.p[k][2 * row];
             b += peers.p[k][2 * row + 1];
         }
+}
+
+// A call without peers (see NoPeerCols).
+struct NoRowPeers {};
+__device__ __forceinline__ void row_pair(const float* __restrict__ own, const NoRowPeers&, int64_t row, float& a, float& b) {
+    a = own[2 * row];
+    b = own[2 * row + 1];
 }
 
 // Two vectors of parameters gathered from their ranks' parts by the leading `blocks` workgroups of the statistics launch, which does
@@ -67,6 +73,11 @@ __device__ __forceinline__ void gather_params(const GatherParams& g) {
             g.out1[i] = g.p1[n][i - k * g.part];
         }
 }
+
+struct NoGather {
+    static constexpr int blocks = 0;
+};
+__device__ __forceinline__ void gather_params(const NoGather&) {}
 
 // Sum of (x-mu) and (x-mu)^2 over one row; every lane returns the full sums.
 template <typename T>
@@ -102,10 +113,10 @@ __device__ __forceinline__ void row_moments(const T* __restrict__ xr, int64_t C,
     s2 = wave_sum(a2);
 }
 
-template <typename T>
+template <typename T, typename GP>
 __global__ __launch_bounds__(kLnBlock) void ln_stats_kernel(int64_t R, int64_t C, const T* __restrict__ x,
                                                             int64_t ld, int mode, const float* __restrict__ mean,
-                                                            float* __restrict__ stats, int vec_ok, const GatherParams gather) {
+                                                            float* __restrict__ stats, int vec_ok, const GP gather) {
     if ((int)blockIdx.x < gather.blocks) return gather_params(gather);
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)((int)blockIdx.x - gather.blocks) * (kLnBlock / 64) + (threadIdx.x >> 6);
@@ -135,14 +146,14 @@ __device__ __forceinline__ void finish_stats(int mode, float s1, float s2, float
     rstd = __builtin_amdgcn_rsqf(var + eps);  // hardware reciprocal square root, 1 ulp
 }
 
-template <typename T, bool FUSED>
+template <typename T, bool FUSED, typename P>
 __global__ __launch_bounds__(kLnBlock) void ln_normalize_kernel(int64_t R, int64_t C, const T* __restrict__ x,
                                                                 int64_t ld, const float* __restrict__ stats,
                                                                 int mode, float inv_h, float eps,
                                                                 const T* __restrict__ gamma,
                                                                 const T* __restrict__ beta, T* __restrict__ y,
                                                                 int64_t ldy, float* __restrict__ mean_rstd,
-                                                                int vec_ok, const RowPeers peers) {
+                                                                int vec_ok, const P peers) {
     constexpr int V = elem<T>::kVec;
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)blockIdx.x * (kLnBlock / 64) + (threadIdx.x >> 6);
@@ -302,11 +313,11 @@ __device__ __forceinline__ void tile_moments(const RowTile<T, NCH, NR>& t, int r
 // checks. On 16384 x 1024 bf16 that is the difference between 0.58 and 0.71 of the HBM peak for the
 // normalise kernel; wavefronts that loop read measurably slower at these sizes, however the loop is
 // pipelined.
-template <typename T, int NCH, int NR, bool EXACT>
+template <typename T, int NCH, int NR, bool EXACT, typename GP>
 __global__ __launch_bounds__(kTileWaves * 64) void ln_stats_tile_kernel(int64_t R, int64_t C,
                                                                         const T* __restrict__ x, int64_t ld, int mode,
                                                                         const float* __restrict__ mean,
-                                                                        float* __restrict__ stats, const GatherParams gather) {
+                                                                        float* __restrict__ stats, const GP gather) {
     if ((int)blockIdx.x < gather.blocks) return gather_params(gather);
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)((int)blockIdx.x - gather.blocks) * kTileWaves + (threadIdx.x >> 6);
@@ -376,11 +387,11 @@ __global__ __launch_bounds__(kTileWaves * 64) void ln_stats_tile_kernel(int64_t 
     }
 }
 
-template <typename T, int NCH, int NR, bool FUSED, bool EXACT>
+template <typename T, int NCH, int NR, bool FUSED, bool EXACT, typename P>
 __global__ __launch_bounds__(kTileWaves * 64) void ln_normalize_tile_kernel(
     int64_t R, int64_t C, const T* __restrict__ x, int64_t ld, const float* __restrict__ stats, int mode, float inv_h,
     float eps, const T* __restrict__ gamma, const T* __restrict__ beta, T* __restrict__ y, int64_t ldy,
-    float* __restrict__ mean_rstd, const RowPeers peers) {
+    float* __restrict__ mean_rstd, const P peers) {
     constexpr int V = elem<T>::kVec;
     const int lane = threadIdx.x & 63;
     const int64_t wave = (int64_t)blockIdx.x * kTileWaves + (threadIdx.x >> 6);
@@ -459,12 +470,12 @@ __global__ __launch_bounds__(kTileWaves * 64) void ln_normalize_tile_kernel(
 
 // Partial statistics of rows wider than a wavefront's registers, laid out like ln_forward_split_kernel:
 // `wpr` wavefronts share a row and add their moments through LDS (one barrier per row).
-template <typename T, int NCH, int MAXW>
+template <typename T, int NCH, int MAXW, typename GP>
 __global__ __launch_bounds__(MAXW * 64) void ln_stats_split_kernel(int64_t R, int64_t C, const T* __restrict__ x,
                                                                    int64_t ld, int mode,
                                                                    const float* __restrict__ mean,
                                                                    float* __restrict__ stats, int wpr,
-                                                                   const GatherParams gather) {
+                                                                   const GP gather) {
     if ((int)blockIdx.x < gather.blocks) return gather_params(gather);
     constexpr int V = elem<T>::kVec;
     __shared__ float lds_sums[2][MAXW][2];  // [trip parity][wavefront][moment]
@@ -647,11 +658,11 @@ __global__ __launch_bounds__(kFwdShortWaves * 64, NCH <= 6 ? 6 : 4) void ln_forw
     if (live && ok) store_raw_stream(y + row * ldy + c0, pack_raw(v, (const T*)nullptr));
 }
 
-template <typename T, int NCH, int NR, bool EXACT>
+template <typename T, int NCH, int NR, bool EXACT, typename CP, typename P>
 __global__ __launch_bounds__(kTileWaves * 64) void ln_bwd_dx_tile_kernel(
     int64_t R, int64_t C, const T* __restrict__ dY, int64_t ld_dy, const T* __restrict__ x, int64_t ld_x,
     const float* __restrict__ mean_rstd, const T* __restrict__ gamma, const float* __restrict__ row_sums, float inv_h,
-    T* __restrict__ dx, int64_t ld_dx, const FinishCols fin, const RowPeers peers) {
+    T* __restrict__ dx, int64_t ld_dx, const FinishCols<CP> fin, const P peers) {
     constexpr int V = elem<T>::kVec;
     if (fin.blocks > 0 && (int)blockIdx.x < fin.blocks) {  // the leading workgroups finish the column sums
         __shared__ float fin_red[kTileWaves * 64];
@@ -1167,14 +1178,14 @@ __global__ __launch_bounds__(kLnBlock) void ln_bwd_cols_generic_kernel(
     col_ws[(int64_t)blockIdx.y * 2 * C + C + c] = db;
 }
 
-template <typename T>
+template <typename T, typename CP, typename P>
 __global__ __launch_bounds__(kLnBlock) void ln_bwd_dx_kernel(int64_t R, int64_t C, const T* __restrict__ dY,
                                                              int64_t ld_dy, const T* __restrict__ x, int64_t ld_x,
                                                              const float* __restrict__ mean_rstd,
                                                              const T* __restrict__ gamma,
                                                              const float* __restrict__ row_sums, float inv_h,
                                                              T* __restrict__ dx, int64_t ld_dx, int vec_ok,
-                                                             const FinishCols fin, const RowPeers peers) {
+                                                             const FinishCols<CP> fin, const P peers) {
     constexpr int V = elem<T>::kVec;
     if (fin.blocks > 0 && (int)blockIdx.x < fin.blocks) {  // the leading workgroups finish the column sums
         __shared__ float fin_red[kLnBlock];
@@ -1261,13 +1272,12 @@ FwdSplitShape fwd_split_shape(int64_t R, int64_t nch) {
     return sh;
 }
 
-template <typename T>
+template <typename T, typename GP = NoGather>
 int stats_impl(int64_t R, int64_t C, const void* x, int64_t ld, int mode, const float* mean, float* stats,
-               hipStream_t s, const GatherParams* params = nullptr) {
-    GatherParams gather = params != nullptr ? *params : GatherParams{};
+               hipStream_t s, GP gather = GP{}) {
     // leading workgroups of `threads` threads that a launch carries for the gathering
     auto extra = [&](int threads) {
-        if (params != nullptr) gather.blocks = (int)((C * (int64_t)(sizeof(T) / 2) + threads - 1) / threads);
+        if constexpr (!std::is_same<GP, NoGather>::value) gather.blocks = (int)((C * (int64_t)(sizeof(T) / 2) + threads - 1) / threads);
         return (unsigned)gather.blocks;
     };
     const int vec_ok = rows_vec_ok<T>(x, ld);
@@ -1276,7 +1286,7 @@ int stats_impl(int64_t R, int64_t C, const void* x, int64_t ld, int mode, const 
         return dispatch_exact<8>(nch, [&](auto nch_c, auto nr_c) {
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
             const unsigned fb = extra(kTileWaves * 64);
-            hipLaunchKernelGGL((ln_stats_tile_kernel<T, NCH, NR, true>), dim3(exact_grid(R, NR) + fb), dim3(kTileWaves * 64),
+            hipLaunchKernelGGL((ln_stats_tile_kernel<T, NCH, NR, true, GP>), dim3(exact_grid(R, NR) + fb), dim3(kTileWaves * 64),
                                0, s, R, C, (const T*)x, ld, mode, mean, stats, gather);
             return check_launch("ln_stats_tile_kernel");
         });
@@ -1285,7 +1295,7 @@ int stats_impl(int64_t R, int64_t C, const void* x, int64_t ld, int mode, const 
         return dispatch_tile(nch, [&](auto nch_c, auto nr_c) {
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
             const unsigned fb = extra(kTileWaves * 64);
-            hipLaunchKernelGGL((ln_stats_tile_kernel<T, NCH, NR, false>), dim3(tile_grid(R, NR) + fb), dim3(kTileWaves * 64),
+            hipLaunchKernelGGL((ln_stats_tile_kernel<T, NCH, NR, false, GP>), dim3(tile_grid(R, NR) + fb), dim3(kTileWaves * 64),
                                0, s, R, C, (const T*)x, ld, mode, mean, stats, gather);
             return check_launch("ln_stats_tile_kernel");
         });
@@ -1294,23 +1304,23 @@ int stats_impl(int64_t R, int64_t C, const void* x, int64_t ld, int mode, const 
     if (vec_ok && (C % elem<T>::kVec) == 0 && sh.takes) {
         const dim3 grid((unsigned)sh.blocks + extra(sh.wpr * sh.nrg * 64)), block(sh.wpr * sh.nrg * 64);
         if (sh.wide)
-            hipLaunchKernelGGL((ln_stats_split_kernel<T, kFwdSplitChunks, 16>), grid, block, 0, s, R, C, (const T*)x,
+            hipLaunchKernelGGL((ln_stats_split_kernel<T, kFwdSplitChunks, 16, GP>), grid, block, 0, s, R, C, (const T*)x,
                                ld, mode, mean, stats, sh.wpr, gather);
         else
-            hipLaunchKernelGGL((ln_stats_split_kernel<T, kFwdSplitChunks, kFwdSplitBlockWaves>), grid, block, 0, s,
+            hipLaunchKernelGGL((ln_stats_split_kernel<T, kFwdSplitChunks, kFwdSplitBlockWaves, GP>), grid, block, 0, s,
                                R, C, (const T*)x, ld, mode, mean, stats, sh.wpr, gather);
         return check_launch("ln_stats_split_kernel");
     }
     const unsigned fb = extra(kLnBlock);
-    hipLaunchKernelGGL(ln_stats_kernel<T>, dim3(ln_grid(R) + fb), dim3(kLnBlock), 0, s, R, C, (const T*)x, ld, mode,
+    hipLaunchKernelGGL((ln_stats_kernel<T, GP>), dim3(ln_grid(R) + fb), dim3(kLnBlock), 0, s, R, C, (const T*)x, ld, mode,
                        mean, stats, vec_ok, gather);
     return check_launch("ln_stats_kernel");
 }
 
-template <typename T, bool FUSED>
+template <typename T, bool FUSED, typename P = NoRowPeers>
 int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float* stats, int mode, int64_t H,
                    float eps, const void* gamma, const void* beta, void* y, int64_t ldy, float* mean_rstd,
-                   hipStream_t s, const RowPeers& peers = RowPeers{}) {
+                   hipStream_t s, const P& peers = P{}) {
     const int vec_ok = rows_vec_ok<T>(x, ld) && rows_vec_ok<T>(y, ldy) && (gamma == nullptr || aligned16(gamma)) &&
                        (beta == nullptr || aligned16(beta));
     const int64_t nch = row_chunks<T>(C);
@@ -1341,7 +1351,7 @@ int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float*
         return dispatch_exact<8>(nch, [&](auto nch_c, auto nr_c) {
             constexpr int NCH = decltype(nch_c)::value;
             constexpr int NR = NCH == 2 ? 2 : decltype(nr_c)::value;
-            hipLaunchKernelGGL((ln_normalize_tile_kernel<T, NCH, NR, FUSED, true>), dim3(exact_grid(R, NR)),
+            hipLaunchKernelGGL((ln_normalize_tile_kernel<T, NCH, NR, FUSED, true, P>), dim3(exact_grid(R, NR)),
                                dim3(kTileWaves * 64), 0, s, R, C, (const T*)x, ld, stats, mode, 1.0f / (float)H, eps,
                                (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd, peers);
             return check_launch("ln_normalize_tile_kernel");
@@ -1350,7 +1360,7 @@ int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float*
     if (vec_ok && (C % elem<T>::kVec) == 0 && nch <= 8) {
         return dispatch_tile(nch, [&](auto nch_c, auto nr_c) {
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
-            hipLaunchKernelGGL((ln_normalize_tile_kernel<T, NCH, NR, FUSED, false>), dim3(tile_grid(R, NR)),
+            hipLaunchKernelGGL((ln_normalize_tile_kernel<T, NCH, NR, FUSED, false, P>), dim3(tile_grid(R, NR)),
                                dim3(kTileWaves * 64), 0, s, R, C, (const T*)x, ld, stats, mode, 1.0f / (float)H, eps,
                                (const T*)gamma, (const T*)beta, (T*)y, ldy, mean_rstd, peers);
             return check_launch("ln_normalize_tile_kernel");
@@ -1371,7 +1381,7 @@ int normalize_impl(int64_t R, int64_t C, const void* x, int64_t ld, const float*
             return check_launch("ln_forward_split_kernel");
         }
     }
-    hipLaunchKernelGGL((ln_normalize_kernel<T, FUSED>), dim3(ln_grid(R)), dim3(kLnBlock), 0, s, R, C, (const T*)x,
+    hipLaunchKernelGGL((ln_normalize_kernel<T, FUSED, P>), dim3(ln_grid(R)), dim3(kLnBlock), 0, s, R, C, (const T*)x,
                        ld, stats, mode, 1.0f / (float)H, eps, (const T*)gamma, (const T*)beta, (T*)y, ldy,
                        mean_rstd, vec_ok, peers);
     return check_launch("ln_normalize_kernel");
@@ -1613,20 +1623,19 @@ int bwd_partials_impl(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const
     return rc;
 }
 
-template <typename T>
+template <typename T, typename CP = NoPeerCols, typename P = NoRowPeers>
 int bwd_dx_impl(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void* x, int64_t ld_x,
                 const float* mean_rstd, const void* gamma, const float* row_sums, int64_t H, void* dx, int64_t ld_dx,
-                hipStream_t s, const FinishCols* finish = nullptr, const RowPeers& peers = RowPeers{}) {
+                hipStream_t s, const FinishCols<CP>& fin = FinishCols<CP>{}, const P& peers = P{}) {
     const int vec_ok = rows_vec_ok<T>(dY, ld_dy) && rows_vec_ok<T>(x, ld_x) && rows_vec_ok<T>(dx, ld_dx) &&
                        (gamma == nullptr || aligned16(gamma));
-    const FinishCols fin = finish != nullptr ? *finish : FinishCols{};
     const unsigned fb = (unsigned)fin.blocks;
     const int64_t nch = row_chunks<T>(C);
     // rows of more than 4 chunks are faster on the looping kernel (the 8-chunk tile needs 160-240 registers)
     if (vec_ok && exact_chunks<T>(C, nch) && nch <= 4 && R <= (int64_t)1 << 30) {
         return dispatch_exact<2>(nch, [&](auto nch_c, auto nr_c) {
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
-            hipLaunchKernelGGL((ln_bwd_dx_tile_kernel<T, NCH, NR, true>), dim3(exact_grid(R, NR) + fb), dim3(kTileWaves * 64),
+            hipLaunchKernelGGL((ln_bwd_dx_tile_kernel<T, NCH, NR, true, CP, P>), dim3(exact_grid(R, NR) + fb), dim3(kTileWaves * 64),
                                0, s, R, C, (const T*)dY, ld_dy, (const T*)x, ld_x, mean_rstd, (const T*)gamma, row_sums,
                                1.0f / (float)H, (T*)dx, ld_dx, fin, peers);
             return check_launch("ln_bwd_dx_tile_kernel");
@@ -1635,13 +1644,13 @@ int bwd_dx_impl(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const void*
     if (vec_ok && (C % elem<T>::kVec) == 0 && nch <= 4) {
         return dispatch_tile(nch, [&](auto nch_c, auto nr_c) {
             constexpr int NCH = decltype(nch_c)::value, NR = decltype(nr_c)::value;
-            hipLaunchKernelGGL((ln_bwd_dx_tile_kernel<T, NCH, NR, false>), dim3(tile_grid(R, NR) + fb), dim3(kTileWaves * 64),
+            hipLaunchKernelGGL((ln_bwd_dx_tile_kernel<T, NCH, NR, false, CP, P>), dim3(tile_grid(R, NR) + fb), dim3(kTileWaves * 64),
                                0, s, R, C, (const T*)dY, ld_dy, (const T*)x, ld_x, mean_rstd, (const T*)gamma, row_sums,
                                1.0f / (float)H, (T*)dx, ld_dx, fin, peers);
             return check_launch("ln_bwd_dx_tile_kernel");
         });
     }
-    hipLaunchKernelGGL(ln_bwd_dx_kernel<T>, dim3(ln_grid(R) + fb), dim3(kLnBlock), 0, s, R, C, (const T*)dY, ld_dy,
+    hipLaunchKernelGGL((ln_bwd_dx_kernel<T, CP, P>), dim3(ln_grid(R) + fb), dim3(kLnBlock), 0, s, R, C, (const T*)dY, ld_dy,
                        (const T*)x, ld_x, mean_rstd, (const T*)gamma, row_sums, 1.0f / (float)H, (T*)dx, ld_dx,
                        vec_ok, fin, peers);
     return check_launch("ln_bwd_dx_kernel");
@@ -1717,7 +1726,7 @@ extern "C" int cw_ln_partial_stats_gather(int64_t R, int64_t C, const void* x, i
     if (const int drc = require_gfx950("cw_ln_partial_stats_gather"); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
     return with_elem_type(io_dtype, [&](auto* tag) {
-        return stats_impl<std::remove_pointer_t<decltype(tag)>>(R, C, x, ld, CW_LN_ONE_PASS, nullptr, stats, s, &g);
+        return stats_impl<std::remove_pointer_t<decltype(tag)>>(R, C, x, ld, CW_LN_ONE_PASS, nullptr, stats, s, g);
     });
 }
 
@@ -1742,8 +1751,9 @@ extern "C" int cw_ln_normalize_peers(int64_t R, int64_t C, const void* x, int64_
     if (const int drc = require_gfx950("cw_ln_normalize"); drc != CW_OK) return drc;
     hipStream_t s = (hipStream_t)stream;
     return with_elem_type(io_dtype, [&](auto* tag) {
-        return normalize_impl<std::remove_pointer_t<decltype(tag)>, false>(R, C, x, ld, stats, mode, H, eps, gamma, beta,
-                                                                           y, ldy, mean_rstd, s, rp);
+        using T = std::remove_pointer_t<decltype(tag)>;
+        if (rp.n > 0) return normalize_impl<T, false>(R, C, x, ld, stats, mode, H, eps, gamma, beta, y, ldy, mean_rstd, s, rp);
+        return normalize_impl<T, false>(R, C, x, ld, stats, mode, H, eps, gamma, beta, y, ldy, mean_rstd, s);
     });
 }
 
@@ -1923,18 +1933,20 @@ extern "C" int cw_ln_bwd_dx_close_peers(int64_t R, int64_t C, const void* dY, in
     if (dY == nullptr || x == nullptr || mean_rstd == nullptr || row_sums == nullptr || dx == nullptr || ld_dy < C ||
         ld_x < C || ld_dx < C)
         return fail(CW_ERR_INVALID, "cw_ln_bwd_dx_close: null pointer or leading dimension < C");
-    FinishCols fin;
-    fin.ws = (const float*)workspace;
-    fin.nparts = n_parts;
-    fin.part_stride = 2 * C;
-    fin.C = C;
-    fin.out0 = dgamma;
-    fin.out1 = dbeta;
-    fin.out_dtype = param_dtype;
-    fin.blocks = n_parts > 0 ? 2 * (int)((C + 63) / 64) : 0;
-    fin.peers = pc;
-    return with_elem_type(io_dtype, [&](auto* tag) {
-        return bwd_dx_impl<std::remove_pointer_t<decltype(tag)>>(R, C, dY, ld_dy, x, ld_x, mean_rstd, gamma, row_sums, H, dx,
-                                                                 ld_dx, s, &fin, rp);
-    });
+    auto run = [&](const auto& cols, const auto& rows) {
+        FinishCols<std::decay_t<decltype(cols)>> fin;
+        fin.ws = (const float*)workspace;
+        fin.nparts = n_parts;
+        fin.part_stride = 2 * C;
+        fin.C = C;
+        fin.out0 = dgamma;
+        fin.out1 = dbeta;
+        fin.out_dtype = param_dtype;
+        fin.blocks = n_parts > 0 ? 2 * (int)((C + 63) / 64) : 0;
+        fin.peers = cols;
+        return with_elem_type(io_dtype, [&](auto* tag) {
+            return bwd_dx_impl<std::remove_pointer_t<decltype(tag)>>(R, C, dY, ld_dy, x, ld_x, mean_rstd, gamma, row_sums, H, dx, ld_dx, s, fin, rows);
+        });
+    };
+    return pc.n_peers > 0 || rp.n > 0 ? run(pc, rp) : run(NoPeerCols{}, NoRowPeers{});
 }
