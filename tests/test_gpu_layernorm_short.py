@@ -106,3 +106,16 @@ def test_a_row_has_the_same_bits_in_any_batch(C, dtype, mode):
     for R in (1, 2, 7, 128, edge, edge + 1):
         for got, whole in zip(ops.ln_forward_fused(x[:R], 1e-5, g, b, mode), want):
             assert torch.equal(got, whole[:R])
+
+
+@pytest.mark.parametrize("R,C", [(128, 1024), (700, 1024), (1536, 2048), (1537, 2048), (300, 4096)])
+def test_residual_gradient_of_an_fp32_stream(R, C):
+    """Added in the kernel in place of a launch behind it: the same sum but for one rounding, where the multiplication before it and the
+    addition are fused (on each kernel that takes it)."""
+    from cubework_amd import ops
+    x, dy, add, g = (randn(s, torch.float32, k, device=DEV) for k, s in enumerate(((R, C), (R, C), (R, C), (C,))))
+    _, mean_rstd = ops.ln_forward_fused(x, 1e-5, g, g)
+    plain, got = (ops.ln_backward_fused(dy, x, mean_rstd, g, dx_addend=a) for a in (None, add))
+    want = plain[0] + add
+    assert ((got[0].double() - want.double()).abs() <= 2.0 ** -24 * (plain[0].double().abs() + 2 * want.double().abs())).all()
+    assert torch.equal(got[1], plain[1]) and torch.equal(got[2], plain[2])
