@@ -289,10 +289,13 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         q.rotate = cfg == 0 ? !ordered || rotated : cfg >= kPairedConfig && !ordered;
         q.partial_bytes = rest * slices * (int64_t)(4096 * c.tm * c.tn) * 4;
         if (max_scratch >= 0 && q.scratch() > max_scratch) return;
-        // TN on the kernels of gemm_tile.h: k-contiguous operands move as pieces of 64 bytes, k-slow ones as whole lines. On the
-        // paired one: the two groups' transposing reads take more LDS cycles than their products.
-        // 64 x 128 tiles of an NT product, at most one a unit: both operands move as whole lines, where the costs were fitted to pieces of 64 bytes
-        // (us, M x N x K, as chosen before / such tiles: 1554 x 768 x 2304 20.3 / 16.0, 489 x 2560 x 2560 22.5 / 17.4, 2561 x 768 x 3072 25.8 / 21.5).
+        // TN on the kernels of gemm_tile.h: both operands are k-slow and move as whole lines, where the costs were fitted to k-contiguous ones
+        // in pieces of 64 bytes (as 128-column tiles still move them; trips of 64 k move lines). On the paired one: the two groups' transposing
+        // reads take more LDS cycles than their products.
+        // 64 x 128 tiles of an NT product, at most one a unit: k-contiguous operands as lines against the same fit
+        // (us, M x N x K, as chosen before / such tiles: 1554 x 768 x 2304 20.3 / 16.0, 489 x 2560 x 2560 22.5 / 17.4, 2561 x 768 x 3072 25.8 / 21.5). Two a
+        // unit, 257 to 512 tiles, are left as fitted: with the factor 150 such products ran 3.6 % faster on average (2091 x 1000 x 1024 15.4 / 13.3),
+        // but up to 12 % slower where rows are not whole lines (1124 x 3072 x 1144 18.1 / 20.5, 558 x 4096 x 1176 19.0 / 21.3).
         const double lines_factor = cfg == 3 && layout == CW_NT && full == tiles && tiles <= 256 ? 0.86 : 1.0;
         const double layout_factor = lines_factor * (cfg == 0 || layout != CW_TN ? 1.0 : cfg == kPairedConfig ? 1.15 : cfg == 2 ? 1.0 : 0.9);
         // Rows that are not whole 128-byte lines cost the paired kernel's loads more the longer a block walks along them (us, M x N x K):
@@ -315,7 +318,7 @@ TilePlan tile_plan(int layout, int64_t M, int64_t N, int64_t K, int n_steps, int
         // All tiles of an output of more than 128 rows and columns sliced: behind the eighth slice the reduction, which requests four together,
         // waits a tenth of that, and up to 32 slices are tried (us, M x N x K, NN, up to 16 / as chosen now): 1023 x 768 x 50257 121 / 90
         // (TN 102 / 86, NT 143 / 103), 1280 x 408 x 50304 94 / 75, 178 x 1536 x 51072 66 / 48, 391 x 2048 x 32000 81 / 66. Of 330 products of
-        // a long k and of the 2415 shapes of the layers this and the slower walks below make 33 more than 3 % faster and none slower. Fewer
+        // a long k and of the 2415 shapes of the layers this and the slower walks below make some thirty more than 3 % faster and none slower. Fewer
         // rows or columns are left to the small tiles: 34 x 3072 x 56535 TN 72 / 87.
         const bool deep = full == 0 && M > 128 && N > 128;
         const double waits = deep && slices > 8 ? 7.2 + 0.1 * (slices - 8) : 0.9 * slices;
