@@ -63,9 +63,10 @@ __device__ __forceinline__ float wave_abs_max(float v) {
 // KIND 0: max |g|;  KIND 2: sum g^2;  KIND 1: sum |g|^p (general p)
 // Bound by memory. Ordinary loads, not streaming ones: the scaling launch reads the same bytes next, and part of them is
 // still in the last-level cache then (norm and scaling of 201 MB of fp32 gradients: 105 -> 99 us, of 1.26 GB: 618 -> 611).
-// A block's chunk in batches of NB loads by NT threads. Of up to kDeepBytes there are two blocks a unit or fewer, whose 4 loads by 256
-// threads do not cover the memory's latency: 8 by 512 (norm and scaling, fp32 28 MB 23.7 -> 18.4 us, 113 MB 60.6 -> 57.0, bf16 57 MB 35.0 ->
-// 30.7, 101 MB 52.8 -> 50.5). More of them fill it (fp32 202 MB 96.7 us, with 8 by 512 97.8; 806 MB 391 and 389).
+// A block's chunk of kChunk elements in batches of NB loads by NT threads. Up to kDeepBytes a launch has two blocks a unit or fewer in fp32, four
+// in 16 bits, whose 4 loads by 256 threads do not cover the memory's latency: 8 by 512 (norm and scaling, us, fp32 40 MB 37.9 -> 29.1, 72 MB
+// 45.7 -> 42.4, 120 MB 62.9 -> 62.2; bf16 40 MB 30.4 -> 28.5, 56 MB 38.7 -> 37.5, 72 to 126 MB within 1.5 % either way, in 40 tensors 1 to
+// 4 % faster). More of them fill it (fp32 202 MB 96.7 us, with 8 by 512 97.8; 806 MB 391 and 389).
 constexpr int64_t kDeepBytes = (int64_t)128 << 20;
 template <typename T, int KIND, int NT, int NB>
 __global__ __launch_bounds__(NT) void multi_norm_kernel(const TensorBatch b, float p, float* __restrict__ ws,
