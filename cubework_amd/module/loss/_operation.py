@@ -74,6 +74,10 @@ def vocab_parallel_cross_entropy_mean(logits, targets, parallel_mode):
     if targets.numel() == 0:  # a mean of nothing: NaN, as torch gives it
         return _VocabParallelCrossEntropy.apply(logits, targets, parallel_mode).mean()
     vocab_start = parallel_mode.local_rank * logits.size(-1)
-    peers = () if parallel_mode.world_size == 1 else parallel_mode.take("vpce_stats")
+    peers = ()
+    if parallel_mode.world_size > 1:
+        peers = parallel_mode.take("vpce_stats")
+        if len(peers) != 4:  # none at all would be a slice without peers to the operator
+            raise ValueError("the peers' max, sumexp, pred and mask are needed")
     loss = ops.mean_loss(logits, targets, vocab_start, peers)
     return _VocabParallelCrossEntropyMean.apply(logits, targets, vocab_start, peers) if loss is None else loss

@@ -68,6 +68,21 @@ def test_no_tokens_and_wrong_targets():
         loss_fn(torch.zeros((3, 8), device=DEV), torch.zeros((2,), dtype=torch.int64, device=DEV))
 
 
+def test_a_slice_whose_peers_are_missing_is_refused():
+    """Statistics staged as nothing are no statistics: not the loss of one slice alone."""
+    from cubework_amd.distributed import ParallelManager as pm
+    from cubework_amd.distributed import initialize
+    from cubework_amd.module.loss import VocabParallelCrossEntropyLoss1D
+
+    initialize("1d", 2, rank=1)
+    x, t = torch.zeros((3, 8), device=DEV), torch.zeros((3,), dtype=torch.int64, device=DEV)
+    for staged in ([], _peers(3, 1, 1)[:3]):
+        pm.PARALLEL_1D.stage("vpce_stats", staged)
+        with pytest.raises(ValueError):
+            VocabParallelCrossEntropyLoss1D()(x, t)
+    initialize("1d", 1)
+
+
 def test_replays_from_a_graph():
     """The arrival count starts at zero on every replay."""
     from cubework_amd import ops
