@@ -111,8 +111,6 @@ class _GatherForwardSplitBackward(torch.autograd.Function):
 
 
 def reduce_grad(input_, parallel_mode):
-    if parallel_mode.world_size == 1:
-        return input_
     return _ReduceGrad.apply(input_, parallel_mode)
 
 

@@ -26,6 +26,11 @@ from ._operation import (gather_forward_split_backward, get_parallel_input, line
                          set_parallel_input, split_forward_gather_backward)
 
 
+def _reduced_grad(input_: Tensor) -> Tensor:
+    """reduce_grad of an input that only the layer reads: without peers there is nothing to reduce and no need of a node."""
+    return input_ if pm.PARALLEL_1D.world_size == 1 else reduce_grad(input_, pm.PARALLEL_1D)
+
+
 class Linear1D_Col(nn.Module):
 
     def __init__(self, in_features: int, out_features: int, bias: bool = True, gather_output: bool = False,
@@ -55,7 +60,7 @@ class Linear1D_Col(nn.Module):
         set_parallel_input(True)
 
     def forward(self, input_: Tensor):
-        input_parallel = reduce_grad(input_, pm.PARALLEL_1D)
+        input_parallel = _reduced_grad(input_)
         bias = self.bias if not self.skip_bias_add else None
         output = linear_nt(input_parallel, self.weight, bias, self.activation)
         if self.gather_output:
@@ -225,4 +230,4 @@ class VocabParallelClassifier1D(nn.Module):
         env.vocab_parallel = True
 
     def forward(self, input_: Tensor) -> Tensor:
-        return linear_nt(reduce_grad(input_, pm.PARALLEL_1D), self.weight, self.bias)
+        return linear_nt(_reduced_grad(input_), self.weight, self.bias)

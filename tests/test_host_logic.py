@@ -208,3 +208,17 @@ def test_attention_head_padding_is_exact_on_the_host():
     # zeros add nothing to q.k (compared in float64: the order of a float32 sum may differ with the length)
     assert torch.equal(torch.einsum("bshd,bthd->bhst", q.double(), k.double()),
                        torch.einsum("bshd,bthd->bhst", qp.double(), kp.double()))
+
+
+def test_reduce_grad_hands_out_a_result_of_its_own():
+    """Without peers too: what is done to it in place is refused and does not reach the input."""
+    from cubework_amd.module.parallel_1d._operation import reduce_grad
+
+    initialize("1d", 1)
+    x = torch.ones(3, 4, requires_grad=True)
+    h = x * 2
+    y = reduce_grad(h, pm.PARALLEL_1D)
+    with pytest.raises(RuntimeError):
+        y.add_(1)
+    (y * 3).sum().backward()
+    assert torch.equal(h, torch.full((3, 4), 2.0)) and torch.equal(x.grad, torch.full((3, 4), 6.0))
