@@ -3,12 +3,13 @@
 // backward beside its launches, a native one 3 to 5.
 //
 // A call that is not the ordinary one returns None, and the caller takes its Python node, which behaves as it always did: tensors that
-// are no plain tensors, tracing, functional transforms, dispatch modes, operands on other devices or of other shapes than the
+// are no plain tensors, tracing, functional transforms, forward-mode levels, dispatch modes, operands on other devices or of other shapes than the
 // operator's own (the Python node raises for those).
 #include "host_ops.h"
 
 #include <ATen/autocast_mode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -21,7 +22,8 @@ using torch::autograd::variable_list;
 
 bool ordinary() {
     return !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
-           !c10::impl::TorchDispatchModeTLS::any_modes_set() && !torch::jit::tracer::isTracing();
+           !c10::impl::TorchDispatchModeTLS::any_modes_set() && !torch::jit::tracer::isTracing() &&
+           torch::autograd::ForwardADLevel::try_get_by_idx(0) == nullptr;
 }
 // A plain CUDA tensor (or parameter), or None where that is allowed (an undefined tensor).
 bool take(py::handle h, Tensor& t, bool optional = false) {

@@ -157,6 +157,7 @@ def test_calls_that_stay_with_the_python_nodes():
     from torch.utils._python_dispatch import TorchDispatchMode
 
     from cubework_amd import _lib, ops
+    from cubework_amd.module.parallel_1d._operation import linear_nt
 
     class Watch(TorchDispatchMode):
         def __torch_dispatch__(self, func, types, args=(), kwargs=None):
@@ -179,6 +180,11 @@ def test_calls_that_stay_with_the_python_nodes():
     assert seen == [None, None]
     with pytest.raises(KeyError):
         ops.linear("NN", x, w, None, "swish")
+    with torch.autograd.forward_ad.dual_level():
+        assert ops.linear("NN", x, w) is None
+        dual = torch.autograd.forward_ad.make_dual(x, x)
+        with pytest.raises(NotImplementedError):
+            linear_nt(dual, w)
 
 
 def test_saved_tensor_hooks_and_checkpoint():
