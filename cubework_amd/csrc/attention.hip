@@ -267,8 +267,8 @@ namespace {
 
 // Wavefronts of a block. Few of them where their blocks all fit the chip at once: a block's wavefronts wait for each other at every tile, and
 // under the causal mask for the longest of them. us, bf16, 8 / 4 / 2 wavefronts (batch x tokens x heads x columns), causal: 1 x 300 x 32 x 128
-// 15.1 / 12.8 / 12.5, 1 x 1024 x 16 x 64 23.9 / 18.6 / 17.8, 2 x 777 x 32 x 64 20.7 / 16.9 / 16.9, 2 x 777 x 32 x 80 26.0 / 25.0 / 27.0. With more
-// blocks than units they read K and V more often: 4 x 2048 x 32 x 64 91.6 / 89.0 / 108, 4 x 2048 x 16 x 64 56 / 50 / 59, x 128 columns 88 / 98 / 126.
+// 15.2 / 13.1 / 12.9, 1 x 1024 x 16 x 64 24.2 / 18.6 / 18.6, 2 x 777 x 32 x 64 21.4 / 17.6 / 18.1, x 80 columns 24.8 / 25.7 / 28.0. With more
+// blocks than units they read K and V more often: 4 x 2048 x 32 x 64 87.6 / 87.9 / 105, 4 x 2048 x 16 x 64 53 / 50 / 56, x 128 columns 82 / 98 / 129.
 // Without the mask all of a block's wavefronts walk alike: blocks of 4 that do not fit cost a second round (1 x 1456 x 32 x 128 47.1 / 58.3,
 // causal 45.1 / 44.5; 1 x 1040 x 32 x 80 31.4 / 37.8, of 16 heads of 1314 34.5 / 33.8).
 // Heads of up to 64 columns leave room for four blocks of 4 a unit; those of more heads than units and many tokens each read their K and V from
