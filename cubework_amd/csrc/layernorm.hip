@@ -1503,14 +1503,17 @@ int bwd_split_launch(const SplitShape& sh, int64_t R, int64_t C, const void* dY,
 #undef CW_SPLIT
 }
 
-// Where the two passes over the rows cost more than the second launch: us with a residual gradient, operands from the Infinity Cache and
-// memory, before / here: up to four chunks a row (bf16, rows x 2048) 128 11.1 / 5.4, 512 11.9 / 8.3, 777 12.6 / 11.2, 1024 13.1 / 13.2;
-// (x 768) 512 10.3 / 7.5, 777 10.5 / 9.5, fp32 9.2 / 9.8; more of them (bf16, x 2560) 512 12.7 / 8.8, 1024 19.3 / 14.0, 1554 23.5 / 21.1,
-// 2048 25.3 / 27.3, (x 4096) 1024 23.9 / 15.7, 2048 31.5 / 28.3; fp32 (x 2048) 1024 17.1 / 14.4, 1554 21.7 / 21.2. Blocks of 4 wavefronts, 4
+// Up to here the second pass over the rows costs less than the second launch (us, operands from memory, before / here, without a residual gradient and
+// with one): bf16, rows x 768 512 8.5 / 7.6 and 10.5 / 7.6, 640 8.8 / 8.9 and 10.5 / 8.9; x 2560 1280 17.8 / 17.4 and 21.6 / 17.7, 1536 18.0 / 20.1
+// and 22.0 / 20.1, 1792 19.5 / 22.8 and 23.6 / 23.2; x 3072 1536 19.7 / 19.2, 1792 20.9 / 22.3 and 24.6 / 23.0; x 4096 1792 23.6 / 22.4 and 27.7 /
+// 23.3; fp32 x 768 576 8.3 / 8.5 and 8.9 / 8.5; x 1280 1024 12.8 / 12.4 and 13.4 / 12.6, 1280 13.5 / 15.7 and 15.5 / 15.8; x 2048 1280 16.4 / 16.1
+// and 18.6 / 16.8, 1408 16.6 / 17.7 and 18.7 / 18.3. From cache it gains at all of these (1536 x 2560 bf16 17.8 / 10.9). Blocks of 4 wavefronts, 4
 // or 16 vectors of columns, 8 rows in flight: slower.
 template <typename T>
-int64_t short_bwd_rows(int64_t nch) {
-    return nch <= kSplitMinChunks ? 640 : sizeof(T) == 2 ? 1792 : 1536;
+int64_t short_bwd_rows(int64_t nch, bool added) {
+    if (nch <= kSplitMinChunks) return added ? 640 : 512;
+    if (sizeof(T) == 4) return nch == 8 ? 1280 : 1024;
+    return added || nch == 8 ? 1792 : nch == 5 ? 1280 : 1536;
 }
 
 template <typename T>
@@ -1523,7 +1526,7 @@ bool bwd_short_takes(int64_t R, int64_t C, const void* dY, int64_t ld_dy, const 
     };
     // the scratch that the entry point asks for, though this launch needs none: with less the others decide
     return dgamma != nullptr && workspace_bytes >= ln_bwd_workspace_bytes(R, C) && C % elem<T>::kVec == 0 && row_chunks<T>(C) <= 8 &&
-           R <= short_bwd_rows<T>(row_chunks<T>(C)) && rows_vec_ok<T>(dY, ld_dy) && rows_vec_ok<T>(x, ld_x) &&
+           R <= short_bwd_rows<T>(row_chunks<T>(C), add.p != nullptr) && rows_vec_ok<T>(dY, ld_dy) && rows_vec_ok<T>(x, ld_x) &&
            (dx == nullptr || rows_vec_ok<T>(dx, ld_dx)) && (gamma == nullptr || aligned16(gamma)) && apart(dY, ld_dy) && apart(x, ld_x) &&
            (add.p == nullptr || rows_vec_ok<T>(add.p, add.ld));
 }

@@ -29,7 +29,8 @@ def _close(got, want, rel, scale=None):
     assert ((got.double() - want).abs() <= rel * scale).all()
 
 
-SHAPES = [(1, 8), (2, 520), (7, 768), (8, 1032), (9, 1536), (63, 2056), (64, 4096), (65, 1024), (257, 2048), (512, 4096), (513, 4096), (640, 768),
+SHAPES = [(512, 768), (513, 768), (1024, 1280), (1025, 1280), (1280, 2048), (1281, 2048), (1280, 2560), (1281, 2560), (1536, 3072), (1537, 3072),
+          (1792, 4096), (1793, 4096), (1, 8), (2, 520), (7, 768), (8, 1032), (9, 1536), (63, 2056), (64, 4096), (65, 1024), (257, 2048), (512, 4096), (513, 4096), (640, 768),
           (641, 768), (819, 2560), (820, 2560), (1024, 2048), (1025, 2048), (1365, 776), (1366, 776), (1536, 2048), (1537, 2048), (1792, 2560),
           (1793, 2560)]
 
@@ -59,7 +60,11 @@ def test_few_rows_forward_and_backward(R, C, dtype, pitched):
     _close(got_db, db, 2.0 ** -20, dy.double().abs().sum(0))
     plain = ops.ln_backward_fused(dy, x, mean_rstd, g, param_dtype=dtype)
     _close(plain[0], dx - add.double(), REL[dtype] * 2)
-    assert plain[1].dtype == dtype and torch.equal(plain[2], got_db.to(dtype))
+    # without the residual gradient another kernel may take the rows: the sums' own bounds, and half a unit of their type
+    unit = 0 if dtype == torch.float32 else torch.finfo(dtype).eps / 2
+    assert plain[1].dtype == dtype
+    _close(plain[1], dg, 1.0, 2.0 ** -19 * bound + unit * 1.001 * dg.abs())
+    _close(plain[2], db, 1.0, 2.0 ** -20 * dy.double().abs().sum(0) + unit * 1.001 * db.abs())
 
 
 def _backward(dy, x, mean_rstd, g, dx, ws_bytes):
