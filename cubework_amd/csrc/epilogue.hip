@@ -209,13 +209,13 @@ void with_peers(const PeerCols* peers, F&& f) {
 // in a graph, bf16): sums of 128 x 2304 3.3 / 5.3, 256 x 4096 4.0 / 6.2, 512 x 768 4.7 / 5.8, 512 x 12288 6.1 / 8.1, from 777 rows on
 // the two are the faster ones at small widths (777 x 768 6.3 / 6.0); with an activation's derivative, which reads and writes three
 // times as much, 128 x 768 3.7 / 5.7, 256 x 768 6.8 / 6.8, 256 x 12288 8.7 / 9.7, 512 x 2304 12.3 / 7.5.
-// The derivatives of the 16-bit GELUs are more work than few blocks of all rows hide: erf at 160 x 768 8.2 / 8.8, 192 x 768 10.5 / 8.8, 256 x 256
-// 10.9 / 8.9; tanh at 224 x 768 6.4 / 6.9, 256 x 400 7.2 / 6.8. ReLU at 256 x 400 5.2 / 6.4, fp32 4.5 / 6.0 (tanh).
+// A 16-bit derivative is more work than few blocks of all rows hide, from memory later than from cache: erf at 160 x 768 8.2 / 8.8, 192 x 768 10.5 / 8.8 from
+// cache, tanh at 224 x 768 6.4 / 6.9 and, from memory, 7.8 / 7.4, ReLU at 256 x 3072 7.4 / 7.3. fp32 at 256 x 400 4.5 / 6.0 (tanh).
 template <typename T, int MODE>
 int64_t short_rows(int act) {
     if (MODE == 0) return 512;
     if (sizeof(T) == 4) return 256;
-    return act == CW_ACT_GELU_ERF ? 160 : act == CW_ACT_GELU_TANH ? 224 : 256;
+    return act == CW_ACT_GELU_ERF || act == CW_ACT_GELU_TANH ? 160 : 224;
 }
 
 template <typename T, int MODE>

@@ -132,7 +132,7 @@ def test_gemm_part_diagnostic_takes_k_of_128(steps):
 @pytest.mark.parametrize("N", [8, 120, 136, 1000])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_column_sums_of_few_rows(M, N, dtype):
-    """One launch up to 512 rows (256 with an activation, 160 or 224 of the GELUs in 16 bits), NaN outside the operands' columns; fp32 sums of M values in any order lie
+    """One launch up to 512 rows (256 with an activation in fp32, 224 in 16 bits, 160 of a GELU), NaN outside the operands' columns; fp32 sums of M values in any order lie
     within M 2^-24 of the sum of magnitudes. dPre does not depend on the kernel."""
     from cubework_amd import ops
 
