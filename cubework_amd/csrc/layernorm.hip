@@ -612,10 +612,9 @@ __global__ __launch_bounds__(MAXW * 64) void ln_forward_split_kernel(
 // the line below fits at once (6 chunks, 682 x 3072: 5.3 -> 4.3 us); 7 and 8 chunks would spill (512 x 4096: 4.4 -> 6.8).
 constexpr int kFwdShortWaves = 8;
 template <typename T, int NCH>
-__global__ __launch_bounds__(kFwdShortWaves * 64, NCH <= 6 ? 6 : 4) void ln_forward_short_kernel(int64_t R, int64_t C, const T* __restrict__ x, int64_t ld, int mode,
-                                                                              float inv_h, float eps, const T* __restrict__ gamma,
-                                                                              const T* __restrict__ beta, T* __restrict__ y, int64_t ldy,
-                                                                              float* __restrict__ mean_rstd) {
+__global__ __launch_bounds__(kFwdShortWaves * 64, NCH <= 6 ? 6 : 4) void ln_forward_short_kernel(
+    int64_t R, int64_t C, const T* __restrict__ x, int64_t ld, int mode, float inv_h, float eps, const T* __restrict__ gamma,
+    const T* __restrict__ beta, T* __restrict__ y, int64_t ldy, float* __restrict__ mean_rstd) {
     constexpr int V = elem<T>::kVec;
     __shared__ raw16_t chunks[kFwdShortWaves][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, first = wave / NCH * NCH;  // wavefront of the row's first chunk
